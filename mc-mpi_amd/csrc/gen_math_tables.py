@@ -29,6 +29,8 @@ from fractions import Fraction
 import math
 import struct
 
+import numpy as np
+
 decimal.getcontext().prec = 80
 
 LOG_BITS = 9
@@ -177,6 +179,37 @@ def exp_table(n):
     return rows
 
 
+def absorb_table(n):
+    """Per k the y = (k 2^36 + j) 2^-43 of smallest |j| <= 2^20 whose exp(-y) is
+    within 2^-71 of a double.  With E = exp(-k/128), d = 2^-43, the fraction of
+    exp(-y) 2^53 is that of E 2^53 (1 - jd + (jd)^2/2 - ...), followed modulo 1
+    in 64-bit fixed point (the cubic term is below 2^-18); the few candidates
+    are then checked exactly."""
+    rows = [(0.0, 1.0)]
+    for k in range(1, n):
+        E = (Decimal(-k) / Decimal(128)).exp()
+        fx = lambda v: int(v.to_integral_value()) % (1 << 64)  # noqa: E731
+        V = E * Decimal(2) ** 53
+        v0 = fx(V * Decimal(2) ** 64)
+        v1 = fx(V * Decimal(2) ** (64 - 43))
+        v2 = fx(V * Decimal(2) ** (64 - 87))
+        j = np.arange(-(1 << 20), (1 << 20) + 1, dtype=np.int64)
+        u = j.astype(np.uint64)
+        with np.errstate(over="ignore"):
+            f = np.uint64(v0) - u * np.uint64(v1) + u * u * np.uint64(v2)
+        near = np.abs(f.view(np.int64)) < np.int64(1 << 47)
+        for c in sorted(j[near].tolist(), key=lambda t: (abs(t), t)):
+            y = Decimal(k) / Decimal(128) + Decimal(c) * Decimal(2) ** -43
+            v = (-y).exp()
+            if abs(v - Decimal(float(v))) < Decimal(2) ** -71:
+                rows.append((float(y), float(v)))
+                break
+        else:
+            raise AssertionError(k)
+        assert Decimal(rows[-1][0]) == y
+    return rows
+
+
 def split_nbits(value, nbits):
     """hi = value rounded to nbits significant bits (as double), then dd tail."""
     q = Fraction(value)  # Decimal -> exact Fraction
@@ -222,6 +255,17 @@ def main():
     w("MC_TAB double mc_exp_tab10[1024][2] = {")
     for j, (hi, lo) in enumerate(exp_table(1024)):
         w(f"  {{{hexf(hi)}, {hexf(lo)}}}, /* {j} */")
+    w("};")
+    w("")
+    # exp(-y_k), y_k near k/128, for the absorbed fraction 1 - exp(-y)
+    w("/* absorbed fraction: y up to this takes mc_absorb_row ... */")
+    w(f"#define MC_ABS_YMAX {hexf(0.6875)}")
+    w("/* ... with {y_k, exp(-y_k)}, k = 0 .. 88: y_k within 2^-23 of k/128, a multiple")
+    w("   of 2^-43, chosen so that the exponential is within 2^-71 of its double */")
+    w("#define MC_ABS_N 89")
+    w("MC_TAB double mc_abs_tab[MC_ABS_N][2] = {")
+    for k, (y, v) in enumerate(absorb_table(89)):
+        w(f"  {{{hexf(y)}, {hexf(v)}}}, /* {k} */")
     w("};")
     w("")
     # ln2 in three pieces; the first has 42 bits so e*LN2_HI is exact |e|<2^11

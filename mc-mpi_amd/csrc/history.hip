@@ -6,61 +6,52 @@
  * Layer::particle_step (src/layer.cpp:123-190).  Unlike the reference CUDA
  * kernel (src/culayer_kernel.cu:19-113: one launch per 325 steps, host
  * round trips and re-sorting between launches), the grid is persistent:
- * a lane whose history ends takes the next particle index from a global
- * work queue (one atomic per wave per refill), so lanes stay busy until the
- * queue is empty and there is one launch per call.
+ * lanes whose histories end take new ones from the wave's run of the work
+ * queue (mc_queue), so lanes stay busy until the queue is empty and there is
+ * one launch per call.
+ *
+ * The event itself is mc_walk_many (mc_walk.h): a short common step with the
+ * general event apart.
  *
  * Tallies: each block accumulates the exact fixed-point tally of its cells
- * in LDS (two 64-bit words per cell, 64-bit LDS atomics with carry) and adds
- * it to the global 128-bit tally once at the end.  Integer sums are exact, so
- * the result is independent of which lane, wave or block handled which
- * history.  For layers too large for LDS the same atomics go to the global
- * (L2-resident) tally.  The per-cell cross-section pairs are staged in LDS
- * when they fit next to the tally, otherwise read through L2.
+ * in LDS (two 64-bit limbs per cell that never carry into each other,
+ * mc_fx_split; for weights too large for them, two words with carry) and adds
+ * it to the global 128-bit tally at the end, and before limbs could overflow.
+ * Integer sums are exact, so the result is independent of which lane, wave or
+ * block handled which history.  For layers too large for LDS the adds go to
+ * the global (L2-resident) tally.  The per-cell cross-section pairs are staged
+ * in LDS when they fit next to the tally, otherwise read through L2.
+ *
+ * Measured against the kernel with mc_event and a tally with carry: a lone
+ * history 450 -> 284 ns per event (10,000 cells); 1,000 histories on the
+ * 100-cell slab, whole call 264 -> 181 us; 1,000 on 10,000 cells 26.0 -> 9.8
+ * ms (dealt over the CUs); 8e6 on 10,000 cells 267 -> 237 ms, there bound by
+ * the cells' L2 reads (37 lines per wave and event).
  */
 #include "internal.h"
+#include "mc_walk.h"
 
 namespace {
 
-template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE>
-__global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refill_k) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const mc_coef K = mc_coef_live();
-  const int m = a.L.m;
-  unsigned long long *t_lo, *t_hi;
-  size_t off = 0;
-  if (LDS_TALLY) {
-    t_lo = reinterpret_cast<unsigned long long *>(smem);
-    t_hi = t_lo + m;
-    off = (size_t)16 * m;
-    for (int c = threadIdx.x; c < m; c += blockDim.x) {
-      t_lo[c] = 0;
-      t_hi[c] = 0;
-    }
-  } else {
-    t_lo = a.fx;
-    t_hi = a.fx + m;
-  }
-  const mc_cell *cells = a.cells;
-  const double *g = a.g;
-  if (LDS_CELLS) {
-    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + off);
-    for (int c = threadIdx.x; c < m; c += blockDim.x) lc[c] = a.cells[c];
-    cells = lc;
-    if (SCORE) {
-      double *lg = reinterpret_cast<double *>(smem + off + sizeof(mc_cell) * (size_t)m);
-      for (int c = threadIdx.x; c < m; c += blockDim.x) lg[c] = a.g[c];
-      g = lg;
-    }
-  }
-  __syncthreads();
+constexpr size_t TAB_BYTES = 16 * MC_ABS_N; /* the absorbed-fraction rows in LDS */
 
-  const int lane = __lane_id();
-  mc_state p;
-  p.index = 0;
+/* A wave's histories, one per lane.  tally(lanes, c, dw) adds deposits;
+   moves(k) is called before every (at most) k events per lane, k <= k_max. */
+template <bool SCORE, typename Tally, typename Moves>
+__device__ __forceinline__ void walk_bank(const mc_transport_args &a, const mc_cell *cells,
+                                          const double *g, const double2 *tab, int refill_k,
+                                          mc_queue q, const mc_walk_k &K,
+                                          unsigned long long *s_tot, int k_max, Tally tally,
+                                          Moves moves) {
+  mc_walk p;
+  p.s2 = 0;
+  p.x = p.mu = p.wmc = p.rh = p.rl = p.fe = p.fs = 0.0;
+  p.c = p.st = 0;
   int64_t idx = 0;
-  bool has = false, done = false, capped = false;
-  uint64_t ev = 0, col = 0;
+  bool has = false, capped = false;
+  mc_mask run = 0, pend = 0; /* lanes whose history goes on / waits for the general event */
+  uint64_t ev = 0;
+  uint32_t col = 0;
   double score = 0.0;
   unsigned long long tot_ev = 0, tot_col = 0, nl = 0, nr = 0, nk = 0;
 
@@ -70,114 +61,173 @@ __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refil
      each refill costs a queue atomic and a pass through this loop) */
   const bool adapt = refill_k <= 0;
   int kk = adapt ? 128 : refill_k;
-  /* wave-uniform bound on every lane's event count: while it stays a whole
-     interval below the cap, no history can reach the cap in the next
-     interval, and the events run without the cap test; recomputed exactly
-     (the largest count in the wave) when it nears the cap */
+  int wait = 1;
+  /* wave-uniform bound on every lane's event count (a waiting event counted);
+     recomputed exactly (the largest in the wave) when an interval could reach
+     the cap, which then shortens the interval: no history passes the cap */
   uint64_t ev_bound = 0;
   for (;;) {
-    if (!done) { /* wave-uniform */
-      const unsigned long long need = __ballot(!has);
+    if (mc_queue_more(q)) { /* wave-uniform */
+      const mc_mask need = mc_lanes(!has);
       if (adapt) {
         const int idle = __popcll(need);
         kk = idle > 16 ? (kk > 8 ? kk >> 1 : 8) : (idle < 4 ? (kk < 256 ? kk << 1 : 256) : kk);
       }
       if (need) {
-        const int cnt = __popcll(need);
-        const int leader = __ffsll((long long)need) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(&a.ctr->next, (unsigned long long)cnt);
-        base = mc_readlane64(base, leader);
-        if (!has) {
-          const int64_t i = (int64_t)(base + (unsigned long long)mc_mbcnt64(need));
-          if (i < a.n) {
-            load_state(a, i, p);
-            mc_refresh_rcp(p);
-            idx = i;
-            has = true;
-            ev = 0;
-            col = 0;
-            score = 0.0;
-          }
+        const int64_t i = mc_queue_take(q, need, &a.ctr->next);
+        bool on = false;
+        if (!has && i >= 0) {
+          mc_state in;
+          load_state(a, i, in);
+          mc_walk_from(p, in, a.L);
+          idx = i;
+          has = true;
+          on = mc_walk_alive(p, a.L);
+          ev = 0;
+          col = 0;
+          score = 0.0;
         }
-        if (base + (unsigned long long)cnt >= (unsigned long long)a.n) done = true;
+        run |= mc_lanes(on);
       }
     }
-    if (__ballot(has) == 0) break; /* wave-uniform */
-    if (ev_bound + (uint64_t)kk >= a.max_events)
-      ev_bound = mc_wave_max_u64(has ? ev : 0ull);
-    const bool below_cap = ev_bound + (uint64_t)kk < a.max_events; /* wave-uniform */
-    ev_bound += (uint64_t)kk;
-    if (has) {
-      /* one event of this lane's history: Layer::particle_step */
-      auto step = [&]() {
-        const int c = p.index - a.L.index_start;
-        bool coll;
-        double di;
-        const double dw = mc_event<true>(p, cells, c, a.L.dx, K, coll, di, nullptr, &col);
-        mc_tally(t_lo, t_hi, a.flags, &a.ctr->status, c, dw);
-        if (SCORE) score = score + g[c] * dw;
-      };
-      /* the same loop twice, so that the common one carries no cap test
-         (the compiler keeps a shared test in the loop even when the flag
-         guarding it is uniform) */
-      if (below_cap) {
-        for (int k = 0; k < kk; ++k) {
-          if (!mc_alive(p, a.L)) break;
-          step();
-          ++ev;
-        }
-      } else {
-        for (int k = 0; k < kk; ++k) {
-          if (!mc_alive(p, a.L) || ev >= a.max_events) break;
-          step();
-          ++ev;
-        }
-      }
-      const bool alive = mc_alive(p, a.L);
-      if (!alive || ev >= a.max_events) {
-        int code = mc_exit_code(p, a.L);
-        if (alive) { /* runaway history stopped by the guard */
-          capped = true;
-          code = 2;
-        }
-        store_state(a, idx, p, code);
-        if (a.events) a.events[idx] = ev;
-        if (a.collisions) a.collisions[idx] = col;
-        if (SCORE) a.score[idx] = score;
-        tot_ev += ev;
-        tot_col += col;
-        nl += code == -1;
-        nr += code == 1;
-        nk += code == 0;
-        has = false;
-      }
+    if (mc_lanes(has) == 0) break; /* wave-uniform */
+    int ki = kk < k_max ? kk : k_max - 1; /* a waiting lane may add one */
+    if (ev_bound + (uint64_t)ki >= a.max_events) {
+      ev_bound = mc_wave_max_u64(has ? ev + (mc_in(pend) ? 1u : 0u) : 0ull);
+      if (ev_bound + (uint64_t)ki >= a.max_events) ki = (int)(a.max_events - ev_bound);
     }
+    ev_bound += (uint64_t)ki;
+    moves(ki + 1);
+    uint32_t ei = 0; /* events of this interval */
+    const int general =
+        mc_walk_many(p, run, pend, ki, wait, cells, tab, K, ei, col,
+                     [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                       tally(lanes, c, dw);
+                       if (SCORE && mc_in(lanes)) score = score + g[c] * dw;
+                     });
+    wait = mc_walk_wait(wait, general, ki);
+    ev += ei;
+    const bool on = mc_in(run), waits = mc_in(pend);
+    if (has && !waits && (!on || ev >= a.max_events)) {
+      mc_state out;
+      mc_walk_to(out, p, a.L);
+      int code = mc_exit_code(out, a.L);
+      if (on) { /* runaway history stopped by the guard */
+        capped = true;
+        code = 2;
+      }
+      store_state(a, idx, out, code);
+      if (a.events) a.events[idx] = ev;
+      if (a.collisions) a.collisions[idx] = col;
+      if (SCORE) a.score[idx] = score;
+      tot_ev += ev;
+      tot_col += col;
+      nl += code == -1;
+      nr += code == 1;
+      nk += code == 0;
+      has = false;
+    }
+    run &= mc_lanes(has);
   }
 
-  tot_ev = mc_wave_sum(tot_ev);
-  tot_col = mc_wave_sum(tot_col);
-  nl = mc_wave_sum(nl);
-  nr = mc_wave_sum(nr);
-  nk = mc_wave_sum(nk);
-  if (lane == 0) {
-    atomicAdd(&a.ctr->events, tot_ev);
-    atomicAdd(&a.ctr->collisions, tot_col);
-    atomicAdd(&a.ctr->n_left, nl);
-    atomicAdd(&a.ctr->n_right, nr);
-    atomicAdd(&a.ctr->n_killed, nk);
-  }
+  mc_totals_wave(s_tot, tot_ev, tot_col, nl, nr, nk);
   if (capped) atomicOr(&a.ctr->status, 1u);
+}
 
+template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE>
+__global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refill_k,
+                                                   int per_cu) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ int s_k;
+  __shared__ unsigned long long s_tot[5];
+  const mc_walk_k K = mc_walk_live(a.L);
+  const mc_queue q = mc_queue_open(a.n, per_cu);
+  const int m = a.L.m;
+  double2 *tab = reinterpret_cast<double2 *>(smem);
+  for (int j = threadIdx.x; j < MC_ABS_N; j += blockDim.x)
+    tab[j] = make_double2(mc_abs_tab[j][0], mc_abs_tab[j][1]);
+  unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + TAB_BYTES), *t1 = t0 + m;
   if (LDS_TALLY) {
+    for (int c = threadIdx.x; c < m; c += blockDim.x) {
+      t0[c] = 0;
+      t1[c] = 0;
+    }
+  }
+  const mc_cell *cells = a.cells;
+  const double *g = a.g;
+  if (LDS_CELLS) {
+    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + TAB_BYTES + (size_t)16 * m);
+    for (int c = threadIdx.x; c < m; c += blockDim.x) lc[c] = a.cells[c];
+    cells = lc;
+    if (SCORE) {
+      double *lg = reinterpret_cast<double *>(smem + TAB_BYTES + (size_t)32 * m);
+      for (int c = threadIdx.x; c < m; c += blockDim.x) lg[c] = a.g[c];
+      g = lg;
+    }
+  }
+  unsigned long long *fx_lo = a.fx, *fx_hi = a.fx + m;
+  uint32_t *flags = a.flags;
+  unsigned int *status = &a.ctr->status;
+  if (threadIdx.x < 5) s_tot[threadIdx.x] = 0;
+  mc_counters *ctr = a.ctr;
+  auto totals = [&]() { /* after a barrier */
+    if (threadIdx.x == 0)
+      mc_totals_block(s_tot, &ctr->events, &ctr->collisions, &ctr->n_left, &ctr->n_right,
+                      &ctr->n_killed);
+  };
+  if (!LDS_TALLY) {
+    __syncthreads();
+    walk_bank<SCORE>(a, cells, g, tab, refill_k, q, K, s_tot, 1 << 30,
+                     [&](mc_mask lanes, int c, double dw) {
+                       if (mc_in(lanes)) mc_tally(fx_lo, fx_hi, flags, status, c, dw);
+                     },
+                     [](int) {});
+    __syncthreads();
+    totals();
+    return;
+  }
+
+  /* the block's weights: the largest among the first histories of its waves
+     (a guess that sets the limbs' range; heavier ones go to the global tally) */
+  if (threadIdx.x == 0) s_k = -1023;
+  __syncthreads();
+  {
+    const uint64_t i = q.next + __lane_id();
+    if (i < q.end) atomicMax(&s_k, mc_ceil_log2(a.aos ? a.aos[i].wmc : a.soa.wmc[i]));
+  }
+  __syncthreads();
+  const int waves = blockDim.x >> 6;
+  const mc_block_tally B = mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), waves);
+  if (B.limbs) { /* block-uniform */
+    int left = B.every;
+    walk_bank<SCORE>(a, cells, g, tab, refill_k, q, K, s_tot, B.every,
+                     [&](mc_mask lanes, int c, double dw) {
+                       mc_tally_limbs(t0, t1, B.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
+                     },
+                     [&](int k) {
+                       if (left < k) { /* wave-uniform */
+                         mc_limbs_move(t0, t1, B.S.L, m, __lane_id(), 64, fx_lo, fx_hi);
+                         left = B.every;
+                       }
+                       left -= k;
+                     });
+    __syncthreads();
+    mc_limbs_move(t0, t1, B.S.L, m, threadIdx.x, blockDim.x, fx_lo, fx_hi);
+  } else {
+    walk_bank<SCORE>(a, cells, g, tab, refill_k, q, K, s_tot, 1 << 30,
+                     [&](mc_mask lanes, int c, double dw) {
+                       if (mc_in(lanes)) mc_tally(t0, t1, flags, status, c, dw);
+                     },
+                     [](int) {});
     __syncthreads();
     for (int c = threadIdx.x; c < m; c += blockDim.x) {
       mc_fx v;
-      v.lo = t_lo[c];
-      v.hi = t_hi[c];
-      mc_fx_atomic_add(&a.fx[c], &a.fx[m + c], v);
+      v.lo = t0[c];
+      v.hi = t1[c];
+      mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], v);
     }
   }
+  totals(); /* the barrier after the walk stands before */
 }
 
 template <bool T, bool C, bool S>
@@ -200,13 +250,10 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
   int grid = o.grid_blocks;
   if (grid <= 0) {
     grid = per_cu * ctx->num_cus;
-    /* no more blocks than there are waves of work */
-    int64_t waves = (a.n + 63) / 64;
-    int64_t blocks_needed = (waves * 64 + block - 1) / block;
-    if (blocks_needed < grid) grid = (int)(blocks_needed > 0 ? blocks_needed : 1);
+    if (a.n < grid) grid = (int)(a.n > 0 ? a.n : 1); /* a block per history at most */
   }
   int k = o.events_per_refill > 0 ? o.events_per_refill : 0; /* 0: adaptive */
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k, per_cu);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
 }
@@ -216,18 +263,19 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
 int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
                       hipStream_t s) {
   const size_t m = (size_t)a.L.m;
-  const size_t tally = 16 * m, cells = sizeof(mc_cell) * m;
-  const bool lds_tally = tally <= ctx->lds_per_block;
+  const size_t tally = 16 * m + TAB_BYTES, cells = sizeof(mc_cell) * m;
+  const size_t budget = ctx->lds_per_block - 256; /* the kernel's static LDS */
+  const bool lds_tally = tally <= budget;
   if (a.score) { /* per-history score of a weighted tally (forward of the adjoint) */
     if (!a.g) return mc_fail(ctx, MCGPU_ERR_ARG, "score output needs target weights g");
     const size_t extra = 8 * m;
-    const bool lds_cells = lds_tally && tally + cells + extra <= 65536;
+    const bool lds_cells = lds_tally && tally + cells + extra <= budget;
     if (lds_tally && lds_cells) return launch_one<true, true, true>(ctx, a, o, s, tally + cells + extra);
     if (lds_tally) return launch_one<true, false, true>(ctx, a, o, s, tally);
-    return launch_one<false, false, true>(ctx, a, o, s, 0);
+    return launch_one<false, false, true>(ctx, a, o, s, TAB_BYTES);
   }
-  const bool lds_cells = lds_tally && tally + cells <= 65536;
+  const bool lds_cells = lds_tally && tally + cells <= budget;
   if (lds_tally && lds_cells) return launch_one<true, true, false>(ctx, a, o, s, tally + cells);
   if (lds_tally) return launch_one<true, false, false>(ctx, a, o, s, tally);
-  return launch_one<false, false, false>(ctx, a, o, s, 0);
+  return launch_one<false, false, false>(ctx, a, o, s, TAB_BYTES);
 }

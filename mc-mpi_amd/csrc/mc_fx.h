@@ -146,4 +146,85 @@ MC_FN_HD double mc_fx_finalize(uint64_t lo, uint64_t hi, uint32_t flags) {
   return mc_fx_to_double(lo, hi);
 }
 
+/* ------------------------------------------------------- two-limb tallies
+   A block's tally in LDS keeps two 64-bit sums per cell that never carry into
+   each other: for a term v, limb 1 takes n1 = v rounded to a multiple of
+   2^(L-88) and limb 0 the signed rest in units of 2^-88, so that
+   n1 * 2^L + n0 is the term's fixed-point integer exactly.  No add needs the
+   other limb's result, so both are plain atomic adds without a returned
+   value.  |n0| <= 2^(L-1); with 0 <= v < 2^V, n1 <= 2^(V+88-L).  After N
+   terms limb 0 stays within a signed and limb 1 within an unsigned 64-bit
+   word while N <= 2^(64-L) and N <= 2^(L-V-24); L = 44 + floor(V/2) makes
+   the two bounds (nearly) equal.  A block moves its limbs to the global
+   128-bit tally (mc_fx_limbs) before N terms can have been added to a cell.
+   Both limbs come from adding constants whose ulp is the limb's unit:
+   c1 = 1.5 * 2^(L-36), 1.5 * 2^-36. */
+typedef struct {
+  double c1;
+  uint32_t c1_hi;  /* high word of c1 (its low word is zero) */
+  uint32_t range;  /* high word of 2^V less that of 2^-36 */
+  int L;
+} mc_fx_split;
+
+#define MC_FX_C2 0x1.8p-36
+#define MC_FX_C2_HI ((uint32_t)((1023 - 36) << 20 | 0x80000))
+#define MC_FX_HI36 ((uint32_t)((1023 - 36) << 20)) /* high word of 2^-36 */
+#define MC_FX_HI88 ((uint32_t)((1023 - 88) << 20)) /* high word of 2^-88 */
+
+/* terms below 2^V, -35 <= V <= 15 */
+MC_FN_HD mc_fx_split mc_fx_split_for(int V) {
+  mc_fx_split S;
+  S.L = 44 + (V >> 1);
+  S.c1_hi = (uint32_t)((1023 + S.L - 36) << 20 | 0x80000);
+  const uint64_t b = (uint64_t)S.c1_hi << 32;
+  __builtin_memcpy(&S.c1, &b, 8);
+  S.range = ((uint32_t)(1023 + V) << 20) - MC_FX_HI36;
+  return S;
+}
+
+/* log2 of the number of terms a cell may take between two moves */
+MC_FN_HD int mc_fx_split_log2_terms(int V) {
+  const int L = 44 + (V >> 1);
+  return 64 - L < L - V - 24 ? 64 - L : L - V - 24;
+}
+
+/* v in [2^-36, 2^V): its unit 2^-88 or coarser, no rounding */
+MC_FN_HD int mc_fx_split_direct(double v, const mc_fx_split *S) {
+  uint64_t b;
+  __builtin_memcpy(&b, &v, 8);
+  return (uint32_t)(b >> 32) - MC_FX_HI36 < S->range;
+}
+
+/* v = 0 or in [2^-88, 2^-36): rounded half up to a multiple of 2^-88 (then as
+   mc_fx_split_direct).  v * 2^88 + 1/2 in one fma: exact, or (across a power
+   of two) rounded without crossing an integer.  Other terms return 0. */
+MC_FN_HD int mc_fx_split_small(double *v) {
+  uint64_t b;
+  __builtin_memcpy(&b, v, 8);
+  const uint32_t h = (uint32_t)(b >> 32);
+  if (!(h - MC_FX_HI88 < MC_FX_HI36 - MC_FX_HI88 || b == 0)) return 0;
+  *v = __builtin_floor(__builtin_fma(*v, 0x1p88, 0.5)) * 0x1p-88;
+  return 1;
+}
+
+/* the limbs of a term that one of the two accepts */
+MC_FN_HD void mc_fx_split_limbs(double v, const mc_fx_split *S, uint64_t *n0, uint64_t *n1) {
+  const double h = v + S->c1;
+  const double rest = v - (h - S->c1);
+  const double l = rest + MC_FX_C2;
+  uint64_t hb, lb;
+  __builtin_memcpy(&hb, &h, 8);
+  __builtin_memcpy(&lb, &l, 8);
+  *n1 = (uint64_t)((uint32_t)(hb >> 32) - S->c1_hi) << 32 | (uint32_t)hb;
+  *n0 = (uint64_t)((uint32_t)(lb >> 32) - MC_FX_C2_HI) << 32 | (uint32_t)lb;
+}
+
+/* n1 * 2^L + n0 as the 128-bit integer (n0 signed, n1 unsigned) */
+MC_FN_HD mc_fx mc_fx_limbs(uint64_t n0, uint64_t n1, int L) {
+  mc_fx r;
+  r.lo = (n1 << L) + n0;
+  r.hi = (n1 >> (64 - L)) + (uint64_t)((int64_t)n0 >> 63) + (r.lo < n0 ? 1u : 0u);
+  return r;
+}
+
 #endif /* MC_FX_H */

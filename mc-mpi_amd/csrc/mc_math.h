@@ -512,4 +512,79 @@ MC_FN double mc_exp_k_row(double x, const mc_exp_row *R, const mc_coef *K) {
   return (yh + yl) * mc_pow2(kk);
 }
 
+/* ------------------------------------------------------ absorbed fraction
+   The transport's deposit is (1 - RN(exp(-y))) * wmc with y = sig_a * di.
+   For y in [0, MC_ABS_YMAX], exp(-y) lies in (1/2, 1], where doubles are the
+   multiples of 2^-53: RN(exp(-y)) is a rounding to a fixed grid, 1 minus it is
+   exact, and only an absolute error matters.  So exp is not formed to full
+   relative accuracy with its own head: the fraction u = 1 - RN(exp(-y)) comes
+   from a short series whose last rounding is certified against the half
+   spacing 2^-54.
+
+   With r = y - y_k (exact: y_k is a multiple of 2^-43, and y within a factor
+   of two of it or k = 0; |r| < 2^-7.99), exp(-y_k) a double to within 2^-71, b = r^2 (1/2 - r/6 + r^2/24 -
+   r^3/120 + r^4/720 - r^5/5040), exp(-r) = 1 - r + b.  Absolute errors: the
+   omitted r^8/8! below 2^-79; b < 2^-17 from r*r, the series and the last
+   fma, each a relative 2^-53 (the series' inner roundings are scaled by r):
+   below 2^-68.3 in all; the last fma and the table's 2^-71, each below
+   2^-70.  Together below 2^-67.3.
+   rem, the exact distance from the rounded value to the computed one, then
+   certifies the rounding when |rem| < 2^-54 - 2^-67 (MC_ABS_REM): the true
+   value is within 2^-54 of the grid point, hence rounds to it.  About one
+   event in 8,000 is not certified and takes the general exp.  */
+#define MC_ABS_REM (0x1p-54 - 0x1p-67)
+#define MC_ABS_THIN 0x1p-8 /* y below this needs no table row */
+
+typedef struct {
+  double c7, c6, c5, c4, c3; /* 1/7!, 1/6!, 1/5!, 1/4!, 1/3! */
+} mc_abs_coef;
+
+MC_FN mc_abs_coef mc_abs_coef_default(void) {
+  mc_abs_coef K;
+  K.c7 = mc_inv_fact[7][0]; K.c6 = mc_inv_fact[6][0]; K.c5 = mc_inv_fact[5][0];
+  K.c4 = mc_inv_fact[4][0]; K.c3 = mc_inv_fact[3][0];
+  return K;
+}
+
+/* 1/2 - r/6 + r^2/24 - r^3/120 + r^4/720 - r^5/5040 */
+MC_FN double mc_abs_series(double r, const mc_abs_coef *K) {
+  double c = mc_fma(-r, K->c7, K->c6);
+  c = mc_fma(-r, c, K->c5);
+  c = mc_fma(-r, c, K->c4);
+  c = mc_fma(-r, c, K->c3);
+  return mc_fma(-r, c, 0.5);
+}
+
+/* u for 0 <= y < MC_ABS_THIN (k = 0, no table row); *rem as above.
+   three4: 3/4; 3/4 + y and 3/4 + u lie in [1/2, 1), on the grid. */
+MC_FN double mc_absorb_thin(double y, double three4, const mc_abs_coef *K, double *rem) {
+  const double c = mc_abs_series(y, K);
+  const double y2 = y * y;
+  const double t = three4 + y;
+  const double res = y - (t - three4);    /* exact, |res| <= 2^-54 */
+  const double lo = mc_fma(-y2, c, res);
+  const double v = t + lo;
+  *rem = lo - (v - t);                    /* exact */
+  return v - three4;
+}
+
+/* k of mc_absorb_row, any y in [0, MC_ABS_YMAX]: at most MC_ABS_N - 1
+   (spacing 2^-7: rounds 128 y) */
+MC_FN unsigned mc_abs_index(double y) {
+  return (unsigned)(uint32_t)mc_asu64(y + 0x1.8p45);
+}
+
+/* u for 0 <= y <= MC_ABS_YMAX from the row {yk, th}, th = exp(-yk) */
+MC_FN double mc_absorb_row(double y, double yk, double th, const mc_abs_coef *K, double *rem) {
+  const double r = y - yk;
+  const double c = mc_abs_series(r, K);
+  const double b = (r * r) * c;
+  const double s = mc_fma(-th, r, th);
+  const double res = mc_fma(-th, r, th - s);
+  const double lo = mc_fma(th, b, res);
+  const double e = s + lo;
+  *rem = lo - (e - s);                    /* exact */
+  return 1.0 - e;
+}
+
 #endif /* MC_MATH_H */

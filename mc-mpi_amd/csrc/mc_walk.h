@@ -1,0 +1,469 @@
+/*
+ * mc_walk.h -- one transport event of Layer::particle_step
+ * (src/layer.cpp:123-190) as the persistent kernels run it: a short common
+ * step for the event that provably crosses its cell, and the general event
+ * (mc_event's operations) for everything else.
+ *
+ * What bounds these kernels is the number of vector instructions per event:
+ * gfx950 issues one 64-bit (or three-operand) wave64 instruction per SIMD
+ * every 4.25 cycles, and a wave on its own one every 8.5 whatever the
+ * instruction, so the count sets both the rate of a full chip and the time of
+ * a lone long history.  The common step has about half the instructions of
+ * mc_event:
+ *  - the state is kept in the form the step uses: the doubled RNG state (the
+ *    generator is a map mod 2^64 with no mask, and its top 32 bits are h's),
+ *    1/mu as a pair, the next edge's number as a double, the cell as an
+ *    offset in the layer;
+ *  - the collision test needs only 20 bits of h: 1 + h (truncated) + sig_i *
+ *    di_edge < 2 - 2^-18 implies 1 - h > sig_i * di_edge * (1 + 2^-40), the
+ *    certificate of mc_event;
+ *  - the absorbed fraction is a rounding on a fixed grid (mc_absorb_thin,
+ *    mc_absorb_row), with no exp to full relative accuracy;
+ *  - the deposit is split into two limbs by floating-point adds and summed by
+ *    two LDS adds without a returned value (mc_fx_split_limbs).
+ * A lane whose event is not certified waits (`pend`) and the wave runs the
+ * general event for its waiting lanes together (see mc_walk_many).
+ */
+#ifndef MC_WALK_H
+#define MC_WALK_H
+
+#include "mc_device.h"
+
+struct mc_walk {
+  uint64_t s2;    /* twice the RNG state (mod 2^64) */
+  double x, mu, wmc;
+  double rh, rl;  /* 1/mu = rh + rl, rh = RN(1/mu); rh = NaN when |mu| <= EPS (or NaN) */
+  double fe, fs;  /* number of the next edge, +-1 */
+  int32_t c, st;  /* cell offset in the layer, +-1 */
+};
+
+__device__ __forceinline__ void mc_walk_turn(mc_walk &p, int32_t index) {
+  const bool back = p.mu < 0;
+  p.st = back ? -1 : 1;
+  p.fs = back ? -1.0 : 1.0;
+  p.fe = (double)(back ? index : index + 1);
+  p.rh = 1.0 / p.mu;
+  p.rl = mc_fma(-p.mu, p.rh, 1.0) * p.rh;
+  if (!(p.mu < -MC_EPS || MC_EPS < p.mu)) p.rh = __builtin_nan("");
+}
+
+__device__ __forceinline__ void mc_walk_from(mc_walk &w, const mc_state &p, const mc_layer_k &L) {
+  w.s2 = p.seed << 1;
+  w.x = p.x;
+  w.mu = p.mu;
+  w.wmc = p.wmc;
+  w.c = p.index - L.index_start;
+  mc_walk_turn(w, p.index);
+}
+
+__device__ __forceinline__ void mc_walk_to(mc_state &p, const mc_walk &w, const mc_layer_k &L) {
+  p.seed = w.s2 >> 1;
+  p.x = w.x;
+  p.mu = w.mu;
+  p.wmc = w.wmc;
+  p.index = w.c + L.index_start;
+}
+
+__device__ __forceinline__ bool mc_walk_alive(const mc_walk &w, const mc_layer_k &L) {
+  return (w.wmc >= L.min_weight) && (uint32_t)w.c < (uint32_t)L.m;
+}
+
+__device__ __forceinline__ void mc_walk_draw(uint64_t &s2) {
+  s2 = MC_RNG_G * s2 + 2 * MC_RNG_C;
+}
+
+/* h of the drawn state: (double)seed * 2^-63, rounded once (as mc_rnd_real) */
+__device__ __forceinline__ double mc_walk_h(uint64_t s2) {
+  return __builtin_fma((double)(uint32_t)(s2 >> 32), 0x1p-32, (double)(uint32_t)s2 * 0x1p-64);
+}
+
+/* wave-uniform values in scalar registers, which the compiler neither folds
+   nor rebuilds from halves at each use */
+struct mc_walk_k {
+  mc_abs_coef A;
+  double rem_max;   /* MC_ABS_REM */
+  double sure_max;  /* 2 - 2^-18 */
+  double q_min;     /* 2^-900 */
+  double three4;    /* 3/4 */
+  double dx, min_weight;
+  int32_t m;
+};
+
+__device__ __forceinline__ mc_walk_k mc_walk_live(const mc_layer_k &L) {
+  mc_walk_k K;
+  K.A = mc_abs_coef_default();
+  K.rem_max = MC_ABS_REM;
+  K.sure_max = 2.0 - 0x1p-18;
+  K.q_min = 0x1p-900;
+  K.three4 = 0.75;
+  K.dx = L.dx;
+  K.min_weight = L.min_weight;
+  K.m = L.m;
+  asm volatile("" : "+v"(K.A.c7), "+s"(K.A.c6), "+s"(K.A.c5), "+s"(K.A.c4), "+s"(K.A.c3));
+  asm volatile("" : "+s"(K.rem_max), "+s"(K.sure_max), "+s"(K.q_min), "+s"(K.three4));
+  asm volatile("" : "+s"(K.dx), "+s"(K.min_weight), "+s"(K.m));
+  return K;
+}
+
+__device__ __forceinline__ uint32_t mc_hi32(double v) { return (uint32_t)(mc_asu64(v) >> 32); }
+
+/* Lanes of the wave as a scalar mask, and back.  Conditions are combined as
+   masks (scalar ands), each ballot of one comparison. */
+typedef unsigned long long mc_mask;
+__device__ __forceinline__ mc_mask mc_lanes(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+__device__ __forceinline__ bool mc_in(mc_mask m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+/* cell c (in [0, m)): an unsigned 32-bit byte offset, so that a global load
+   takes the uniform base in scalar registers */
+__device__ __forceinline__ mc_cell mc_cell_at(const mc_cell *cells, uint32_t c) {
+  return *reinterpret_cast<const mc_cell *>(reinterpret_cast<const char *>(cells) + (c << 4));
+}
+
+/* The common step on cell `cell`, for every lane of the wave: the draw, then
+   the crossing's next edge xn, flight q and absorbed fraction u.  Returns
+   the lanes whose event certainly is that crossing, u certified; for the
+   others mc_walk_general finishes the event.  run: the lanes that matter.
+   tab: the rows of mc_abs_tab (LDS).
+   The edge quotient a / mu: q0 = a rh + RN(a rl) rounded once is within 1 ulp,
+   and one Markstein step with rh = RN(1/mu) makes it the correctly rounded
+   quotient (as in mc_div_by_rcp, one fma fewer since q0 is closer); q > 2^-900
+   keeps every product normal, and |mu| <= EPS (rh NaN) fails every test. */
+__device__ __forceinline__ mc_mask mc_walk_cross(mc_walk &p, mc_mask run, const mc_cell cell,
+                                                 const double2 *tab, const mc_walk_k &K,
+                                                 double &xn, double &q, double &u) {
+  mc_walk_draw(p.s2);
+  xn = p.fe * K.dx;
+  const double a = xn - p.x;
+  const double q0 = mc_fma(a, p.rh, a * p.rl);
+  q = mc_fma(mc_fma(-p.mu, q0, a), p.rh, q0);
+  /* 1 + h with h's top 20 bits (any low word: h is at most 2^-20 above) */
+  const uint32_t sh = (uint32_t)(p.s2 >> 32);
+  const double h1 = mc_asf64((uint64_t)__builtin_amdgcn_alignbit(0x3FFu, sh, 12) << 32);
+  const double t = mc_fma(cell.sig_i, q, h1);
+  const double y = cell.sig_a * q;
+  mc_mask ok = run & mc_lanes(t < K.sure_max) & mc_lanes(q > K.q_min);
+  double rem;
+  /* y in [0, MC_ABS_THIN) by its high word (negative and NaN fail) */
+  const mc_mask thin = mc_lanes(mc_hi32(y) < (uint32_t)((1023 - 8) << 20));
+  if ((run & ~thin) == 0) { /* wave-uniform: every live lane is thin */
+    u = mc_absorb_thin(y, K.three4, &K.A, &rem);
+  } else {
+    ok &= mc_lanes(y >= 0.0) & mc_lanes(y <= MC_ABS_YMAX);
+    const unsigned k = mc_abs_index(y);
+    const double2 row = tab[k < MC_ABS_N ? k : 0u];
+    u = mc_absorb_row(y, row.x, row.y, &K.A, &rem);
+  }
+  return ok & mc_lanes(__builtin_fabs(rem) < K.rem_max);
+}
+
+/* The general event, after mc_walk_cross has drawn: mc_event's operations.
+   Returns the deposit; coll, di as mc_event's. */
+__device__ __forceinline__ double mc_walk_general(mc_walk &p, const mc_cell cell, const double dx,
+                                                  bool &coll, double &di) {
+  const mc_coef K = mc_coef_default();
+  const double h = mc_walk_h(p.s2);
+  const double xn = p.fe * dx;
+  const bool flat = !(p.mu < -MC_EPS || MC_EPS < p.mu);
+  const double di_edge = flat ? MC_MAXREAL : mc_div_by_rcp(xn - p.x, p.mu, p.rh);
+  const double reach = cell.sig_i * di_edge;
+  const int sure_cross =
+      (int)!(cell.sig_i > MC_EPS) | (int)((1.0 - h) > mc_fma(reach, 0x1p-40, reach));
+  di = di_edge;
+  coll = false;
+  if (!sure_cross) {
+    const double dq = -mc_log_k(h, &K) / cell.sig_i;
+    coll = dq < di_edge;
+    if (coll) di = dq;
+  }
+  const double dw = (1 - mc_exp_k(-cell.sig_a * di, &K)) * p.wmc;
+  p.wmc -= dw;
+  if (coll) {
+    p.x += di * p.mu;
+    mc_walk_draw(p.s2);
+    p.mu = 2 * mc_walk_h(p.s2) - 1;
+    /* the index from the edge ahead: fe is index + 1 moving up, index moving down */
+    mc_walk_turn(p, (int32_t)p.fe - (p.st > 0 ? 1 : 0));
+  } else {
+    p.x = xn;
+    p.fe += p.fs;
+    p.c += p.st;
+  }
+  return dw;
+}
+
+/* The waiting lanes (per 64 live ones) at which the wave runs the general
+   event.  Running it for one lane costs the wave about three common steps;
+   letting w lanes wait leaves w/2 of 64 idle on average.  With a chance p per
+   event the sum is least at w = sqrt(128 * 64 * 3 p), which is 400 times the
+   general events per iteration (64 p / w) at that w: move towards it. */
+__device__ __forceinline__ int mc_walk_wait(int wait, int general, int iterations) {
+  const int want = 400 * general;
+  if (want > wait * iterations) return wait < 16 ? wait + 1 : 16;
+  return wait > 1 ? wait - 1 : 1;
+}
+
+/* Up to ki events of every lane in `run` (lanes whose history goes on; `pend`:
+   lanes whose drawn event waits for the general form; both wave-uniform
+   masks, disjoint).  on_event(lanes, c, cell, coll, di, dw, wmc) is called by
+   the whole wave for an event of `lanes` in cell c (wmc: the weight after
+   it).  ei counts a lane's events, col its collisions.  Returns how often the
+   general event ran.
+   Every lane computes the common step (lanes not in `run` on whatever they
+   hold, with the cell index clamped); only the lanes of a certified crossing
+   commit it.  An iteration in which no lane stops or waits costs one scalar
+   comparison; the next cell is loaded before the tally's adds, so that its
+   latency passes under them and the next draw. */
+template <typename F>
+__device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &pend, int ki,
+                                            int wait, const mc_cell *cells, const double2 *tab,
+                                            const mc_walk_k &K, uint32_t &ei, uint32_t &col,
+                                            F on_event) {
+  int general = 0;
+  const uint32_t top = (uint32_t)K.m - 1u;
+  for (;;) {
+    const int live = __popcll(run | pend);
+    if (live == 0) break;
+    const int nwait = ki > 0 ? (wait * live + 63) >> 6 : 1;
+    if (run != 0 && ki > 0 && __popcll(pend) < nwait) {
+      const int k0 = ki;
+      uint64_t s2 = p.s2; /* the state of the lanes not in run: the draw below is for all */
+      mc_cell cell = mc_cell_at(cells, (uint32_t)p.c < top ? (uint32_t)p.c : top);
+      for (;;) {
+        double xn, q, u;
+        const mc_mask ok = mc_walk_cross(p, run, cell, tab, K, xn, q, u);
+        const mc_cell here = cell;
+        const int c = p.c;
+        const double dw = u * p.wmc;
+        if (mc_in(ok)) {
+          p.wmc -= dw;
+          p.x = xn;
+          p.fe += p.fs;
+          p.c += p.st;
+          cell = mc_cell_at(cells, (uint32_t)p.c < top ? (uint32_t)p.c : top);
+        }
+        const mc_mask on =
+            ok & mc_lanes(p.wmc >= K.min_weight) & mc_lanes((uint32_t)p.c < (uint32_t)K.m);
+        on_event(ok, c, here, false, q, dw, p.wmc);
+        --ki;
+        if (__builtin_expect(on != run, 0)) { /* wave-uniform: a lane stopped or waits */
+          if (mc_in(run & ~on)) {
+            s2 = p.s2;
+            ei += (uint32_t)(k0 - ki) - (mc_in(ok) ? 0u : 1u);
+          }
+          pend |= run & ~ok;
+          run = on;
+          if (run == 0 || __popcll(pend) >= nwait) break;
+        }
+        if (ki == 0) break;
+      }
+      if (mc_in(run))
+        ei += (uint32_t)(k0 - ki);
+      else
+        p.s2 = s2;
+    }
+    if (pend != 0 && (run == 0 || __popcll(pend) >= nwait)) {
+      ++general;
+      const int c = p.c;
+      mc_cell cell;
+      cell.sig_a = cell.sig_i = 0.0;
+      bool coll = false, on = false;
+      double di = 0.0, dw = 0.0;
+      if (mc_in(pend)) {
+        cell = mc_cell_at(cells, (uint32_t)c);
+        dw = mc_walk_general(p, cell, K.dx, coll, di);
+        ++ei;
+        col += coll ? 1u : 0u;
+        on = p.wmc >= K.min_weight && (uint32_t)p.c < (uint32_t)K.m;
+      }
+      on_event(pend, c, cell, coll, di, dw, p.wmc);
+      run |= mc_lanes(on);
+      pend = 0;
+    }
+    if (ki == 0) break;
+  }
+  return general;
+}
+
+/* -------------------------------------------------------------- work queue */
+
+/* The histories 0 .. n-1 of a call, taken by waves in runs: the first run of
+   each wave is its own by position (no atomic), later ones come from the
+   call's counter, a quarter of what is left per wave at a time.  With one
+   atomic per refill instead, short histories wait for the counter: one
+   address takes about one atomic every 7 ns from a full chip.
+   First runs go to wave 0 of every block, then to wave 1 of every block, ...:
+   few histories spread over all CUs and SIMDs.  A SIMD runs two waves as fast
+   as one (each issues at most every 8.5 cycles, the SIMD every 4.25), four
+   at half speed, and a wave's lanes wait for each other's general events; so
+   up to 64 histories for each of the first eight waves of a CU are dealt out
+   evenly among those waves. */
+struct mc_queue {
+  uint64_t n, next, end; /* the wave's run [next, end) */
+  uint64_t first, seen;  /* where the counter's zero stands; the last place seen */
+  uint32_t waves;
+  bool dry;              /* no run left to take */
+};
+
+__device__ __forceinline__ uint64_t mc_run_size(uint64_t left, uint32_t waves) {
+  const uint64_t s = left / (4u * (uint64_t)waves);
+  return s < 64 ? 64 : (s > 4096 ? 4096 : s);
+}
+
+/* per_cu: blocks on a CU */
+__device__ __forceinline__ mc_queue mc_queue_open(int64_t n, int per_cu) {
+  mc_queue q;
+  const uint32_t per_block = blockDim.x >> 6;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t pos = wave * gridDim.x + blockIdx.x;
+  q.n = (uint64_t)n;
+  q.waves = gridDim.x * per_block;
+  const uint32_t few = (per_block * (uint32_t)per_cu > 8u ? (8u + per_cu - 1) / per_cu : per_block) *
+                       gridDim.x;
+  const uint64_t size = q.n <= 64ull * few ? (q.n + few - 1) / few : mc_run_size(q.n, q.waves);
+  q.next = pos * size;
+  q.end = q.next + size;
+  q.first = q.seen = q.waves * size;
+  if (q.end > q.n) q.end = q.n;
+  if (q.next > q.n) q.next = q.n;
+  q.dry = q.first >= q.n;
+  return q;
+}
+
+/* whether the wave can still take histories */
+__device__ __forceinline__ bool mc_queue_more(const mc_queue &q) {
+  return !q.dry || q.next < q.end;
+}
+
+/* a history for each lane of `need` (called by the whole wave): its index, or
+   -1 when none is left */
+__device__ __forceinline__ int64_t mc_queue_take(mc_queue &q, mc_mask need,
+                                                 unsigned long long *counter) {
+  const uint64_t cnt = (uint64_t)__popcll(need), have = q.end - q.next;
+  const uint64_t rank = (uint64_t)mc_mbcnt64(need);
+  uint64_t i = q.next + rank;
+  if (cnt <= have || q.dry) {
+    if (rank >= have) i = ~0ull;
+    q.next = cnt < have ? q.next + cnt : q.end;
+  } else { /* wave-uniform */
+    const uint64_t size = mc_run_size(q.n - q.seen, q.waves); /* seen < n: not dry */
+    unsigned long long base = 0;
+    if (__lane_id() == 0) base = atomicAdd(counter, (unsigned long long)size);
+    base = mc_readlane64(base, 0) + q.first;
+    uint64_t end = base + size;
+    if (end >= q.n) {
+      q.dry = true;
+      end = q.n;
+    }
+    if (base > q.n) base = q.n;
+    q.seen = base;
+    if (rank >= have) i = base + (rank - have) < end ? base + (rank - have) : ~0ull;
+    const uint64_t used = cnt - have;
+    q.next = base + used < end ? base + used : end;
+    q.end = end;
+  }
+  return (int64_t)i;
+}
+
+/* The call's totals: lanes to the wave's, to the block's (LDS words s_tot[5],
+   zeroed), to the counter block.  One global atomic per block and nonzero
+   total: with one per wave the five addresses of a full chip's 4,096 waves
+   alone took 0.14 ms. */
+__device__ __forceinline__ void mc_totals_wave(unsigned long long *s_tot, unsigned long long ev,
+                                               unsigned long long col, unsigned long long nl,
+                                               unsigned long long nr, unsigned long long nk) {
+  const unsigned long long v[5] = {mc_wave_sum(ev), mc_wave_sum(col), mc_wave_sum(nl),
+                                   mc_wave_sum(nr), mc_wave_sum(nk)};
+  if (__lane_id() == 0)
+    for (int i = 0; i < 5; ++i)
+      if (v[i]) atomicAdd(&s_tot[i], v[i]);
+}
+
+/* by one thread of the block, after a barrier */
+__device__ __forceinline__ void mc_totals_block(const unsigned long long *s_tot,
+                                                unsigned long long *ev, unsigned long long *col,
+                                                unsigned long long *nl, unsigned long long *nr,
+                                                unsigned long long *nk) {
+  unsigned long long *const to[5] = {ev, col, nl, nr, nk};
+  for (int i = 0; i < 5; ++i)
+    if (s_tot[i]) atomicAdd(to[i], s_tot[i]);
+}
+
+/* ------------------------------------------------------------- block tally */
+
+/* How a block's LDS tally takes terms.  Limbs (mc_fx_split) when the weights
+   allow a useful interval between moves, else 128-bit adds with carry. */
+struct mc_block_tally {
+  mc_fx_split S;
+  int every;  /* events per lane between two moves of the limbs (per wave) */
+  int limbs;  /* 0: words (lo, hi) with carry */
+};
+
+/* V for a layer of m cells with weights up to 2^k: thin cells absorb a small
+   part of the weight, and a smaller V means rarer moves; the few larger terms
+   go to the global tally directly.  (On a 1-long slab of m cells a term above
+   2^-6 of the weight needs |mu| below about 64 / m.) */
+__device__ __forceinline__ mc_block_tally mc_block_tally_for(int m, int k, int waves) {
+  mc_block_tally B;
+  const int V = k - (m < 1024 ? 0 : (m < 4096 ? 4 : 6));
+  const int Vc = V < -30 ? -30 : (V > 2 ? 2 : V);
+  B.limbs = V <= 2; /* an interval of at least 512 events per lane */
+  B.S = mc_fx_split_for(Vc);
+  const int lg = mc_fx_split_log2_terms(Vc);
+  B.every = (int)((1u << (lg < 30 ? lg : 30)) / (64u * (unsigned)waves));
+  return B;
+}
+
+/* smallest k with 2^k >= v (v >= 0, not subnormal); large for inf and NaN */
+__device__ __forceinline__ int mc_ceil_log2(double v) {
+  const uint64_t b = mc_asu64(v) & 0x7FFFFFFFFFFFFFFFULL;
+  return (int)(b >> 52) - 1023 + ((b & 0x000FFFFFFFFFFFFFULL) ? 1 : 0);
+}
+
+/* a term that neither limb conversion takes: to the global tally */
+__device__ __noinline__ static void mc_tally_general(unsigned long long *fx_lo,
+                                                     unsigned long long *fx_hi, uint32_t *flags,
+                                                     unsigned int *status, int c, double dw) {
+  const mc_fx_flagged g = mc_fx_from_double_general(dw);
+  if (g.flags) {
+    atomicOr(&flags[c], g.flags);
+    if (g.flags & 8u) atomicOr(status, 2u);
+  }
+  mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], g.v);
+}
+
+/* add dw of `lanes` to cell c of the limb tally (t0, t1), called by the whole
+   wave; fx_lo, fx_hi: global tally */
+__device__ __forceinline__ void mc_tally_limbs(unsigned long long *t0, unsigned long long *t1,
+                                               const mc_fx_split &S, unsigned long long *fx_lo,
+                                               unsigned long long *fx_hi, uint32_t *flags,
+                                               unsigned int *status, mc_mask lanes, int c,
+                                               double dw) {
+  mc_mask take = lanes & mc_lanes(mc_fx_split_direct(dw, &S));
+  if (__builtin_expect(take != lanes, 0)) { /* wave-uniform: small, large or special terms */
+    bool small = false;
+    if (mc_in(lanes & ~take)) {
+      small = mc_fx_split_small(&dw);
+      if (!small) mc_tally_general(fx_lo, fx_hi, flags, status, c, dw);
+    }
+    take |= mc_lanes(small);
+  }
+  if (mc_in(take)) {
+    uint64_t n0, n1;
+    mc_fx_split_limbs(dw, &S, &n0, &n1);
+    atomicAdd(&t0[c], (unsigned long long)n0);
+    atomicAdd(&t1[c], (unsigned long long)n1);
+  }
+}
+
+/* move the limbs of cells first, first + step, ... to the global tally; any
+   wave may do it while others add (each limb is exchanged with zero) */
+__device__ __forceinline__ void mc_limbs_move(unsigned long long *t0, unsigned long long *t1, int L,
+                                              int m, int first, int step, unsigned long long *fx_lo,
+                                              unsigned long long *fx_hi) {
+  for (int c = first; c < m; c += step) {
+    const uint64_t n0 = atomicExch(&t0[c], 0ull), n1 = atomicExch(&t1[c], 0ull);
+    mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx_limbs(n0, n1, L));
+  }
+}
+
+#endif /* MC_WALK_H */
