@@ -17,11 +17,17 @@
  *    and replayed; zeroing is done by kernels (no memset nodes).
  * Per history the arithmetic is the single-slab kernels' arithmetic, so each
  * slab's results are bit-identical to transporting it alone.
+ *
+ * The event is the common step of mc_walk.h; what bounds a launch besides it
+ * is the tiles: a block waits for its tile's longest history, and few large
+ * tiles leave CUs idle.  Measured, 512 slabs of 32 to 8,192 cells with 100 to
+ * 1e5 histories each: 110.0 -> 72.5 ms with mc_walk.h and tiles cut to an
+ * eighth of a CU's share.
  */
 #include <algorithm>
 #include <vector>
 
-#include "internal.h"
+#include "mc_walk.h"
 
 namespace {
 
@@ -42,177 +48,123 @@ struct batch_args {
   uint64_t max_events;
 };
 
-/* Per-lane counters of one block, carried across its tiles. */
-struct batch_lane {
-  bool capped;
-  unsigned int ev_pending, col_pending;
+struct tile_io {
+  const batch_args &a;
+  __device__ __forceinline__ void load(int64_t i, mc_state &p) {
+    p.seed = a.soa.seed[i];
+    p.x = a.soa.x[i];
+    p.mu = a.soa.mu[i];
+    p.wmc = a.soa.wmc[i];
+    p.index = a.soa.index[i];
+  }
+  __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t, uint32_t) {
+    a.soa.seed[i] = p.seed;
+    a.soa.x[i] = p.x;
+    a.soa.mu[i] = p.mu;
+    a.soa.wmc[i] = p.wmc;
+    a.soa.index[i] = p.index;
+    if (a.result8) a.result8[i] = (int8_t)code;
+    return false;
+  }
 };
 
-/* One tile: its histories, lanes refilled from the LDS queue s_next.  The
-   tally and cell pointers are LDS or global according to the template
-   arguments, so every access compiles to the matching instruction. */
-template <bool LDS_TALLY, bool LDS_CELLS, bool HI_COND>
-__device__ __forceinline__ void batch_tile(const batch_args &a, const mc_tile_k &tile,
-                                           const mc_slab_k &sl, const mc_layer_k &L,
-                                           unsigned long long *t_lo, unsigned long long *t_hi,
-                                           const mc_cell *cells, unsigned long long *s_next,
-                                           unsigned long long *s_tot, uint32_t max_ev,
-                                           int refill_k, const mc_coef &K, batch_lane &bl) {
-  const int lane = __lane_id();
-  mc_state p;
-  p.index = 0;
-  int64_t idx = 0;
-  bool has = false, done = false;
-  uint32_t ev = 0, col = 0;
-  for (;;) {
-    if (!done) {
-      const unsigned long long need = __ballot(!has);
-      if (need) {
-        const int cnt = __popcll(need);
-        const int leader = __ffsll((long long)need) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(s_next, (unsigned long long)cnt);
-        base = mc_readlane64(base, leader);
-        if (!has) {
-          const int64_t i = (int64_t)(base + (unsigned long long)mc_mbcnt64(need));
-          if (i < tile.end) {
-            p.seed = a.soa.seed[i];
-            p.x = a.soa.x[i];
-            p.mu = a.soa.mu[i];
-            mc_refresh_rcp(p);
-            p.wmc = a.soa.wmc[i];
-            p.index = a.soa.index[i];
-            idx = i;
-            has = true;
-            ev = 0;
-            col = 0;
-          }
-        }
-        if (base + (unsigned long long)cnt >= (unsigned long long)tile.end) done = true;
-      }
-    }
-    if (__ballot(has) == 0) break;
-    if (has) {
-      for (int k = 0; k < refill_k; ++k) {
-        if (!mc_alive(p, L) || ev >= max_ev) break;
-        const int c = p.index - L.index_start;
-        bool coll;
-        double di;
-        const double dw = mc_event<true>(p, cells, c, L.dx, K, coll, di, nullptr, &col);
-        ++ev;
-        mc_tally<false, HI_COND>(t_lo, t_hi, a.flags + sl.cell_off, &a.ctr->status, c, dw);
-      }
-      const bool alive = mc_alive(p, L);
-      if (!alive || ev >= max_ev) {
-        int code = mc_exit_code(p, L);
-        if (alive) {
-          bl.capped = true;
-          code = 2;
-        }
-        a.soa.seed[idx] = p.seed;
-        a.soa.x[idx] = p.x;
-        a.soa.mu[idx] = p.mu;
-        a.soa.wmc[idx] = p.wmc;
-        a.soa.index[idx] = p.index;
-        if (a.result8) a.result8[idx] = (int8_t)code;
-        bl.ev_pending += ev;
-        bl.col_pending += col;
-        atomicAdd(&s_tot[code == -1 ? 2 : (code == 1 ? 3 : 4)], code == 2 ? 0ull : 1ull);
-        has = false;
-        if (bl.ev_pending > 0x40000000u) { /* keep the 32-bit lane counters safe */
-          atomicAdd(&s_tot[0], (unsigned long long)bl.ev_pending);
-          atomicAdd(&s_tot[1], (unsigned long long)bl.col_pending);
-          bl.ev_pending = bl.col_pending = 0;
-        }
-      }
-    }
-  }
-}
-
-/* HI_COND: every particle weight is below 2^-24 (see mc_fx_atomic_add_always) */
-template <bool HI_COND>
+/* The tile loop is the history kernel's (mc_walk_bank) with the tile's LDS
+   counter as its queue; the tally and cell pointers are LDS or global in
+   branches of their own, so every access compiles to the matching
+   instruction. */
 __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const mc_coef K = mc_coef_live();
-  __shared__ int s_tile;
+  __shared__ int s_tile, s_k;
   __shared__ unsigned long long s_next;
-  __shared__ unsigned long long s_tot[5];
-  unsigned long long *t_lds = reinterpret_cast<unsigned long long *>(smem);
-  const int lane = __lane_id();
+  __shared__ unsigned long long s_tot[MC_TOTALS];
+  double2 *tab = reinterpret_cast<double2 *>(smem);
+  mc_tab_fill(tab);
+  unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES);
   const int B = blockDim.x;
   const int tid = threadIdx.x;
-  if (tid < 5) s_tot[tid] = 0;
-  batch_lane bl;
-  bl.capped = false;
-  bl.ev_pending = bl.col_pending = 0;
-  const uint32_t max_ev = a.max_events > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)a.max_events;
+  if (tid < MC_TOTALS) s_tot[tid] = 0;
+  if (tid == 0) s_k = -1023;
+  tile_io io{a};
 
   for (;;) {
     if (tid == 0) s_tile = (int)atomicAdd(&a.ctr->next, 1ull);
     __syncthreads();
-    const int t = s_tile;
+    const int t = __builtin_amdgcn_readfirstlane(s_tile);
     if (t >= a.n_tiles) break; /* block-uniform */
     const mc_tile_k tile = a.tiles[t];
-    const mc_slab_k sl = a.slabs[tile.slab];
-    const int m = sl.m;
+    const mc_slab_k sl = a.slabs[__builtin_amdgcn_readfirstlane(tile.slab)];
     mc_layer_k L;
-    L.index_start = sl.index_start;
-    L.m = m;
-    L.dx = sl.dx;
-    L.min_weight = sl.min_weight;
+    L.index_start = __builtin_amdgcn_readfirstlane(sl.index_start);
+    L.m = __builtin_amdgcn_readfirstlane(sl.m);
+    L.dx = mc_uniform(sl.dx);
+    L.min_weight = mc_uniform(sl.min_weight);
+    const int m = L.m;
+    const int64_t cell_off = (int64_t)mc_readlane64((unsigned long long)sl.cell_off, 0);
     const bool lds_tally = m <= a.lds_tally_max_m; /* block-uniform */
     const bool lds_cells = m <= a.lds_cells_max_m; /* implies lds_tally */
-    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + (size_t)16 * m);
+    unsigned long long *t1 = t0 + m;
+    mc_cell *lc = reinterpret_cast<mc_cell *>(t1 + m);
+    const mc_cell *gc = a.cells + cell_off;
     if (lds_tally) {
       for (int c = tid; c < m; c += B) {
-        t_lds[c] = 0;
-        t_lds[m + c] = 0;
-        if (lds_cells) lc[c] = a.cells[sl.cell_off + c];
+        t0[c] = 0;
+        t1[c] = 0;
+        if (lds_cells) lc[c] = gc[c];
       }
     }
     if (tid == 0) s_next = (unsigned long long)tile.begin;
+    /* the tile's weights, from one history per thread (as the history kernel) */
+    if (tile.begin + tid < tile.end) atomicMax(&s_k, mc_ceil_log2(a.soa.wmc[tile.begin + tid]));
     __syncthreads();
 
-    if (lds_cells)
-      batch_tile<true, true, HI_COND>(a, tile, sl, L, t_lds, t_lds + m, lc, &s_next, s_tot, max_ev,
-                             refill_k, K, bl);
-    else if (lds_tally)
-      batch_tile<true, false, HI_COND>(a, tile, sl, L, t_lds, t_lds + m, a.cells + sl.cell_off, &s_next,
-                              s_tot, max_ev, refill_k, K, bl);
-    else
-      batch_tile<false, false, HI_COND>(a, tile, sl, L, a.fx + sl.cell_off,
-                               a.fx + a.total_cells + sl.cell_off, a.cells + sl.cell_off,
-                               &s_next, s_tot, max_ev, refill_k, K, bl);
+    const mc_walk_k K = mc_walk_live(L);
+    const mc_block_tally bt =
+        mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), B >> 6);
+    mc_tile_queue queue{&s_next, mc_readlane64((unsigned long long)tile.end, 0), false};
+    unsigned long long *fx_lo = a.fx + cell_off, *fx_hi = fx_lo + a.total_cells;
+    uint32_t *flags = a.flags + cell_off;
+    unsigned int *status = &a.ctr->status;
+    auto limbs = [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+      mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
+    };
+    const mc_mover mover{t0, t1, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every};
+    if (lds_tally && bt.limbs) {
+      if (lds_cells)
+        mc_walk_bank(io, queue, L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
+                     mover);
+      else
+        mc_walk_bank(io, queue, L, K, gc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
+                     mover);
+    } else if (lds_tally) { /* heavy weights */
+      mc_walk_bank(io, queue, L, K, gc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) mc_tally(t0, t1, flags, status, c, dw);
+                   },
+                   [](int) {});
+    } else {
+      mc_walk_bank(io, queue, L, K, gc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) mc_tally(fx_lo, fx_hi, flags, status, c, dw);
+                   },
+                   [](int) {});
+    }
 
     __syncthreads();
-    if (lds_tally) {
+    if (lds_tally && bt.limbs) {
+      mc_limbs_move(t0, t1, bt.S.L, m, tid, B, fx_lo, fx_hi);
+    } else if (lds_tally) {
       for (int c = tid; c < m; c += B) {
         mc_fx v;
-        v.lo = t_lds[c];
-        v.hi = t_lds[m + c];
-        if (v.lo | v.hi) /* cells the tile never reached add nothing */
-          mc_fx_atomic_add(&a.fx[sl.cell_off + c], &a.fx[a.total_cells + sl.cell_off + c], v);
+        v.lo = t0[c];
+        v.hi = t1[c];
+        mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], v);
       }
     }
+    if (tid == 0) s_k = -1023;
     __syncthreads();
   }
-
-  {
-    const unsigned long long e = mc_wave_sum(bl.ev_pending), cl = mc_wave_sum(bl.col_pending);
-    if (lane == 0) {
-      atomicAdd(&s_tot[0], e);
-      atomicAdd(&s_tot[1], cl);
-    }
-  }
-  if (bl.capped) atomicOr(&a.ctr->status, 1u);
-  __syncthreads();
-  if (tid == 0) {
-    atomicAdd(&a.ctr->events, s_tot[0]);
-    atomicAdd(&a.ctr->collisions, s_tot[1]);
-    atomicAdd(&a.ctr->n_left, s_tot[2]);
-    atomicAdd(&a.ctr->n_right, s_tot[3]);
-    atomicAdd(&a.ctr->n_killed, s_tot[4]);
-  }
+  /* the break follows a barrier after the last tile's totals */
+  if (tid == 0) mc_totals_out(s_tot, a.ctr);
 }
 
 __global__ void k_batch_setup(int64_t total, const double *sigs, const double *ar, mc_cell *cells,
@@ -249,25 +201,22 @@ int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, in
     return mc_fail(ctx, MCGPU_ERR_ARG, "block_size must be a multiple of 64 and <= 1024");
   mc_batched_shape sh;
   sh.block = block;
-  sh.refill = refill > 0 ? refill : 8;
+  sh.refill = refill > 0 ? refill : 0; /* 0: adaptive */
   /* LDS: the largest slab's tally plus its cross sections, as far as they fit
-     (128 B are left for the kernel's static LDS); slabs whose tally does not
-     fit add into the global tally directly */
-  const size_t budget = ctx->lds_per_block - 128;
-  sh.lds = std::min(budget, (size_t)32 * (size_t)std::max(max_m, 1));
-  sh.lds_cells_max_m = (int)(sh.lds / 32);
-  sh.lds_tally_max_m = (int)(sh.lds / 16);
+     (next to the absorbed-fraction rows and the kernel's static LDS); slabs
+     whose tally does not fit add into the global tally directly */
+  const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES;
+  const size_t lds = std::min(budget, (size_t)32 * (size_t)std::max(max_m, 1));
+  sh.lds = lds + MC_TAB_BYTES;
+  sh.lds_cells_max_m = (int)(lds / 32);
+  sh.lds_tally_max_m = (int)(lds / 16);
   if (sh.lds > 65536)
-  {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_batched<false>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_batched),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_batched<true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds);
-  }
   sh.grid = grid;
   if (sh.grid <= 0) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batched<false>, block, sh.lds) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batched, block, sh.lds) !=
             hipSuccess ||
         per_cu < 1)
       per_cu = 1;
@@ -281,7 +230,7 @@ int mc_launch_batched(mcgpu_context *ctx, const mc_batched_shape &sh, const mc_s
                       const mc_tile_k *tiles, int32_t n_tiles, const mcgpu_bank &bank,
                       const mc_cell *cells, unsigned long long *fx, int64_t total_cells,
                       uint32_t *flags, int8_t *result8, mc_counters *ctr, uint64_t max_events,
-                      bool small_weights, hipStream_t s) {
+                      hipStream_t s) {
   batch_args a;
   a.slabs = slabs;
   a.tiles = tiles;
@@ -296,10 +245,7 @@ int mc_launch_batched(mcgpu_context *ctx, const mc_batched_shape &sh, const mc_s
   a.result8 = result8;
   a.ctr = ctr;
   a.max_events = max_events;
-  if (small_weights)
-    hipLaunchKernelGGL(k_batched<true>, dim3(sh.grid), dim3(sh.block), sh.lds, s, a, sh.refill);
-  else
-    hipLaunchKernelGGL(k_batched<false>, dim3(sh.grid), dim3(sh.block), sh.lds, s, a, sh.refill);
+  hipLaunchKernelGGL(k_batched, dim3(sh.grid), dim3(sh.block), sh.lds, s, a, sh.refill);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
 }
@@ -341,17 +287,30 @@ int batch_tiles(mcgpu_batch *b) {
   mcgpu_context *ctx = b->ctx;
   const int ppl = b->opt.particles_per_lane > 0 ? b->opt.particles_per_lane : 16;
   const int64_t T = (int64_t)ppl * b->block;
+  /* automatic: at most 16 histories per lane, fewer where a slab's tiles would
+     be more than an eighth of a CU's share of the work (few or uneven slabs),
+     at least one (a block waits for its tile's longest history) */
+  double share = 0.0;
+  if (b->opt.particles_per_lane <= 0) {
+    for (const mcgpu_slab &h : b->host_slabs) share += (double)h.n * (h.max_index - h.min_index);
+    share /= 8.0 * ctx->num_cus;
+  }
   std::vector<mc_tile_k> tiles;
   std::vector<double> work;
   for (size_t s = 0; s < b->host_slabs.size(); ++s) {
     const mcgpu_slab &h = b->host_slabs[s];
     const int m = h.max_index - h.min_index;
-    for (int64_t p0 = 0; p0 < h.n; p0 += T) {
+    int64_t Ts = T;
+    if (share > 0.0) {
+      const double most = share / m;
+      if (most < (double)T) Ts = std::max<int64_t>(b->block, ((int64_t)most + 63) / 64 * 64);
+    }
+    for (int64_t p0 = 0; p0 < h.n; p0 += Ts) {
       mc_tile_k t;
       t.slab = (int32_t)s;
       t.pad_ = 0;
       t.begin = h.particle_offset + p0;
-      t.end = h.particle_offset + std::min(h.n, p0 + T);
+      t.end = h.particle_offset + std::min(h.n, p0 + Ts);
       tiles.push_back(t);
       work.push_back((double)(t.end - t.begin) * (double)m);
     }
@@ -383,7 +342,8 @@ int batch_capture(mcgpu_batch *b) {
   int rc = batch_tiles(b);
   if (rc) return rc;
   mc_batched_shape sh;
-  if ((rc = mc_batched_plan_shape(ctx, b->max_m, b->block, b->opt.grid_blocks, b->refill, &sh)))
+  if ((rc = mc_batched_plan_shape(ctx, b->max_m, b->block, b->opt.grid_blocks,
+                                  b->opt.events_per_refill, &sh)))
     return rc;
   b->lds = sh.lds;
   b->lds_cells_max_m = sh.lds_cells_max_m;
@@ -415,7 +375,7 @@ int batch_capture(mcgpu_batch *b) {
   MC_HIP(ctx, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   hipLaunchKernelGGL(k_batch_setup, dim3((unsigned)((tc + 255) / 256)), dim3(256), 0, b->stream,
                      tc, b->sigs, b->ar, b->d_cells, b->d_fx, b->d_flags, b->d_ctr);
-  hipLaunchKernelGGL(k_batched<false>, dim3(sh.grid), dim3(sh.block), sh.lds, b->stream, a,
+  hipLaunchKernelGGL(k_batched, dim3(sh.grid), dim3(sh.block), sh.lds, b->stream, a,
                      sh.refill);
   hipLaunchKernelGGL(k_batch_finalize, dim3((unsigned)((tc + 255) / 256)), dim3(256), 0,
                      b->stream, tc, (const unsigned long long *)b->d_fx,

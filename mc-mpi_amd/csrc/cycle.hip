@@ -495,7 +495,6 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
 
   /* the initial bank, host AoS -> device SoA */
   pool_guard init, work;
-  double wmax = k.nb_particles_create > 0 ? std::fabs(k.wmc) : 0.0;
   if (n0 > 0) {
     if ((rc = alloc_pool(ctx, n0, &init.p, nullptr))) return rc;
     std::vector<uint64_t> hs(n0);
@@ -508,7 +507,6 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
       hm[i] = q.mu;
       hw[i] = q.wmc;
       hi[i] = q.index;
-      wmax = std::max(wmax, std::fabs(q.wmc));
     }
     MC_HIP(ctx, hipMemcpyAsync(init.p.seed, hs.data(), 8 * n0, hipMemcpyHostToDevice, s));
     MC_HIP(ctx, hipMemcpyAsync(init.p.x, hx.data(), 8 * n0, hipMemcpyHostToDevice, s));
@@ -622,8 +620,7 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
     const mcgpu_bank bank{work.p.seed, work.p.x, work.p.mu, work.p.wmc, work.p.index};
     MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
     if ((rc = mc_launch_batched(ctx, sh, d_slabs, d_tiles, (int32_t)h_tiles.size(), bank, d_cells,
-                                d_fx, G * m, d_flags, nullptr, d_ctr, max_events,
-                                wmax < 0x1p-24, s)))
+                                d_fx, G * m, d_flags, nullptr, d_ctr, max_events, s)))
       return rc;
     MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
     hipLaunchKernelGGL(k_one_finalize, dim3(blocks_for(m, 256)), dim3(256), 0, s, m, G,
@@ -885,11 +882,6 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
     cap = new_cap;
     return MCGPU_OK;
   };
-  /* weights only decrease; when every initial one is below 2^-24 the
-     tally's high words only take carries (mc_launch_batched, small_weights) */
-  double wmax = 0.0;
-  for (int r = 0; r < R; ++r)
-    if (ranks[r].nb_particles_create > 0) wmax = std::max(wmax, std::fabs(ranks[r].wmc));
   {
     std::vector<int64_t> c0(R);
     for (int r = 0; r < R; ++r) c0[r] = need_of(r);
@@ -908,8 +900,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
         hm[i] = q.mu;
         hw[i] = q.wmc;
         hi[i] = q.index;
-        wmax = std::max(wmax, std::fabs(q.wmc));
-      }
+        }
       const int64_t b = base[r];
       MC_HIP(ctx, hipMemcpyAsync(pool.p.seed + b, hs.data(), 8 * n, hipMemcpyHostToDevice, s));
       MC_HIP(ctx, hipMemcpyAsync(pool.p.x + b, hx.data(), 8 * n, hipMemcpyHostToDevice, s));
@@ -1013,8 +1004,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
     MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
     if (n_tiles > 0 &&
         (rc = mc_launch_batched(ctx, sh, d_slabs, d_tiles, (int32_t)n_tiles, bank, d_cells, d_fx,
-                                tc, d_flags, pool.result8, d_ctr, max_events,
-                                wmax < 0x1p-24, s)))
+                                tc, d_flags, pool.result8, d_ctr, max_events, s)))
       return rc;
     MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
     hipLaunchKernelGGL(k_cyc_finalize, dim3(blocks_for(tc, 256)), dim3(256), 0, s, tc,

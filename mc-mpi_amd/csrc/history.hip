@@ -33,120 +33,35 @@
 
 namespace {
 
-constexpr size_t TAB_BYTES = 16 * MC_ABS_N; /* the absorbed-fraction rows in LDS */
-
-/* A wave's histories, one per lane.  tally(lanes, c, dw) adds deposits;
-   moves(k) is called before every (at most) k events per lane, k <= k_max. */
-template <bool SCORE, typename Tally, typename Moves>
-__device__ __forceinline__ void walk_bank(const mc_transport_args &a, const mc_cell *cells,
-                                          const double *g, const double2 *tab, int refill_k,
-                                          mc_queue q, const mc_walk_k &K,
-                                          unsigned long long *s_tot, int k_max, Tally tally,
-                                          Moves moves) {
-  mc_walk p;
-  p.s2 = 0;
-  p.x = p.mu = p.wmc = p.rh = p.rl = p.fe = p.fs = 0.0;
-  p.c = p.st = 0;
-  int64_t idx = 0;
-  bool has = false, capped = false;
-  mc_mask run = 0, pend = 0; /* lanes whose history goes on / waits for the general event */
-  uint64_t ev = 0;
-  uint32_t col = 0;
-  double score = 0.0;
-  unsigned long long tot_ev = 0, tot_col = 0, nl = 0, nr = 0, nk = 0;
-
-  /* events between refills: refill_k if positive, else adapted per wave
-     from the lanes found idle at each refill (many idle: the histories are
-     short against the interval, halve it; almost none: double it, since
-     each refill costs a queue atomic and a pass through this loop) */
-  const bool adapt = refill_k <= 0;
-  int kk = adapt ? 128 : refill_k;
-  int wait = 1;
-  /* wave-uniform bound on every lane's event count (a waiting event counted);
-     recomputed exactly (the largest in the wave) when an interval could reach
-     the cap, which then shortens the interval: no history passes the cap */
-  uint64_t ev_bound = 0;
-  for (;;) {
-    if (mc_queue_more(q)) { /* wave-uniform */
-      const mc_mask need = mc_lanes(!has);
-      if (adapt) {
-        const int idle = __popcll(need);
-        kk = idle > 16 ? (kk > 8 ? kk >> 1 : 8) : (idle < 4 ? (kk < 256 ? kk << 1 : 256) : kk);
-      }
-      if (need) {
-        const int64_t i = mc_queue_take(q, need, &a.ctr->next);
-        bool on = false;
-        if (!has && i >= 0) {
-          mc_state in;
-          load_state(a, i, in);
-          mc_walk_from(p, in, a.L);
-          idx = i;
-          has = true;
-          on = mc_walk_alive(p, a.L);
-          ev = 0;
-          col = 0;
-          score = 0.0;
-        }
-        run |= mc_lanes(on);
-      }
-    }
-    if (mc_lanes(has) == 0) break; /* wave-uniform */
-    int ki = kk < k_max ? kk : k_max - 1; /* a waiting lane may add one */
-    if (ev_bound + (uint64_t)ki >= a.max_events) {
-      ev_bound = mc_wave_max_u64(has ? ev + (mc_in(pend) ? 1u : 0u) : 0ull);
-      if (ev_bound + (uint64_t)ki >= a.max_events) ki = (int)(a.max_events - ev_bound);
-    }
-    ev_bound += (uint64_t)ki;
-    moves(ki + 1);
-    uint32_t ei = 0; /* events of this interval */
-    const int general =
-        mc_walk_many(p, run, pend, ki, wait, cells, tab, K, ei, col,
-                     [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-                       tally(lanes, c, dw);
-                       if (SCORE && mc_in(lanes)) score = score + g[c] * dw;
-                     });
-    wait = mc_walk_wait(wait, general, ki);
-    ev += ei;
-    const bool on = mc_in(run), waits = mc_in(pend);
-    if (has && !waits && (!on || ev >= a.max_events)) {
-      mc_state out;
-      mc_walk_to(out, p, a.L);
-      int code = mc_exit_code(out, a.L);
-      if (on) { /* runaway history stopped by the guard */
-        capped = true;
-        code = 2;
-      }
-      store_state(a, idx, out, code);
-      if (a.events) a.events[idx] = ev;
-      if (a.collisions) a.collisions[idx] = col;
-      if (SCORE) a.score[idx] = score;
-      tot_ev += ev;
-      tot_col += col;
-      nl += code == -1;
-      nr += code == 1;
-      nk += code == 0;
-      has = false;
-    }
-    run &= mc_lanes(has);
+template <bool SCORE> struct bank_io {
+  const mc_transport_args &a;
+  double score;
+  __device__ __forceinline__ void load(int64_t i, mc_state &p) {
+    load_state(a, i, p);
+    score = 0.0;
   }
-
-  mc_totals_wave(s_tot, tot_ev, tot_col, nl, nr, nk);
-  if (capped) atomicOr(&a.ctr->status, 1u);
-}
+  __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t ev,
+                                        uint32_t col) {
+    store_state(a, i, p, code);
+    if (a.events) a.events[i] = ev;
+    if (a.collisions) a.collisions[i] = col;
+    if (SCORE) a.score[i] = score;
+    return false;
+  }
+};
 
 template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE>
 __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refill_k,
                                                    int per_cu) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_k;
-  __shared__ unsigned long long s_tot[5];
+  __shared__ unsigned long long s_tot[MC_TOTALS];
   const mc_walk_k K = mc_walk_live(a.L);
-  const mc_queue q = mc_queue_open(a.n, per_cu);
+  mc_call_queue queue{mc_queue_open(a.n, per_cu), &a.ctr->next};
   const int m = a.L.m;
   double2 *tab = reinterpret_cast<double2 *>(smem);
-  for (int j = threadIdx.x; j < MC_ABS_N; j += blockDim.x)
-    tab[j] = make_double2(mc_abs_tab[j][0], mc_abs_tab[j][1]);
-  unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + TAB_BYTES), *t1 = t0 + m;
+  mc_tab_fill(tab);
+  unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES), *t1 = t0 + m;
   if (LDS_TALLY) {
     for (int c = threadIdx.x; c < m; c += blockDim.x) {
       t0[c] = 0;
@@ -156,78 +71,62 @@ __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refil
   const mc_cell *cells = a.cells;
   const double *g = a.g;
   if (LDS_CELLS) {
-    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + TAB_BYTES + (size_t)16 * m);
+    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + MC_TAB_BYTES + (size_t)16 * m);
     for (int c = threadIdx.x; c < m; c += blockDim.x) lc[c] = a.cells[c];
     cells = lc;
     if (SCORE) {
-      double *lg = reinterpret_cast<double *>(smem + TAB_BYTES + (size_t)32 * m);
+      double *lg = reinterpret_cast<double *>(smem + MC_TAB_BYTES + (size_t)32 * m);
       for (int c = threadIdx.x; c < m; c += blockDim.x) lg[c] = a.g[c];
       g = lg;
     }
   }
-  unsigned long long *fx_lo = a.fx, *fx_hi = a.fx + m;
-  uint32_t *flags = a.flags;
-  unsigned int *status = &a.ctr->status;
-  if (threadIdx.x < 5) s_tot[threadIdx.x] = 0;
-  mc_counters *ctr = a.ctr;
-  auto totals = [&]() { /* after a barrier */
-    if (threadIdx.x == 0)
-      mc_totals_block(s_tot, &ctr->events, &ctr->collisions, &ctr->n_left, &ctr->n_right,
-                      &ctr->n_killed);
-  };
-  if (!LDS_TALLY) {
-    __syncthreads();
-    walk_bank<SCORE>(a, cells, g, tab, refill_k, q, K, s_tot, 1 << 30,
-                     [&](mc_mask lanes, int c, double dw) {
-                       if (mc_in(lanes)) mc_tally(fx_lo, fx_hi, flags, status, c, dw);
-                     },
-                     [](int) {});
-    __syncthreads();
-    totals();
-    return;
-  }
-
+  if (threadIdx.x < MC_TOTALS) s_tot[threadIdx.x] = 0;
   /* the block's weights: the largest among the first histories of its waves
      (a guess that sets the limbs' range; heavier ones go to the global tally) */
   if (threadIdx.x == 0) s_k = -1023;
   __syncthreads();
-  {
-    const uint64_t i = q.next + __lane_id();
-    if (i < q.end) atomicMax(&s_k, mc_ceil_log2(a.aos ? a.aos[i].wmc : a.soa.wmc[i]));
+  if (LDS_TALLY) {
+    const uint64_t i = queue.q.next + __lane_id();
+    if (i < queue.q.end) atomicMax(&s_k, mc_ceil_log2(a.aos ? a.aos[i].wmc : a.soa.wmc[i]));
+    __syncthreads();
   }
-  __syncthreads();
-  const int waves = blockDim.x >> 6;
-  const mc_block_tally B = mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), waves);
-  if (B.limbs) { /* block-uniform */
-    int left = B.every;
-    walk_bank<SCORE>(a, cells, g, tab, refill_k, q, K, s_tot, B.every,
-                     [&](mc_mask lanes, int c, double dw) {
-                       mc_tally_limbs(t0, t1, B.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
-                     },
-                     [&](int k) {
-                       if (left < k) { /* wave-uniform */
-                         mc_limbs_move(t0, t1, B.S.L, m, __lane_id(), 64, fx_lo, fx_hi);
-                         left = B.every;
-                       }
-                       left -= k;
-                     });
+
+  bank_io<SCORE> io{a, 0.0};
+  unsigned long long *fx_lo = a.fx, *fx_hi = a.fx + m;
+  uint32_t *flags = a.flags;
+  unsigned int *status = &a.ctr->status;
+  const mc_block_tally B =
+      mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), blockDim.x >> 6);
+  if (LDS_TALLY && B.limbs) { /* block-uniform */
+    mc_walk_bank(io, queue, a.L, K, cells, tab, refill_k, B.every, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                   mc_tally_limbs(t0, t1, B.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
+                   if (SCORE && mc_in(lanes)) io.score = io.score + g[c] * dw;
+                 },
+                 mc_mover{t0, t1, fx_lo, fx_hi, m, B.S.L, B.every, B.every});
     __syncthreads();
     mc_limbs_move(t0, t1, B.S.L, m, threadIdx.x, blockDim.x, fx_lo, fx_hi);
   } else {
-    walk_bank<SCORE>(a, cells, g, tab, refill_k, q, K, s_tot, 1 << 30,
-                     [&](mc_mask lanes, int c, double dw) {
-                       if (mc_in(lanes)) mc_tally(t0, t1, flags, status, c, dw);
-                     },
-                     [](int) {});
+    unsigned long long *lo = LDS_TALLY ? t0 : fx_lo, *hi = LDS_TALLY ? t1 : fx_hi;
+    mc_walk_bank(io, queue, a.L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                   if (mc_in(lanes)) {
+                     mc_tally(lo, hi, flags, status, c, dw);
+                     if (SCORE) io.score = io.score + g[c] * dw;
+                   }
+                 },
+                 [](int) {});
     __syncthreads();
-    for (int c = threadIdx.x; c < m; c += blockDim.x) {
-      mc_fx v;
-      v.lo = t0[c];
-      v.hi = t1[c];
-      mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], v);
+    if (LDS_TALLY) {
+      for (int c = threadIdx.x; c < m; c += blockDim.x) {
+        mc_fx v;
+        v.lo = t0[c];
+        v.hi = t1[c];
+        mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], v);
+      }
     }
   }
-  totals(); /* the barrier after the walk stands before */
+  if (threadIdx.x == 0) mc_totals_out(s_tot, a.ctr);
 }
 
 template <bool T, bool C, bool S>
@@ -263,7 +162,7 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
 int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
                       hipStream_t s) {
   const size_t m = (size_t)a.L.m;
-  const size_t tally = 16 * m + TAB_BYTES, cells = sizeof(mc_cell) * m;
+  const size_t tally = 16 * m + MC_TAB_BYTES, cells = sizeof(mc_cell) * m;
   const size_t budget = ctx->lds_per_block - 256; /* the kernel's static LDS */
   const bool lds_tally = tally <= budget;
   if (a.score) { /* per-history score of a weighted tally (forward of the adjoint) */
@@ -272,10 +171,10 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
     const bool lds_cells = lds_tally && tally + cells + extra <= budget;
     if (lds_tally && lds_cells) return launch_one<true, true, true>(ctx, a, o, s, tally + cells + extra);
     if (lds_tally) return launch_one<true, false, true>(ctx, a, o, s, tally);
-    return launch_one<false, false, true>(ctx, a, o, s, TAB_BYTES);
+    return launch_one<false, false, true>(ctx, a, o, s, MC_TAB_BYTES);
   }
   const bool lds_cells = lds_tally && tally + cells <= budget;
   if (lds_tally && lds_cells) return launch_one<true, true, false>(ctx, a, o, s, tally + cells);
   if (lds_tally) return launch_one<true, false, false>(ctx, a, o, s, tally);
-  return launch_one<false, false, false>(ctx, a, o, s, TAB_BYTES);
+  return launch_one<false, false, false>(ctx, a, o, s, MC_TAB_BYTES);
 }

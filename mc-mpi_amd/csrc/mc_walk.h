@@ -27,7 +27,9 @@
 #ifndef MC_WALK_H
 #define MC_WALK_H
 
-#include "mc_device.h"
+#include "internal.h"
+
+constexpr size_t MC_TAB_BYTES = 16 * MC_ABS_N; /* the absorbed-fraction rows in LDS */
 
 struct mc_walk {
   uint64_t s2;    /* twice the RNG state (mod 2^64) */
@@ -103,6 +105,11 @@ __device__ __forceinline__ mc_walk_k mc_walk_live(const mc_layer_k &L) {
   asm volatile("" : "+s"(K.rem_max), "+s"(K.sure_max), "+s"(K.q_min), "+s"(K.three4));
   asm volatile("" : "+s"(K.dx), "+s"(K.min_weight), "+s"(K.m));
   return K;
+}
+
+/* a wave-uniform value read from memory, in scalar registers */
+__device__ __forceinline__ double mc_uniform(double v) {
+  return mc_asf64(mc_readlane64(mc_asu64(v), 0));
 }
 
 __device__ __forceinline__ uint32_t mc_hi32(double v) { return (uint32_t)(mc_asu64(v) >> 32); }
@@ -329,13 +336,10 @@ __device__ __forceinline__ mc_queue mc_queue_open(int64_t n, int per_cu) {
   return q;
 }
 
-/* whether the wave can still take histories */
 __device__ __forceinline__ bool mc_queue_more(const mc_queue &q) {
   return !q.dry || q.next < q.end;
 }
 
-/* a history for each lane of `need` (called by the whole wave): its index, or
-   -1 when none is left */
 __device__ __forceinline__ int64_t mc_queue_take(mc_queue &q, mc_mask need,
                                                  unsigned long long *counter) {
   const uint64_t cnt = (uint64_t)__popcll(need), have = q.end - q.next;
@@ -364,28 +368,145 @@ __device__ __forceinline__ int64_t mc_queue_take(mc_queue &q, mc_mask need,
   return (int64_t)i;
 }
 
-/* The call's totals: lanes to the wave's, to the block's (LDS words s_tot[5],
-   zeroed), to the counter block.  One global atomic per block and nonzero
-   total: with one per wave the five addresses of a full chip's 4,096 waves
-   alone took 0.14 ms. */
-__device__ __forceinline__ void mc_totals_wave(unsigned long long *s_tot, unsigned long long ev,
-                                               unsigned long long col, unsigned long long nl,
-                                               unsigned long long nr, unsigned long long nk) {
-  const unsigned long long v[5] = {mc_wave_sum(ev), mc_wave_sum(col), mc_wave_sum(nl),
-                                   mc_wave_sum(nr), mc_wave_sum(nk)};
-  if (__lane_id() == 0)
-    for (int i = 0; i < 5; ++i)
-      if (v[i]) atomicAdd(&s_tot[i], v[i]);
-}
+/* whether the wave can still take histories; a history for each lane of `need`
+   or -1 (called by the whole wave) */
+struct mc_call_queue {
+  mc_queue q;
+  unsigned long long *counter;
+  __device__ __forceinline__ bool more() const { return mc_queue_more(q); }
+  __device__ __forceinline__ int64_t take(mc_mask need) { return mc_queue_take(q, need, counter); }
+};
+
+/* the histories [.., end) of a block's tile, from its LDS counter */
+struct mc_tile_queue {
+  unsigned long long *counter; /* LDS */
+  uint64_t end;
+  bool dry;
+  __device__ __forceinline__ bool more() const { return !dry; }
+  __device__ __forceinline__ int64_t take(mc_mask need) {
+    const uint64_t cnt = (uint64_t)__popcll(need);
+    unsigned long long base = 0;
+    if (__lane_id() == 0) base = atomicAdd(counter, (unsigned long long)cnt);
+    base = mc_readlane64(base, 0);
+    dry = base + cnt >= end;
+    const uint64_t i = base + (uint64_t)mc_mbcnt64(need);
+    return i < end ? (int64_t)i : -1;
+  }
+};
+
+/* The block's totals, LDS words zeroed by the block: events, collisions, left,
+   right, killed; then whether a history hit the cap.  One global atomic per
+   block and nonzero total (mc_totals_out): with one per wave the five
+   addresses of a full chip's 4,096 waves alone took 0.14 ms. */
+constexpr int MC_TOTALS = 6;
 
 /* by one thread of the block, after a barrier */
-__device__ __forceinline__ void mc_totals_block(const unsigned long long *s_tot,
-                                                unsigned long long *ev, unsigned long long *col,
-                                                unsigned long long *nl, unsigned long long *nr,
-                                                unsigned long long *nk) {
-  unsigned long long *const to[5] = {ev, col, nl, nr, nk};
-  for (int i = 0; i < 5; ++i)
-    if (s_tot[i]) atomicAdd(to[i], s_tot[i]);
+__device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, mc_counters *ctr) {
+  if (s_tot[0]) atomicAdd(&ctr->events, s_tot[0]);
+  if (s_tot[1]) atomicAdd(&ctr->collisions, s_tot[1]);
+  if (s_tot[2]) atomicAdd(&ctr->n_left, s_tot[2]);
+  if (s_tot[3]) atomicAdd(&ctr->n_right, s_tot[3]);
+  if (s_tot[4]) atomicAdd(&ctr->n_killed, s_tot[4]);
+  if (s_tot[5]) atomicOr(&ctr->status, 1u);
+}
+
+/* A wave's histories, one per lane, until its queue is empty.
+   io.load(i, state) reads history i (and resets what the caller keeps per
+   lane); io.store(i, state, code, ev, col) takes a finished one and returns
+   whether the lane goes on with the state it leaves in `state` (a replay);
+   on_event as in mc_walk_many; moves(k) is called before every (at most) k
+   events per lane, k <= k_max.
+   refill_k: events between refills; 0: adapted per wave from the lanes found
+   idle at each refill (many idle: the histories are short against the
+   interval, halve it; almost none: double it, since each refill costs a pass
+   through this loop). */
+template <typename IO, typename Queue, typename Event, typename Moves>
+__device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_layer_k &L,
+                                             const mc_walk_k &K, const mc_cell *cells,
+                                             const double2 *tab, int refill_k, int k_max,
+                                             uint64_t max_events, unsigned long long *s_tot,
+                                             Event on_event, Moves moves) {
+  mc_walk p;
+  p.s2 = 0;
+  p.x = p.mu = p.wmc = p.rh = p.rl = p.fe = p.fs = 0.0;
+  p.c = p.st = 0;
+  int64_t idx = 0;
+  bool has = false;
+  mc_mask run = 0, pend = 0; /* lanes whose history goes on / waits for the general event */
+  uint64_t ev = 0;
+  uint32_t col = 0;
+  const bool adapt = refill_k <= 0;
+  int kk = adapt ? 128 : refill_k;
+  int wait = 1;
+  /* wave-uniform bound on every lane's event count (a waiting event counted);
+     recomputed exactly (the largest in the wave) when an interval could reach
+     the cap, which then shortens the interval: no history passes the cap */
+  uint64_t ev_bound = 0;
+  for (;;) {
+    if (queue.more()) { /* wave-uniform */
+      const mc_mask need = mc_lanes(!has);
+      if (adapt) {
+        const int idle = __popcll(need);
+        kk = idle > 16 ? (kk > 8 ? kk >> 1 : 8) : (idle < 4 ? (kk < 256 ? kk << 1 : 256) : kk);
+      }
+      if (need) {
+        const int64_t i = queue.take(need);
+        bool on = false;
+        if (!has && i >= 0) {
+          mc_state in;
+          io.load(i, in);
+          mc_walk_from(p, in, L);
+          idx = i;
+          has = true;
+          on = mc_walk_alive(p, L);
+          ev = 0;
+          col = 0;
+        }
+        run |= mc_lanes(on);
+      }
+    }
+    if (mc_lanes(has) == 0) break; /* wave-uniform */
+    int ki = kk < k_max ? kk : k_max - 1; /* a waiting lane may add one */
+    if (ev_bound + (uint64_t)ki >= max_events) {
+      ev_bound = mc_wave_max_u64(has ? ev + (mc_in(pend) ? 1u : 0u) : 0ull);
+      if (ev_bound + (uint64_t)ki >= max_events) ki = (int)(max_events - ev_bound);
+    }
+    ev_bound += (uint64_t)ki;
+    moves(ki + 1);
+    uint32_t ei = 0; /* events of this interval */
+    const int general = mc_walk_many(p, run, pend, ki, wait, cells, tab, K, ei, col, on_event);
+    wait = mc_walk_wait(wait, general, ki);
+    ev += ei;
+    const bool on = mc_in(run), waits = mc_in(pend);
+    const bool ends = has && !waits && (!on || ev >= max_events);
+    if (mc_lanes(ends) == 0) continue; /* wave-uniform */
+    bool again = false;
+    int code = 3;
+    if (ends) {
+      mc_state out;
+      mc_walk_to(out, p, L);
+      code = on ? 2 : mc_exit_code(out, L); /* on: a runaway history stopped by the guard */
+      atomicAdd(&s_tot[0], (unsigned long long)ev);
+      atomicAdd(&s_tot[1], (unsigned long long)col);
+      has = io.store(idx, out, code, ev, col);
+      if (has) {
+        mc_walk_from(p, out, L);
+        again = mc_walk_alive(p, L);
+        ev = 0;
+        col = 0;
+      }
+    }
+    const int nl = __popcll(mc_lanes(code == -1)), nr = __popcll(mc_lanes(code == 1)),
+              nk = __popcll(mc_lanes(code == 0));
+    const bool capped = mc_lanes(code == 2) != 0;
+    if (__lane_id() == 0) {
+      if (nl) atomicAdd(&s_tot[2], (unsigned long long)nl);
+      if (nr) atomicAdd(&s_tot[3], (unsigned long long)nr);
+      if (nk) atomicAdd(&s_tot[4], (unsigned long long)nk);
+      if (capped) atomicOr(&s_tot[5], 1ull);
+    }
+    run = (run & mc_lanes(has)) | mc_lanes(again);
+  }
 }
 
 /* ------------------------------------------------------------- block tally */
@@ -462,8 +583,27 @@ __device__ __forceinline__ void mc_limbs_move(unsigned long long *t0, unsigned l
                                               unsigned long long *fx_hi) {
   for (int c = first; c < m; c += step) {
     const uint64_t n0 = atomicExch(&t0[c], 0ull), n1 = atomicExch(&t1[c], 0ull);
-    mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx_limbs(n0, n1, L));
+    if (n0 | n1) mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx_limbs(n0, n1, L));
   }
 }
+
+/* the rows of mc_abs_tab into LDS (all threads of the block; then a barrier) */
+__device__ __forceinline__ void mc_tab_fill(double2 *tab) {
+  for (int j = threadIdx.x; j < MC_ABS_N; j += blockDim.x)
+    tab[j] = make_double2(mc_abs_tab[j][0], mc_abs_tab[j][1]);
+}
+
+/* The moves(k) of a limb tally: whole tables of m cells, by this wave. */
+struct mc_mover {
+  unsigned long long *t0, *t1, *fx_lo, *fx_hi;
+  int m, L, every, left;
+  __device__ __forceinline__ void operator()(int k) {
+    if (left < k) { /* wave-uniform */
+      mc_limbs_move(t0, t1, L, m, __lane_id(), 64, fx_lo, fx_hi);
+      left = every;
+    }
+    left -= k;
+  }
+};
 
 #endif /* MC_WALK_H */
