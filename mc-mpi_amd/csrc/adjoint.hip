@@ -20,7 +20,7 @@
  * When T_h was not stored, each lane first replays the history once to
  * compute it, then replays it again for the gradient.
  */
-#include "internal.h"
+#include "mc_adjoint.h"
 
 namespace {
 
@@ -37,23 +37,35 @@ struct adj_args {
   uint64_t max_events;
 };
 
-template <bool LDS, bool HAVE_SCORE>
-__global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k) {
+/* LDS_T: the two limb tallies in LDS; LDS_C: the cells and target weights too */
+template <bool LDS_T, bool LDS_C, bool HAVE_SCORE>
+__global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int per_cu) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const mc_coef K = mc_coef_live();
+  __shared__ int s_k, s_g;
+  __shared__ unsigned long long s_tot[MC_TOTALS];
+  const mc_walk_k K = mc_walk_live(a.L);
+  mc_call_queue queue{mc_queue_open(a.n, per_cu), &a.ctr->next};
   const int m = a.L.m;
-  unsigned long long *tl = a.fx; /* 4m words */
+  double2 *tab = reinterpret_cast<double2 *>(smem);
+  mc_tab_fill(tab);
+  mc_grad_tally G;
+  G.t = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES);
+  G.fx = a.fx;
+  G.stride = m;
+  G.flags_a = a.flags;
+  G.flags_i = a.flags + m;
+  G.status = &a.ctr->status;
+  G.m = m;
   const mc_cell *cells = a.cells;
   const double *g = a.g;
-  if (LDS) {
-    tl = reinterpret_cast<unsigned long long *>(smem);
-    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + 32 * (size_t)m);
-    double *lg = reinterpret_cast<double *>(smem + 48 * (size_t)m);
+  if (threadIdx.x < MC_TOTALS) s_tot[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_k = s_g = -1023;
+  if (LDS_T)
+    for (int c = threadIdx.x; c < 4 * m; c += blockDim.x) G.t[c] = 0;
+  if (LDS_C) {
+    mc_cell *lc = reinterpret_cast<mc_cell *>(G.t + 4 * m);
+    double *lg = reinterpret_cast<double *>(lc + m);
     for (int c = threadIdx.x; c < m; c += blockDim.x) {
-      tl[c] = 0;
-      tl[m + c] = 0;
-      tl[2 * m + c] = 0;
-      tl[3 * m + c] = 0;
       lc[c] = a.cells[c];
       lg[c] = a.g[c];
     }
@@ -61,118 +73,42 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k) {
     g = lg;
   }
   __syncthreads();
-
-  const int lane = __lane_id();
-  const uint32_t max_ev = a.max_events > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)a.max_events;
-  mc_state p;
-  p.index = 0;
-  int64_t idx = 0;
-  bool has = false, done = false, capped = false;
-  int phase = 1;       /* 0: score replay, 1: gradient replay */
-  uint32_t ev = 0;
-  double T = 0.0, P = 0.0;
-  unsigned long long tot_ev = 0;
-
-  /* events between refills: refill_k if positive, else adapted per wave as
-     in the history kernel (halved when many lanes were idle at a refill,
-     doubled when almost none were) */
-  const bool adapt = refill_k <= 0;
-  int kk = adapt ? 128 : refill_k;
-  for (;;) {
-    if (!done) {
-      const unsigned long long need = __ballot(!has);
-      if (adapt) {
-        const int idle = __popcll(need);
-        kk = idle > 16 ? (kk > 8 ? kk >> 1 : 8) : (idle < 4 ? (kk < 256 ? kk << 1 : 256) : kk);
-      }
-      if (need) {
-        const int cnt = __popcll(need);
-        const int leader = __ffsll((long long)need) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(&a.ctr->next, (unsigned long long)cnt);
-        base = mc_readlane64(base, leader);
-        if (!has) {
-          const int64_t i = (int64_t)(base + (unsigned long long)mc_mbcnt64(need));
-          if (i < a.n) {
-            p.seed = a.init.seed[i];
-            p.x = a.init.x[i];
-            p.mu = a.init.mu[i];
-            mc_refresh_rcp(p);
-            p.wmc = a.init.wmc[i];
-            p.index = a.init.index[i];
-            idx = i;
-            has = true;
-            ev = 0;
-            P = 0.0;
-            if (HAVE_SCORE) {
-              T = a.score[i];
-              phase = 1;
-            } else {
-              T = 0.0;
-              phase = 0;
-            }
-          }
-        }
-        if (base + (unsigned long long)cnt >= (unsigned long long)a.n) done = true;
-      }
-    }
-    if (__ballot(has) == 0) break;
-    if (has) {
-      for (int k = 0; k < kk; ++k) {
-        if (!mc_alive(p, a.L) || ev >= max_ev) break;
-        const int c = p.index - a.L.index_start;
-        mc_cell cell;
-        bool coll;
-        double di;
-        const double dw = mc_event<true>(p, cells, c, a.L.dx, K, coll, di, &cell);
-        ++ev;
-        if (!HAVE_SCORE && phase == 0) {
-          T = T + g[c] * dw;
-          continue;
-        }
-        const double gc = g[c];
-        double term_a, term_i;
-        const bool has_i = mc_adjoint_terms(cell, coll, di, dw, gc, p.wmc, T, P, term_a, term_i);
-        mc_tally<true>(tl, tl + m, a.flags, &a.ctr->status, c, term_a);
-        if (has_i) mc_tally<true>(tl + 2 * m, tl + 3 * m, a.flags + m, &a.ctr->status, c, term_i);
-        P = P + gc * dw;
-      }
-      const bool alive = mc_alive(p, a.L);
-      if (!alive || ev >= max_ev) {
-        if (alive) capped = true;
-        tot_ev += ev;
-        if (!HAVE_SCORE && phase == 0 && !alive) {
-          /* score known: replay the same history for the gradient */
-          p.seed = a.init.seed[idx];
-          p.x = a.init.x[idx];
-          p.mu = a.init.mu[idx];
-          mc_refresh_rcp(p);
-          p.wmc = a.init.wmc[idx];
-          p.index = a.init.index[idx];
-          ev = 0;
-          P = 0.0;
-          phase = 1;
-        } else {
-          has = false;
-        }
-      }
-    }
-  }
-
-  tot_ev = mc_wave_sum(tot_ev);
-  if (lane == 0) atomicAdd(&a.ctr->events, tot_ev);
-  if (capped) atomicOr(&a.ctr->status, 1u);
-  if (LDS) {
-    __syncthreads();
+  if (LDS_T) { /* the split: the largest target weight, the first histories' weights */
+    int kg = -1023;
     for (int c = threadIdx.x; c < m; c += blockDim.x) {
-      mc_fx v;
-      v.lo = tl[c];
-      v.hi = tl[m + c];
-      mc_fx_atomic_add(&a.fx[c], &a.fx[m + c], v);
-      v.lo = tl[2 * m + c];
-      v.hi = tl[3 * m + c];
-      mc_fx_atomic_add(&a.fx[2 * m + c], &a.fx[3 * m + c], v);
+      const int k = mc_ceil_log2(g[c]);
+      kg = k > kg ? k : kg;
     }
+    atomicMax(&s_g, kg);
+    const uint64_t i = queue.q.next + __lane_id();
+    if (i < queue.q.end) atomicMax(&s_k, mc_ceil_log2(a.init.wmc[i]));
+    __syncthreads();
+  }
+  const bool limbs =
+      mc_grad_split(G, __builtin_amdgcn_readfirstlane(s_k + s_g), blockDim.x >> 6);
+
+  mc_grad_io<HAVE_SCORE> io{a.init, a.score, 0.0, 0.0, 1};
+  if (LDS_T && limbs) { /* block-uniform */
+    mc_walk_bank(io, queue, a.L, K, cells, tab, refill_k, G.every, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+                     double wmc) {
+                   mc_grad_event<MC_GRAD_LIMBS>(io, G, g, lanes, c, cell, coll, di, dw, wmc);
+                 },
+                 mc_grad_mover{G, G.every});
+  } else {
+    constexpr int MODE = LDS_T ? MC_GRAD_CARRY : MC_GRAD_GLOBAL;
+    mc_walk_bank(io, queue, a.L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+                     double wmc) {
+                   mc_grad_event<MODE>(io, G, g, lanes, c, cell, coll, di, dw, wmc);
+                 },
+                 [](int) {});
+  }
+  __syncthreads();
+  if (LDS_T) mc_grad_move(G, threadIdx.x, blockDim.x, limbs);
+  if (threadIdx.x == 0) { /* this call counts events alone */
+    s_tot[1] = s_tot[2] = s_tot[3] = s_tot[4] = 0;
+    mc_totals_out(s_tot, a.ctr);
   }
 }
 
@@ -248,10 +184,10 @@ int cells_setup(mcgpu_context *ctx, int m, const double *sig_a, const double *si
   return MCGPU_OK;
 }
 
-template <bool LDS, bool S>
+template <bool T, bool C, bool S>
 int launch_adj(mcgpu_context *ctx, const adj_args &a, const mcgpu_options &o, hipStream_t s,
                size_t lds) {
-  auto kern = k_adjoint<LDS, S>;
+  auto kern = k_adjoint<T, C, S>;
   if (lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -268,13 +204,24 @@ int launch_adj(mcgpu_context *ctx, const adj_args &a, const mcgpu_options &o, hi
   int grid = o.grid_blocks;
   if (grid <= 0) {
     grid = per_cu * ctx->num_cus;
-    const int64_t blocks_needed = (a.n + block - 1) / block;
-    if (blocks_needed < grid) grid = (int)(blocks_needed > 0 ? blocks_needed : 1);
+    if (a.n < grid) grid = (int)(a.n > 0 ? a.n : 1); /* a block per history at most */
   }
   const int k = o.events_per_refill > 0 ? o.events_per_refill : 0; /* 0: adaptive */
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k, per_cu);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
+}
+
+/* the two tallies, cells and target weights in LDS when they fit, else the
+   tallies, else nothing */
+template <bool S>
+int launch_adj_fit(mcgpu_context *ctx, const adj_args &a, const mcgpu_options &o, hipStream_t s) {
+  const size_t m = (size_t)a.L.m, budget = ctx->lds_per_block - 256;
+  if (MC_TAB_BYTES + 56 * m <= budget)
+    return launch_adj<true, true, S>(ctx, a, o, s, MC_TAB_BYTES + 56 * m);
+  if (MC_TAB_BYTES + 32 * m <= budget)
+    return launch_adj<true, false, S>(ctx, a, o, s, MC_TAB_BYTES + 32 * m);
+  return launch_adj<false, false, S>(ctx, a, o, s, MC_TAB_BYTES);
 }
 
 } // namespace
@@ -367,14 +314,9 @@ int mcgpu_adjoint_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *initial
   a.flags = (uint32_t *)ctx->flags;
   a.ctr = (mc_counters *)ctx->counters;
   a.max_events = o.max_events_per_history ? o.max_events_per_history : (1ULL << 27);
-  const size_t lds = 56 * (size_t)m; /* two tallies, cells, target weights */
-  const bool in_lds = lds <= ctx->lds_per_block;
   MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
   if (n > 0) {
-    if (history_score)
-      rc = in_lds ? launch_adj<true, true>(ctx, a, o, s, lds) : launch_adj<false, true>(ctx, a, o, s, 0);
-    else
-      rc = in_lds ? launch_adj<true, false>(ctx, a, o, s, lds) : launch_adj<false, false>(ctx, a, o, s, 0);
+    rc = history_score ? launch_adj_fit<true>(ctx, a, o, s) : launch_adj_fit<false>(ctx, a, o, s);
     if (rc) return rc;
   }
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));

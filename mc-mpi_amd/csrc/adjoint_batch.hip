@@ -20,7 +20,7 @@
 #include <algorithm>
 #include <vector>
 
-#include "internal.h"
+#include "mc_adjoint.h"
 
 namespace {
 
@@ -61,342 +61,219 @@ struct bcell_args {
 __device__ __forceinline__ int next_tile(mc_counters *ctr, int *s_tile) {
   if (threadIdx.x == 0) *s_tile = (int)atomicAdd(&ctr->next, 1ull);
   __syncthreads();
-  return *s_tile;
+  return __builtin_amdgcn_readfirstlane(*s_tile);
 }
 
-/* Per-lane counters of one block, carried across its tiles. */
-struct blane {
-  bool capped;
-  unsigned long long ev, col;
+/* a tile and its slab, every field wave-uniform */
+struct btile {
+  mc_layer_k L;
+  int64_t cell_off;
+  uint64_t begin, end;
 };
 
-/* One tile of the forward: its histories, lanes refilled from the LDS queue
-   s_next.  Called with LDS or global accumulator/cell pointers from two
-   places, so each inlined copy uses the matching memory instructions. */
-template <bool SCORE>
-__device__ __forceinline__ void fwd_tile(const bcell_args &a, const btile_k &tile,
-                                         const bslab_k &sl, const mc_layer_k &L,
-                                         unsigned long long *t_lo, unsigned long long *t_hi,
-                                         const mc_cell *cells, const double *g,
-                                         unsigned long long *s_next, unsigned long long *s_tot,
-                                         uint32_t max_ev, int refill_k, const mc_coef &K,
-                                         blane &bl) {
-  const int lane = __lane_id();
-  mc_state p;
-  p.index = 0;
-  int64_t idx = 0;
-  bool has = false, done = false;
-  uint32_t ev = 0, col = 0;
-  double score = 0.0;
-  for (;;) {
-    if (!done) {
-      const unsigned long long need = __ballot(!has);
-      if (need) {
-        const int cnt = __popcll(need);
-        const int leader = __ffsll((long long)need) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(s_next, (unsigned long long)cnt);
-        base = mc_readlane64(base, leader);
-        if (!has) {
-          const int64_t i = (int64_t)(base + (unsigned long long)mc_mbcnt64(need));
-          if (i < tile.end) {
-            p.seed = a.bank.seed[i];
-            p.x = a.bank.x[i];
-            p.mu = a.bank.mu[i];
-            mc_refresh_rcp(p);
-            p.wmc = a.bank.wmc[i];
-            p.index = a.bank.index[i];
-            idx = i;
-            has = true;
-            ev = 0;
-            col = 0;
-            score = 0.0;
-          }
-        }
-        if (base + (unsigned long long)cnt >= (unsigned long long)tile.end) done = true;
-      }
-    }
-    if (__ballot(has) == 0) break;
-    if (has) {
-      for (int k = 0; k < refill_k; ++k) {
-        if (!mc_alive(p, L) || ev >= max_ev) break;
-        const int c = p.index - L.index_start;
-        bool coll;
-        double di;
-        const double dw = mc_event<true>(p, cells, c, L.dx, K, coll, di);
-        ++ev;
-        col += coll ? 1u : 0u;
-        mc_tally(t_lo, t_hi, a.flags + sl.cell_off, &a.ctr->status, c, dw);
-        if (SCORE) score = score + g[c] * dw;
-      }
-      const bool alive = mc_alive(p, L);
-      if (!alive || ev >= max_ev) {
-        int code = mc_exit_code(p, L);
-        if (alive) {
-          bl.capped = true;
-          code = 2;
-        }
-        a.bank.seed[idx] = p.seed;
-        a.bank.x[idx] = p.x;
-        a.bank.mu[idx] = p.mu;
-        a.bank.wmc[idx] = p.wmc;
-        a.bank.index[idx] = p.index;
-        if (a.result8) a.result8[idx] = (int8_t)code;
-        if (SCORE) a.score_out[idx] = score;
-        bl.ev += ev;
-        bl.col += col;
-        atomicAdd(&s_tot[code == -1 ? 2 : (code == 1 ? 3 : 4)], code == 2 ? 0ull : 1ull);
-        has = false;
-      }
-    }
-  }
+__device__ __forceinline__ btile read_tile(const bcell_args &a, int t) {
+  const btile_k tile = a.tiles[t];
+  const bslab_k sl = a.slabs[__builtin_amdgcn_readfirstlane(tile.slab)];
+  btile b;
+  b.L.index_start = __builtin_amdgcn_readfirstlane(sl.index_start);
+  b.L.m = __builtin_amdgcn_readfirstlane(sl.m);
+  b.L.dx = mc_uniform(sl.dx);
+  b.L.min_weight = mc_uniform(sl.min_weight);
+  b.cell_off = (int64_t)mc_readlane64((unsigned long long)sl.cell_off, 0);
+  b.begin = mc_readlane64((unsigned long long)tile.begin, 0);
+  b.end = mc_readlane64((unsigned long long)tile.end, 0);
+  return b;
 }
 
-/* Forward: mcgpu_forward_cells per slab (history kernel arithmetic). */
+template <bool SCORE> struct fwd_io {
+  const bcell_args &a;
+  double score;
+  __device__ __forceinline__ void load(int64_t i, mc_state &p) {
+    p.seed = a.bank.seed[i];
+    p.x = a.bank.x[i];
+    p.mu = a.bank.mu[i];
+    p.wmc = a.bank.wmc[i];
+    p.index = a.bank.index[i];
+    score = 0.0;
+  }
+  __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t, uint32_t) {
+    a.bank.seed[i] = p.seed;
+    a.bank.x[i] = p.x;
+    a.bank.mu[i] = p.mu;
+    a.bank.wmc[i] = p.wmc;
+    a.bank.index[i] = p.index;
+    if (a.result8) a.result8[i] = (int8_t)code;
+    if (SCORE) a.score_out[i] = score;
+    return false;
+  }
+};
+
+/* Forward: mcgpu_forward_cells per slab.  Per tile as the batched transport
+   (k_batched), with each history's score. */
 template <bool SCORE>
 __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const mc_coef K = mc_coef_live();
-  __shared__ int s_tile;
+  __shared__ int s_tile, s_k;
   __shared__ unsigned long long s_next;
-  __shared__ unsigned long long s_tot[5];
-  const int lane = __lane_id();
+  __shared__ unsigned long long s_tot[MC_TOTALS];
   const int B = blockDim.x, tid = threadIdx.x;
-  if (tid < 5) s_tot[tid] = 0;
-  blane bl;
-  bl.capped = false;
-  bl.ev = bl.col = 0;
-  const uint32_t max_ev = a.max_events > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)a.max_events;
-  unsigned long long *t_lds = reinterpret_cast<unsigned long long *>(smem);
+  if (tid < MC_TOTALS) s_tot[tid] = 0;
+  if (tid == 0) s_k = -1023;
+  double2 *tab = reinterpret_cast<double2 *>(smem);
+  mc_tab_fill(tab);
+  unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES);
+  fwd_io<SCORE> io{a, 0.0};
 
   for (;;) {
     const int t = next_tile(a.ctr, &s_tile);
     if (t >= a.n_tiles) break;
-    const btile_k tile = a.tiles[t];
-    const bslab_k sl = a.slabs[tile.slab];
-    const int m = sl.m;
-    mc_layer_k L;
-    L.index_start = sl.index_start;
-    L.m = m;
-    L.dx = sl.dx;
-    L.min_weight = sl.min_weight;
+    const btile b = read_tile(a, t);
+    const int m = b.L.m;
     const bool in_lds = m <= a.lds_max_m; /* block-uniform */
-    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + (size_t)16 * m);
-    double *lg = reinterpret_cast<double *>(smem + (size_t)32 * m);
+    unsigned long long *t1 = t0 + m;
+    mc_cell *lc = reinterpret_cast<mc_cell *>(t1 + m);
+    double *lg = reinterpret_cast<double *>(lc + m);
     if (in_lds) {
       for (int c = tid; c < m; c += B) {
-        t_lds[c] = 0;
-        t_lds[m + c] = 0;
-        lc[c] = a.cells[sl.cell_off + c];
-        if (SCORE) lg[c] = a.g[sl.cell_off + c];
+        t0[c] = 0;
+        t1[c] = 0;
+        lc[c] = a.cells[b.cell_off + c];
+        if (SCORE) lg[c] = a.g[b.cell_off + c];
       }
     }
-    if (tid == 0) s_next = (unsigned long long)tile.begin;
+    if (tid == 0) s_next = b.begin;
+    if (b.begin + tid < b.end) atomicMax(&s_k, mc_ceil_log2(a.bank.wmc[b.begin + tid]));
     __syncthreads();
 
-    if (in_lds)
-      fwd_tile<SCORE>(a, tile, sl, L, t_lds, t_lds + m, lc, lg, &s_next, s_tot, max_ev,
-                      refill_k, K, bl);
-    else
-      fwd_tile<SCORE>(a, tile, sl, L, a.fx + sl.cell_off, a.fx + a.total + sl.cell_off,
-                      a.cells + sl.cell_off, a.g ? a.g + sl.cell_off : nullptr, &s_next, s_tot,
-                      max_ev, refill_k, K, bl);
-
+    const mc_walk_k K = mc_walk_live(b.L);
+    const mc_block_tally bt = mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), B >> 6);
+    mc_tile_queue queue{&s_next, b.end, false};
+    unsigned long long *fx_lo = a.fx + b.cell_off, *fx_hi = fx_lo + a.total;
+    uint32_t *flags = a.flags + b.cell_off;
+    unsigned int *status = &a.ctr->status;
+    const double *gg = SCORE ? a.g + b.cell_off : nullptr;
+    if (in_lds && bt.limbs) {
+      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
+                     if (SCORE && mc_in(lanes)) io.score = io.score + lg[c] * dw;
+                   },
+                   mc_mover{t0, t1, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every});
+    } else if (in_lds) { /* weights too heavy for the limbs */
+      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) {
+                       mc_tally(t0, t1, flags, status, c, dw);
+                       if (SCORE) io.score = io.score + lg[c] * dw;
+                     }
+                   },
+                   [](int) {});
+    } else {
+      mc_walk_bank(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
+                   s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) {
+                       mc_tally(fx_lo, fx_hi, flags, status, c, dw);
+                       if (SCORE) io.score = io.score + gg[c] * dw;
+                     }
+                   },
+                   [](int) {});
+    }
     __syncthreads();
     if (in_lds) {
-      for (int c = tid; c < m; c += B) {
-        mc_fx v;
-        v.lo = t_lds[c];
-        v.hi = t_lds[m + c];
-        mc_fx_atomic_add(&a.fx[sl.cell_off + c], &a.fx[a.total + sl.cell_off + c], v);
-      }
+      if (bt.limbs)
+        mc_limbs_move(t0, t1, bt.S.L, m, tid, B, fx_lo, fx_hi);
+      else
+        for (int c = tid; c < m; c += B)
+          mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx{t0[c], t1[c]});
     }
+    if (tid == 0) s_k = -1023;
     __syncthreads();
   }
-
-  {
-    const unsigned long long e = mc_wave_sum(bl.ev), cl = mc_wave_sum(bl.col);
-    if (lane == 0) {
-      atomicAdd(&s_tot[0], e);
-      atomicAdd(&s_tot[1], cl);
-    }
-  }
-  if (bl.capped) atomicOr(&a.ctr->status, 1u);
-  __syncthreads();
-  if (tid == 0) {
-    atomicAdd(&a.ctr->events, s_tot[0]);
-    atomicAdd(&a.ctr->collisions, s_tot[1]);
-    atomicAdd(&a.ctr->n_left, s_tot[2]);
-    atomicAdd(&a.ctr->n_right, s_tot[3]);
-    atomicAdd(&a.ctr->n_killed, s_tot[4]);
-  }
-}
-
-/* One tile of the adjoint (replay from the initial bank); pointers as in
-   fwd_tile. */
-template <bool HAVE_SCORE>
-__device__ __forceinline__ void adj_tile(const bcell_args &a, const btile_k &tile,
-                                         const bslab_k &sl, const mc_layer_k &L,
-                                         unsigned long long *ga_lo, unsigned long long *ga_hi,
-                                         unsigned long long *gi_lo, unsigned long long *gi_hi,
-                                         const mc_cell *cells, const double *g,
-                                         unsigned long long *s_next, uint32_t max_ev,
-                                         int refill_k, const mc_coef &K, blane &bl) {
-  const int lane = __lane_id();
-  uint32_t *fa = a.flags + sl.cell_off, *fi = a.flags + a.total + sl.cell_off;
-  mc_state p;
-  p.index = 0;
-  int64_t idx = 0;
-  bool has = false, done = false;
-  int phase = 1; /* 0: score replay, 1: gradient replay */
-  uint32_t ev = 0;
-  double T = 0.0, P = 0.0;
-  for (;;) {
-    if (!done) {
-      const unsigned long long need = __ballot(!has);
-      if (need) {
-        const int cnt = __popcll(need);
-        const int leader = __ffsll((long long)need) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(s_next, (unsigned long long)cnt);
-        base = mc_readlane64(base, leader);
-        if (!has) {
-          const int64_t i = (int64_t)(base + (unsigned long long)mc_mbcnt64(need));
-          if (i < tile.end) {
-            p.seed = a.bank.seed[i];
-            p.x = a.bank.x[i];
-            p.mu = a.bank.mu[i];
-            mc_refresh_rcp(p);
-            p.wmc = a.bank.wmc[i];
-            p.index = a.bank.index[i];
-            idx = i;
-            has = true;
-            ev = 0;
-            P = 0.0;
-            if (HAVE_SCORE) {
-              T = a.score_in[i];
-              phase = 1;
-            } else {
-              T = 0.0;
-              phase = 0;
-            }
-          }
-        }
-        if (base + (unsigned long long)cnt >= (unsigned long long)tile.end) done = true;
-      }
-    }
-    if (__ballot(has) == 0) break;
-    if (has) {
-      for (int k = 0; k < refill_k; ++k) {
-        if (!mc_alive(p, L) || ev >= max_ev) break;
-        const int c = p.index - L.index_start;
-        mc_cell cell;
-        bool coll;
-        double di;
-        const double dw = mc_event<true>(p, cells, c, L.dx, K, coll, di, &cell);
-        ++ev;
-        if (!HAVE_SCORE && phase == 0) {
-          T = T + g[c] * dw;
-          continue;
-        }
-        const double gc = g[c];
-        double term_a, term_i;
-        const bool has_i = mc_adjoint_terms(cell, coll, di, dw, gc, p.wmc, T, P, term_a, term_i);
-        mc_tally<true>(ga_lo, ga_hi, fa, &a.ctr->status, c, term_a);
-        if (has_i) mc_tally<true>(gi_lo, gi_hi, fi, &a.ctr->status, c, term_i);
-        P = P + gc * dw;
-      }
-      const bool alive = mc_alive(p, L);
-      if (!alive || ev >= max_ev) {
-        if (alive) bl.capped = true;
-        bl.ev += ev;
-        if (!HAVE_SCORE && phase == 0 && !alive) {
-          p.seed = a.bank.seed[idx];
-          p.x = a.bank.x[idx];
-          p.mu = a.bank.mu[idx];
-          mc_refresh_rcp(p);
-          p.wmc = a.bank.wmc[idx];
-          p.index = a.bank.index[idx];
-          ev = 0;
-          P = 0.0;
-          phase = 1;
-        } else {
-          has = false;
-        }
-      }
-    }
-  }
+  if (tid == 0) mc_totals_out(s_tot, a.ctr);
 }
 
 /* Adjoint: mcgpu_adjoint_cells per slab (replay from the initial bank). */
 template <bool HAVE_SCORE>
 __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const mc_coef K = mc_coef_live();
-  __shared__ int s_tile;
+  __shared__ int s_tile, s_k, s_g;
   __shared__ unsigned long long s_next;
-  const int lane = __lane_id();
+  __shared__ unsigned long long s_tot[MC_TOTALS];
   const int B = blockDim.x, tid = threadIdx.x;
-  blane bl;
-  bl.capped = false;
-  bl.ev = bl.col = 0;
-  const uint32_t max_ev = a.max_events > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)a.max_events;
-  const int64_t T4 = a.total;
-  unsigned long long *w_lds = reinterpret_cast<unsigned long long *>(smem);
+  if (tid < MC_TOTALS) s_tot[tid] = 0;
+  if (tid == 0) s_k = s_g = -1023;
+  double2 *tab = reinterpret_cast<double2 *>(smem);
+  mc_tab_fill(tab);
+  mc_grad_tally G;
+  G.t = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES);
+  G.stride = a.total;
+  G.status = &a.ctr->status;
+  mc_grad_io<HAVE_SCORE> io{a.bank, a.score_in, 0.0, 0.0, 1};
 
   for (;;) {
     const int t = next_tile(a.ctr, &s_tile);
     if (t >= a.n_tiles) break;
-    const btile_k tile = a.tiles[t];
-    const bslab_k sl = a.slabs[tile.slab];
-    const int m = sl.m;
-    mc_layer_k L;
-    L.index_start = sl.index_start;
-    L.m = m;
-    L.dx = sl.dx;
-    L.min_weight = sl.min_weight;
+    const btile b = read_tile(a, t);
+    const int m = b.L.m;
     const bool in_lds = m <= a.lds_max_m; /* block-uniform */
-    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + (size_t)32 * m);
-    double *lg = reinterpret_cast<double *>(smem + (size_t)48 * m);
+    mc_cell *lc = reinterpret_cast<mc_cell *>(G.t + 4 * m);
+    double *lg = reinterpret_cast<double *>(lc + m);
+    const double *gg = a.g + b.cell_off;
+    G.fx = a.fx + b.cell_off;
+    G.flags_a = a.flags + b.cell_off;
+    G.flags_i = a.flags + a.total + b.cell_off;
+    G.m = m;
     if (in_lds) {
+      int kg = -1023;
       for (int c = tid; c < m; c += B) {
-        w_lds[c] = 0;
-        w_lds[m + c] = 0;
-        w_lds[2 * m + c] = 0;
-        w_lds[3 * m + c] = 0;
-        lc[c] = a.cells[sl.cell_off + c];
-        lg[c] = a.g[sl.cell_off + c];
+        for (int w = 0; w < 4; ++w) G.t[w * m + c] = 0;
+        lc[c] = a.cells[b.cell_off + c];
+        const double v = gg[c];
+        lg[c] = v;
+        const int k = mc_ceil_log2(v);
+        kg = k > kg ? k : kg;
       }
+      atomicMax(&s_g, kg);
     }
-    if (tid == 0) s_next = (unsigned long long)tile.begin;
+    if (tid == 0) s_next = b.begin;
+    if (b.begin + tid < b.end) atomicMax(&s_k, mc_ceil_log2(a.bank.wmc[b.begin + tid]));
     __syncthreads();
 
-    if (in_lds)
-      adj_tile<HAVE_SCORE>(a, tile, sl, L, w_lds, w_lds + m, w_lds + 2 * m, w_lds + 3 * m, lc, lg,
-                           &s_next, max_ev, refill_k, K, bl);
+    const mc_walk_k K = mc_walk_live(b.L);
+    const bool limbs = mc_grad_split(G, __builtin_amdgcn_readfirstlane(s_k + s_g), B >> 6);
+    mc_tile_queue queue{&s_next, b.end, false};
+    if (in_lds && limbs)
+      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, G.every, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+                       double wmc) {
+                     mc_grad_event<MC_GRAD_LIMBS>(io, G, lg, lanes, c, cell, coll, di, dw, wmc);
+                   },
+                   mc_grad_mover{G, G.every});
+    else if (in_lds)
+      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+                       double wmc) {
+                     mc_grad_event<MC_GRAD_CARRY>(io, G, lg, lanes, c, cell, coll, di, dw, wmc);
+                   },
+                   [](int) {});
     else
-      adj_tile<HAVE_SCORE>(a, tile, sl, L, a.fx + sl.cell_off, a.fx + T4 + sl.cell_off,
-                           a.fx + 2 * T4 + sl.cell_off, a.fx + 3 * T4 + sl.cell_off,
-                           a.cells + sl.cell_off, a.g + sl.cell_off, &s_next, max_ev, refill_k,
-                           K, bl);
-
+      mc_walk_bank(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
+                   s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+                       double wmc) {
+                     mc_grad_event<MC_GRAD_GLOBAL>(io, G, gg, lanes, c, cell, coll, di, dw, wmc);
+                   },
+                   [](int) {});
     __syncthreads();
-    if (in_lds) {
-      for (int c = tid; c < m; c += B) {
-        mc_fx v;
-        v.lo = w_lds[c];
-        v.hi = w_lds[m + c];
-        mc_fx_atomic_add(&a.fx[sl.cell_off + c], &a.fx[T4 + sl.cell_off + c], v);
-        v.lo = w_lds[2 * m + c];
-        v.hi = w_lds[3 * m + c];
-        mc_fx_atomic_add(&a.fx[2 * T4 + sl.cell_off + c], &a.fx[3 * T4 + sl.cell_off + c], v);
-      }
-    }
+    if (in_lds) mc_grad_move(G, tid, B, limbs);
+    if (tid == 0) s_k = s_g = -1023;
     __syncthreads();
   }
-  const unsigned long long e = mc_wave_sum(bl.ev);
-  if (lane == 0) atomicAdd(&a.ctr->events, e);
-  if (bl.capped) atomicOr(&a.ctr->status, 1u);
+  if (tid == 0) { /* this call counts events alone */
+    s_tot[1] = s_tot[2] = s_tot[3] = s_tot[4] = 0;
+    mc_totals_out(s_tot, a.ctr);
+  }
 }
 
 /* cells from (sig_a, sig_i); zeroed accumulators (words per cell) and counters */
@@ -435,13 +312,18 @@ __global__ void k_batch_cells_finalize(int64_t total, const unsigned long long *
 /* Validates the slab table and builds the device slab and tile tables in
    ctx->tables; returns the largest slab's cell count in *max_m. */
 int build_tables(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
-                 int64_t total_cells, int64_t tile_size, const bslab_k **d_slabs,
+                 int64_t total_cells, int ppl, int block, int grid, const bslab_k **d_slabs,
                  const btile_k **d_tiles, int32_t *n_tiles, int *max_m, int64_t *max_particle) {
   std::vector<bslab_k> ks(n_slabs);
   std::vector<btile_k> tiles;
   std::vector<double> work;
   *max_m = 0;
   *max_particle = 0;
+  const int64_t most = (int64_t)(ppl > 0 ? ppl : 16) * block;
+  double share = 0.0; /* automatic: at most 16 histories per lane (mc_tile_size) */
+  if (ppl <= 0)
+    for (int s = 0; s < n_slabs; ++s)
+      share += (double)slabs[s].n * ((double)slabs[s].max_index - slabs[s].min_index) / grid;
   for (int s = 0; s < n_slabs; ++s) {
     const mcgpu_slab &h = slabs[s];
     const int m = h.max_index - h.min_index;
@@ -455,6 +337,7 @@ int build_tables(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
     ks[s].cell_off = h.cell_offset;
     *max_m = std::max(*max_m, m);
     *max_particle = std::max(*max_particle, h.particle_offset + h.n);
+    const int64_t tile_size = ppl > 0 ? most : mc_tile_size(most, share, h.n, m, block);
     for (int64_t p0 = 0; p0 < h.n; p0 += tile_size) {
       btile_k t;
       t.slab = s;
@@ -506,46 +389,51 @@ int read_batch_counters(mcgpu_context *ctx, hipStream_t s, mcgpu_stats *stats) {
   return MCGPU_OK;
 }
 
+/* o's block, grid and refill as batch_prepare set them */
 template <typename K>
 int launch_persistent(mcgpu_context *ctx, K kern, const bcell_args &a, const mcgpu_options &o,
                       size_t lds, hipStream_t s) {
-  if (lds > 65536)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  const int block = o.block_size > 0 ? o.block_size : 1024;
-  int grid = o.grid_blocks;
-  if (grid <= 0) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, lds) != hipSuccess ||
-        per_cu < 1)
-      per_cu = 1;
-    grid = per_cu * ctx->num_cus;
-  }
-  const int k = o.events_per_refill > 0 ? o.events_per_refill : 8;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k);
+  hipLaunchKernelGGL(kern, dim3(o.grid_blocks), dim3(o.block_size), lds, s, a, o.events_per_refill);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
 }
 
-/* Common set-up of both batched calls: options, tables, cells, accumulators,
-   LDS size.  fx_words / flag_words: accumulator words per cell. */
-int batch_prepare(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
+/* Common set-up of both batched calls: options and launch shape of `kern`,
+   tables, cells, accumulators, LDS size.  fx_words / flag_words: accumulator
+   words per cell. */
+template <typename K>
+int batch_prepare(mcgpu_context *ctx, K kern, int32_t n_slabs, const mcgpu_slab *slabs,
                   int64_t total_cells, const mcgpu_bank *bank, const double *sig_a,
                   const double *sig_i, int fx_words, int flag_words, size_t lds_bytes_per_cell,
                   const mcgpu_options *opt, hipStream_t s, mcgpu_options *o, bcell_args *a,
                   size_t *lds) {
   mcgpu_default_options(o);
   if (opt) *o = *opt;
-  const int block = o->block_size > 0 ? o->block_size : 1024;
-  if (block > 1024 || block % 64)
+  if (o->block_size > 1024 || o->block_size % 64)
     return mc_fail(ctx, MCGPU_ERR_ARG, "block_size must be a multiple of 64 and <= 1024");
-  o->block_size = block;
-  const int ppl = o->particles_per_lane > 0 ? o->particles_per_lane : 16;
   memset(a, 0, sizeof *a);
   int max_m = 0;
+  for (int s_ = 0; s_ < n_slabs; ++s_)
+    max_m = std::max(max_m, slabs[s_].max_index - slabs[s_].min_index);
+  /* LDS for the largest slab that fits; larger slabs use the global accumulators */
+  const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES; /* and the static LDS */
+  a->lds_max_m = (int)std::min<size_t>((size_t)max_m, budget / lds_bytes_per_cell);
+  *lds = MC_TAB_BYTES + lds_bytes_per_cell * (size_t)a->lds_max_m;
+  if (*lds > 65536)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds);
+  int per_cu = 0;
+  if (o->block_size <= 0)
+    o->block_size = mc_auto_block(kern, *lds, &per_cu);
+  else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, o->block_size, *lds) !=
+               hipSuccess || per_cu < 1)
+    per_cu = 1;
+  const int block = o->block_size;
+  if (o->grid_blocks <= 0) o->grid_blocks = per_cu * ctx->num_cus;
+  if (o->events_per_refill < 0) o->events_per_refill = 0; /* 0: adaptive */
   int64_t max_particle = 0;
-  int rc = build_tables(ctx, n_slabs, slabs, total_cells, (int64_t)ppl * block, &a->slabs,
-                        &a->tiles, &a->n_tiles, &max_m, &max_particle);
+  int rc = build_tables(ctx, n_slabs, slabs, total_cells, o->particles_per_lane, block,
+                        o->grid_blocks, &a->slabs, &a->tiles, &a->n_tiles, &max_m, &max_particle);
   if (rc) return rc;
   if (max_particle > 0 && (!bank->seed || !bank->x || !bank->mu || !bank->wmc || !bank->index))
     return mc_fail(ctx, MCGPU_ERR_ARG, "batch: bank has a null array");
@@ -559,11 +447,6 @@ int batch_prepare(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
                      (unsigned long long *)ctx->fx, fx_words, (uint32_t *)ctx->flags, flag_words,
                      (mc_counters *)ctx->counters);
   MC_HIP(ctx, hipGetLastError());
-  /* LDS for the largest slab that fits; larger slabs use the global accumulators */
-  const size_t budget = ctx->lds_per_block - 128; /* the kernels' static LDS */
-  int lds_max_m = (int)std::min<size_t>((size_t)max_m, budget / lds_bytes_per_cell);
-  *lds = lds_bytes_per_cell * (size_t)lds_max_m;
-  a->lds_max_m = lds_max_m;
   a->bank = *bank;
   a->cells = (const mc_cell *)ctx->cells;
   a->fx = (unsigned long long *)ctx->fx;
@@ -594,7 +477,8 @@ int mcgpu_forward_cells_batch(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_s
   bcell_args a;
   size_t lds = 0;
   const bool score = history_score != nullptr;
-  int rc = batch_prepare(ctx, n_slabs, slabs, total_cells, bank, sig_a, sig_i, 2, 1,
+  const auto kern = score ? k_forward_cells_batch<true> : k_forward_cells_batch<false>;
+  int rc = batch_prepare(ctx, kern, n_slabs, slabs, total_cells, bank, sig_a, sig_i, 2, 1,
                          score ? 40 : 32, opt, s, &o, &a, &lds);
   if (rc) return rc;
   a.g = g;
@@ -602,8 +486,7 @@ int mcgpu_forward_cells_batch(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_s
   a.result8 = result;
   MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
   if (a.n_tiles > 0) {
-    rc = score ? launch_persistent(ctx, k_forward_cells_batch<true>, a, o, lds, s)
-               : launch_persistent(ctx, k_forward_cells_batch<false>, a, o, lds, s);
+    rc = launch_persistent(ctx, kern, a, o, lds, s);
     if (rc) return rc;
   }
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
@@ -630,15 +513,15 @@ int mcgpu_adjoint_cells_batch(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_s
   mcgpu_options o;
   bcell_args a;
   size_t lds = 0;
-  int rc = batch_prepare(ctx, n_slabs, slabs, total_cells, initial, sig_a, sig_i, 4, 2, 56, opt,
+  const auto kern = history_score ? k_adjoint_cells_batch<true> : k_adjoint_cells_batch<false>;
+  int rc = batch_prepare(ctx, kern, n_slabs, slabs, total_cells, initial, sig_a, sig_i, 4, 2, 56, opt,
                          s, &o, &a, &lds);
   if (rc) return rc;
   a.g = g;
   a.score_in = history_score;
   MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
   if (a.n_tiles > 0) {
-    rc = history_score ? launch_persistent(ctx, k_adjoint_cells_batch<true>, a, o, lds, s)
-                       : launch_persistent(ctx, k_adjoint_cells_batch<false>, a, o, lds, s);
+    rc = launch_persistent(ctx, kern, a, o, lds, s);
     if (rc) return rc;
   }
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));

@@ -21,8 +21,8 @@
  * The event is the common step of mc_walk.h; what bounds a launch besides it
  * is the tiles: a block waits for its tile's longest history, and few large
  * tiles leave CUs idle.  Measured, 512 slabs of 32 to 8,192 cells with 100 to
- * 1e5 histories each: 110.0 -> 72.5 ms with mc_walk.h and tiles cut to an
- * eighth of a CU's share.
+ * 1e5 histories each: 110.0 -> 50.2 ms with mc_walk.h and the tile sizes of
+ * mc_tile_size.
  */
 #include <algorithm>
 #include <vector>
@@ -197,10 +197,9 @@ __global__ void k_batch_finalize(int64_t total, const unsigned long long *fx,
 
 int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, int refill,
                           mc_batched_shape *out) {
-  if (block > 1024 || block < 64 || block % 64)
+  if (block > 1024 || block < 0 || block % 64)
     return mc_fail(ctx, MCGPU_ERR_ARG, "block_size must be a multiple of 64 and <= 1024");
   mc_batched_shape sh;
-  sh.block = block;
   sh.refill = refill > 0 ? refill : 0; /* 0: adaptive */
   /* LDS: the largest slab's tally plus its cross sections, as far as they fit
      (next to the absorbed-fraction rows and the kernel's static LDS); slabs
@@ -213,9 +212,11 @@ int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, in
   if (sh.lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_batched),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds);
+  int per_cu = 0;
+  if (block == 0) block = mc_auto_block(k_batched, sh.lds, &per_cu);
+  sh.block = block;
   sh.grid = grid;
   if (sh.grid <= 0) {
-    int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batched, block, sh.lds) !=
             hipSuccess ||
         per_cu < 1)
@@ -287,24 +288,16 @@ int batch_tiles(mcgpu_batch *b) {
   mcgpu_context *ctx = b->ctx;
   const int ppl = b->opt.particles_per_lane > 0 ? b->opt.particles_per_lane : 16;
   const int64_t T = (int64_t)ppl * b->block;
-  /* automatic: at most 16 histories per lane, fewer where a slab's tiles would
-     be more than an eighth of a CU's share of the work (few or uneven slabs),
-     at least one (a block waits for its tile's longest history) */
-  double share = 0.0;
-  if (b->opt.particles_per_lane <= 0) {
-    for (const mcgpu_slab &h : b->host_slabs) share += (double)h.n * (h.max_index - h.min_index);
-    share /= 8.0 * ctx->num_cus;
-  }
+  double share = 0.0; /* automatic: at most 16 histories per lane (mc_tile_size) */
+  if (b->opt.particles_per_lane <= 0)
+    for (const mcgpu_slab &h : b->host_slabs)
+      share += (double)h.n * (h.max_index - h.min_index) / b->grid;
   std::vector<mc_tile_k> tiles;
   std::vector<double> work;
   for (size_t s = 0; s < b->host_slabs.size(); ++s) {
     const mcgpu_slab &h = b->host_slabs[s];
     const int m = h.max_index - h.min_index;
-    int64_t Ts = T;
-    if (share > 0.0) {
-      const double most = share / m;
-      if (most < (double)T) Ts = std::max<int64_t>(b->block, ((int64_t)most + 63) / 64 * 64);
-    }
+    const int64_t Ts = b->opt.particles_per_lane > 0 ? T : mc_tile_size(T, share, h.n, m, b->block);
     for (int64_t p0 = 0; p0 < h.n; p0 += Ts) {
       mc_tile_k t;
       t.slab = (int32_t)s;
@@ -335,20 +328,18 @@ int batch_tiles(mcgpu_batch *b) {
 
 int batch_capture(mcgpu_batch *b) {
   mcgpu_context *ctx = b->ctx;
-  b->block = b->opt.block_size > 0 ? b->opt.block_size : 1024;
-  if (b->block > 1024 || b->block % 64)
-    return mc_fail(ctx, MCGPU_ERR_ARG, "block_size must be a multiple of 64 and <= 1024");
   b->refill = b->opt.events_per_refill > 0 ? b->opt.events_per_refill : 8;
-  int rc = batch_tiles(b);
-  if (rc) return rc;
+  int rc;
   mc_batched_shape sh;
-  if ((rc = mc_batched_plan_shape(ctx, b->max_m, b->block, b->opt.grid_blocks,
-                                  b->opt.events_per_refill, &sh)))
+  if ((rc = mc_batched_plan_shape(ctx, b->max_m, b->opt.block_size > 0 ? b->opt.block_size : 0,
+                                  b->opt.grid_blocks, b->opt.events_per_refill, &sh)))
     return rc;
+  b->block = sh.block;
   b->lds = sh.lds;
   b->lds_cells_max_m = sh.lds_cells_max_m;
   b->lds_tally_max_m = sh.lds_tally_max_m;
   b->grid = sh.grid;
+  if ((rc = batch_tiles(b))) return rc;
   if (b->exec) {
     (void)hipGraphExecDestroy(b->exec);
     b->exec = nullptr;

@@ -199,8 +199,26 @@ struct mc_batched_shape {
   int lds_tally_max_m; /* slabs with m <= this keep their tally in LDS */
 };
 
-/* Launch shape for slabs of up to max_m cells; grid <= 0 takes resident
-   blocks per CU x CUs. */
+/* Histories of a tile of a slab of n histories and m cells: n in equal tiles
+   of at most `most`, or, when `share` (a block's part of all slabs' histories
+   x cells) is given, of at most half of it (few or uneven slabs), though of at
+   least one history per thread of the block.  A block waits for its tile's
+   longest history, several times the mean one, so many small tiles cost more
+   than they balance: forward and adjoint of 64 slabs of 50,000 histories on
+   1,000 cells took 34.7 ms in tiles of 16,384, 50.5 ms at an eighth of a
+   block's part (1,600) and 31.6 ms at a half; 512 slabs of 32 to 8,192 cells
+   72.5 ms at an eighth and 50.2 ms at a half. */
+inline int64_t mc_tile_size(int64_t most, double share, int64_t n, int m, int block) {
+  double fit = (double)most;
+  if (share > 0.0 && share / (2.0 * m) < fit) fit = share / (2.0 * m);
+  if (fit < (double)block) fit = (double)block;
+  const int64_t tiles = (int64_t)((double)n / fit) + ((double)n / fit > (int64_t)((double)n / fit));
+  if (tiles <= 1) return n > 0 ? n : 1;
+  return ((n + tiles - 1) / tiles + 63) / 64 * 64;
+}
+
+/* Launch shape for slabs of up to max_m cells; block 0 takes the size with
+   the most resident waves, grid <= 0 resident blocks per CU x CUs. */
 int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, int refill,
                           mc_batched_shape *out);
 /* One launch over n_tiles tiles; fx / flags / ctr must be zeroed first

@@ -227,4 +227,33 @@ MC_FN_HD mc_fx mc_fx_limbs(uint64_t n0, uint64_t n1, int L) {
   return r;
 }
 
+/* Terms of either sign (the gradients'): |v| < 2^V, limb 1 signed, so half as
+   many terms.  Rounding as in mc_fx_from_double_general: the magnitude half
+   up.  (Most terms are zero: callers skip those before the test.) */
+MC_FN_HD int mc_fx_split_signed_log2_terms(int V) {
+  const int L = 44 + (V >> 1);
+  return 64 - L < L - V - 25 ? 64 - L : L - V - 25;
+}
+
+MC_FN_HD int mc_fx_split_signed_direct(double v, const mc_fx_split *S) {
+  uint64_t b;
+  __builtin_memcpy(&b, &v, 8);
+  return ((uint32_t)(b >> 32) & 0x7FFFFFFFu) - MC_FX_HI36 < S->range;
+}
+
+MC_FN_HD int mc_fx_split_signed_small(double *v) {
+  double a = __builtin_fabs(*v);
+  if (!mc_fx_split_small(&a)) return 0;
+  *v = __builtin_copysign(a, *v);
+  return 1;
+}
+
+MC_FN_HD mc_fx mc_fx_signed_limbs(uint64_t n0, uint64_t n1, int L) {
+  mc_fx r;
+  r.lo = (n1 << L) + n0;
+  r.hi = (uint64_t)((int64_t)n1 >> (64 - L)) + (uint64_t)((int64_t)n0 >> 63) +
+         (r.lo < n0 ? 1u : 0u);
+  return r;
+}
+
 #endif /* MC_FX_H */

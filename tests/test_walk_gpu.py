@@ -74,3 +74,61 @@ def test_runs_from_the_counter(ctx, oracle, n):
     """More histories than the first runs hold: few blocks, many later runs."""
     _say(f"n={n}, later runs")
     _check(ctx, oracle, 25, n, n, 1.0, 1e-2, grid_blocks=3, block_size=64)
+
+
+def _gradient(ctx, oracle, m, n, seed, wscale, gscale, with_score, batched):
+    """Forward with scores and adjoint against the oracle, one slab (or the
+    slab twice in a batch): scores, tally and both gradients, bit for bit."""
+    import mcgpu
+    import torch
+    rng = np.random.default_rng(seed)
+    sa, ss = rng.lognormal(0, 0.5, m), rng.lognormal(0, 0.5, m)
+    ss[::7] = 5e-5  # not sampled there: no sig_i term
+    _, _, dx, bank = _case(m, n, seed, wscale * rng.uniform(0.5, 1.0, n))
+    g = gscale * rng.uniform(-1, 1, m) * (rng.random(m) < 0.3)
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+    zeros = lambda k: torch.zeros(k, dtype=torch.float64, device="cuda")  # noqa: E731
+    min_w = 1e-3 * wscale
+    o = oracle.forward_cells(0, m, dx, min_w, sa, ss, bank, g=g)
+    oa, oi = oracle.adjoint_cells(0, m, dx, min_w, sa, ss, bank, g,
+                                  score=o["score"] if with_score else None)
+    k = 2 if batched else 1
+    rep = lambda x: dev(np.tile(x, k))  # noqa: E731
+    init = mcgpu.bank_to_device(np.tile(bank, k))
+    work = {f: v.clone() for f, v in init.items()}
+    w, ga, gi = zeros(k * m), zeros(k * m), zeros(k * m)
+    score = torch.empty(k * n, dtype=torch.float64, device="cuda")
+    if batched:
+        slabs = [(0, m, dx, min_w, s * m, s * n, n) for s in range(k)]
+        ctx.forward_cells_batch(slabs, work, rep(sa), rep(ss), w, g=rep(g), history_score=score)
+        ctx.adjoint_cells_batch(slabs, init, rep(sa), rep(ss), rep(g), ga, gi,
+                                history_score=score if with_score else None)
+    else:
+        ctx.forward_cells(work, dev(sa), dev(ss), w, 0, m, dx, min_w, g=dev(g),
+                          history_score=score)
+        ctx.adjoint_cells(init, dev(sa), dev(ss), 0, m, dx, min_w, dev(g), ga, gi,
+                          history_score=score if with_score else None)
+    same = lambda t, x: np.array_equal(t.cpu().numpy().view(np.uint64),  # noqa: E731
+                                       np.tile(x, k).view(np.uint64))
+    assert same(score, o["score"])
+    assert same(w, o["tally_exact"])
+    assert same(ga, oa) and same(gi, oi)
+    assert oa.any() and oi.any()
+
+
+@pytest.mark.parametrize("batched", [False, True])
+@pytest.mark.parametrize("wscale,gscale", [(1.0, 1e-9), (1.0, 20.0), (1.0, 1e4), (1e-8, 1.0),
+                                           (1e3, 1.0)])
+def test_gradient_terms_of_every_scale(ctx, oracle, wscale, gscale, batched):
+    _say(f"gradient, weights {wscale} targets {gscale} batched={batched}")
+    _gradient(ctx, oracle, 90, 500, 3, wscale, gscale, True, batched)
+
+
+@pytest.mark.parametrize("with_score", [True, False])
+@pytest.mark.parametrize("m,batched", [(2890, False), (2900, False), (5100, False), (2880, True),
+                                       (4100, True)])
+def test_gradient_layers_around_the_lds_limits(ctx, oracle, m, batched, with_score):
+    """Cells, targets and tallies in LDS (56 B a cell); the tallies alone
+    (32 B, one slab); neither."""
+    _say(f"gradient, m={m} batched={batched} with_score={with_score}")
+    _gradient(ctx, oracle, m, 120, m, 1.0, 1.0, with_score, batched)

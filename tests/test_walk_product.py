@@ -43,6 +43,21 @@ void pw_limbs(const double *v, long n, int V, uint64_t *out, int8_t *taken, uint
     out[2 * i + 1] = r.hi;
   }
 }
+void pw_signed_limbs(const double *v, long n, int V, uint64_t *out, int8_t *taken, uint64_t *n0s,
+                     uint64_t *n1s) {
+  const mc_fx_split S = mc_fx_split_for(V);
+  for (long i = 0; i < n; ++i) {
+    double x = v[i];
+    taken[i] = mc_fx_split_signed_direct(x, &S) ? 1 : (mc_fx_split_signed_small(&x) ? 2 : 0);
+    out[2 * i] = out[2 * i + 1] = n0s[i] = n1s[i] = 0;
+    if (!taken[i]) continue;
+    mc_fx_split_limbs(x, &S, &n0s[i], &n1s[i]);
+    const mc_fx r = mc_fx_signed_limbs(n0s[i], n1s[i], S.L);
+    out[2 * i] = r.lo;
+    out[2 * i + 1] = r.hi;
+  }
+}
+int pw_signed_log2_terms(int V) { return mc_fx_split_signed_log2_terms(V); }
 int pw_L(int V) { return mc_fx_split_for(V).L; }
 int pw_log2_terms(int V) { return mc_fx_split_log2_terms(V); }
 void pw_join(const uint64_t *n0, const uint64_t *n1, long n, int L, uint64_t *out) {
@@ -67,7 +82,7 @@ def pw(tmp_path_factory):
     L = C.CDLL(str(so))
     p, n, i = C.c_void_p, C.c_long, C.c_int
     L.pw_absorb.argtypes = [p, n, i, p, p]
-    L.pw_limbs.argtypes = [p, n, i, p, p, p, p]
+    L.pw_limbs.argtypes = L.pw_signed_limbs.argtypes = [p, n, i, p, p, p, p]
     L.pw_join.argtypes = [p, p, n, i, p]
     return L
 
@@ -145,6 +160,33 @@ def test_limbs_equal_the_fixed_point_term(pw, oracle, V):
     assert n1[t].max() <= 2 ** max(V + 88 - L, 52 - L)
     lg = pw.pw_log2_terms(V)
     assert lg + L - 1 <= 63 and lg + V + 88 - L <= 64
+
+
+@pytest.mark.parametrize("V", [-30, -3, 0, 2, 5])
+def test_signed_limbs_equal_the_fixed_point_term(pw, oracle, V):
+    """The same for terms of either sign (the gradients')."""
+    rng = np.random.default_rng(25)
+    p2 = np.ldexp(1.0, np.arange(-1074, 42))
+    v = np.concatenate([p2, np.nextafter(p2, 0), np.nextafter(p2, np.inf), p2 * 1.5,
+                        rng.uniform(1, 2, 400_000) * np.ldexp(1.0, rng.integers(-95, V + 2, 400_000)),
+                        (2 * rng.integers(0, 2 ** 51, 200_000) + 1) * np.ldexp(
+                            0.5 ** 88, -rng.integers(0, 52, 200_000)) * 0.5, [np.inf, np.nan]])
+    v = np.concatenate([v, -v])
+    n = len(v)
+    out, n0, n1 = np.zeros(2 * n, np.uint64), np.zeros(n, np.uint64), np.zeros(n, np.uint64)
+    taken = np.zeros(n, np.int8)
+    pw.pw_signed_limbs(v.ctypes.data, n, V, out.ctypes.data, taken.ctypes.data, n0.ctypes.data,
+                       n1.ctypes.data)
+    a = np.abs(v)
+    t = taken != 0
+    assert np.array_equal(t, (a == 0) | ((a >= 2.0 ** -88) & (a < max(2.0 ** V, 2.0 ** -36))))
+    want, fl = oracle.fx_convert(v)
+    assert not fl[t].any()
+    assert np.array_equal(out.reshape(-1, 2)[t], want.reshape(-1, 2)[t])
+    L, lg = pw.pw_L(V), pw.pw_signed_log2_terms(V)
+    assert np.abs(n0[t].view(np.int64)).max() <= 2 ** (L - 1)
+    assert np.abs(n1[t].view(np.int64)).max() <= 2 ** max(V + 88 - L, 52 - L)
+    assert lg + L - 1 <= 63 and lg + V + 88 - L <= 63
 
 
 def test_limb_sums_join_with_borrow_and_carry(pw):
