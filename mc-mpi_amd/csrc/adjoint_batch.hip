@@ -88,13 +88,15 @@ __device__ __forceinline__ btile read_tile(const bcell_args &a, int t) {
 template <bool SCORE> struct fwd_io {
   const bcell_args &a;
   double score;
-  __device__ __forceinline__ void load(int64_t i, mc_state &p) {
+  static constexpr bool RESUMES = false;
+  __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
     p.seed = a.bank.seed[i];
     p.x = a.bank.x[i];
     p.mu = a.bank.mu[i];
     p.wmc = a.bank.wmc[i];
     p.index = a.bank.index[i];
     score = 0.0;
+    return 0;
   }
   __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t, uint32_t) {
     a.bank.seed[i] = p.seed;

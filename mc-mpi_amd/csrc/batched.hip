@@ -50,12 +50,14 @@ struct batch_args {
 
 struct tile_io {
   const batch_args &a;
-  __device__ __forceinline__ void load(int64_t i, mc_state &p) {
+  static constexpr bool RESUMES = false;
+  __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
     p.seed = a.soa.seed[i];
     p.x = a.soa.x[i];
     p.mu = a.soa.mu[i];
     p.wmc = a.soa.wmc[i];
     p.index = a.soa.index[i];
+    return 0;
   }
   __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t, uint32_t) {
     a.soa.seed[i] = p.seed;

@@ -25,12 +25,17 @@
  *  - when the pool has room for a chunk, it is refilled from the call's bank
  *    through the global work queue (one atomic per refill), so pools stay
  *    full until the bank is exhausted;
- *  - the exact fixed-point tally lives in LDS for the block's lifetime and is
- *    added to the global tally once (same arithmetic as the history kernel).
+ *  - once the bank is exhausted the pools would only empty from pass to pass,
+ *    each event still paying the pipeline's four stages: a wave then finishes
+ *    its pool's particles one history per lane (mc_walk_bank, the pool as its
+ *    queue).  1e6 particles on the 10,000-cell slab: 215 -> 64 ms; 2e7: 1,406
+ *    -> 1,282 ms;
+ *  - the exact fixed-point tally lives in LDS for the block's lifetime (limbs
+ *    as the history kernel's, or words with carry for heavy weights).
  * Results are bit-identical to the history kernel and the oracle: histories
  * are independent and the tally is an exact integer sum.
  */
-#include "internal.h"
+#include "mc_walk.h"
 
 namespace {
 
@@ -263,6 +268,55 @@ __device__ __forceinline__ void exit_state(const sargs &v, int64_t i, const mc_s
   if (c) gbl(c)[i] = col;
 }
 
+/* The particles left in a wave's pool, as the queue and the bank of
+   mc_walk_bank: slots [next, n), dead ones passed over. */
+struct pool_queue {
+  rsrc_t src;
+  int F_CW, n, next;
+  __device__ __forceinline__ bool more() const { return next < n; }
+  __device__ __forceinline__ int64_t take(mc_mask need) {
+    int slot = -1;
+    while (need != 0 && next < n) { /* wave-uniform */
+      const int s = next + mc_mbcnt64(need);
+      next += __popcll(need);
+      bool live = false;
+      if (mc_in(need) && s < n) live = ld32(src, 4 * s, F_CW) != DEAD_CW;
+      if (live) slot = s;
+      need &= ~mc_lanes(live);
+    }
+    return slot;
+  }
+};
+
+template <bool COLL> struct pool_io {
+  static constexpr bool RESUMES = true;
+  const sargs &v;
+  rsrc_t src;
+  mc_layer_k L;
+  int P;
+  unsigned pass;
+  uint32_t id, col0;
+  __device__ __forceinline__ uint64_t load(int64_t slot, mc_state &p) {
+    const int s = (int)slot;
+    uint64_t w;
+    ld128(src, 16 * s, 0, p.seed, w);
+    p.wmc = as_f64(w);
+    p.mu = as_f64(ld64(src, 8 * s, 24 * P));
+    const double x = as_f64(ld64(src, 8 * s, 16 * P));
+    const uint32_t cw = ld32(src, 4 * s, 32 * P);
+    id = ld32(src, 4 * s, 36 * P);
+    const uint32_t t0 = ld32(src, 4 * s, 40 * P);
+    col0 = COLL ? ld32(src, 4 * s, 44 * P) : 0u;
+    p.index = (int32_t)(cw & ~ON_EDGE) + L.index_start;
+    p.x = (cw & ON_EDGE) ? (p.mu < 0 ? p.index + 1 : p.index) * L.dx : x;
+    return pass - t0;
+  }
+  __device__ __forceinline__ bool store(int64_t, mc_state &p, int code, uint64_t ev, uint32_t col) {
+    exit_state(fresh(v), (int64_t)id, p, code, (uint32_t)ev, col0 + col);
+    return false;
+  }
+};
+
 /* Threads per block at most: 1024, 16 waves per CU when the block's tally
    fills the LDS.  The four stages keep about 60 values per lane live across
    the calls of the rare math paths, which leave only the callee-saved
@@ -276,7 +330,7 @@ constexpr int EVENT_MAX_BLOCK = 1024;
 /* the kernel's own LDS (block totals, the arguments), an upper bound: the
    tally and cells take what is left of the block's */
 constexpr size_t EVENT_STATIC_LDS = 2048;
-static_assert(5 * 8 + sizeof(mc_transport_args) + 64 <= EVENT_STATIC_LDS, "static LDS bound");
+static_assert(MC_TOTALS * 8 + sizeof(mc_transport_args) + 64 <= EVENT_STATIC_LDS, "static LDS bound");
 
 template <bool LDS_TALLY, bool LDS_CELLS, bool COLL>
 __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
@@ -286,8 +340,9 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
   /* the log and exp coefficients in vector registers (as constants each use
      would take two scalar moves) */
   const mc_coef K = mc_coef_live();
-  /* block totals: events, collisions, left, right, killed */
-  __shared__ unsigned long long s_tot[5];
+  /* block totals: events, collisions, left, right, killed, capped */
+  __shared__ unsigned long long s_tot[MC_TOTALS];
+  __shared__ int s_k;
   __shared__ mc_transport_args s_a;
   const sargs &v = s_a;
   if (threadIdx.x == 0) s_a = a;
@@ -316,8 +371,19 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
   mc_cell *cells_l = reinterpret_cast<mc_cell *>(smem + off);
   if (LDS_CELLS)
     for (int c = threadIdx.x; c < m; c += blockDim.x) cells_l[c] = ld_cell(cells_g + c);
-  if (threadIdx.x < 5) s_tot[threadIdx.x] = 0;
+  if (threadIdx.x < MC_TOTALS) s_tot[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_k = -1023;
   __syncthreads();
+  if (LDS_TALLY) { /* the block's weights, from one particle per thread (as k_history) */
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t j = i < a.n ? i : (int64_t)threadIdx.x;
+    if (j < a.n) atomicMax(&s_k, mc_ceil_log2(a.aos ? a.aos[j].wmc : a.soa.wmc[j]));
+    __syncthreads();
+  }
+  const mc_block_tally B =
+      mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), blockDim.x >> 6);
+  const bool limbs = LDS_TALLY && B.limbs && (P >> 6) <= B.every; /* block-uniform */
+  mc_mover moves{t_lo, t_hi, a.fx, a.fx + m, m, B.S.L, B.every, B.every};
 
   /* this wave's pool: two halves of P slots */
   const int lane = __lane_id();
@@ -349,7 +415,8 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
     atomicAdd(&s_tot[code == -1 ? 2 : (code == 1 ? 3 : 4)], code == 2 ? 0ull : 1ull);
   };
 
-  for (unsigned pass = 0;;) {
+  unsigned pass = 0;
+  for (;;) {
     /* ---- refill from the work queue (wave-uniform condition) */
     if (!queue_done && n_pool <= P - 64) {
       const int want = P - n_pool;
@@ -384,8 +451,8 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
       /* slots written by one lane are read by another lane of this wave */
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     }
+    if (queue_done) break;
     if (n_pool == 0) {
-      if (queue_done) break;
       ++pass;
       continue;
     }
@@ -393,12 +460,14 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
     /* ---- a segment: the passes up to the next compaction (one pass when
        the pool holds fewer than four chunks), streamed through the stages */
     const int nch = (n_pool + 63) >> 6;
-    const unsigned last = nch >= 4 ? pass + (ce - pass % ce) % ce : pass;
+    unsigned last = nch >= 4 ? pass + (ce - pass % ce) % ce : pass;
+    if (limbs && (int)(last - pass + 1) * nch > B.every) last = pass + (unsigned)(B.every / nch) - 1;
     const int total = (int)(last - pass + 1) * nch;
     const bool ends_compacting = last % ce == 0;
     /* the event cap can bind in this segment (a count after pass q is at
        most q + 1): the passes then read every slot's count origin */
     const bool cap_live = (unsigned long long)last + 1 >= max_ev;
+    if (limbs) moves(total);
     const rsrc_t src = half_rsrc(mine + cur * half_bytes, P);
     const rsrc_t dst = half_rsrc(mine + (cur ^ 1) * half_bytes, P);
     int wpos = 0; /* wave-uniform output position of the compaction */
@@ -446,6 +515,7 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
            that is a compaction pass (passes before it are not) */
         const bool compact = ends_compacting && c_q == last;
         bool keep = false, on_edge = false;
+        double d_dw = 0.0;
         if (c_live) {
           if (c_event) {
             const double e = mc_exp_k_row(c_arg, &c_row, &K);
@@ -456,7 +526,8 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
             ++lane_ev;
             c_col += c_coll ? 1u : 0u;
             lane_col += c_coll ? 1u : 0u;
-            mc_tally_with(t_lo, t_hi, c_cell, dw, [&](uint32_t g) {
+            d_dw = dw;
+            if (!limbs) mc_tally_with(t_lo, t_hi, c_cell, dw, [&](uint32_t g) {
               const sargs &w = fresh(v);
               __hip_atomic_fetch_or(gbl(w.flags) + c_cell, g, __ATOMIC_RELAXED,
                                     __HIP_MEMORY_SCOPE_AGENT);
@@ -479,6 +550,9 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
             finish(c_p, id, c_q - t0 + done, c_col);
           }
         }
+        if (limbs)
+          mc_tally_limbs(t_lo, t_hi, B.S, fresh(v).fx, fresh(v).fx + m, fresh(v).flags,
+                         &fresh(v).ctr->status, mc_lanes(c_live && c_event), c_cell, d_dw);
         /* the write-back: the offsets per path, then the same stores on both
            (a store on one path only would make the compiler assume fewer
            operations in flight after the branches and wait longer at the
@@ -619,24 +693,45 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
     pass = last + 1;
   }
 
-  mc_counters *ctr = a.ctr;
-  if (capped) atomicOr(&ctr->status, 1u);
-
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    atomicAdd(&ctr->events, s_tot[0]);
-    atomicAdd(&ctr->collisions, s_tot[1]);
-    atomicAdd(&ctr->n_left, s_tot[2]);
-    atomicAdd(&ctr->n_right, s_tot[3]);
-    atomicAdd(&ctr->n_killed, s_tot[4]);
+  /* ---- the bank is exhausted: what is left in the pool, a history per lane */
+  if (n_pool > 0) {
+    const rsrc_t src = half_rsrc(mine + cur * half_bytes, P);
+    pool_queue queue{src, F_CW, n_pool, 0};
+    pool_io<COLL> io{v, src, L, P, pass, 0u, 0u};
+    const mc_walk_k W = mc_walk_live(L);
+    const mc_cell *cells = LDS_CELLS ? cells_l : a.cells;
+    const double2 *tab = reinterpret_cast<const double2 *>(mc_abs_tab);
+    unsigned long long *fx_lo = a.fx, *fx_hi = a.fx + m;
+    uint32_t *flags = a.flags;
+    unsigned int *status = &a.ctr->status;
+    if (limbs)
+      mc_walk_bank(io, queue, L, W, cells, tab, 0, B.every, max_ev, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     mc_tally_limbs(t_lo, t_hi, B.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
+                   },
+                   moves);
+    else
+      mc_walk_bank(io, queue, L, W, cells, tab, 0, 1 << 30, max_ev, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) mc_tally(t_lo, t_hi, flags, status, c, dw);
+                   },
+                   [](int) {});
   }
+
+  if (capped) atomicOr(&s_tot[5], 1ull);
+  __syncthreads();
+  if (threadIdx.x == 0) mc_totals_out(s_tot, a.ctr);
   if (LDS_TALLY) {
     unsigned long long *fx = a.fx;
-    for (int c = threadIdx.x; c < m; c += blockDim.x) {
-      mc_fx t;
-      t.lo = t_lo[c];
-      t.hi = t_hi[c];
-      mc_fx_atomic_add(&fx[c], &fx[m + c], t);
+    if (limbs) {
+      mc_limbs_move(t_lo, t_hi, B.S.L, m, threadIdx.x, blockDim.x, fx, fx + m);
+    } else {
+      for (int c = threadIdx.x; c < m; c += blockDim.x) {
+        mc_fx t;
+        t.lo = t_lo[c];
+        t.hi = t_hi[c];
+        mc_fx_atomic_add(&fx[c], &fx[m + c], t);
+      }
     }
   }
 }

@@ -263,7 +263,7 @@ def main():
     w("/* ... with {y_k, exp(-y_k)}, k = 0 .. 88: y_k within 2^-23 of k/128, a multiple")
     w("   of 2^-43, chosen so that the exponential is within 2^-71 of its double */")
     w("#define MC_ABS_N 89")
-    w("MC_TAB double mc_abs_tab[MC_ABS_N][2] = {")
+    w("MC_TAB double MC_ALIGN16 mc_abs_tab[MC_ABS_N][2] = {")
     for k, (y, v) in enumerate(absorb_table(89)):
         w(f"  {{{hexf(y)}, {hexf(v)}}}, /* {k} */")
     w("};")

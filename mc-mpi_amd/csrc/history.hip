@@ -36,9 +36,11 @@ namespace {
 template <bool SCORE> struct bank_io {
   const mc_transport_args &a;
   double score;
-  __device__ __forceinline__ void load(int64_t i, mc_state &p) {
+  static constexpr bool RESUMES = false;
+  __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
     load_state(a, i, p);
     score = 0.0;
+    return 0;
   }
   __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t ev,
                                         uint32_t col) {

@@ -110,10 +110,12 @@ template <bool HAVE_SCORE> struct mc_grad_io {
     p.index = init.index[i];
     P = 0.0;
   }
-  __device__ __forceinline__ void load(int64_t i, mc_state &p) {
+  static constexpr bool RESUMES = false;
+  __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
     read(i, p);
     T = HAVE_SCORE ? score[i] : 0.0;
     phase = HAVE_SCORE ? 1 : 0;
+    return 0;
   }
   __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t, uint32_t) {
     if (HAVE_SCORE || phase == 1 || code == 2) return false;

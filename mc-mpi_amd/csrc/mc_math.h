@@ -49,6 +49,7 @@
 #define MC_TAB static const
 #endif
 
+#define MC_ALIGN16 __attribute__((aligned(16)))
 #include "mc_math_tables.h"
 
 /* ---------------------------------------------------------------- basics */

@@ -412,8 +412,10 @@ __device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, m
 
 /* A wave's histories, one per lane, until its queue is empty.
    io.load(i, state) reads history i (and resets what the caller keeps per
-   lane); io.store(i, state, code, ev, col) takes a finished one and returns
-   whether the lane goes on with the state it leaves in `state` (a replay);
+   lane) and returns the events it has had before; io.store(i, state, code, ev,
+   col) takes a finished one (ev with those before, col without) and returns
+   whether the lane goes on, from no events, with the state it leaves in
+   `state` (a replay);
    on_event as in mc_walk_many; moves(k) is called before every (at most) k
    events per lane, k <= k_max.
    refill_k: events between refills; 0: adapted per wave from the lanes found
@@ -433,7 +435,7 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
   int64_t idx = 0;
   bool has = false;
   mc_mask run = 0, pend = 0; /* lanes whose history goes on / waits for the general event */
-  uint64_t ev = 0;
+  uint64_t ev = 0, before = 0; /* events of the lane's history; those before this call */
   uint32_t col = 0;
   const bool adapt = refill_k <= 0;
   int kk = adapt ? 128 : refill_k;
@@ -454,22 +456,24 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
         bool on = false;
         if (!has && i >= 0) {
           mc_state in;
-          io.load(i, in);
+          ev = io.load(i, in);
           mc_walk_from(p, in, L);
           idx = i;
           has = true;
-          on = mc_walk_alive(p, L);
-          ev = 0;
+          on = mc_walk_alive(p, L) && ev < max_events;
+          if (IO::RESUMES) before = ev;
           col = 0;
         }
         run |= mc_lanes(on);
+        if (IO::RESUMES) ev_bound = max_events; /* recomputed below */
       }
     }
     if (mc_lanes(has) == 0) break; /* wave-uniform */
     int ki = kk < k_max ? kk : k_max - 1; /* a waiting lane may add one */
     if (ev_bound + (uint64_t)ki >= max_events) {
       ev_bound = mc_wave_max_u64(has ? ev + (mc_in(pend) ? 1u : 0u) : 0ull);
-      if (ev_bound + (uint64_t)ki >= max_events) ki = (int)(max_events - ev_bound);
+      if (ev_bound + (uint64_t)ki >= max_events)
+        ki = ev_bound < max_events ? (int)(max_events - ev_bound) : 0;
     }
     ev_bound += (uint64_t)ki;
     moves(ki + 1);
@@ -485,14 +489,15 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
     if (ends) {
       mc_state out;
       mc_walk_to(out, p, L);
-      code = on ? 2 : mc_exit_code(out, L); /* on: a runaway history stopped by the guard */
-      atomicAdd(&s_tot[0], (unsigned long long)ev);
+      /* at the cap and alive: a runaway history stopped by the guard */
+      code = ev >= max_events && mc_walk_alive(p, L) ? 2 : mc_exit_code(out, L);
+      atomicAdd(&s_tot[0], (unsigned long long)(ev - before));
       atomicAdd(&s_tot[1], (unsigned long long)col);
       has = io.store(idx, out, code, ev, col);
       if (has) {
         mc_walk_from(p, out, L);
         again = mc_walk_alive(p, L);
-        ev = 0;
+        ev = before = 0;
         col = 0;
       }
     }

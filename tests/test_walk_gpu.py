@@ -27,13 +27,13 @@ def _case(m, n, seed, wmc):
     return sigs, ar, 1.0 / m, bank
 
 
-def _check(ctx, oracle, m, n, seed, wmc, min_w, **opts):
+def _check(ctx, oracle, m, n, seed, wmc, min_w, kernel="history", **opts):
     import mcgpu
     sigs, ar, dx, bank = _case(m, n, seed, wmc)
     o = oracle.simulate_bank(64, 0, m, dx, min_w, sigs, ar, bank, nthread=8)
     b, w = bank.copy(), np.zeros(m)
     result, st, rc = ctx.simulate(b, sigs, ar, w, 0, m, dx, min_w,
-                                  options=mcgpu.make_options("history", **opts))
+                                  options=mcgpu.make_options(kernel, **opts))
     assert rc == 0
     for f in ("seed", "x", "mu", "wmc", "index"):
         assert np.array_equal(b[f], o["bank"][f]), f
@@ -74,6 +74,20 @@ def test_runs_from_the_counter(ctx, oracle, n):
     """More histories than the first runs hold: few blocks, many later runs."""
     _say(f"n={n}, later runs")
     _check(ctx, oracle, 25, n, n, 1.0, 1e-2, grid_blocks=3, block_size=64)
+
+
+@pytest.mark.parametrize("compaction_interval", [1, 3, 64])
+@pytest.mark.parametrize("scale", [1e-8, 1.0, 1e3])
+@pytest.mark.parametrize("n", [50, 700, 5000])
+def test_event_kernel_passes_then_drain(ctx, oracle, n, scale, compaction_interval):
+    """Two waves of 256 pool slots each: banks that never leave the drain, that
+    just fill the pools, and that pass through them many times, with on-edge
+    and dead slots at the switch and every form of tally."""
+    _say(f"event n={n} weights {scale} ci={compaction_interval}")
+    rng = np.random.default_rng(n)
+    _check(ctx, oracle, 45, n, n, scale * rng.uniform(0.5, 1.0, n), 1e-2 * scale, kernel="event",
+           grid_blocks=1, block_size=128, particles_per_lane=4,
+           compaction_interval=compaction_interval)
 
 
 def _gradient(ctx, oracle, m, n, seed, wscale, gscale, with_score, batched):
