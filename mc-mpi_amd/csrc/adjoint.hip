@@ -44,7 +44,7 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
   __shared__ int s_k, s_g;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   const mc_walk_k K = mc_walk_live(a.L);
-  mc_call_queue queue{mc_queue_open(a.n, per_cu), &a.ctr->next};
+  mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
   const int m = a.L.m;
   double2 *tab = reinterpret_cast<double2 *>(smem);
   mc_tab_fill(tab);

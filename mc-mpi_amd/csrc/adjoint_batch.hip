@@ -89,6 +89,9 @@ template <bool SCORE> struct fwd_io {
   const bcell_args &a;
   double score;
   static constexpr bool RESUMES = false;
+  __device__ __forceinline__ int code(const mc_state &p, bool at_cap, const mc_layer_k &L) {
+    return mc_end_code(p, at_cap, L);
+  }
   __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
     p.seed = a.bank.seed[i];
     p.x = a.bank.x[i];

@@ -51,6 +51,9 @@ struct batch_args {
 struct tile_io {
   const batch_args &a;
   static constexpr bool RESUMES = false;
+  __device__ __forceinline__ int code(const mc_state &p, bool at_cap, const mc_layer_k &L) {
+    return mc_end_code(p, at_cap, L);
+  }
   __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
     p.seed = a.soa.seed[i];
     p.x = a.soa.x[i];

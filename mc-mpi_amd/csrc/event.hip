@@ -290,6 +290,9 @@ struct pool_queue {
 
 template <bool COLL> struct pool_io {
   static constexpr bool RESUMES = true;
+  __device__ __forceinline__ int code(const mc_state &p, bool at_cap, const mc_layer_k &l) {
+    return mc_end_code(p, at_cap, l);
+  }
   const sargs &v;
   rsrc_t src;
   mc_layer_k L;

@@ -111,6 +111,9 @@ template <bool HAVE_SCORE> struct mc_grad_io {
     P = 0.0;
   }
   static constexpr bool RESUMES = false;
+  __device__ __forceinline__ int code(const mc_state &p, bool at_cap, const mc_layer_k &L) {
+    return mc_end_code(p, at_cap, L);
+  }
   __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
     read(i, p);
     T = HAVE_SCORE ? score[i] : 0.0;

@@ -291,6 +291,11 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
   return general;
 }
 
+/* exit code of a history that ends in state p (2: alive, stopped by the cap) */
+__device__ __forceinline__ int mc_end_code(const mc_state &p, bool at_cap, const mc_layer_k &L) {
+  return at_cap && mc_alive(p, L) ? 2 : mc_exit_code(p, L);
+}
+
 /* -------------------------------------------------------------- work queue */
 
 /* The histories 0 .. n-1 of a call, taken by waves in runs: the first run of
@@ -316,16 +321,17 @@ __device__ __forceinline__ uint64_t mc_run_size(uint64_t left, uint32_t waves) {
   return s < 64 ? 64 : (s > 4096 ? 4096 : s);
 }
 
-/* per_cu: blocks on a CU */
-__device__ __forceinline__ mc_queue mc_queue_open(int64_t n, int per_cu) {
+/* per_cu: blocks on a CU; this is block `block` of `blocks` that share the queue */
+__device__ __forceinline__ mc_queue mc_queue_open(int64_t n, int per_cu, uint32_t block,
+                                                  uint32_t blocks) {
   mc_queue q;
   const uint32_t per_block = blockDim.x >> 6;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t pos = wave * gridDim.x + blockIdx.x;
+  const uint32_t pos = wave * blocks + block;
   q.n = (uint64_t)n;
-  q.waves = gridDim.x * per_block;
+  q.waves = blocks * per_block;
   const uint32_t few = (per_block * (uint32_t)per_cu > 8u ? (8u + per_cu - 1) / per_cu : per_block) *
-                       gridDim.x;
+                       blocks;
   const uint64_t size = q.n <= 64ull * few ? (q.n + few - 1) / few : mc_run_size(q.n, q.waves);
   q.next = pos * size;
   q.end = q.next + size;
@@ -415,7 +421,8 @@ __device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, m
    lane) and returns the events it has had before; io.store(i, state, code, ev,
    col) takes a finished one (ev with those before, col without) and returns
    whether the lane goes on, from no events, with the state it leaves in
-   `state` (a replay);
+   `state` (a replay); io.code(state, at_cap, L) is its exit code (3: none to
+   count);
    on_event as in mc_walk_many; moves(k) is called before every (at most) k
    events per lane, k <= k_max.
    refill_k: events between refills; 0: adapted per wave from the lanes found
@@ -490,7 +497,7 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
       mc_state out;
       mc_walk_to(out, p, L);
       /* at the cap and alive: a runaway history stopped by the guard */
-      code = ev >= max_events && mc_walk_alive(p, L) ? 2 : mc_exit_code(out, L);
+      code = io.code(out, ev >= max_events, L);
       atomicAdd(&s_tot[0], (unsigned long long)(ev - before));
       atomicAdd(&s_tot[1], (unsigned long long)col);
       has = io.store(idx, out, code, ev, col);

@@ -146,3 +146,91 @@ def test_gradient_layers_around_the_lds_limits(ctx, oracle, m, batched, with_sco
     (32 B, one slab); neither."""
     _say(f"gradient, m={m} batched={batched} with_score={with_score}")
     _gradient(ctx, oracle, m, 120, m, 1.0, 1.0, with_score, batched)
+
+
+@pytest.mark.parametrize("m,n,opts", [(10_136, 900, {}), (20_500, 400, {}), (20_500, 3000, {}),
+                                      (31_000, 64, {"grid_blocks": 5, "block_size": 128}),
+                                      (31_000, 64, {"grid_blocks": 2})])
+@pytest.mark.parametrize("host", [True, False])
+def test_wide_layers_in_windows(ctx, oracle, m, n, opts, host):
+    """Layers of more cells than a block's LDS tally holds: two windows just
+    above the limit, three and four of them, and too few blocks for them (the
+    global tally).  Histories cross the windows' edges both ways; counts add up
+    over the sweeps."""
+    import mcgpu
+    import torch
+    _say(f"windows m={m} n={n} {opts} host={host}")
+    sigs, ar, dx, bank = _case(m, n, m + n, 1.0)
+    sigs *= 3.0
+    lo = 700
+    bank["index"] += lo
+    bank["x"] = (bank["index"] + 0.25) * dx
+    min_w = 1e-2
+    bank["wmc"][::50] = 1e-3  # finished as they come
+    o = oracle.simulate_bank(64, lo, m, dx, min_w, sigs, ar, bank, nthread=8)
+    options = mcgpu.make_options("history", **opts)
+    if host:
+        b, w = bank.copy(), np.zeros(m)
+        result, st, rc = ctx.simulate(b, sigs, ar, w, lo, lo + m, dx, min_w, options=options)
+    else:
+        db = mcgpu.bank_to_device(bank)
+        dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+        dw, dr = dev(np.zeros(m)), dev(np.zeros(n, np.int8))
+        ev, co = dev(np.zeros(n, np.int64)), dev(np.full(n, 5))
+        st, rc = ctx.simulate_device(db, dev(sigs), dev(ar), dw, lo, lo + m, dx, min_w, result=dr,
+                                     events=ev, collisions=co, options=options)
+        b, w, result = mcgpu.bank_from_device(db), dw.cpu().numpy(), dr.cpu().numpy()
+        assert np.array_equal(ev.cpu().numpy(), o["events"])
+        assert np.array_equal(co.cpu().numpy(), o["collisions"])
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f]), f
+    assert np.array_equal(result.astype(np.int32), o["result"])
+    assert st["events"] == int(o["events"].sum())
+    assert st["collisions"] == int(o["collisions"].sum())
+    assert st["n_left"] + st["n_right"] + st["n_killed"] == n
+    assert np.array_equal(w, o["tally_exact"])
+
+
+def test_wide_layer_event_cap_counts_over_sweeps(ctx, oracle):
+    """A cap that histories reach after several sweeps ends them at exactly
+    that count; shorter ones are the oracle's."""
+    import mcgpu
+    import torch
+    m, n, cap = 10_400, 300, 9000
+    sigs, ar, dx, bank = _case(m, n, 9, 1.0)
+    _say("windows, event cap")
+    o = oracle.simulate_bank(64, 0, m, dx, 1e-3, sigs, ar, bank, nthread=8)
+    db = mcgpu.bank_to_device(bank)
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+    dr, ev = dev(np.zeros(n, np.int8)), dev(np.zeros(n, np.int64))
+    st, rc = ctx.simulate_device(db, dev(sigs), dev(ar), dev(np.zeros(m)), 0, m, dx, 1e-3,
+                                 result=dr, events=ev, allow=(mcgpu.ERR_EVENT_CAP,),
+                                 options=mcgpu.make_options("history", max_events_per_history=cap))
+    longer = o["events"] > cap
+    assert longer.any() and not longer.all() and rc == mcgpu.ERR_EVENT_CAP
+    e, r, b = ev.cpu().numpy(), dr.cpu().numpy(), mcgpu.bank_from_device(db)
+    assert np.all(e[longer] == cap) and np.all(r[longer] == 2)
+    assert np.array_equal(e[~longer], o["events"][~longer])
+    assert np.array_equal(r[~longer], o["result"][~longer])
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f][~longer], o["bank"][f][~longer]), f
+    assert st["events"] == int(np.minimum(o["events"], cap).sum())
+
+
+def test_wide_layer_scores(ctx, oracle):
+    """forward_cells with per-history scores over windows: the same sums in
+    event order."""
+    import mcgpu
+    import torch
+    m, n = 12_000, 200
+    rng = np.random.default_rng(8)
+    sa, ss, g = rng.lognormal(0, 0.5, m), rng.lognormal(0, 0.5, m), rng.uniform(-1, 1, m)
+    _, _, dx, bank = _case(m, n, 8, 1.0)
+    _say("windows, scores")
+    o = oracle.forward_cells(0, m, dx, 1e-3, sa, ss, bank, g=g)
+    db = mcgpu.bank_to_device(bank)
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+    w, sc = dev(np.zeros(m)), dev(np.full(n, 7.0))
+    ctx.forward_cells(db, dev(sa), dev(ss), w, 0, m, dx, 1e-3, g=dev(g), history_score=sc)
+    assert np.array_equal(w.cpu().numpy(), o["tally_exact"])
+    assert np.array_equal(sc.cpu().numpy().view(np.uint64), o["score"].view(np.uint64))
