@@ -64,12 +64,9 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
     for (int c = threadIdx.x; c < 4 * m; c += blockDim.x) G.t[c] = 0;
   if (LDS_C) {
     mc_cell *lc = reinterpret_cast<mc_cell *>(G.t + 4 * m);
-    double *lg = reinterpret_cast<double *>(lc + m);
-    for (int c = threadIdx.x; c < m; c += blockDim.x) {
-      lc[c] = a.cells[c];
-      lg[c] = a.g[c];
-    }
-    cells = lc;
+    double *lg = reinterpret_cast<double *>(lc + m + 2);
+    for (int c = threadIdx.x; c < m; c += blockDim.x) lg[c] = a.g[c];
+    cells = mc_cells_fill(lc, a.cells, m);
     g = lg;
   }
   __syncthreads();
@@ -89,18 +86,18 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
 
   mc_grad_io<HAVE_SCORE> io{a.init, a.score, 0.0, 0.0, 1};
   if (LDS_T && limbs) { /* block-uniform */
-    mc_walk_bank(io, queue, a.L, K, cells, tab, refill_k, G.every, a.max_events, s_tot,
-                 [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+    mc_walk_bank<LDS_C>(io, queue, a.L, K, cells, tab, refill_k, G.every, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
                      double wmc) {
-                   mc_grad_event<MC_GRAD_LIMBS>(io, G, g, lanes, c, cell, coll, di, dw, wmc);
+                   mc_grad_event<MC_GRAD_LIMBS>(io, G, g, lanes, c8, cell, coll, di, dw, wmc);
                  },
                  mc_grad_mover{G, G.every});
   } else {
     constexpr int MODE = LDS_T ? MC_GRAD_CARRY : MC_GRAD_GLOBAL;
-    mc_walk_bank(io, queue, a.L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
-                 [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+    mc_walk_bank<LDS_C>(io, queue, a.L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
                      double wmc) {
-                   mc_grad_event<MODE>(io, G, g, lanes, c, cell, coll, di, dw, wmc);
+                   mc_grad_event<MODE>(io, G, g, lanes, c8, cell, coll, di, dw, wmc);
                  },
                  [](int) {});
   }
@@ -217,8 +214,8 @@ int launch_adj(mcgpu_context *ctx, const adj_args &a, const mcgpu_options &o, hi
 template <bool S>
 int launch_adj_fit(mcgpu_context *ctx, const adj_args &a, const mcgpu_options &o, hipStream_t s) {
   const size_t m = (size_t)a.L.m, budget = ctx->lds_per_block - 256;
-  if (MC_TAB_BYTES + 56 * m <= budget)
-    return launch_adj<true, true, S>(ctx, a, o, s, MC_TAB_BYTES + 56 * m);
+  if (MC_TAB_BYTES + MC_PAD_BYTES + 56 * m <= budget)
+    return launch_adj<true, true, S>(ctx, a, o, s, MC_TAB_BYTES + MC_PAD_BYTES + 56 * m);
   if (MC_TAB_BYTES + 32 * m <= budget)
     return launch_adj<true, false, S>(ctx, a, o, s, MC_TAB_BYTES + 32 * m);
   return launch_adj<false, false, S>(ctx, a, o, s, MC_TAB_BYTES);

@@ -137,14 +137,14 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     const bool in_lds = m <= a.lds_max_m; /* block-uniform */
     unsigned long long *t1 = t0 + m;
     mc_cell *lc = reinterpret_cast<mc_cell *>(t1 + m);
-    double *lg = reinterpret_cast<double *>(lc + m);
+    double *lg = reinterpret_cast<double *>(lc + m + 2);
     if (in_lds) {
       for (int c = tid; c < m; c += B) {
         t0[c] = 0;
         t1[c] = 0;
-        lc[c] = a.cells[b.cell_off + c];
         if (SCORE) lg[c] = a.g[b.cell_off + c];
       }
+      lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
     }
     if (tid == 0) s_next = b.begin;
     if (b.begin + tid < b.end) atomicMax(&s_k, mc_ceil_log2(a.bank.wmc[b.begin + tid]));
@@ -158,28 +158,28 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     unsigned int *status = &a.ctr->status;
     const double *gg = SCORE ? a.g + b.cell_off : nullptr;
     if (in_lds && bt.limbs) {
-      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-                     mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
-                     if (SCORE && mc_in(lanes)) io.score = io.score + lg[c] * dw;
+      mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                     mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+                     if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(lg, c8) * dw;
                    },
                    mc_mover{t0, t1, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every});
     } else if (in_lds) { /* weights too heavy for the limbs */
-      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+      mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
                      if (mc_in(lanes)) {
-                       mc_tally(t0, t1, flags, status, c, dw);
-                       if (SCORE) io.score = io.score + lg[c] * dw;
+                       mc_tally(t0, t1, flags, status, c8 >> 3, dw);
+                       if (SCORE) io.score = io.score + *mc_word(lg, c8) * dw;
                      }
                    },
                    [](int) {});
     } else {
-      mc_walk_bank(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
+      mc_walk_bank<false>(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
                    s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
                      if (mc_in(lanes)) {
-                       mc_tally(fx_lo, fx_hi, flags, status, c, dw);
-                       if (SCORE) io.score = io.score + gg[c] * dw;
+                       mc_tally(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
+                       if (SCORE) io.score = io.score + *mc_word(gg, c8) * dw;
                      }
                    },
                    [](int) {});
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
     const int m = b.L.m;
     const bool in_lds = m <= a.lds_max_m; /* block-uniform */
     mc_cell *lc = reinterpret_cast<mc_cell *>(G.t + 4 * m);
-    double *lg = reinterpret_cast<double *>(lc + m);
+    double *lg = reinterpret_cast<double *>(lc + m + 2);
     const double *gg = a.g + b.cell_off;
     G.fx = a.fx + b.cell_off;
     G.flags_a = a.flags + b.cell_off;
@@ -233,13 +233,13 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
       int kg = -1023;
       for (int c = tid; c < m; c += B) {
         for (int w = 0; w < 4; ++w) G.t[w * m + c] = 0;
-        lc[c] = a.cells[b.cell_off + c];
         const double v = gg[c];
         lg[c] = v;
         const int k = mc_ceil_log2(v);
         kg = k > kg ? k : kg;
       }
       atomicMax(&s_g, kg);
+      lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
     }
     if (tid == 0) s_next = b.begin;
     if (b.begin + tid < b.end) atomicMax(&s_k, mc_ceil_log2(a.bank.wmc[b.begin + tid]));
@@ -249,25 +249,25 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
     const bool limbs = mc_grad_split(G, __builtin_amdgcn_readfirstlane(s_k + s_g), B >> 6);
     mc_tile_queue queue{&s_next, b.end, false};
     if (in_lds && limbs)
-      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, G.every, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+      mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, G.every, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
                        double wmc) {
-                     mc_grad_event<MC_GRAD_LIMBS>(io, G, lg, lanes, c, cell, coll, di, dw, wmc);
+                     mc_grad_event<MC_GRAD_LIMBS>(io, G, lg, lanes, c8, cell, coll, di, dw, wmc);
                    },
                    mc_grad_mover{G, G.every});
     else if (in_lds)
-      mc_walk_bank(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+      mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
                        double wmc) {
-                     mc_grad_event<MC_GRAD_CARRY>(io, G, lg, lanes, c, cell, coll, di, dw, wmc);
+                     mc_grad_event<MC_GRAD_CARRY>(io, G, lg, lanes, c8, cell, coll, di, dw, wmc);
                    },
                    [](int) {});
     else
-      mc_walk_bank(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
+      mc_walk_bank<false>(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
                    s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
+                   [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
                        double wmc) {
-                     mc_grad_event<MC_GRAD_GLOBAL>(io, G, gg, lanes, c, cell, coll, di, dw, wmc);
+                     mc_grad_event<MC_GRAD_GLOBAL>(io, G, gg, lanes, c8, cell, coll, di, dw, wmc);
                    },
                    [](int) {});
     __syncthreads();
@@ -421,9 +421,9 @@ int batch_prepare(mcgpu_context *ctx, K kern, int32_t n_slabs, const mcgpu_slab 
   for (int s_ = 0; s_ < n_slabs; ++s_)
     max_m = std::max(max_m, slabs[s_].max_index - slabs[s_].min_index);
   /* LDS for the largest slab that fits; larger slabs use the global accumulators */
-  const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES; /* and the static LDS */
+  const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES - MC_PAD_BYTES; /* static LDS */
   a->lds_max_m = (int)std::min<size_t>((size_t)max_m, budget / lds_bytes_per_cell);
-  *lds = MC_TAB_BYTES + lds_bytes_per_cell * (size_t)a->lds_max_m;
+  *lds = MC_TAB_BYTES + MC_PAD_BYTES + lds_bytes_per_cell * (size_t)a->lds_max_m;
   if (*lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds);

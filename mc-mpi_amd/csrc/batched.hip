@@ -114,8 +114,8 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
       for (int c = tid; c < m; c += B) {
         t0[c] = 0;
         t1[c] = 0;
-        if (lds_cells) lc[c] = gc[c];
       }
+      if (lds_cells) lc = mc_cells_fill(lc, gc, m);
     }
     if (tid == 0) s_next = (unsigned long long)tile.begin;
     /* the tile's weights, from one history per thread (as the history kernel) */
@@ -129,27 +129,27 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     unsigned long long *fx_lo = a.fx + cell_off, *fx_hi = fx_lo + a.total_cells;
     uint32_t *flags = a.flags + cell_off;
     unsigned int *status = &a.ctr->status;
-    auto limbs = [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-      mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
+    auto limbs = [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+      mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
     };
     const mc_mover mover{t0, t1, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every};
     if (lds_tally && bt.limbs) {
       if (lds_cells)
-        mc_walk_bank(io, queue, L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
+        mc_walk_bank<true>(io, queue, L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
                      mover);
       else
-        mc_walk_bank(io, queue, L, K, gc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
+        mc_walk_bank<false>(io, queue, L, K, gc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
                      mover);
     } else if (lds_tally) { /* heavy weights */
-      mc_walk_bank(io, queue, L, K, gc, tab, refill_k, 1 << 30, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-                     if (mc_in(lanes)) mc_tally(t0, t1, flags, status, c, dw);
+      mc_walk_bank<false>(io, queue, L, K, gc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) mc_tally(t0, t1, flags, status, c8 >> 3, dw);
                    },
                    [](int) {});
     } else {
-      mc_walk_bank(io, queue, L, K, gc, tab, refill_k, 1 << 30, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-                     if (mc_in(lanes)) mc_tally(fx_lo, fx_hi, flags, status, c, dw);
+      mc_walk_bank<false>(io, queue, L, K, gc, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) mc_tally(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
                    },
                    [](int) {});
     }
@@ -210,9 +210,9 @@ int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, in
      (next to the absorbed-fraction rows and the kernel's static LDS); slabs
      whose tally does not fit add into the global tally directly */
   const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES;
-  const size_t lds = std::min(budget, (size_t)32 * (size_t)std::max(max_m, 1));
+  const size_t lds = std::min(budget, (size_t)32 * (size_t)std::max(max_m, 1) + MC_PAD_BYTES);
   sh.lds = lds + MC_TAB_BYTES;
-  sh.lds_cells_max_m = (int)(lds / 32);
+  sh.lds_cells_max_m = (int)((lds - MC_PAD_BYTES) / 32);
   sh.lds_tally_max_m = (int)(lds / 16);
   if (sh.lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_batched),

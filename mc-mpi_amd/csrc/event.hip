@@ -555,7 +555,7 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
         }
         if (limbs)
           mc_tally_limbs(t_lo, t_hi, B.S, fresh(v).fx, fresh(v).fx + m, fresh(v).flags,
-                         &fresh(v).ctr->status, mc_lanes(c_live && c_event), c_cell, d_dw);
+                         &fresh(v).ctr->status, mc_lanes(c_live && c_event), 8 * c_cell, d_dw);
         /* the write-back: the offsets per path, then the same stores on both
            (a store on one path only would make the compiler assume fewer
            operations in flight after the branches and wait longer at the
@@ -708,15 +708,15 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
     uint32_t *flags = a.flags;
     unsigned int *status = &a.ctr->status;
     if (limbs)
-      mc_walk_bank(io, queue, L, W, cells, tab, 0, B.every, max_ev, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-                     mc_tally_limbs(t_lo, t_hi, B.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
+      mc_walk_bank<false>(io, queue, L, W, cells, tab, 0, B.every, max_ev, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                     mc_tally_limbs(t_lo, t_hi, B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
                    },
                    moves);
     else
-      mc_walk_bank(io, queue, L, W, cells, tab, 0, 1 << 30, max_ev, s_tot,
-                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-                     if (mc_in(lanes)) mc_tally(t_lo, t_hi, flags, status, c, dw);
+      mc_walk_bank<false>(io, queue, L, W, cells, tab, 0, 1 << 30, max_ev, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) mc_tally(t_lo, t_hi, flags, status, c8 >> 3, dw);
                    },
                    [](int) {});
   }

@@ -212,11 +212,10 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
   const mc_cell *cells = a.cells + off;
   const double *g = SCORE ? a.g + off : nullptr;
   if (LDS_CELLS) {
-    mc_cell *lc = reinterpret_cast<mc_cell *>(smem + MC_TAB_BYTES + (size_t)16 * m);
-    for (int c = threadIdx.x; c < m; c += blockDim.x) lc[c] = cells[c];
-    cells = lc;
+    mc_cell *lc = reinterpret_cast<mc_cell *>(t1 + m);
+    cells = mc_cells_fill(lc, cells, m);
     if (SCORE) {
-      double *lg = reinterpret_cast<double *>(smem + MC_TAB_BYTES + (size_t)32 * m);
+      double *lg = reinterpret_cast<double *>(lc + m + 2);
       for (int c = threadIdx.x; c < m; c += blockDim.x) lg[c] = g[c];
       g = lg;
     }
@@ -237,21 +236,21 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
   const mc_block_tally B =
       mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), blockDim.x >> 6);
   if (LDS_TALLY && B.limbs) { /* block-uniform */
-    mc_walk_bank(io, queue, L, K, cells, tab, refill_k, B.every, a.max_events, s_tot,
-                 [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
-                   mc_tally_limbs(t0, t1, B.S, fx_lo, fx_hi, flags, status, lanes, c, dw);
-                   if (SCORE && mc_in(lanes)) io.score = io.score + g[c] * dw;
+    mc_walk_bank<LDS_CELLS>(io, queue, L, K, cells, tab, refill_k, B.every, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                   mc_tally_limbs(t0, t1, B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+                   if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(g, c8) * dw;
                  },
                  mc_mover{t0, t1, fx_lo, fx_hi, m, B.S.L, B.every, B.every});
     __syncthreads();
     mc_limbs_move(t0, t1, B.S.L, m, threadIdx.x, blockDim.x, fx_lo, fx_hi);
   } else {
     unsigned long long *lo = LDS_TALLY ? t0 : fx_lo, *hi = LDS_TALLY ? t1 : fx_hi;
-    mc_walk_bank(io, queue, L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
-                 [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+    mc_walk_bank<LDS_CELLS>(io, queue, L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
+                 [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
                    if (mc_in(lanes)) {
-                     mc_tally(lo, hi, flags, status, c, dw);
-                     if (SCORE) io.score = io.score + g[c] * dw;
+                     mc_tally(lo, hi, flags, status, c8 >> 3, dw);
+                     if (SCORE) io.score = io.score + *mc_word(g, c8) * dw;
                    }
                  },
                  [](int) {});
@@ -389,7 +388,7 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
 int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
                       hipStream_t s) {
   const size_t m = (size_t)a.L.m;
-  const size_t tally = 16 * m + MC_TAB_BYTES, cells = sizeof(mc_cell) * m;
+  const size_t tally = 16 * m + MC_TAB_BYTES, cells = sizeof(mc_cell) * m + MC_PAD_BYTES;
   const size_t budget = ctx->lds_per_block - 256; /* the kernel's static LDS */
   const bool lds_tally = tally <= budget;
   /* wide layers: equal windows that fill the LDS; with scratch for them (not

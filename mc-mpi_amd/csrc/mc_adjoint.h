@@ -37,18 +37,18 @@ enum { MC_GRAD_GLOBAL, MC_GRAD_LIMBS, MC_GRAD_CARRY }; /* fx; t as limbs; t with
 
 /* which: 0 sig_a, 1 sig_i; called by the whole wave */
 template <int MODE>
-__device__ __forceinline__ void mc_grad_add(const mc_grad_tally &G, int which, mc_mask lanes, int c,
+__device__ __forceinline__ void mc_grad_add(const mc_grad_tally &G, int which, mc_mask lanes, int c8,
                                             double v) {
   lanes &= mc_lanes(v != 0.0); /* (NaN differs from 0) */
   unsigned long long *fx = G.fx + 2 * which * G.stride;
   uint32_t *flags = which ? G.flags_i : G.flags_a;
   if (MODE == MC_GRAD_GLOBAL) {
-    if (mc_in(lanes)) mc_tally<true>(fx, fx + G.stride, flags, G.status, c, v);
+    if (mc_in(lanes)) mc_tally<true>(fx, fx + G.stride, flags, G.status, c8 >> 3, v);
     return;
   }
   if (MODE == MC_GRAD_CARRY) {
     unsigned long long *t = G.t + 2 * which * G.m;
-    if (mc_in(lanes)) mc_tally<true>(t, t + G.m, flags, G.status, c, v);
+    if (mc_in(lanes)) mc_tally<true>(t, t + G.m, flags, G.status, c8 >> 3, v);
     return;
   }
   mc_mask take = lanes & mc_lanes(mc_fx_split_signed_direct(v, &G.S));
@@ -56,14 +56,14 @@ __device__ __forceinline__ void mc_grad_add(const mc_grad_tally &G, int which, m
     bool small = false;
     if (mc_in(lanes & ~take)) {
       small = mc_fx_split_signed_small(&v);
-      if (!small) mc_tally_general(fx, fx + G.stride, flags, G.status, c, v);
+      if (!small) mc_tally_general(fx, fx + G.stride, flags, G.status, c8 >> 3, v);
     }
     take |= mc_lanes(small);
   }
   if (mc_in(take)) {
     uint64_t n0, n1;
     mc_fx_split_limbs(v, &G.S, &n0, &n1);
-    unsigned long long *t = G.t + 2 * which * G.m + c;
+    unsigned long long *t = mc_word(G.t + 2 * which * G.m, c8);
     atomicAdd(t, (unsigned long long)n0);
     atomicAdd(t + G.m, (unsigned long long)n1);
   }
@@ -131,11 +131,11 @@ template <bool HAVE_SCORE> struct mc_grad_io {
 /* one event of `lanes` (mc_walk_many's on_event) */
 template <int MODE, bool HAVE_SCORE>
 __device__ __forceinline__ void mc_grad_event(mc_grad_io<HAVE_SCORE> &io, const mc_grad_tally &G,
-                                              const double *g, mc_mask lanes, int c,
+                                              const double *g, mc_mask lanes, int c8,
                                               const mc_cell &cell, bool coll, double di, double dw,
                                               double wmc) {
   double gc = 0.0;
-  if (mc_in(lanes)) gc = g[c];
+  if (mc_in(lanes)) gc = *mc_word(g, c8);
   if (!HAVE_SCORE) {
     const mc_mask first = lanes & mc_lanes(io.phase == 0);
     if (mc_in(first)) io.T = io.T + gc * dw;
@@ -143,8 +143,8 @@ __device__ __forceinline__ void mc_grad_event(mc_grad_io<HAVE_SCORE> &io, const 
   }
   double term_a, term_i;
   mc_adjoint_terms(cell, coll, di, dw, gc, wmc, io.T, io.P, term_a, term_i);
-  mc_grad_add<MODE>(G, 0, lanes, c, term_a);
-  mc_grad_add<MODE>(G, 1, lanes & mc_lanes(cell.sig_i > MC_EPS), c, term_i);
+  mc_grad_add<MODE>(G, 0, lanes, c8, term_a);
+  mc_grad_add<MODE>(G, 1, lanes & mc_lanes(cell.sig_i > MC_EPS), c8, term_i);
   if (mc_in(lanes)) io.P = io.P + gc * dw;
 }
 

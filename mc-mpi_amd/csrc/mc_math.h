@@ -155,6 +155,15 @@ MC_FN double mc_div_by_rcp(double a, double b, double y) {
   return mc_fma(r1, y, q1);
 }
 
+/* a / b for 1/b = rh + rl (rh = RN(1/b), rl = RN((1 - b rh) rh)): q0 is within
+   1 ulp of the quotient, and one Markstein step with rh makes it the correctly
+   rounded one.  Without a test of the range: exact where 2^-60 <= |b| <= 2^64
+   and a is 0 or 2^-752 <= |a| <= 2^700. */
+MC_FN double mc_div_by_pair(double a, double b, double rh, double rl) {
+  const double q0 = mc_fma(a, rh, a * rl);
+  return mc_fma(mc_fma(-b, q0, a), rh, q0);
+}
+
 /* ------------------------------------------------------------------- log */
 
 /* log(x) as double-double, all steps in double-double (about 2^-100 rel). */

@@ -234,3 +234,35 @@ def test_wide_layer_scores(ctx, oracle):
     ctx.forward_cells(db, dev(sa), dev(ss), w, 0, m, dx, 1e-3, g=dev(g), history_score=sc)
     assert np.array_equal(w.cpu().numpy(), o["tally_exact"])
     assert np.array_equal(sc.cpu().numpy().view(np.uint64), o["score"].view(np.uint64))
+
+
+@pytest.mark.parametrize("kernel", ["history", "event"])
+@pytest.mark.parametrize("dx", [1e-190, 1e-3, 1.0, 1e190])
+def test_particles_at_the_bounds_of_the_common_step(ctx, oracle, dx, kernel):
+    """Directions from grazing to far above 1, positions of 0, tiny, on and
+    beyond an edge, and cell widths for which the common step is not used."""
+    import mcgpu
+    _say(f"bounds of the common step dx={dx} {kernel}")
+    m = 24
+    sigs, ar, _, bank = _case(m, 2000, 61, 1.0)
+    sigs = sigs * 0.2 / dx
+    rng = np.random.default_rng(62)
+    bank["x"] = (bank["index"] + rng.random(2000)) * dx
+    edge = rng.integers(0, 2000, 500)
+    bank["x"][edge] = (bank["index"][edge] + rng.integers(0, 2, 500)) * dx
+    bank["x"][::97] += 0.5 * dx
+    first = bank["index"] == 0
+    bank["x"][first] = rng.choice([0.0, 5e-324, 2.0 ** -701, 2.0 ** -700, 1e-150], first.sum()) * dx
+    eps = 1e-4
+    mus = np.array([0.0, eps, np.nextafter(eps, 1), 1e-9, 1.0, 3.0, 2.0 ** 64, 2.0 ** 65, 1e150])
+    bank["mu"][::3] = (mus[rng.integers(0, mus.size, 667)] * rng.choice([-1.0, 1.0], 667))
+    o = oracle.simulate_bank(64, 0, m, dx, 1e-2, sigs, ar, bank, nthread=8)
+    b, w = bank.copy(), np.zeros(m)
+    result, st, rc = ctx.simulate(b, sigs, ar, w, 0, m, dx, 1e-2,
+                                  options=mcgpu.make_options(kernel))
+    assert rc == 0
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f], equal_nan=f not in ("seed", "index")), f
+    assert np.array_equal(result, o["result"])
+    assert st["events"] == int(o["events"].sum())
+    assert np.array_equal(w, o["tally_exact"])

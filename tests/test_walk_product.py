@@ -57,6 +57,19 @@ void pw_signed_limbs(const double *v, long n, int V, uint64_t *out, int8_t *take
     out[2 * i + 1] = r.hi;
   }
 }
+void pw_quotient(const double *a, const double *b, long n, double *q) {
+  for (long i = 0; i < n; ++i) {
+    const double rh = 1.0 / b[i], rl = mc_fma(-b[i], rh, 1.0) * rh;
+    q[i] = mc_div_by_pair(a[i], b[i], rh, rl);
+  }
+}
+/* 1 + (the top 20 of h's 32 high bits) + sig_i di < 2 - 2^-18 */
+void pw_crosses(const uint32_t *sh, const double *sig_i, const double *di, long n, int8_t *sure) {
+  for (long i = 0; i < n; ++i) {
+    const double h1 = mc_asf64((uint64_t)(0x3FF00000u | (sh[i] >> 12)) << 32);
+    sure[i] = mc_fma(sig_i[i], di[i], h1) < 2.0 - 0x1p-18;
+  }
+}
 int pw_signed_log2_terms(int V) { return mc_fx_split_signed_log2_terms(V); }
 int pw_L(int V) { return mc_fx_split_for(V).L; }
 int pw_log2_terms(int V) { return mc_fx_split_log2_terms(V); }
@@ -84,6 +97,8 @@ def pw(tmp_path_factory):
     L.pw_absorb.argtypes = [p, n, i, p, p]
     L.pw_limbs.argtypes = L.pw_signed_limbs.argtypes = [p, n, i, p, p, p, p]
     L.pw_join.argtypes = [p, p, n, i, p]
+    L.pw_quotient.argtypes = [p, p, n, p]
+    L.pw_crosses.argtypes = [p, p, p, n, p]
     return L
 
 
@@ -204,3 +219,51 @@ def test_limb_sums_join_with_borrow_and_carry(pw):
         for i in range(5000):
             s = (int(n1[i]) << L) + int(n0[i])
             assert (int(out[2 * i + 1]) << 64 | int(out[2 * i])) == s % (1 << 128)
+
+
+def test_edge_quotient_is_the_ieee_division(pw):
+    """a / b by the pair equals the division over the stated ranges: random,
+    next to a representable or halfway quotient, powers of two, and zero."""
+    rng = np.random.default_rng(26)
+    n = 3_000_000
+    b = rng.uniform(1, 2, n) * np.ldexp(1.0, rng.integers(-60, 64, n)) * rng.choice([-1.0, 1.0], n)
+    b[: n // 2] = rng.uniform(-1, 1, n // 2)
+    b[np.abs(b) < 1e-12] = 1.0
+    a = rng.uniform(1, 2, n) * np.ldexp(1.0, rng.integers(-752, 700, n)) * rng.choice([-1.0, 1.0], n)
+    k = slice(0, n // 2, 2)
+    q = rng.uniform(1, 2, a[k].size)
+    a[k] = q * b[k]  # quotients next to a double
+    a[k] = np.nextafter(a[k], rng.choice([-np.inf, 0, np.inf], a[k].size))
+    k = slice(1, n // 2, 2)
+    a[k] = rng.integers(0, 1000, a[k].size) * 1e-3 - rng.uniform(0, 1, a[k].size)
+    p2 = np.ldexp(1.0, np.arange(-60, 65))
+    b = np.concatenate([b, p2, np.nextafter(p2[1:-1], 0), np.nextafter(p2[:-1], np.inf), [1.0, -3.0]])
+    a = np.concatenate([a, rng.uniform(-1, 1, b.size - n)])
+    a[-2:] = 0.0
+    got = np.empty_like(a)
+    pw.pw_quotient(a.ctypes.data, b.ctypes.data, a.size, got.ctypes.data)
+    assert np.array_equal(got, a / b)
+
+
+def test_crossing_by_20_bits_never_takes_a_collision(pw, oracle):
+    """Where the 20-bit sum certifies a crossing, the sampled flight
+    -log(h) / sig_i is not below the way to the edge; cells whose sum lies next
+    to the limit are in the sample, and both answers occur."""
+    rng = np.random.default_rng(27)
+    n = 1_000_000
+    sh = rng.integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32)
+    h = sh * 2.0 ** -32 + rng.integers(0, 2 ** 31, n) * 2.0 ** -63
+    sig = 2.0 ** rng.uniform(-30, 12, n)
+    reach = 2.0 ** rng.uniform(-30, 0.1, n)
+    reach[::2] = np.maximum(1 - h[::2], 2.0 ** -30) * (1 + rng.normal(0, 1, n // 2) * 2.0 ** -17)
+    reach[::8] = 0.0
+    di = reach / sig
+    sure = np.empty(n, np.int8)
+    pw.pw_crosses(sh.ctypes.data, sig.ctypes.data, di.ctypes.data, n, sure.ctypes.data)
+    sure = sure != 0
+    assert 0.1 < sure.mean() < 0.9
+    h = np.maximum(h, 2.0 ** -63)
+    flight = -oracle.math_eval("log", h) / sig
+    assert not (flight[sure] < di[sure]).any()
+    near = sure & (1 - h < reach * (1 + 2.0 ** -14)) & (reach > 2.0 ** -3)
+    assert near.any()
