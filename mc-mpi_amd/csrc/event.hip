@@ -274,6 +274,8 @@ struct pool_queue {
   rsrc_t src;
   int F_CW, n, next;
   __device__ __forceinline__ bool more() const { return next < n; }
+  static constexpr bool LEAVES = false;
+  __device__ __forceinline__ int least() const { return 8; }
   __device__ __forceinline__ int64_t take(mc_mask need) {
     int slot = -1;
     while (need != 0 && next < n) { /* wave-uniform */

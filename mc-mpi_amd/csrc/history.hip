@@ -18,8 +18,8 @@
  * mc_fx_split; for weights too large for them, two words with carry) and adds
  * it to the global 128-bit tally at the end, and before limbs could overflow.
  * Integer sums are exact, so the result is independent of which lane, wave or
- * block handled which history.  For layers too large for LDS the adds go to
- * the global (L2-resident) tally.  The per-cell cross-section pairs are staged
+ * block handled which history.  Layers too large for LDS are transported in
+ * windows (below).  The per-cell cross-section pairs are staged
  * in LDS when they fit next to the tally, otherwise read through L2.
  *
  * Measured against the kernel with mc_event and a tally with carry: a lone
@@ -58,22 +58,57 @@ template <bool SCORE> struct bank_io {
 };
 
 /* ------------------------------------------------------------- wide layers
-   A layer of more cells than a block's LDS tally holds is cut into windows.
-   A sweep transports the histories of every window, each block one window's;
-   a history that crosses into another window is parked there for the next
-   sweep, until none is left.  A history crosses a window's edge a few times at
-   most (windows are thousands of cells, flights a good part of the layer), so
-   parking costs little, where a global tally costs two returning atomics in
-   memory per event: 200,000 histories on 20,000 cells 540 -> 118 ms. */
+   A layer of more cells than a block's LDS tally holds is cut into windows
+   whose cells and tally fit; each block transports the histories of one
+   window.  A history that crosses into another window is parked: its state
+   goes to memory and its number into that window's ring, from which the
+   window's blocks refill their lanes.  A block that has run dry, or has few
+   histories left while many wait elsewhere, empties its tally, parks what it
+   has and takes the window with the most waiting histories per block.  So all
+   windows are worked at once, wherever the histories are, and the whole call
+   is one launch; a history crosses a window's edge a few times at most
+   (windows are thousands of cells, flights a good part of the layer).
+   Histories whose ring slot was lost (a full ring, a wave that gave up
+   waiting for it) are found by the next sweep; usually there is none.
+   Measured against a global tally (two returning atomics in memory per event)
+   and against sweeps in which a parked history waits for the next launch:
+   200,000 histories on 20,000 cells 540, 106 and 45 ms; 2 M 161 ms (228 by
+   sweeps); 200,000 on 50,000 cells 102 ms (236); 1,000 on 20,000 21.6 ms (56).
+   Layers whose tally alone fits keep one window: 10,000 cells and 2 M
+   histories take 67 ms in two windows and 70 in one, 300,000 25 and 22, 2 M on
+   6,000 cells 46 and 37 (histories that refill a lane at the same edge walk on
+   together and meet in the LDS banks). */
 constexpr int MC_MAX_WINDOWS = 64;
 
 struct mc_windows {
   int32_t nw, W;            /* window w: cells [w W, (w + 1) W) of the layer */
-  uint32_t *count;          /* [nw] histories of this sweep */
+  uint32_t *count;          /* [nw] histories at the sweep's start */
   unsigned long long *next; /* [nw] queue counters */
-  const uint32_t *list;     /* histories, by window */
-  int32_t *win;             /* [n] a history's window, -1 when finished */
+  const uint32_t *list;     /* those histories, by window */
+  int32_t *at;              /* [n] the cell of a parked history, -1 when finished */
   uint64_t *ev;             /* [n] its events so far */
+  /* histories parked in the course of a sweep: window w's are a ring of cap
+     slots at parked + w cap, put[w] - got[w] of them waiting */
+  uint32_t *parked, *put, *got; /* [nw cap], [nw], [nw] */
+  uint32_t *blocks;             /* [nw] blocks that transport window w */
+  uint32_t *left;               /* histories not known to be finished */
+  uint32_t cap;
+  int patience; /* looks of an idle block before it ends */
+};
+constexpr uint32_t MC_NOT_PUT = 0xFFFFFFFFu;
+
+/* words of different windows lie on different lines */
+constexpr int MC_WINDOW_STEP = 32;
+
+/* LDS words of a block */
+struct mc_window_block {
+  unsigned long long run; /* the block's run of parked histories: next, end << 32 */
+  unsigned int looked;    /* clock of the last look at the windows' counts */
+  int looking;
+  int busy;               /* lanes with a history */
+  int leave;              /* the block parks its histories and takes another window */
+  uint32_t done;          /* histories finished */
+  int w;                  /* the window chosen */
 };
 
 /* windows of a sweep and the blocks they get: one each, the rest by count */
@@ -101,34 +136,260 @@ __device__ __forceinline__ mc_window_share mc_window_of(const mc_windows &win) {
   return s;
 }
 
+/* Words that another block may have written, or will read, within the sweep:
+   past the caches of this XCD (agent scope) */
+template <typename T> __device__ __forceinline__ T ld_shared(const T *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> __device__ __forceinline__ void st_shared(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <typename T> __device__ __forceinline__ T ld_block(const T *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 template <bool SCORE> struct window_io {
   static constexpr bool RESUMES = true;
   const mc_transport_args &a;
   const mc_windows &win;
-  const uint32_t *list;
+  int32_t w; /* the block's window */
+  mc_window_block *blk;
   double score;
-  int64_t j;
-  int to; /* window a history is parked in, -1: finished */
-  __device__ __forceinline__ uint64_t load(int64_t i, mc_state &p) {
-    j = list[i];
-    load_state(a, j, p);
-    if (SCORE) score = a.score[j];
-    return win.ev[j];
+  int to; /* cell a history is parked in, -1: finished */
+  __device__ __forceinline__ uint64_t load(int64_t j, mc_state &p) {
+    if (a.aos) {
+      const mcgpu_particle *q = a.aos + j;
+      p.seed = ld_shared(&q->seed);
+      p.x = ld_shared(&q->x);
+      p.mu = ld_shared(&q->mu);
+      p.wmc = ld_shared(&q->wmc);
+      p.index = ld_shared(&q->index);
+    } else {
+      p.seed = ld_shared(&a.soa.seed[j]);
+      p.x = ld_shared(&a.soa.x[j]);
+      p.mu = ld_shared(&a.soa.mu[j]);
+      p.wmc = ld_shared(&a.soa.wmc[j]);
+      p.index = ld_shared(&a.soa.index[j]);
+    }
+    if (SCORE) score = ld_shared(&a.score[j]);
+    return ld_shared(&win.ev[j]);
   }
   __device__ __forceinline__ int code(const mc_state &p, bool at_cap, const mc_layer_k &) {
-    to = mc_alive(p, a.L) && !at_cap ? (p.index - a.L.index_start) / win.W : -1;
+    to = mc_alive(p, a.L) && !at_cap ? p.index - a.L.index_start : -1;
     return to >= 0 ? 3 : mc_end_code(p, at_cap, a.L);
   }
-  __device__ __forceinline__ bool store(int64_t, mc_state &p, int code, uint64_t ev, uint32_t col) {
-    store_state(a, j, p, code);
-    win.ev[j] = ev;
-    win.win[j] = to;
-    if (a.events) a.events[j] = ev;
-    if (a.collisions) a.collisions[j] += col;
-    if (SCORE) a.score[j] = score;
+  __device__ __forceinline__ bool store(int64_t j, mc_state &p, int code, uint64_t ev,
+                                        uint32_t col) {
+    if (a.collisions) st_shared(&a.collisions[j], ld_shared(&a.collisions[j]) + col);
+    if (SCORE) st_shared(&a.score[j], score);
+    if (to < 0) {
+      store_state(a, j, p, code);
+      if (a.events) a.events[j] = ev;
+      win.at[j] = -1;
+      atomicAdd(&blk->done, 1u);
+      return false;
+    }
+    if (a.aos) {
+      mcgpu_particle *q = a.aos + j;
+      st_shared(&q->seed, p.seed);
+      st_shared(&q->x, p.x);
+      st_shared(&q->mu, p.mu);
+      st_shared(&q->wmc, p.wmc);
+      st_shared(&q->index, p.index);
+    } else {
+      st_shared(&a.soa.seed[j], p.seed);
+      st_shared(&a.soa.x[j], p.x);
+      st_shared(&a.soa.mu[j], p.mu);
+      st_shared(&a.soa.wmc[j], p.wmc);
+      st_shared(&a.soa.index[j], p.index);
+    }
+    st_shared(&win.ev[j], ev);
+    st_shared(&win.at[j], (int32_t)to);
+    /* all of it in memory before the history's number can be seen there */
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int32_t v = to / win.W;
+    if (win.cap) {
+      put(j, v, v < w);
+      put(j, v, v == w);
+      put(j, v, v > w);
+    }
     return false;
   }
+  /* the lanes with `mine`, all of the same window v */
+  __device__ __forceinline__ void put(int64_t j, int32_t v, bool mine) {
+    if (!mine) return;
+    const mc_mask lanes = mc_lanes(true);
+    const uint32_t rank = (uint32_t)mc_mbcnt64(lanes);
+    uint32_t base = 0;
+    if (rank == 0) base = atomicAdd(&win.put[v * MC_WINDOW_STEP], (uint32_t)__popcll(lanes));
+    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+    st_shared(&win.parked[(size_t)v * win.cap + (base + rank) % win.cap], (uint32_t)j);
+  }
 };
+
+/* the parked histories of window v (0: none), read past the caches */
+__device__ __forceinline__ uint32_t mc_window_waiting(const mc_windows &win, int v) {
+  const uint32_t got = ld_shared(win.got + v * MC_WINDOW_STEP);
+  const uint32_t have = ld_shared(win.put + v * MC_WINDOW_STEP) - got;
+  return (int32_t)have > 0 ? have : 0u;
+}
+
+/* `want` of a window's parked histories, or a share of many, for a block (by
+   one lane): its run, 0 if there are none */
+__device__ __forceinline__ unsigned long long mc_window_claim(const mc_windows &win, int w,
+                                                              uint32_t want) {
+  uint32_t *got = win.got + w * MC_WINDOW_STEP;
+  uint32_t at = ld_shared(got);
+  for (int t = 0; t < 8; ++t) {
+    const uint32_t have = ld_shared(win.put + w * MC_WINDOW_STEP) - at;
+    if ((int32_t)have <= 0) return 0;
+    const uint32_t share = have / (2u * gridDim.x);
+    uint32_t size = share > want ? share : want;
+    size = size < have ? size : have;
+    const uint32_t was = atomicCAS(got, at, at + size);
+    if (was == at) return (unsigned long long)at | ((unsigned long long)(at + size) << 32);
+    at = was;
+  }
+  return 0;
+}
+
+/* A wave's histories of a window: those of its list, then those parked in it
+   meanwhile.  Nothing waits long for a history to be parked: one that no wave
+   takes is in the next sweep's list. */
+struct mc_window_queue {
+  static constexpr bool LEAVES = true;
+  mc_call_queue open; /* none after the block's first window */
+  const uint32_t *list;
+  const mc_windows &win;
+  mc_window_block *blk;
+  int32_t w;
+  int lanes; /* of the wave, counted in blk->busy */
+  bool starved;
+  __device__ __forceinline__ bool more() const { return true; }
+  __device__ __forceinline__ int least() const { return starved ? 64 : 8; }
+  __device__ __forceinline__ int64_t take(mc_mask need) {
+    int64_t j = -1;
+    if (open.more()) { /* wave-uniform */
+      const int64_t i = open.take(need);
+      if (mc_in(need) && i >= 0) j = list[i];
+      need &= ~mc_lanes(j >= 0);
+      if (need == 0 || open.more()) return j;
+    }
+    const uint32_t cnt = (uint32_t)__popcll(need);
+    uint32_t next = 0, have = 0;
+    if (__lane_id() == 0 && win.cap) {
+      unsigned long long run = ld_block(&blk->run);
+      if ((int32_t)((uint32_t)(run >> 32) - (uint32_t)run) > 0) {
+        run = atomicAdd(&blk->run, (unsigned long long)cnt); /* next stays below 2^32: see look */
+        next = (uint32_t)run;
+        const int32_t d = (int32_t)((uint32_t)(run >> 32) - next);
+        have = d > 0 ? (uint32_t)d : 0u;
+      }
+    }
+    next = (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
+    have = (uint32_t)__builtin_amdgcn_readfirstlane((int)have);
+    const uint32_t rank = (uint32_t)mc_mbcnt64(need);
+    starved = have < cnt;
+    if (mc_in(need) && rank < have) {
+      uint32_t *slot = win.parked + (size_t)w * win.cap + (next + rank) % win.cap;
+      uint32_t v = MC_NOT_PUT;
+      /* put[] counts it, so its number is on the way; if it does not come in
+         time, it stays for the next sweep */
+      for (int t = 0; t < 1024 && v == MC_NOT_PUT; ++t) v = ld_shared(slot);
+      if (v != MC_NOT_PUT) v = atomicExch(slot, MC_NOT_PUT);
+      if (v != MC_NOT_PUT) j = v;
+    }
+    return j;
+  }
+  /* counts the wave's lanes in use; when the block's run is used up, one wave
+     every 40,000 cycles takes another, or finds that the block had better
+     leave for another window.  Returns whether the wave is to park its
+     histories and leave. */
+  __device__ __forceinline__ bool leave(int used) {
+    if (used != lanes) {
+      if (__lane_id() == 0) atomicAdd(&blk->busy, used - lanes);
+      lanes = used;
+    }
+    if (starved && win.cap) look();
+    return __builtin_amdgcn_readfirstlane(ld_block(&blk->leave)) != 0 && !open.more();
+  }
+  __device__ __forceinline__ bool has_run() const {
+    const unsigned long long run = ld_block(&blk->run);
+    return (int32_t)((uint32_t)(run >> 32) - (uint32_t)run) > 0;
+  }
+  __device__ __forceinline__ void look() {
+    const unsigned int now = (unsigned int)__builtin_readcyclecounter();
+    int mine = 0;
+    if (__lane_id() == 0) {
+      if ((int32_t)(now - ld_block(&blk->looked)) > 40000 && atomicCAS(&blk->looking, 0, 1) == 0) {
+        mine = !has_run() && ld_block(&blk->leave) == 0; /* under the lock: no other wave claims */
+        if (!mine) atomicExch(&blk->looking, 0);
+      }
+    }
+    if (!__builtin_amdgcn_readfirstlane(mine)) return;
+    const int v = (int)__lane_id();
+    const int busy = __builtin_amdgcn_readfirstlane(ld_block(&blk->busy));
+    const int idle = (int)blockDim.x - busy;
+    const uint32_t have = v < win.nw ? mc_window_waiting(win, v) : 0u;
+    if (v == 0) blk->looked = now;
+    if (mc_lanes(v == w && have != 0)) {
+      if (v == 0) {
+        const unsigned long long run = mc_window_claim(win, w, idle > 64 ? (uint32_t)idle : 64u);
+        if (run) atomicExch(&blk->run, run);
+      }
+    } else if (busy * 4 < (int)blockDim.x) {
+      const uint32_t least = busy > 128 ? 4u * (uint32_t)busy : 512u;
+      if (mc_lanes(have >= least) && v == 0) atomicExch(&blk->leave, 1);
+    }
+    if (v == 0) atomicExch(&blk->looking, 0);
+  }
+  /* with no history: whether the block still transports some of the window */
+  __device__ __forceinline__ bool wait() const {
+    if (win.cap == 0) return false;
+    if (__builtin_amdgcn_readfirstlane(has_run())) return true;
+    if (__builtin_amdgcn_readfirstlane(ld_block(&blk->busy)) == 0) return false;
+    __builtin_amdgcn_s_sleep(127);
+    return true;
+  }
+};
+
+/* by the first wave of a block without histories: a window with parked ones
+   and a run of them, in blk; blk->w = -1: none came up while the block waited */
+__device__ __forceinline__ void mc_window_choose(const mc_windows &win, mc_window_block *blk) {
+  const int v = (int)__lane_id();
+  int chosen = -1;
+  unsigned long long run = 0;
+  for (int t = 0; t < win.patience; ++t) { /* wave-uniform */
+    uint64_t key = 0;
+    if (v < win.nw) {
+      const uint32_t have = mc_window_waiting(win, v);
+      const uint32_t there = ld_shared(win.blocks + v * MC_WINDOW_STEP);
+      if (have) key = ((((uint64_t)have << 6) / (there + 1u) + 1u) << 8) | (uint64_t)v;
+    }
+    const uint64_t best = mc_wave_max_u64(key);
+    if (best) {
+      const int w = __builtin_amdgcn_readfirstlane((int)(best & 255u));
+      if (v == 0) {
+        run = mc_window_claim(win, w, blockDim.x);
+        if (run) atomicAdd(&win.blocks[w * MC_WINDOW_STEP], 1u);
+      }
+      if (mc_readlane64(run, 0)) {
+        chosen = w;
+        break;
+      }
+    } else {
+      if (__builtin_amdgcn_readfirstlane((int)ld_shared(win.left)) <= 0) break;
+      for (int r = 0; r < 10; ++r) __builtin_amdgcn_s_sleep(127);
+    }
+  }
+  if (v == 0) {
+    blk->w = chosen;
+    blk->run = run;
+    blk->busy = blk->leave = 0;
+  }
+}
 
 __global__ void k_windows_clear(mc_windows win, uint32_t *cursor) {
   const int t = threadIdx.x;
@@ -136,6 +397,9 @@ __global__ void k_windows_clear(mc_windows win, uint32_t *cursor) {
   win.count[t] = 0;
   cursor[t] = 0;
   win.next[t] = 0;
+  win.put[t * MC_WINDOW_STEP] = win.got[t * MC_WINDOW_STEP] = 0;
+  win.blocks[t * MC_WINDOW_STEP] = 0;
+  if (t == 0) *win.left = 0;
 }
 
 /* the histories of each window; OPEN: their first windows, from the bank */
@@ -150,31 +414,37 @@ template <bool OPEN> __global__ void k_windows_count(mc_transport_args a, mc_win
       mc_state p;
       load_state(a, i, p);
       const uint32_t c = (uint32_t)p.index - (uint32_t)a.L.index_start;
-      w = c < (uint32_t)a.L.m ? (int)(c / (uint32_t)win.W) : 0;
-      win.win[i] = w;
+      w = c < (uint32_t)a.L.m ? (int)c : 0;
+      win.at[i] = w;
       win.ev[i] = 0;
       if (a.collisions) a.collisions[i] = 0;
       if (a.score) a.score[i] = 0.0;
     } else {
-      w = win.win[i];
+      w = win.at[i];
     }
-    if (w >= 0) atomicAdd(&s_n[w], 1u);
+    if (w >= 0) atomicAdd(&s_n[w / win.W], 1u);
   }
   __syncthreads();
-  if (threadIdx.x < (unsigned)win.nw && s_n[threadIdx.x])
+  if (threadIdx.x < (unsigned)win.nw && s_n[threadIdx.x]) {
     atomicAdd(&win.count[threadIdx.x], s_n[threadIdx.x]);
+    atomicAdd(win.left, s_n[threadIdx.x]);
+  }
 }
 
-/* the histories of each window one after the other (cursors zeroed) */
+/* the histories of each window one after the other (cursors zeroed), and
+   room for those parked in the sweep */
 __global__ void k_windows_list(int64_t n, mc_windows win, uint32_t *list, uint32_t *cursor) {
   __shared__ uint32_t s_n[MC_MAX_WINDOWS], s_at[MC_MAX_WINDOWS];
   const int t = threadIdx.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + t; i < (size_t)win.nw * win.cap;
+       i += (size_t)gridDim.x * blockDim.x)
+    win.parked[i] = MC_NOT_PUT;
   for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n;
        base += (int64_t)gridDim.x * blockDim.x) { /* block-uniform */
     if (t < MC_MAX_WINDOWS) s_n[t] = 0;
     __syncthreads();
     const int64_t i = base + t;
-    const int w = i < n ? win.win[i] : -1;
+    const int at = i < n ? win.at[i] : -1, w = at >= 0 ? at / win.W : -1;
     uint32_t r = 0;
     if (w >= 0) r = atomicAdd(&s_n[w], 1u);
     __syncthreads();
@@ -191,9 +461,9 @@ __global__ void k_windows_list(int64_t n, mc_windows win, uint32_t *list, uint32
 
 /* one block's part of layer L (cells and global tally words at cells, fx_lo,
    fx_hi, ...): LDS, the walk, the tally and totals */
-template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE, typename IO>
+template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE, typename IO, typename Queue>
 __device__ __forceinline__ void history_block(const mc_transport_args &a, const mc_layer_k &L,
-                                              int off, IO &io, mc_call_queue &queue, double wmc,
+                                              int off, IO &io, Queue &queue, double wmc,
                                               int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_k;
@@ -278,21 +548,62 @@ __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refil
 }
 
 /* one sweep over the windows of a wide layer */
-template <bool SCORE>
+template <bool LDS_CELLS, bool SCORE>
 __global__ __launch_bounds__(1024) void k_history_windows(mc_transport_args a, mc_windows win,
                                                           int refill_k, int per_cu) {
+  __shared__ mc_window_block blk;
   const mc_window_share sh = mc_window_of(win);
-  if (sh.w < 0) return; /* block-uniform: no window left for this block */
-  const int w = __builtin_amdgcn_readfirstlane(sh.w), off = w * win.W;
-  mc_layer_k L = a.L;
-  L.index_start += off;
-  L.m = a.L.m - off < win.W ? a.L.m - off : win.W;
-  mc_call_queue queue{mc_queue_open(win.count[w], per_cu, sh.block, sh.blocks), &win.next[w]};
-  window_io<SCORE> io{a, win, win.list + sh.first, 0.0, 0, -1};
-  const uint64_t i = queue.q.next + __lane_id();
-  double wmc = 0.0;
-  if (i < queue.q.end) wmc = a.aos ? a.aos[io.list[i]].wmc : a.soa.wmc[io.list[i]];
-  history_block<true, false, SCORE>(a, L, off, io, queue, wmc, refill_k);
+  if (threadIdx.x == 0) {
+    blk = {0, 0, 0, 0, 0, 0, sh.w};
+    if (sh.w >= 0) atomicAdd(&win.blocks[sh.w * MC_WINDOW_STEP], 1u);
+  }
+  __syncthreads();
+  int w = __builtin_amdgcn_readfirstlane(sh.w);
+  for (bool first = true;; first = false) {
+    if (!first || w < 0) { /* block-uniform */
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        if (w >= 0) atomicSub(&win.blocks[w * MC_WINDOW_STEP], 1u);
+        if (blk.done) atomicSub(win.left, blk.done);
+        blk.done = 0;
+      }
+      if (threadIdx.x < 64) mc_window_choose(win, &blk);
+      __syncthreads();
+      w = __builtin_amdgcn_readfirstlane(blk.w);
+      if (w < 0) return;
+    }
+    const int off = w * win.W;
+    mc_layer_k L = a.L;
+    L.index_start += off;
+    L.m = a.L.m - off < win.W ? a.L.m - off : win.W;
+    const bool listed = first && sh.w >= 0;
+    mc_window_queue queue{
+        {mc_queue_open(listed ? win.count[w] : 0, per_cu, listed ? sh.block : 0u,
+                       listed ? sh.blocks : 1u), &win.next[w]},
+        win.list + sh.first, win, &blk, w, 0, false};
+    window_io<SCORE> io{a, win, w, &blk, 0.0, -1};
+    const uint64_t i = queue.open.q.next + __lane_id();
+    int64_t j = -1;
+    if (i < queue.open.q.end) {
+      j = queue.list[i];
+    } else { /* threads look at the run's first histories; none is taken yet */
+      const uint32_t next = (uint32_t)blk.run, end = (uint32_t)(blk.run >> 32);
+      if (threadIdx.x < end - next) {
+        const uint32_t v =
+            ld_shared(&win.parked[(size_t)w * win.cap + (next + threadIdx.x) % win.cap]);
+        if (v != MC_NOT_PUT) j = v;
+      }
+    }
+    double wmc = 0.0;
+    if (j >= 0) wmc = ld_shared(a.aos ? &a.aos[j].wmc : &a.soa.wmc[j]);
+    history_block<true, LDS_CELLS, SCORE>(a, L, off, io, queue, wmc, refill_k);
+  }
+}
+
+/* LDS bytes of a window of W cells, with its cells (and targets) or without */
+constexpr size_t window_lds(size_t W, bool cells, bool score) {
+  return MC_TAB_BYTES + 16 * W +
+         (cells ? sizeof(mc_cell) * W + MC_PAD_BYTES + (score ? 8 * W : 0) : 0);
 }
 
 template <bool T, bool C, bool S>
@@ -323,13 +634,15 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
   return MCGPU_OK;
 }
 
-/* Sweeps over a wide layer's windows until no history is parked.  Scratch (16
-   bytes per history) from the context; MCGPU_ERR_NOMEM: there is none. */
-template <bool S>
+/* Sweeps over a wide layer's windows, cells in LDS or not, until no history is
+   parked.  Scratch from the context (16 bytes per history and 4 per history
+   and window); MCGPU_ERR_NOMEM: there is none. */
+template <bool LDS_CELLS, bool S>
 int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-                   hipStream_t s, int nw, int W) {
-  auto kern = k_history_windows<S>;
-  const size_t lds = MC_TAB_BYTES + 16 * (size_t)W;
+                   hipStream_t s, int nw) {
+  auto kern = k_history_windows<LDS_CELLS, S>;
+  const int W = (a.L.m + nw - 1) / nw;
+  const size_t lds = window_lds((size_t)W, LDS_CELLS, S);
   if (lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -340,25 +653,37 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, lds) != hipSuccess ||
            per_cu < 1)
     per_cu = 1;
-  const int grid = o.grid_blocks > 0 ? o.grid_blocks : per_cu * ctx->num_cus;
+  const int resident = per_cu * ctx->num_cus, grid = o.grid_blocks > 0 ? o.grid_blocks : resident;
   const int k = o.events_per_refill > 0 ? o.events_per_refill : 0;
 
-  /* ev[n], win[n], list[n], queue counters, counts, cursors */
-  const size_t n = (size_t)a.n, words = (16 * n + 255) / 256 * 256;
-  int rc = mc_ensure(ctx, &ctx->work, &ctx->work_bytes, words + 16 * MC_MAX_WINDOWS);
+  /* ev[n], at[n], list[n], parked[nw cap], queue counters, counts, cursors,
+     left, and put, got, blocks a line apart */
+  const size_t n = (size_t)a.n;
+  const size_t cap = 4 * n * (size_t)nw <= ((size_t)1 << 31) ? n : 0; /* 0: no ring */
+  const size_t words = (16 * n + 4 * cap * (size_t)nw + 255) / 256 * 256;
+  int rc = mc_ensure(ctx, &ctx->work, &ctx->work_bytes,
+                     words + (20 + 12 * MC_WINDOW_STEP) * MC_MAX_WINDOWS);
   if (rc) return rc;
   unsigned char *base = (unsigned char *)ctx->work;
   mc_windows win;
   win.nw = nw;
   win.W = W;
+  win.cap = (uint32_t)cap;
+  /* an idle block looks for parked histories for some 30 ms; at once it ends
+     if there is no ring, or if blocks that have not started wait for its place */
+  win.patience = cap == 0 ? 0 : (grid <= resident ? 1000 : 1);
   win.ev = (uint64_t *)base;
-  win.win = (int32_t *)(base + 8 * n);
+  win.at = (int32_t *)(base + 8 * n);
   uint32_t *list = (uint32_t *)(base + 12 * n);
   win.list = list;
+  win.parked = (uint32_t *)(base + 16 * n);
   win.next = (unsigned long long *)(base + words);
   win.count = (uint32_t *)(win.next + MC_MAX_WINDOWS);
   uint32_t *cursor = win.count + MC_MAX_WINDOWS;
-  uint32_t host[MC_MAX_WINDOWS];
+  win.left = cursor + MC_MAX_WINDOWS;
+  win.put = win.left + MC_MAX_WINDOWS;
+  win.got = win.put + MC_MAX_WINDOWS * MC_WINDOW_STEP;
+  win.blocks = win.got + MC_MAX_WINDOWS * MC_WINDOW_STEP;
   const unsigned blocks = (unsigned)std::min<size_t>((n + 1023) / 1024, 4 * (size_t)ctx->num_cus);
 
   for (bool first = true;; first = false) {
@@ -370,10 +695,9 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
       hipLaunchKernelGGL(k_windows_count<false>, dim3(blocks), dim3(1024), 0, s, a, win);
     MC_HIP(ctx, hipGetLastError());
     if (!first) { /* the first sweep's histories are all of them */
-      MC_HIP(ctx, hipMemcpyAsync(host, win.count, 4 * (size_t)nw, hipMemcpyDeviceToHost, s));
+      uint32_t left = 0;
+      MC_HIP(ctx, hipMemcpyAsync(&left, win.left, 4, hipMemcpyDeviceToHost, s));
       MC_HIP(ctx, hipStreamSynchronize(s));
-      uint64_t left = 0;
-      for (int w = 0; w < nw; ++w) left += host[w];
       if (left == 0) return MCGPU_OK;
     }
     hipLaunchKernelGGL(k_windows_list, dim3(blocks), dim3(1024), 0, s, a.n, win, list, cursor);
@@ -381,6 +705,24 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
     hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, win, k, per_cu);
     MC_HIP(ctx, hipGetLastError());
   }
+}
+
+/* the windows of a layer of m cells */
+int windows_of(size_t m, size_t budget, bool cells, bool score) {
+  const size_t fixed = window_lds(0, cells, score);
+  const size_t most = (budget - fixed) / (window_lds(1, cells, score) - fixed);
+  return (int)std::min<size_t>((m + most - 1) / most, 1u << 30);
+}
+
+template <bool S>
+int launch_wide(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
+                hipStream_t s, size_t budget) {
+  const int all = windows_of((size_t)a.L.m, budget, true, S);
+  const int tally = windows_of((size_t)a.L.m, budget, false, S);
+  const int limit = o.grid_blocks > 0 ? std::min(o.grid_blocks, MC_MAX_WINDOWS) : MC_MAX_WINDOWS;
+  if (all <= limit) return launch_windows<true, S>(ctx, a, o, s, all);
+  if (tally <= limit) return launch_windows<false, S>(ctx, a, o, s, tally);
+  return MCGPU_ERR_NOMEM;
 }
 
 } // namespace
@@ -391,16 +733,13 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
   const size_t tally = 16 * m + MC_TAB_BYTES, cells = sizeof(mc_cell) * m + MC_PAD_BYTES;
   const size_t budget = ctx->lds_per_block - 256; /* the kernel's static LDS */
   const bool lds_tally = tally <= budget;
-  /* wide layers: equal windows that fill the LDS; with scratch for them (not
-     in the no-allocation entry point, whose context is quiet) and at least a
-     block per window.  Else the global tally. */
-  const size_t most = (budget - MC_TAB_BYTES) / 16, nw = (m + most - 1) / most;
+  /* wide layers: windows, with scratch for them (not in the no-allocation
+     entry point, whose context is quiet) and at least a block per window.  Else
+     the global tally. */
   const bool block_ok = o.block_size <= 1024 && o.block_size % 64 == 0;
-  if (!lds_tally && !ctx->quiet && nw <= MC_MAX_WINDOWS && a.n < (int64_t)0xFFFFFFFFu &&
-      block_ok && (o.grid_blocks <= 0 || (size_t)o.grid_blocks >= nw) && !(a.score && !a.g)) {
-    const int W = (int)((m + nw - 1) / nw);
-    const int rc = a.score ? launch_windows<true>(ctx, a, o, s, (int)nw, W)
-                           : launch_windows<false>(ctx, a, o, s, (int)nw, W);
+  if (!lds_tally && !ctx->quiet && a.n < (int64_t)0xFFFFFFFFu && block_ok && !(a.score && !a.g)) {
+    const int rc = a.score ? launch_wide<true>(ctx, a, o, s, budget)
+                           : launch_wide<false>(ctx, a, o, s, budget);
     if (rc != MCGPU_ERR_NOMEM) return rc;
     ctx->err.clear();
   }

@@ -423,6 +423,8 @@ struct mc_call_queue {
   mc_queue q;
   unsigned long long *counter;
   __device__ __forceinline__ bool more() const { return mc_queue_more(q); }
+  static constexpr bool LEAVES = false;
+  __device__ __forceinline__ int least() const { return 8; }
   __device__ __forceinline__ int64_t take(mc_mask need) { return mc_queue_take(q, need, counter); }
 };
 
@@ -432,6 +434,8 @@ struct mc_tile_queue {
   uint64_t end;
   bool dry;
   __device__ __forceinline__ bool more() const { return !dry; }
+  static constexpr bool LEAVES = false;
+  __device__ __forceinline__ int least() const { return 8; }
   __device__ __forceinline__ int64_t take(mc_mask need) {
     const uint64_t cnt = (uint64_t)__popcll(need);
     unsigned long long base = 0;
@@ -499,7 +503,8 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
       const mc_mask need = mc_lanes(!has);
       if (adapt) {
         const int idle = __popcll(need);
-        kk = idle > 16 ? (kk > 8 ? kk >> 1 : 8) : (idle < 4 ? (kk < 256 ? kk << 1 : 256) : kk);
+        kk = idle > 16 ? kk >> 1 : (idle < 4 ? kk << 1 : kk);
+        kk = kk < queue.least() ? queue.least() : (kk < 256 ? kk : 256);
       }
       if (need) {
         const int64_t i = queue.take(need);
@@ -516,6 +521,15 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
         }
         run |= mc_lanes(on);
         if (IO::RESUMES) ev_bound = max_events; /* recomputed below */
+      }
+    }
+    if constexpr (Queue::LEAVES) {
+      const bool leaves = queue.leave(__popcll(mc_lanes(has)));
+      if (leaves) { /* wave-uniform: the histories are stored as they stand */
+        if (mc_in(pend)) p.s2 = mc_walk_undraw(p.s2);
+        pend = run = 0;
+      } else if (mc_lanes(has) == 0 && queue.wait()) {
+        continue;
       }
     }
     if (mc_lanes(has) == 0) break; /* wave-uniform */

@@ -266,3 +266,26 @@ def test_particles_at_the_bounds_of_the_common_step(ctx, oracle, dx, kernel):
     assert np.array_equal(result, o["result"])
     assert st["events"] == int(o["events"].sum())
     assert np.array_equal(w, o["tally_exact"])
+
+
+@pytest.mark.parametrize("m,n,opts", [(10_200, 12_000, {"grid_blocks": 8, "block_size": 256}),
+                                      (16_000, 6000, {}), (10_200, 3000, {"grid_blocks": 700})])
+def test_wide_layer_histories_from_one_edge(ctx, oracle, m, n, opts):
+    """All histories start in the first window: every block begins there, and
+    blocks change windows as histories are parked, several times over."""
+    import mcgpu
+    _say(f"windows from one edge m={m} n={n} {opts}")
+    sigs, ar, dx, bank = _case(m, n, m + n, 1.0)
+    bank["index"] = 0
+    bank["x"] = 0.0
+    bank["mu"] = np.abs(bank["mu"])
+    o = oracle.simulate_bank(64, 0, m, dx, 5e-2, sigs, ar, bank, nthread=8)
+    b, w = bank.copy(), np.zeros(m)
+    result, st, rc = ctx.simulate(b, sigs, ar, w, 0, m, dx, 5e-2,
+                                  options=mcgpu.make_options("history", **opts))
+    assert rc == 0
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f]), f
+    assert np.array_equal(result, o["result"])
+    assert st["events"] == int(o["events"].sum())
+    assert np.array_equal(w, o["tally_exact"])
