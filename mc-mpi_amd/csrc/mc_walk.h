@@ -234,12 +234,35 @@ __device__ __forceinline__ int mc_walk_wait(int wait, int general, int iteration
   return wait > 1 ? wait - 1 : 1;
 }
 
+/* Histories that set out together from one cell in one direction stay in the
+   same cell as long as none collides (an event moves each by one cell), and a
+   wave's adds to one LDS word follow one another.  So such lanes set out one
+   event apart: their cells, and the words they add to, then lie side by side.
+   The window kernel lets two or more wait (they start at a window's edge),
+   the others four or more, in layers of 256 cells on: in shorter ones the
+   events spent waiting cost more than the adds (100,000 histories through
+   host buffers on 100 cells 1.63 ms against 1.67 with it).
+   Measured without and with: 2 M histories into both faces of a 1,000-cell
+   layer 10.4 -> 4.9 ms, forward and gradient of 1,000 cells and 1 M histories
+   11.6 -> 10.2 ms, 512 slabs 46.9 -> 43.1 ms, 2 M histories in windows of
+   20,000 cells 176 -> 123 ms.  With each event of a start a call of
+   mc_walk_many, short histories lost: the cycle loop 12.9 -> 14.1 ms, now
+   13.0. */
+constexpr int MC_APART_CELLS = 256;
+
+/* the next lane to set out (fresh may be empty) */
+__device__ __forceinline__ mc_mask mc_sets_out(mc_mask &fresh) {
+  const mc_mask one = fresh & (0 - fresh);
+  fresh ^= one;
+  return one;
+}
+
 /* Up to ki events of every lane in `run` (lanes whose history goes on; `pend`:
-   lanes whose drawn event waits for the general form; both wave-uniform
-   masks, disjoint).  on_event(lanes, c8, cell, coll, di, dw, wmc) is called by
-   the whole wave for an event of `lanes` in cell c8 / 8 (wmc: the weight after
-   it).  ei counts a lane's events, col its collisions.  Returns how often the
-   general event ran.
+   lanes whose drawn event waits for the general form; `fresh`: lanes that set
+   out one after the other, one per event; all wave-uniform masks, disjoint).
+   on_event(lanes, c8, cell, coll, di, dw, wmc) is called by the whole wave for
+   an event of `lanes` in cell c8 / 8 (wmc: the weight after it).  ei counts a
+   lane's events, col its collisions.  Returns how often the general event ran.
    Every lane computes the common step (lanes not in `run` on whatever they
    hold); only the lanes of a certified crossing commit it.  A history's end
    shows at its next step, whose draw is taken back: the step's own tests and
@@ -256,8 +279,9 @@ __device__ __forceinline__ int mc_walk_wait(int wait, int general, int iteration
    cycles stood at 90 % of the time) 81.0 -> 64.6 ms; 1,000 on 1,000 cells,
    where the longest history's events follow one another, 1.09 -> 0.92 ms. */
 template <bool PAD, typename F>
-__device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &pend, int ki,
-                                            int wait, const mc_cell *cells, const double2 *tab,
+__device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &pend,
+                                            mc_mask &fresh, int ki, int wait,
+                                            const mc_cell *cells, const double2 *tab,
                                             const mc_walk_k &K, uint32_t &ei, uint32_t &col,
                                             F on_event) {
   int general = 0;
@@ -267,14 +291,16 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
     return mc_cell_at(cells, (uint32_t)c8 < K.top8 ? (uint32_t)c8 : K.top8);
   };
   for (;;) {
-    const int live = __popcll(run | pend);
+    const int live = __popcll(run | pend | fresh);
     if (live == 0) break;
     const int nwait = ki > 0 ? (wait * live + 63) >> 6 : 1;
-    if (run != 0 && ki > 0 && __popcll(pend) < nwait) {
+    if ((run | fresh) != 0 && ki > 0 && __popcll(pend) < nwait) {
       const int k0 = ki;
+      run |= mc_sets_out(fresh);
+      mc_mask all = run | fresh;
       uint64_t s2 = p.s2; /* the state of the lanes not in run: the draw below is for all */
       mc_cell cell;
-      if (mc_in(run)) cell = cell_of(p.c8);
+      if (mc_in(all)) cell = cell_of(p.c8);
       for (;;) {
         double xn, q, u;
         mc_mask ok = mc_walk_cross(p, run, cell, tab, K, xn, q, u);
@@ -292,7 +318,7 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
         }
         on_event(ok, c8, here, false, q, dw, p.wmc);
         --ki;
-        if (__builtin_expect(ok != run, 0)) { /* wave-uniform: a lane stopped or waits */
+        if (__builtin_expect(ok != all, 0)) { /* wave-uniform: a lane stopped, waits or sets out */
           const mc_mask out = run & ~ok;
           const mc_mask waits = out & mc_lanes(p.wmc >= K.min_weight) &
                                 mc_lanes((uint32_t)p.c8 < K.m8);
@@ -302,6 +328,15 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
           }
           pend |= waits;
           run = ok;
+          if (fresh != 0) {
+            const mc_mask sets_out = mc_sets_out(fresh);
+            if (mc_in(sets_out)) {
+              p.s2 = s2;
+              ei -= (uint32_t)(k0 - ki);
+            }
+            run |= sets_out;
+          }
+          all = run | fresh;
           if (run == 0 || __popcll(pend) >= nwait) break;
         }
         if (ki == 0) break;
@@ -311,7 +346,7 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
       else
         p.s2 = s2;
     }
-    if (pend != 0 && (run == 0 || __popcll(pend) >= nwait)) {
+    if (pend != 0 && ((run | fresh) == 0 || __popcll(pend) >= nwait)) {
       ++general;
       const int c8 = p.c8;
       mc_cell cell;
@@ -489,6 +524,8 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
   int64_t idx = 0;
   bool has = false;
   mc_mask run = 0, pend = 0; /* lanes whose history goes on / waits for the general event */
+  mc_mask fresh = 0;         /* lanes whose history has not set out yet */
+  const int apart = Queue::LEAVES ? 2 : (L.m >= MC_APART_CELLS ? 4 : 65);
   uint64_t ev = 0, before = 0; /* events of the lane's history; those before this call */
   uint32_t col = 0;
   const bool adapt = refill_k <= 0;
@@ -519,7 +556,16 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
           if (IO::RESUMES) before = ev;
           col = 0;
         }
-        run |= mc_lanes(on);
+        mc_mask out = mc_lanes(on);
+        if (!Queue::LEAVES && out) { /* of other cells: at once */
+          const int c8 = __builtin_amdgcn_readlane(p.c8, __builtin_ctzll(out));
+          const mc_mask here = out & mc_lanes(p.c8 == c8);
+          run |= out & ~here;
+          out = here;
+        }
+        const int up = __popcll(out & mc_lanes(p.st8 > 0)), down = __popcll(out) - up;
+        mc_mask &to = (up > down ? up : down) >= apart ? fresh : run;
+        to |= out;
         if (IO::RESUMES) ev_bound = max_events; /* recomputed below */
       }
     }
@@ -527,7 +573,7 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
       const bool leaves = queue.leave(__popcll(mc_lanes(has)));
       if (leaves) { /* wave-uniform: the histories are stored as they stand */
         if (mc_in(pend)) p.s2 = mc_walk_undraw(p.s2);
-        pend = run = 0;
+        pend = run = fresh = 0;
       } else if (mc_lanes(has) == 0 && queue.wait()) {
         continue;
       }
@@ -542,10 +588,11 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
     ev_bound += (uint64_t)ki;
     moves(ki + 1);
     uint32_t ei = 0; /* events of this interval */
-    const int general = mc_walk_many<PAD>(p, run, pend, ki, wait, cells, tab, K, ei, col, on_event);
+    const int general =
+        mc_walk_many<PAD>(p, run, pend, fresh, ki, wait, cells, tab, K, ei, col, on_event);
     wait = mc_walk_wait(wait, general, ki);
     ev += ei;
-    const bool on = mc_in(run), waits = mc_in(pend);
+    const bool on = mc_in(run | fresh), waits = mc_in(pend);
     const bool ends = has && !waits && (!on || ev >= max_events);
     if (mc_lanes(ends) == 0) continue; /* wave-uniform */
     bool again = false;

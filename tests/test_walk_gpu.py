@@ -289,3 +289,30 @@ def test_wide_layer_histories_from_one_edge(ctx, oracle, m, n, opts):
     assert np.array_equal(result, o["result"])
     assert st["events"] == int(o["events"].sum())
     assert np.array_equal(w, o["tally_exact"])
+
+
+@pytest.mark.parametrize("events_per_refill", [0, 1, 3])
+@pytest.mark.parametrize("m,n", [(255, 500), (256, 3), (256, 4), (256, 65), (700, 1300)])
+def test_histories_that_set_out_apart(ctx, oracle, m, n, events_per_refill):
+    """Histories from one cell, most of them in one direction, some that end at
+    once, in layers around the size from which they set out one event apart."""
+    import mcgpu
+    _say(f"one cell m={m} n={n} events_per_refill={events_per_refill}")
+    sigs, ar, dx, bank = _case(m, n, m + n, 1.0)
+    bank["index"] = m // 3
+    bank["x"] = bank["index"] * dx
+    bank["mu"] = np.where(np.arange(n) % 5 == 4, -1.0, 1.0) * np.abs(bank["mu"])
+    bank["wmc"][::7] = 1e-3
+    bank["index"][3::11] = m
+    o = oracle.simulate_bank(64, 0, m, dx, 1e-2, sigs, ar, bank, nthread=8)
+    b, w = bank.copy(), np.zeros(m)
+    result, st, rc = ctx.simulate(
+        b, sigs, ar, w, 0, m, dx, 1e-2,
+        options=mcgpu.make_options("history", events_per_refill=events_per_refill, block_size=64,
+                                   grid_blocks=1 + n // 200))
+    assert rc == 0
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f]), f
+    assert np.array_equal(result, o["result"])
+    assert st["events"] == int(o["events"].sum())
+    assert np.array_equal(w, o["tally_exact"])
