@@ -41,7 +41,7 @@ struct adj_args {
 template <bool LDS_T, bool LDS_C, bool HAVE_SCORE>
 __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int per_cu) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_k, s_g;
+  __shared__ mc_scale s_scale;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   const mc_walk_k K = mc_walk_live(a.L);
   mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
   const mc_cell *cells = a.cells;
   const double *g = a.g;
   if (threadIdx.x < MC_TOTALS) s_tot[threadIdx.x] = 0;
-  if (threadIdx.x == 0) s_k = s_g = -1023;
+  if (threadIdx.x == 0) mc_scale_clear(&s_scale);
   if (LDS_T)
     for (int c = threadIdx.x; c < 4 * m; c += blockDim.x) G.t[c] = 0;
   if (LDS_C) {
@@ -70,19 +70,23 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
     g = lg;
   }
   __syncthreads();
-  if (LDS_T) { /* the split: the largest target weight, the first histories' weights */
+  if (LDS_T) { /* the split */
     int kg = -1023;
     for (int c = threadIdx.x; c < m; c += blockDim.x) {
       const int k = mc_ceil_log2(g[c]);
       kg = k > kg ? k : kg;
     }
-    atomicMax(&s_g, kg);
+    atomicMax(&s_scale.g, kg);
+    mc_scale_scatter(&s_scale, cells, m);
     const uint64_t i = queue.q.next + __lane_id();
-    if (i < queue.q.end) atomicMax(&s_k, mc_ceil_log2(a.init.wmc[i]));
+    if (i < queue.q.end) atomicMax(&s_scale.w, mc_ceil_log2(a.init.wmc[i]));
+    const uint64_t j =
+        mc_scale_place(0, (uint64_t)a.n, (uint64_t)threadIdx.x * gridDim.x + blockIdx.x,
+                       (uint64_t)blockDim.x * gridDim.x);
+    if (j < (uint64_t)a.n) atomicMax(&s_scale.w, mc_ceil_log2(a.init.wmc[j]));
     __syncthreads();
   }
-  const bool limbs =
-      mc_grad_split(G, __builtin_amdgcn_readfirstlane(s_k + s_g), blockDim.x >> 6);
+  const bool limbs = mc_grad_split(G, s_scale, a.L.dx, blockDim.x >> 6);
 
   mc_grad_io<HAVE_SCORE> io{a.init, a.score, 0.0, 0.0, 1};
   if (LDS_T && limbs) { /* block-uniform */

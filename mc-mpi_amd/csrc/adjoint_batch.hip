@@ -118,12 +118,13 @@ template <bool SCORE> struct fwd_io {
 template <bool SCORE>
 __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_tile, s_k;
+  __shared__ int s_tile;
+  __shared__ mc_scale s_scale;
   __shared__ unsigned long long s_next;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   const int B = blockDim.x, tid = threadIdx.x;
   if (tid < MC_TOTALS) s_tot[tid] = 0;
-  if (tid == 0) s_k = -1023;
+  if (tid == 0) mc_scale_clear(&s_scale);
   double2 *tab = reinterpret_cast<double2 *>(smem);
   mc_tab_fill(tab);
   unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES);
@@ -147,11 +148,15 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
       lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
     }
     if (tid == 0) s_next = b.begin;
-    if (b.begin + tid < b.end) atomicMax(&s_k, mc_ceil_log2(a.bank.wmc[b.begin + tid]));
+    {
+      const uint64_t i = mc_scale_place(b.begin, b.end, tid, B);
+      if (i < (uint64_t)b.end) atomicMax(&s_scale.w, mc_ceil_log2(a.bank.wmc[i]));
+    }
+    if (in_lds && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, a.cells + b.cell_off, m, b.L.dx);
     __syncthreads();
 
     const mc_walk_k K = mc_walk_live(b.L);
-    const mc_block_tally bt = mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), B >> 6);
+    const mc_block_tally bt = mc_block_tally_for(m, s_scale, B >> 6);
     mc_tile_queue queue{&s_next, b.end, false};
     unsigned long long *fx_lo = a.fx + b.cell_off, *fx_hi = fx_lo + a.total;
     uint32_t *flags = a.flags + b.cell_off;
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
         for (int c = tid; c < m; c += B)
           mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx{t0[c], t1[c]});
     }
-    if (tid == 0) s_k = -1023;
+    if (tid == 0) mc_scale_clear(&s_scale);
     __syncthreads();
   }
   if (tid == 0) mc_totals_out(s_tot, a.ctr);
@@ -202,12 +207,13 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
 template <bool HAVE_SCORE>
 __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_tile, s_k, s_g;
+  __shared__ int s_tile;
+  __shared__ mc_scale s_scale;
   __shared__ unsigned long long s_next;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   const int B = blockDim.x, tid = threadIdx.x;
   if (tid < MC_TOTALS) s_tot[tid] = 0;
-  if (tid == 0) s_k = s_g = -1023;
+  if (tid == 0) mc_scale_clear(&s_scale);
   double2 *tab = reinterpret_cast<double2 *>(smem);
   mc_tab_fill(tab);
   mc_grad_tally G;
@@ -238,15 +244,19 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
         const int k = mc_ceil_log2(v);
         kg = k > kg ? k : kg;
       }
-      atomicMax(&s_g, kg);
+      atomicMax(&s_scale.g, kg);
+      mc_scale_scatter(&s_scale, a.cells + b.cell_off, m);
       lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
     }
     if (tid == 0) s_next = b.begin;
-    if (b.begin + tid < b.end) atomicMax(&s_k, mc_ceil_log2(a.bank.wmc[b.begin + tid]));
+    {
+      const uint64_t i = mc_scale_place(b.begin, b.end, tid, B);
+      if (i < (uint64_t)b.end) atomicMax(&s_scale.w, mc_ceil_log2(a.bank.wmc[i]));
+    }
     __syncthreads();
 
     const mc_walk_k K = mc_walk_live(b.L);
-    const bool limbs = mc_grad_split(G, __builtin_amdgcn_readfirstlane(s_k + s_g), B >> 6);
+    const bool limbs = mc_grad_split(G, s_scale, b.L.dx, B >> 6);
     mc_tile_queue queue{&s_next, b.end, false};
     if (in_lds && limbs)
       mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, G.every, a.max_events, s_tot,
@@ -272,7 +282,7 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
                    [](int) {});
     __syncthreads();
     if (in_lds) mc_grad_move(G, tid, B, limbs);
-    if (tid == 0) s_k = s_g = -1023;
+    if (tid == 0) mc_scale_clear(&s_scale);
     __syncthreads();
   }
   if (tid == 0) { /* this call counts events alone */

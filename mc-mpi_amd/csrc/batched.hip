@@ -79,7 +79,8 @@ struct tile_io {
    instruction. */
 __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_tile, s_k;
+  __shared__ int s_tile;
+  __shared__ mc_scale s_scale;
   __shared__ unsigned long long s_next;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   double2 *tab = reinterpret_cast<double2 *>(smem);
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
   const int B = blockDim.x;
   const int tid = threadIdx.x;
   if (tid < MC_TOTALS) s_tot[tid] = 0;
-  if (tid == 0) s_k = -1023;
+  if (tid == 0) mc_scale_clear(&s_scale);
   tile_io io{a};
 
   for (;;) {
@@ -119,12 +120,15 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     }
     if (tid == 0) s_next = (unsigned long long)tile.begin;
     /* the tile's weights, from one history per thread (as the history kernel) */
-    if (tile.begin + tid < tile.end) atomicMax(&s_k, mc_ceil_log2(a.soa.wmc[tile.begin + tid]));
+    {
+      const uint64_t i = mc_scale_place(tile.begin, tile.end, tid, B);
+      if (i < (uint64_t)tile.end) atomicMax(&s_scale.w, mc_ceil_log2(a.soa.wmc[i]));
+    }
+    if (lds_tally && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, gc, m, L.dx);
     __syncthreads();
 
     const mc_walk_k K = mc_walk_live(L);
-    const mc_block_tally bt =
-        mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), B >> 6);
+    const mc_block_tally bt = mc_block_tally_for(m, s_scale, B >> 6);
     mc_tile_queue queue{&s_next, mc_readlane64((unsigned long long)tile.end, 0), false};
     unsigned long long *fx_lo = a.fx + cell_off, *fx_hi = fx_lo + a.total_cells;
     uint32_t *flags = a.flags + cell_off;
@@ -165,7 +169,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
         mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], v);
       }
     }
-    if (tid == 0) s_k = -1023;
+    if (tid == 0) mc_scale_clear(&s_scale);
     __syncthreads();
   }
   /* the break follows a barrier after the last tile's totals */

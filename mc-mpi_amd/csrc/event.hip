@@ -347,7 +347,7 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
   const mc_coef K = mc_coef_live();
   /* block totals: events, collisions, left, right, killed, capped */
   __shared__ unsigned long long s_tot[MC_TOTALS];
-  __shared__ int s_k;
+  __shared__ mc_scale s_scale;
   __shared__ mc_transport_args s_a;
   const sargs &v = s_a;
   if (threadIdx.x == 0) s_a = a;
@@ -377,16 +377,20 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
   if (LDS_CELLS)
     for (int c = threadIdx.x; c < m; c += blockDim.x) cells_l[c] = ld_cell(cells_g + c);
   if (threadIdx.x < MC_TOTALS) s_tot[threadIdx.x] = 0;
-  if (threadIdx.x == 0) s_k = -1023;
+  if (threadIdx.x == 0) mc_scale_clear(&s_scale);
   __syncthreads();
   if (LDS_TALLY) { /* the block's weights, from one particle per thread (as k_history) */
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t j = i < a.n ? i : (int64_t)threadIdx.x;
-    if (j < a.n) atomicMax(&s_k, mc_ceil_log2(a.aos ? a.aos[j].wmc : a.soa.wmc[j]));
+    auto look = [&](uint64_t i) {
+      if (i < (uint64_t)a.n)
+        atomicMax(&s_scale.w, mc_ceil_log2(a.aos ? a.aos[i].wmc : a.soa.wmc[i]));
+    };
+    look(threadIdx.x);
+    look(mc_scale_place(0, (uint64_t)a.n, (uint64_t)threadIdx.x * gridDim.x + blockIdx.x,
+                        (uint64_t)blockDim.x * gridDim.x));
+    if (m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, a.cells, m, a.L.dx);
     __syncthreads();
   }
-  const mc_block_tally B =
-      mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), blockDim.x >> 6);
+  const mc_block_tally B = mc_block_tally_for(m, s_scale, blockDim.x >> 6);
   const bool limbs = LDS_TALLY && B.limbs && (P >> 6) <= B.every; /* block-uniform */
   mc_mover moves{t_lo, t_hi, a.fx, a.fx + m, m, B.S.L, B.every, B.every};
 

@@ -460,13 +460,14 @@ __global__ void k_windows_list(int64_t n, mc_windows win, uint32_t *list, uint32
 }
 
 /* one block's part of layer L (cells and global tally words at cells, fx_lo,
-   fx_hi, ...): LDS, the walk, the tally and totals */
+   fx_hi, ...): LDS, the walk, the tally and totals.  k: mc_ceil_log2 of the
+   weights this thread has looked at */
 template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE, typename IO, typename Queue>
 __device__ __forceinline__ void history_block(const mc_transport_args &a, const mc_layer_k &L,
-                                              int off, IO &io, Queue &queue, double wmc,
+                                              int off, IO &io, Queue &queue, int k,
                                               int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_k;
+  __shared__ mc_scale s_scale;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   const mc_walk_k K = mc_walk_live(L);
   const int m = L.m;
@@ -491,20 +492,18 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
     }
   }
   if (threadIdx.x < MC_TOTALS) s_tot[threadIdx.x] = 0;
-  /* the block's weights: the largest among the first histories of its waves
-     (a guess that sets the limbs' range; heavier ones go to the global tally) */
-  if (threadIdx.x == 0) s_k = -1023;
+  if (threadIdx.x == 0) mc_scale_clear(&s_scale);
   __syncthreads();
   if (LDS_TALLY) {
-    atomicMax(&s_k, mc_ceil_log2(wmc));
+    atomicMax(&s_scale.w, k);
+    if (m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, cells, m, L.dx);
     __syncthreads();
   }
 
   unsigned long long *fx_lo = a.fx + off, *fx_hi = fx_lo + a.L.m;
   uint32_t *flags = a.flags + off;
   unsigned int *status = &a.ctr->status;
-  const mc_block_tally B =
-      mc_block_tally_for(m, __builtin_amdgcn_readfirstlane(s_k), blockDim.x >> 6);
+  const mc_block_tally B = mc_block_tally_for(m, s_scale, blockDim.x >> 6);
   if (LDS_TALLY && B.limbs) { /* block-uniform */
     mc_walk_bank<LDS_CELLS>(io, queue, L, K, cells, tab, refill_k, B.every, a.max_events, s_tot,
                  [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
@@ -541,10 +540,17 @@ template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE>
 __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refill_k, int per_cu) {
   mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
   bank_io<SCORE> io{a, 0.0};
-  const uint64_t i = queue.q.next + __lane_id();
-  double wmc = 0.0;
-  if (LDS_TALLY && i < queue.q.end) wmc = a.aos ? a.aos[i].wmc : a.soa.wmc[i];
-  history_block<LDS_TALLY, LDS_CELLS, SCORE>(a, a.L, 0, io, queue, wmc, refill_k);
+  int k = -1023;
+  if (LDS_TALLY) { /* the first histories, and one anywhere */
+    auto look = [&](uint64_t i, uint64_t end) {
+      const int of = i < end ? mc_ceil_log2(a.aos ? a.aos[i].wmc : a.soa.wmc[i]) : -1023;
+      k = of > k ? of : k;
+    };
+    look(queue.q.next + __lane_id(), queue.q.end);
+    look(mc_scale_place(0, (uint64_t)a.n, (uint64_t)threadIdx.x * gridDim.x + blockIdx.x,
+                        (uint64_t)blockDim.x * gridDim.x), (uint64_t)a.n);
+  }
+  history_block<LDS_TALLY, LDS_CELLS, SCORE>(a, a.L, 0, io, queue, k, refill_k);
 }
 
 /* one sweep over the windows of a wide layer */
@@ -584,8 +590,13 @@ __global__ __launch_bounds__(1024) void k_history_windows(mc_transport_args a, m
     window_io<SCORE> io{a, win, w, &blk, 0.0, -1};
     const uint64_t i = queue.open.q.next + __lane_id();
     int64_t j = -1;
+    const uint64_t at =
+        mc_scale_place(0, queue.open.q.n, (uint64_t)threadIdx.x * sh.blocks + sh.block,
+                       (uint64_t)blockDim.x * sh.blocks);
     if (i < queue.open.q.end) {
       j = queue.list[i];
+    } else if (at < queue.open.q.n) { /* its own share is short: one of all */
+      j = queue.list[at];
     } else { /* threads look at the run's first histories; none is taken yet */
       const uint32_t next = (uint32_t)blk.run, end = (uint32_t)(blk.run >> 32);
       if (threadIdx.x < end - next) {
@@ -594,9 +605,9 @@ __global__ __launch_bounds__(1024) void k_history_windows(mc_transport_args a, m
         if (v != MC_NOT_PUT) j = v;
       }
     }
-    double wmc = 0.0;
-    if (j >= 0) wmc = ld_shared(a.aos ? &a.aos[j].wmc : &a.soa.wmc[j]);
-    history_block<true, LDS_CELLS, SCORE>(a, L, off, io, queue, wmc, refill_k);
+    int k = -1023;
+    if (j >= 0) k = mc_ceil_log2(ld_shared(a.aos ? &a.aos[j].wmc : &a.soa.wmc[j]));
+    history_block<true, LDS_CELLS, SCORE>(a, L, off, io, queue, k, refill_k);
   }
 }
 

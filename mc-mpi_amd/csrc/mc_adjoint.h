@@ -21,11 +21,28 @@ struct mc_grad_tally {
   int every;
 };
 
-/* V: terms are at most about the largest target weight times the particle
-   weight (times the flight length, below 1); larger ones go to fx.  Returns
-   whether limbs serve (an interval of at least 128 events per lane between
-   moves); if not, t holds words with carry. */
-__device__ __forceinline__ bool mc_grad_split(mc_grad_tally &G, int k, int waves) {
+/* the largest sig_i of a block's cells, by all its threads */
+__device__ __forceinline__ void mc_scale_scatter(mc_scale *s, const mc_cell *cells, int m) {
+  double most = 0.0;
+  for (int c = threadIdx.x; c < m; c += blockDim.x) {
+    const double b = cells[c].sig_i;
+    most = b > most ? b : most;
+  }
+  atomicMax(&s->b, mc_ceil_log2(most));
+}
+
+/* V: a term is at most about the largest target weight times the particle
+   weight times a flight, or, where the history collides, 1 / sig_i: 1, 64
+   cells (terms above need |mu| < 1/64, one crossing in 4,096) or 1 over the
+   largest sig_i, whichever is most.  Larger terms go to fx.  Returns whether
+   limbs serve (an interval of at least 128 events per lane between moves); if
+   not, t holds words with carry. */
+__device__ __forceinline__ bool mc_grad_split(mc_grad_tally &G, const mc_scale &s, double dx,
+                                              int waves) {
+  const int flight = mc_ceil_log2(dx) + 6, b = __builtin_amdgcn_readfirstlane(s.b);
+  const int free_path = b < -13 ? 0 : 1 - b; /* none: nothing scatters (MC_EPS < 2^-13) */
+  const int longest = flight > free_path ? flight : free_path;
+  const int k = __builtin_amdgcn_readfirstlane(s.w + s.g) + (longest > 0 ? longest : 0);
   const int V = k < -30 ? -30 : (k > 5 ? 5 : k);
   G.S = mc_fx_split_for(V);
   const int lg = mc_fx_split_signed_log2_terms(V);

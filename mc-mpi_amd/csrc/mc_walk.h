@@ -635,25 +635,70 @@ struct mc_block_tally {
   int limbs;  /* 0: words (lo, hi) with carry */
 };
 
-/* V for a layer of m cells with weights up to 2^k: thin cells absorb a small
-   part of the weight, and a smaller V means rarer moves; the few larger terms
-   go to the global tally directly.  (On a 1-long slab of m cells a term above
-   2^-6 of the weight needs |mu| below about 64 / m.) */
-__device__ __forceinline__ mc_block_tally mc_block_tally_for(int m, int k, int waves) {
+/* smallest k with 2^k >= v (v >= 0, not subnormal); large for inf and NaN */
+__device__ __forceinline__ int mc_ceil_log2(double v) {
+  const uint64_t b = mc_asu64(v) & 0x7FFFFFFFFFFFFFFFULL;
+  return (int)(b >> 52) - 1023 + ((b & 0x000FFFFFFFFFFFFFULL) ? 1 : 0);
+}
+
+/* What a block expects of its terms, in LDS: binary exponents of the largest
+   weight, of the largest sig_a dx, and (gradients) of the largest target
+   weight and sig_i.  A guess that sets the split; larger terms go to the
+   global tally, where a full chip's adds to one word follow one another at
+   about 7 ns each, so they have to stay rare. */
+struct mc_scale {
+  int w, thick, g, b;
+};
+
+/* by one thread, before a barrier */
+__device__ __forceinline__ void mc_scale_clear(mc_scale *s) { *s = {-1023, -1023, -1023, -1023}; }
+
+/* the weights of histories first .. end - 1, as one history per thread of
+   `threads` finds them, spread over all; pos: this thread's place */
+__device__ __forceinline__ uint64_t mc_scale_place(uint64_t first, uint64_t end, uint64_t pos,
+                                                   uint64_t threads) {
+  const uint64_t n = end - first;
+  if (n <= threads) return first + pos; /* may be end or beyond */
+  const uint64_t i = (uint64_t)((double)pos * ((double)n / (double)threads));
+  return first + (i < n ? i : n - 1);
+}
+
+/* the cells of a block's layer, by all its threads */
+__device__ __forceinline__ void mc_scale_cells(mc_scale *s, const mc_cell *cells, int m,
+                                               double dx) {
+  double most = 0.0;
+  for (int c = threadIdx.x; c < m; c += blockDim.x) {
+    const double a = cells[c].sig_a;
+    most = a > most ? a : most;
+  }
+  atomicMax(&s->thick, mc_ceil_log2(most * dx));
+}
+
+/* V: terms up to the largest weight in a layer of few cells.  In one of many
+   cells a smaller V (a cell absorbs a small part of the weight) means rarer
+   moves: the largest weight times 16 sig_a dx of the thickest cell (terms
+   above need |mu| < 1/16 there, one crossing in 256), but no less than 2^-4
+   or 2^-6 of the weight, where moves are rare enough.  With V from the number
+   of cells alone, 2 M histories into the face of a layer of 10,000 cells with
+   a mean sig_a dx of 0.011 took 67 ms, nearly every term in the global tally;
+   now 2.0.  Largest weights seen by one history per thread, over the whole
+   bank: a bank sorted by weight is seen whole. */
+constexpr int MC_THICK_CELLS = 1024;
+__device__ __forceinline__ mc_block_tally mc_block_tally_for(int m, const mc_scale &s, int waves) {
   mc_block_tally B;
-  const int V = k - (m < 1024 ? 0 : (m < 4096 ? 4 : 6));
+  const int k = __builtin_amdgcn_readfirstlane(s.w);
+  int less = 0;
+  if (m >= MC_THICK_CELLS) {
+    const int most = m < 4096 ? 4 : 6, thin = -4 - __builtin_amdgcn_readfirstlane(s.thick);
+    less = thin < 0 ? 0 : (thin < most ? thin : most);
+  }
+  const int V = k - less;
   const int Vc = V < -30 ? -30 : (V > 2 ? 2 : V);
   B.limbs = V <= 2; /* an interval of at least 512 events per lane */
   B.S = mc_fx_split_for(Vc);
   const int lg = mc_fx_split_log2_terms(Vc);
   B.every = (int)((1u << (lg < 30 ? lg : 30)) / (64u * (unsigned)waves));
   return B;
-}
-
-/* smallest k with 2^k >= v (v >= 0, not subnormal); large for inf and NaN */
-__device__ __forceinline__ int mc_ceil_log2(double v) {
-  const uint64_t b = mc_asu64(v) & 0x7FFFFFFFFFFFFFFFULL;
-  return (int)(b >> 52) - 1023 + ((b & 0x000FFFFFFFFFFFFFULL) ? 1 : 0);
 }
 
 /* a term that neither limb conversion takes: to the global tally */

@@ -316,3 +316,29 @@ def test_histories_that_set_out_apart(ctx, oracle, m, n, events_per_refill):
     assert np.array_equal(result, o["result"])
     assert st["events"] == int(o["events"].sum())
     assert np.array_equal(w, o["tally_exact"])
+
+
+@pytest.mark.parametrize("kernel", ["history", "event"])
+@pytest.mark.parametrize("thick", [0.03, 1.0, 30.0])
+@pytest.mark.parametrize("m", [1023, 1024, 4096])
+def test_thick_cells_and_sorted_weights(ctx, oracle, m, thick, kernel):
+    """Cells that absorb much of the weight, where the split follows the
+    thickest one, and weights that rise through the bank."""
+    import mcgpu
+    n = 3000
+    _say(f"thick cells m={m} {thick} {kernel}")
+    sigs, ar, dx, bank = _case(m, n, m, np.geomspace(1e-6, 1.0, 3000))
+    sigs = sigs * thick * m
+    bank["index"][::2] = 0
+    bank["x"][::2] = 0.0
+    bank["mu"][::2] = np.abs(bank["mu"][::2])
+    o = oracle.simulate_bank(64, 0, m, dx, 1e-8, sigs, ar, bank, nthread=8)
+    b, w = bank.copy(), np.zeros(m)
+    result, st, rc = ctx.simulate(b, sigs, ar, w, 0, m, dx, 1e-8,
+                                  options=mcgpu.make_options(kernel))
+    assert rc == 0
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f]), f
+    assert np.array_equal(result, o["result"])
+    assert st["events"] == int(o["events"].sum())
+    assert np.array_equal(w, o["tally_exact"])
