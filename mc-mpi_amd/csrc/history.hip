@@ -74,10 +74,9 @@ template <bool SCORE> struct bank_io {
    and against sweeps in which a parked history waits for the next launch:
    200,000 histories on 20,000 cells 540, 106 and 45 ms; 2 M 161 ms (228 by
    sweeps); 200,000 on 50,000 cells 102 ms (236); 1,000 on 20,000 21.6 ms (56).
-   Layers whose tally alone fits keep one window: 10,000 cells and 2 M
-   histories take 67 ms in two windows and 70 in one, 300,000 25 and 22, 2 M on
-   6,000 cells 46 and 37 (histories that refill a lane at the same edge walk on
-   together and meet in the LDS banks). */
+   Histories taken up together at an edge set out one event apart (mc_walk.h);
+   before, they met in the LDS banks, and 8 M histories on 10,000 cells took
+   208 ms in two windows (now 161; 234 in one, whose cells do not fit). */
 constexpr int MC_MAX_WINDOWS = 64;
 
 struct mc_windows {
@@ -96,6 +95,9 @@ struct mc_windows {
   int patience; /* looks of an idle block before it ends */
 };
 constexpr uint32_t MC_NOT_PUT = 0xFFFFFFFFu;
+
+/* the rings' words of a call at most (2 GiB) */
+constexpr size_t MC_RING_WORDS = (size_t)1 << 29;
 
 /* words of different windows lie on different lines */
 constexpr int MC_WINDOW_STEP = 32;
@@ -670,7 +672,7 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   /* ev[n], at[n], list[n], parked[nw cap], queue counters, counts, cursors,
      left, and put, got, blocks a line apart */
   const size_t n = (size_t)a.n;
-  const size_t cap = 4 * n * (size_t)nw <= ((size_t)1 << 31) ? n : 0; /* 0: no ring */
+  const size_t cap = n * (size_t)nw <= MC_RING_WORDS ? n : 0; /* 0: no ring */
   const size_t words = (16 * n + 4 * cap * (size_t)nw + 255) / 256 * 256;
   int rc = mc_ensure(ctx, &ctx->work, &ctx->work_bytes,
                      words + (20 + 12 * MC_WINDOW_STEP) * MC_MAX_WINDOWS);
@@ -732,7 +734,7 @@ int launch_wide(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_opti
   const int tally = windows_of((size_t)a.L.m, budget, false, S);
   const int limit = o.grid_blocks > 0 ? std::min(o.grid_blocks, MC_MAX_WINDOWS) : MC_MAX_WINDOWS;
   if (all <= limit) return launch_windows<true, S>(ctx, a, o, s, all);
-  if (tally <= limit) return launch_windows<false, S>(ctx, a, o, s, tally);
+  if (tally > 1 && tally <= limit) return launch_windows<false, S>(ctx, a, o, s, tally);
   return MCGPU_ERR_NOMEM;
 }
 
@@ -744,11 +746,26 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
   const size_t tally = 16 * m + MC_TAB_BYTES, cells = sizeof(mc_cell) * m + MC_PAD_BYTES;
   const size_t budget = ctx->lds_per_block - 256; /* the kernel's static LDS */
   const bool lds_tally = tally <= budget;
-  /* wide layers: windows, with scratch for them (not in the no-allocation
-     entry point, whose context is quiet) and at least a block per window.  Else
-     the global tally. */
+  const size_t targets = a.score ? 8 * m : 0;
+  const bool lds_cells = lds_tally && tally + cells + targets <= budget;
+  /* Windows, with scratch for them (not in the no-allocation entry point, whose
+     context is quiet) and at least a block per window: for a layer whose tally
+     does not fit (else the global tally), and for one whose tally fits but not
+     its cells, if there are many histories per lane and many cells beyond
+     those that fit.  Reading cells through L2 holds the long run back (37 lines
+     per wave and event); windows lose to it where blocks that change windows
+     run on few histories.  One window and two, in ms: 10,000 cells (4,934
+     beyond) 8 M histories 234 and 161, 1 M 39.8 and 37.6, 500,000 25.5 and
+     26.2; 8,500 cells 1 M 33.1 and 30.8; 7,000 cells 4 M 77 and 67, 1 M 26.9
+     and 27.6; 6,000 cells 8 M 116 and 106, 4 M 62.6 and 65.5. */
+  const size_t lanes = 1024 * (size_t)(o.grid_blocks > 0 ? o.grid_blocks : ctx->num_cus);
+  const size_t beyond = (tally + cells + targets - std::min(budget, tally + cells + targets)) /
+                        (sizeof(mc_cell) + 16 + (a.score ? 8 : 0));
+  const bool long_run = !lds_cells && (double)a.n * (double)beyond >= 2e4 * (double)lanes &&
+                        (size_t)a.n <= MC_RING_WORDS / 4;
   const bool block_ok = o.block_size <= 1024 && o.block_size % 64 == 0;
-  if (!lds_tally && !ctx->quiet && a.n < (int64_t)0xFFFFFFFFu && block_ok && !(a.score && !a.g)) {
+  if ((!lds_tally || long_run) && !ctx->quiet && a.n < (int64_t)0xFFFFFFFFu && block_ok &&
+      !(a.score && !a.g)) {
     const int rc = a.score ? launch_wide<true>(ctx, a, o, s, budget)
                            : launch_wide<false>(ctx, a, o, s, budget);
     if (rc != MCGPU_ERR_NOMEM) return rc;
@@ -756,14 +773,11 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
   }
   if (a.score) { /* per-history score of a weighted tally (forward of the adjoint) */
     if (!a.g) return mc_fail(ctx, MCGPU_ERR_ARG, "score output needs target weights g");
-    const size_t extra = 8 * m;
-    const bool lds_cells = lds_tally && tally + cells + extra <= budget;
-    if (lds_tally && lds_cells) return launch_one<true, true, true>(ctx, a, o, s, tally + cells + extra);
+    if (lds_cells) return launch_one<true, true, true>(ctx, a, o, s, tally + cells + targets);
     if (lds_tally) return launch_one<true, false, true>(ctx, a, o, s, tally);
     return launch_one<false, false, true>(ctx, a, o, s, MC_TAB_BYTES);
   }
-  const bool lds_cells = lds_tally && tally + cells <= budget;
-  if (lds_tally && lds_cells) return launch_one<true, true, false>(ctx, a, o, s, tally + cells);
+  if (lds_cells) return launch_one<true, true, false>(ctx, a, o, s, tally + cells);
   if (lds_tally) return launch_one<true, false, false>(ctx, a, o, s, tally);
   return launch_one<false, false, false>(ctx, a, o, s, MC_TAB_BYTES);
 }

@@ -318,6 +318,14 @@ def test_histories_that_set_out_apart(ctx, oracle, m, n, events_per_refill):
     assert np.array_equal(w, o["tally_exact"])
 
 
+@pytest.mark.parametrize("n", [8290, 8320])
+def test_long_run_of_a_layer_whose_cells_do_not_fit(ctx, oracle, n):
+    """10,000 cells on two blocks, around the number of histories from which the
+    layer goes in two windows."""
+    _say(f"cells that do not fit, n={n}")
+    _check(ctx, oracle, 10_000, n, 71, 1.0, 5e-2, grid_blocks=2)
+
+
 @pytest.mark.parametrize("kernel", ["history", "event"])
 @pytest.mark.parametrize("thick", [0.03, 1.0, 30.0])
 @pytest.mark.parametrize("m", [1023, 1024, 4096])
