@@ -44,6 +44,7 @@ struct bcell_args {
   const btile_k *tiles;
   int32_t n_tiles;
   int32_t lds_max_m;      /* slabs with m <= this stage their cells in LDS */
+  uint32_t lds;           /* dynamic LDS bytes */
   mcgpu_bank bank;        /* forward: in/out; adjoint: initial bank, read only */
   const mc_cell *cells;   /* [total] */
   const double *g;        /* [total] */
@@ -136,13 +137,16 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     const btile b = read_tile(a, t);
     const int m = b.L.m;
     const bool in_lds = m <= a.lds_max_m; /* block-uniform */
-    unsigned long long *t1 = t0 + m;
-    mc_cell *lc = reinterpret_cast<mc_cell *>(t1 + m);
+    const int sh = in_lds ? mc_limbs_copies(m, a.lds - MC_TAB_BYTES - MC_PAD_BYTES -
+                                                   (sizeof(mc_cell) + (SCORE ? 8 : 0)) * m)
+                          : 0;
+    const mc_limbs T = mc_limbs_at(t0, m, sh), mine = mc_limbs_mine(T);
+    unsigned long long *t1 = t0 + m; /* words with carry: one copy */
+    mc_cell *lc = reinterpret_cast<mc_cell *>(t0 + (2 * (size_t)m << sh));
     double *lg = reinterpret_cast<double *>(lc + m + 2);
     if (in_lds) {
+      for (int c = tid; c < 2 * m << sh; c += B) t0[c] = 0;
       for (int c = tid; c < m; c += B) {
-        t0[c] = 0;
-        t1[c] = 0;
         if (SCORE) lg[c] = a.g[b.cell_off + c];
       }
       lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
@@ -165,10 +169,10 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     if (in_lds && bt.limbs) {
       mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot,
                    [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
-                     mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+                     mc_tally_limbs(mine, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
                      if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(lg, c8) * dw;
                    },
-                   mc_mover{t0, t1, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every});
+                   mc_mover{T, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every});
     } else if (in_lds) { /* weights too heavy for the limbs */
       mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
                    [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
@@ -192,7 +196,7 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     __syncthreads();
     if (in_lds) {
       if (bt.limbs)
-        mc_limbs_move(t0, t1, bt.S.L, m, tid, B, fx_lo, fx_hi);
+        mc_limbs_move(T, bt.S.L, m, tid, B, fx_lo, fx_hi);
       else
         for (int c = tid; c < m; c += B)
           mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx{t0[c], t1[c]});
@@ -434,6 +438,8 @@ int batch_prepare(mcgpu_context *ctx, K kern, int32_t n_slabs, const mcgpu_slab 
   const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES - MC_PAD_BYTES; /* static LDS */
   a->lds_max_m = (int)std::min<size_t>((size_t)max_m, budget / lds_bytes_per_cell);
   *lds = MC_TAB_BYTES + MC_PAD_BYTES + lds_bytes_per_cell * (size_t)a->lds_max_m;
+  if (flag_words == 1) *lds = mc_lds_with_copies(*lds, a->lds_max_m); /* the forward */
+  a->lds = (uint32_t)*lds;
   if (*lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds);

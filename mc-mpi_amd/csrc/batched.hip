@@ -35,6 +35,7 @@ struct batch_args {
   const mc_slab_k *slabs;
   const mc_tile_k *tiles;
   int32_t n_tiles;
+  uint32_t lds;            /* dynamic LDS bytes of a block */
   int32_t lds_cells_max_m; /* slabs with m <= this stage cross sections in LDS */
   int32_t lds_tally_max_m; /* slabs with m <= this keep their tally in LDS; larger
                               ones add straight into the global tally */
@@ -108,14 +109,15 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     const int64_t cell_off = (int64_t)mc_readlane64((unsigned long long)sl.cell_off, 0);
     const bool lds_tally = m <= a.lds_tally_max_m; /* block-uniform */
     const bool lds_cells = m <= a.lds_cells_max_m; /* implies lds_tally */
-    unsigned long long *t1 = t0 + m;
-    mc_cell *lc = reinterpret_cast<mc_cell *>(t1 + m);
+    const int sh = lds_cells ? mc_limbs_copies(m, a.lds - MC_TAB_BYTES - MC_PAD_BYTES -
+                                                      sizeof(mc_cell) * m)
+                             : 0;
+    const mc_limbs T = mc_limbs_at(t0, m, sh), mine = mc_limbs_mine(T);
+    unsigned long long *t1 = t0 + m; /* words with carry: one copy */
+    mc_cell *lc = reinterpret_cast<mc_cell *>(t0 + (2 * (size_t)m << sh));
     const mc_cell *gc = a.cells + cell_off;
     if (lds_tally) {
-      for (int c = tid; c < m; c += B) {
-        t0[c] = 0;
-        t1[c] = 0;
-      }
+      for (int c = tid; c < 2 * m << sh; c += B) t0[c] = 0;
       if (lds_cells) lc = mc_cells_fill(lc, gc, m);
     }
     if (tid == 0) s_next = (unsigned long long)tile.begin;
@@ -134,9 +136,9 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     uint32_t *flags = a.flags + cell_off;
     unsigned int *status = &a.ctr->status;
     auto limbs = [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
-      mc_tally_limbs(t0, t1, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+      mc_tally_limbs(mine, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
     };
-    const mc_mover mover{t0, t1, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every};
+    const mc_mover mover{T, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every};
     if (lds_tally && bt.limbs) {
       if (lds_cells)
         mc_walk_bank<true>(io, queue, L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
@@ -160,7 +162,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
 
     __syncthreads();
     if (lds_tally && bt.limbs) {
-      mc_limbs_move(t0, t1, bt.S.L, m, tid, B, fx_lo, fx_hi);
+      mc_limbs_move(T, bt.S.L, m, tid, B, fx_lo, fx_hi);
     } else if (lds_tally) {
       for (int c = tid; c < m; c += B) {
         mc_fx v;
@@ -215,7 +217,7 @@ int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, in
      whose tally does not fit add into the global tally directly */
   const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES;
   const size_t lds = std::min(budget, (size_t)32 * (size_t)std::max(max_m, 1) + MC_PAD_BYTES);
-  sh.lds = lds + MC_TAB_BYTES;
+  sh.lds = mc_lds_with_copies(lds + MC_TAB_BYTES, max_m);
   sh.lds_cells_max_m = (int)((lds - MC_PAD_BYTES) / 32);
   sh.lds_tally_max_m = (int)(lds / 16);
   if (sh.lds > 65536)
@@ -247,6 +249,7 @@ int mc_launch_batched(mcgpu_context *ctx, const mc_batched_shape &sh, const mc_s
   a.n_tiles = n_tiles;
   a.lds_cells_max_m = sh.lds_cells_max_m;
   a.lds_tally_max_m = sh.lds_tally_max_m;
+  a.lds = (uint32_t)sh.lds;
   a.soa = bank;
   a.cells = cells;
   a.fx = fx;
@@ -363,6 +366,7 @@ int batch_capture(mcgpu_batch *b) {
   a.n_tiles = b->n_tiles;
   a.lds_cells_max_m = b->lds_cells_max_m;
   a.lds_tally_max_m = b->lds_tally_max_m;
+  a.lds = (uint32_t)b->lds;
   a.soa = b->bank;
   a.cells = b->d_cells;
   a.fx = b->d_fx;

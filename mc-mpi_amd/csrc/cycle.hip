@@ -298,6 +298,8 @@ __global__ void k_cyc_exchange(const rank_in *rin, const rank_sum *sum, pool_k p
   copy_particle(esc, src, pool, rin[q].pool_base + s.keep + k);
 }
 
+constexpr int64_t MC_POOL_BYTES = 8 + 8 + 8 + 8 + 4 + 1; /* of a particle in the pool */
+
 inline unsigned blocks_for(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 /* device allocations of one run, freed on every exit path */
@@ -452,7 +454,7 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
   /* work buffer and per-cycle tallies of one group */
   const int64_t pcap = std::max(S, std::min<int64_t>(all, (int64_t)1 << 26));
   const int64_t gcap = std::max<int64_t>(1, ((int64_t)1 << 23) / m);
-  const int64_t max_tiles = pcap / T + gcap + 1;
+  const int64_t max_tiles = pcap / (o.particles_per_lane > 0 ? T : block) + gcap + 1;
 
   cycle_mem mem;
   auto dalloc = [&](void **p, size_t bytes) -> int {
@@ -570,6 +572,12 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
     if (G == 0) break;
     /* ---- lay out the particles, tables, one launch, weights in cycle order */
     MC_HIP(ctx, hipEventRecord(ev_start, s));
+    /* Tiles of a whole block's part (twice the share: mc_tile_size takes half):
+       every resident block gets one, and none a second to wait for.  2 M
+       histories in 20 cycles: 13.3 ms in tiles of 4,096 (half the blocks
+       without one), 9.2 in tiles of half a part, 8.7. */
+    double share = 0.0;
+    for (const one_cycle &c : cyc) share += 2.0 * (double)c.n * m / sh.grid;
     h_slabs.assign(G, mc_slab_k{});
     h_tiles.clear();
     for (int64_t g = 0; g < G; ++g) {
@@ -601,12 +609,13 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
       sl.min_weight = k.particle_min_weight;
       sl.cell_off = g * m;
       const int64_t end = cyc[g].first + cyc[g].n;
-      for (int64_t p0 = cyc[g].first; p0 < end; p0 += T) {
+      const int64_t Tg = o.particles_per_lane > 0 ? T : mc_tile_size(T, share, cyc[g].n, m, block);
+      for (int64_t p0 = cyc[g].first; p0 < end; p0 += Tg) {
         mc_tile_k t;
         t.slab = (int32_t)g;
         t.pad_ = 0;
         t.begin = p0;
-        t.end = std::min(end, p0 + T);
+        t.end = std::min(end, p0 + Tg);
         h_tiles.push_back(t);
       }
     }
@@ -838,6 +847,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
     seed[r] = ranks[r].seed;
     ranks[r].n_left = ranks[r].n_right = ranks[r].n_killed = 0;
   }
+  const auto m_of = [&](int r) { return ranks[r].max_index - ranks[r].min_index; };
   /* room for the bank, one creation and two received buffers */
   auto need_of = [&](int r) {
     return size[r] + (create[r] > 0 ? std::max(MAX_PARTICLES_VECTOR, S) : 0) + 2 * S;
@@ -883,9 +893,22 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
     return MCGPU_OK;
   };
   {
-    std::vector<int64_t> c0(R);
-    for (int r = 0; r < R; ++r) c0[r] = need_of(r);
-    if ((rc = build_pool(c0))) return rc;
+    /* Room for every particle in every rank, up to 1 GiB in all: banks that
+       grow as the particles spread are moved each time, 2.7 ms for a pool of
+       2 M (12 of 34 ms in a run of 2 M particles on eight ranks). */
+    const int64_t all = (((int64_t)1 << 30) / MC_POOL_BYTES) / R;
+    std::vector<int64_t> c0(R), c1(R);
+    for (int r = 0; r < R; ++r) {
+      c0[r] = need_of(r);
+      c1[r] = std::max(c0[r], std::min(nb_particles + 2 * S, all));
+    }
+    rc = build_pool(c1);
+    if (rc) {
+      (void)hipGetLastError();
+      ctx->err.clear();
+      rc = build_pool(c0);
+    }
+    if (rc) return rc;
     /* initial banks: host AoS -> device SoA */
     for (int r = 0; r < R; ++r) {
       const int64_t n = size[r];
@@ -952,6 +975,12 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
 
     /* 1. lazy creation (src/layer.cpp:247-248, :89-121) */
     int64_t n_tiles = 0, n_chunks = 0;
+    double share = 0.0; /* of a block, twice over: see sync_one_rank */
+    for (int r = 0; r < R; ++r) {
+      int64_t have = size[r];
+      if (have < S && create[r] > 0) have += create[r];
+      share += 2.0 * (double)std::min(have, S) * m_of(r) / sh.grid;
+    }
     for (int r = 0; r < R; ++r) {
       mcgpu_cycle_rank &k = ranks[r];
       if (size[r] < S && create[r] > 0) {
@@ -970,12 +999,14 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
       /* 2. tiles of the last n particles, 3. partition chunks */
       const int64_t n = std::min(size[r], S);
       const int64_t end = base[r] + size[r];
-      for (int64_t p0 = end - n; p0 < end; p0 += T) {
+      const int64_t Tr =
+          o.particles_per_lane > 0 ? T : mc_tile_size(16 * block, share, n, m_of(r), block);
+      for (int64_t p0 = end - n; p0 < end; p0 += Tr) {
         mc_tile_k t;
         t.slab = r;
         t.pad_ = 0;
         t.begin = p0;
-        t.end = std::min(end, p0 + T);
+        t.end = std::min(end, p0 + Tr);
         h_tiles[n_tiles++] = t;
       }
       rank_in &ri = h_rin[r];

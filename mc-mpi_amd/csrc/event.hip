@@ -392,7 +392,8 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
   }
   const mc_block_tally B = mc_block_tally_for(m, s_scale, blockDim.x >> 6);
   const bool limbs = LDS_TALLY && B.limbs && (P >> 6) <= B.every; /* block-uniform */
-  mc_mover moves{t_lo, t_hi, a.fx, a.fx + m, m, B.S.L, B.every, B.every};
+  const mc_limbs T{t_lo, t_hi, 0};
+  mc_mover moves{T, a.fx, a.fx + m, m, B.S.L, B.every, B.every};
 
   /* this wave's pool: two halves of P slots */
   const int lane = __lane_id();
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
           }
         }
         if (limbs)
-          mc_tally_limbs(t_lo, t_hi, B.S, fresh(v).fx, fresh(v).fx + m, fresh(v).flags,
+          mc_tally_limbs(T, B.S, fresh(v).fx, fresh(v).fx + m, fresh(v).flags,
                          &fresh(v).ctr->status, mc_lanes(c_live && c_event), 8 * c_cell, d_dw);
         /* the write-back: the offsets per path, then the same stores on both
            (a store on one path only would make the compiler assume fewer
@@ -716,7 +717,7 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
     if (limbs)
       mc_walk_bank<false>(io, queue, L, W, cells, tab, 0, B.every, max_ev, s_tot,
                    [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
-                     mc_tally_limbs(t_lo, t_hi, B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+                     mc_tally_limbs(T, B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
                    },
                    moves);
     else
@@ -733,7 +734,7 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
   if (LDS_TALLY) {
     unsigned long long *fx = a.fx;
     if (limbs) {
-      mc_limbs_move(t_lo, t_hi, B.S.L, m, threadIdx.x, blockDim.x, fx, fx + m);
+      mc_limbs_move(T, B.S.L, m, threadIdx.x, blockDim.x, fx, fx + m);
     } else {
       for (int c = threadIdx.x; c < m; c += blockDim.x) {
         mc_fx t;

@@ -466,7 +466,7 @@ __global__ void k_windows_list(int64_t n, mc_windows win, uint32_t *list, uint32
    weights this thread has looked at */
 template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE, typename IO, typename Queue>
 __device__ __forceinline__ void history_block(const mc_transport_args &a, const mc_layer_k &L,
-                                              int off, IO &io, Queue &queue, int k,
+                                              int off, IO &io, Queue &queue, int k, int sh,
                                               int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ mc_scale s_scale;
@@ -475,17 +475,15 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
   const int m = L.m;
   double2 *tab = reinterpret_cast<double2 *>(smem);
   mc_tab_fill(tab);
-  unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES), *t1 = t0 + m;
-  if (LDS_TALLY) {
-    for (int c = threadIdx.x; c < m; c += blockDim.x) {
-      t0[c] = 0;
-      t1[c] = 0;
-    }
-  }
+  unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES);
+  unsigned long long *t1 = t0 + m; /* words with carry: one copy */
+  const mc_limbs T = mc_limbs_at(t0, m, sh), mine = mc_limbs_mine(T);
+  if (LDS_TALLY)
+    for (int c = threadIdx.x; c < 2 * m << sh; c += blockDim.x) t0[c] = 0;
   const mc_cell *cells = a.cells + off;
   const double *g = SCORE ? a.g + off : nullptr;
   if (LDS_CELLS) {
-    mc_cell *lc = reinterpret_cast<mc_cell *>(t1 + m);
+    mc_cell *lc = reinterpret_cast<mc_cell *>(t0 + (2 * (size_t)m << sh));
     cells = mc_cells_fill(lc, cells, m);
     if (SCORE) {
       double *lg = reinterpret_cast<double *>(lc + m + 2);
@@ -509,12 +507,12 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
   if (LDS_TALLY && B.limbs) { /* block-uniform */
     mc_walk_bank<LDS_CELLS>(io, queue, L, K, cells, tab, refill_k, B.every, a.max_events, s_tot,
                  [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
-                   mc_tally_limbs(t0, t1, B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+                   mc_tally_limbs(mine, B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
                    if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(g, c8) * dw;
                  },
-                 mc_mover{t0, t1, fx_lo, fx_hi, m, B.S.L, B.every, B.every});
+                 mc_mover{T, fx_lo, fx_hi, m, B.S.L, B.every, B.every});
     __syncthreads();
-    mc_limbs_move(t0, t1, B.S.L, m, threadIdx.x, blockDim.x, fx_lo, fx_hi);
+    mc_limbs_move(T, B.S.L, m, threadIdx.x, blockDim.x, fx_lo, fx_hi);
   } else {
     unsigned long long *lo = LDS_TALLY ? t0 : fx_lo, *hi = LDS_TALLY ? t1 : fx_hi;
     mc_walk_bank<LDS_CELLS>(io, queue, L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
@@ -539,7 +537,8 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
 }
 
 template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE>
-__global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refill_k, int per_cu) {
+__global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refill_k, int per_cu,
+                                                  int sh) {
   mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
   bank_io<SCORE> io{a, 0.0};
   int k = -1023;
@@ -552,7 +551,8 @@ __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refil
     look(mc_scale_place(0, (uint64_t)a.n, (uint64_t)threadIdx.x * gridDim.x + blockIdx.x,
                         (uint64_t)blockDim.x * gridDim.x), (uint64_t)a.n);
   }
-  history_block<LDS_TALLY, LDS_CELLS, SCORE>(a, a.L, 0, io, queue, k, refill_k);
+  history_block<LDS_TALLY, LDS_CELLS, SCORE>(a, a.L, 0, io, queue, k, LDS_CELLS ? sh : 0,
+                                             refill_k);
 }
 
 /* one sweep over the windows of a wide layer */
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(1024) void k_history_windows(mc_transport_args a, m
     }
     int k = -1023;
     if (j >= 0) k = mc_ceil_log2(ld_shared(a.aos ? &a.aos[j].wmc : &a.soa.wmc[j]));
-    history_block<true, LDS_CELLS, SCORE>(a, L, off, io, queue, k, refill_k);
+    history_block<true, LDS_CELLS, SCORE>(a, L, off, io, queue, k, 0, refill_k);
   }
 }
 
@@ -623,6 +623,12 @@ template <bool T, bool C, bool S>
 int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
                hipStream_t s, size_t lds) {
   auto kern = k_history<T, C, S>;
+  int sh = 0;
+  if (C) {
+    const size_t other = lds - 16 * (size_t)a.L.m;
+    lds = mc_lds_with_copies(lds, a.L.m);
+    sh = mc_limbs_copies(a.L.m, lds - other);
+  }
   if (lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -642,7 +648,7 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
     if (a.n < grid) grid = (int)(a.n > 0 ? a.n : 1); /* a block per history at most */
   }
   int k = o.events_per_refill > 0 ? o.events_per_refill : 0; /* 0: adaptive */
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k, per_cu);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k, per_cu, sh);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
 }
