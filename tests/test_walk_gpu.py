@@ -350,3 +350,27 @@ def test_thick_cells_and_sorted_weights(ctx, oracle, m, thick, kernel):
     assert np.array_equal(result, o["result"])
     assert st["events"] == int(o["events"].sum())
     assert np.array_equal(w, o["tally_exact"])
+
+
+@pytest.mark.parametrize("m", [1, 2, 74, 75, 144, 145, 273, 491, 817, 818])
+def test_tally_copies(ctx, oracle, m):
+    """Layers around the sizes at which the block keeps fewer copies of its
+    tally, histories all from one face and from anywhere."""
+    import mcgpu
+    n = 1500
+    _say(f"tally copies m={m}")
+    sigs, ar, dx, bank = _case(m, n, m + 5, 1.0)
+    bank["index"][::2] = 0
+    bank["x"][::2] = 0.0
+    bank["mu"][::2] = np.abs(bank["mu"][::2])
+    o = oracle.simulate_bank(64, 0, m, dx, 1e-2, sigs, ar, bank, nthread=8)
+    for grid in (0, 1):
+        b, w = bank.copy(), np.zeros(m)
+        result, st, rc = ctx.simulate(b, sigs, ar, w, 0, m, dx, 1e-2,
+                                      options=mcgpu.make_options("history", grid_blocks=grid))
+        assert rc == 0
+        for f in ("seed", "x", "mu", "wmc", "index"):
+            assert np.array_equal(b[f], o["bank"][f]), f
+        assert np.array_equal(result, o["result"])
+        assert st["events"] == int(o["events"].sum())
+        assert np.array_equal(w, o["tally_exact"])
