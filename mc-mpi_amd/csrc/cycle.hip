@@ -572,12 +572,8 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
     if (G == 0) break;
     /* ---- lay out the particles, tables, one launch, weights in cycle order */
     MC_HIP(ctx, hipEventRecord(ev_start, s));
-    /* Tiles of a whole block's part (twice the share: mc_tile_size takes half):
-       every resident block gets one, and none a second to wait for.  2 M
-       histories in 20 cycles: 13.3 ms in tiles of 4,096 (half the blocks
-       without one), 9.2 in tiles of half a part, 8.7. */
-    double share = 0.0;
-    for (const one_cycle &c : cyc) share += 2.0 * (double)c.n * m / sh.grid;
+    double share = 0.0; /* of a block (mc_tile_size) */
+    for (const one_cycle &c : cyc) share += (double)c.n * m / sh.grid;
     h_slabs.assign(G, mc_slab_k{});
     h_tiles.clear();
     for (int64_t g = 0; g < G; ++g) {
@@ -975,11 +971,11 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
 
     /* 1. lazy creation (src/layer.cpp:247-248, :89-121) */
     int64_t n_tiles = 0, n_chunks = 0;
-    double share = 0.0; /* of a block, twice over: see sync_one_rank */
+    double share = 0.0; /* of a block (mc_tile_size) */
     for (int r = 0; r < R; ++r) {
       int64_t have = size[r];
       if (have < S && create[r] > 0) have += create[r];
-      share += 2.0 * (double)std::min(have, S) * m_of(r) / sh.grid;
+      share += (double)std::min(have, S) * m_of(r) / sh.grid;
     }
     for (int r = 0; r < R; ++r) {
       mcgpu_cycle_rank &k = ranks[r];

@@ -201,16 +201,18 @@ struct mc_batched_shape {
 
 /* Histories of a tile of a slab of n histories and m cells: n in equal tiles
    of at most `most`, or, when `share` (a block's part of all slabs' histories
-   x cells) is given, of at most half of it (few or uneven slabs), though of at
-   least one history per thread of the block.  A block waits for its tile's
-   longest history, several times the mean one, so many small tiles cost more
-   than they balance: forward and adjoint of 64 slabs of 50,000 histories on
-   1,000 cells took 34.7 ms in tiles of 16,384, 50.5 ms at an eighth of a
-   block's part (1,600) and 31.6 ms at a half; 512 slabs of 32 to 8,192 cells
-   72.5 ms at an eighth and 50.2 ms at a half. */
+   x cells) is given, of at most that (few or uneven slabs), though of at least
+   one history per thread of the block.  A block waits for its tile's longest
+   history, several times the mean one, so small tiles cost more than they
+   balance.  In tiles of 4/3, 1, 1/1.3, 1/2 and 1/3 of a part: 512 slabs of 32
+   to 8,192 cells 39.8, 39.3, 41.8, 45.5 and 46.5 ms; forward and adjoint of 64
+   slabs of 50,000 histories on 1,000 cells 27.1, 24.3, 26.0, 28.0 and 29.5 ms;
+   the cycle loop of 20 cycles of 100,000 histories with one rank 8.7 ms in
+   whole parts, 9.2 in halves, 13.3 in tiles of 4,096 (half the blocks without
+   one). */
 inline int64_t mc_tile_size(int64_t most, double share, int64_t n, int m, int block) {
   double fit = (double)most;
-  if (share > 0.0 && share / (2.0 * m) < fit) fit = share / (2.0 * m);
+  if (share > 0.0 && share / m < fit) fit = share / m;
   if (fit < (double)block) fit = (double)block;
   const int64_t tiles = (int64_t)((double)n / fit) + ((double)n / fit > (int64_t)((double)n / fit));
   if (tiles <= 1) return n > 0 ? n : 1;
