@@ -22,7 +22,7 @@
  * windows (below).  The per-cell cross-section pairs are staged
  * in LDS when they fit next to the tally, otherwise read through L2.
  *
- * Measured against the kernel with mc_event and a tally with carry: a lone
+ * Measured against the kernel with the full event and a tally with carry: a lone
  * history 450 -> 284 ns per event (10,000 cells); 1,000 histories on the
  * 100-cell slab, whole call 264 -> 181 us; 1,000 on 10,000 cells 26.0 -> 9.8
  * ms (dealt over the CUs); 8e6 on 10,000 cells 267 -> 237 ms, there bound by

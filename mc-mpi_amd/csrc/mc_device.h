@@ -114,10 +114,7 @@ struct mc_state {
   double mu;
   double wmc;
   int32_t index;
-  double inv_mu; /* RN(1/mu), kept by the kernels that divide by reciprocal */
 };
-
-__device__ __forceinline__ void mc_refresh_rcp(mc_state &p) { p.inv_mu = 1.0 / p.mu; }
 
 /* Layer constants read by the step (include/layer/layer.hpp:465-485) */
 struct mc_layer_k {
@@ -132,7 +129,7 @@ struct mc_layer_k {
 #define MC_MAXREAL 1.7976931348623157e308
 
 /* the log/exp coefficients as values the compiler cannot fold; made once at
-   kernel entry and passed to every mc_event of the kernel */
+   kernel entry and passed to every event of the kernel */
 __device__ __forceinline__ mc_coef mc_coef_live() {
   mc_coef K = mc_coef_default();
   asm volatile("" : "+v"(K.l8), "+v"(K.l7), "+v"(K.l6), "+v"(K.l5), "+v"(K.l4), "+v"(K.l3));
@@ -141,9 +138,13 @@ __device__ __forceinline__ mc_coef mc_coef_live() {
 }
 
 /* One transport event: Layer::particle_step (src/layer.cpp:123-190) in FP64
-   with correctly rounded log/exp, on cell c (cells[c]).  Returns the
-   absorbed weight dw (tallied by the caller to cell c); `collided` reports
-   which branch was taken and di_out the flight length.
+   with correctly rounded log/exp, on `cell`, up to the exp argument: the draw,
+   the edge distance (IEEE division), the collision decision (certified
+   crossing, else the correctly rounded log and division), the collision's new
+   x and mu, or the crossing's x; returns -sig_a * di and the new cell index.
+   The caller (the event kernel, which loads the exp table row one step before
+   it evaluates) then forms dw = (1 - mc_exp_k_row(arg, row, K)) * wmc, wmc -=
+   dw, index = index_new.  The persistent kernels' form is in mc_walk.h.
    The reference draws the flight length di = -log(h) / sig_i and the edge
    distance di_edge, and the particle collides iff di < di_edge (both
    correctly rounded quotients here).  On fine meshes most events cross the
@@ -154,70 +155,7 @@ __device__ __forceinline__ mc_coef mc_coef_live() {
    the particle crosses: such an event needs no log at all.  Only when that
    is not certain (h near 1, a collision, a thick cell, |mu| <= EPS) are the
    correctly rounded log and the division formed and compared exactly, as the
-   reference does.  Results are identical either way.
-   RCP: the edge distance divides by the particle's stored RN(1/mu)
-   (mc_div_by_rcp; same result), refreshed when mu changes, for kernels that
-   keep the state in registers. */
-template <bool RCP = false, typename Count = uint64_t>
-__device__ __forceinline__ double mc_event(mc_state &p, const mc_cell *cells, int c,
-                                           const double dx, const mc_coef &K, bool &collided,
-                                           double &di_out, mc_cell *cell_out = nullptr,
-                                           Count *col_count = nullptr) {
-  /* The edge quotient is formed unconditionally and then selected; when
-     |mu| <= EPS the discarded quotient may be inf or NaN and is never used.
-     *cell_out (if given) receives the cell; *col_count (if given) is
-     incremented on a collision, inside the collision's own branch. */
-  /* an unsigned 32-bit byte offset (c is in [0, m)): the load takes the
-     uniform base in scalar registers and the offset as is */
-  const mc_cell cell =
-      *reinterpret_cast<const mc_cell *>(reinterpret_cast<const char *>(cells) + ((uint32_t)c << 4));
-  if (cell_out) *cell_out = cell;
-  const double h = mc_rnd_real(p.seed);
-
-  const bool back = p.mu < 0;
-  int index_new = back ? p.index - 1 : p.index + 1;
-  const double x_new_edge = (back ? p.index : p.index + 1) * dx;
-  const double q_edge = RCP ? mc_div_by_rcp(x_new_edge - p.x, p.mu, p.inv_mu)
-                            : (x_new_edge - p.x) / p.mu;
-  const double di_edge = (p.mu < -MC_EPS || MC_EPS < p.mu) ? q_edge : MC_MAXREAL;
-
-  const double reach = cell.sig_i * di_edge;
-  /* bitwise, not short-circuit: one test, no branch */
-  const int sure_cross =
-      (int)!(cell.sig_i > MC_EPS) | (int)((1.0 - h) > mc_fma(reach, 0x1p-40, reach));
-  double di = di_edge;
-  collided = false;
-  if (!sure_cross) {
-    const double nlog = -mc_log_k(h, &K);
-    const double dq = cell.sig_i > MC_EPS ? nlog / cell.sig_i : MC_MAXREAL;
-    collided = dq < di_edge;
-    if (collided) di = dq;
-  }
-  if (collided) {
-    index_new = p.index;
-    p.x += di * p.mu;
-    p.mu = 2 * mc_rnd_real(p.seed) - 1;
-    if (RCP) mc_refresh_rcp(p);
-    if (col_count) ++*col_count;
-  } else {
-    p.x = x_new_edge;
-  }
-
-  const double dw = (1 - mc_exp_k(-cell.sig_a * di, &K)) * p.wmc;
-  p.wmc -= dw;
-  p.index = index_new;
-  di_out = di;
-  return dw;
-}
-
-/* mc_event in two halves, for a kernel that loads the exp table row one
-   step before it evaluates (the event kernel's pipeline).  mc_event_decide
-   is mc_event up to the exp argument: the draw, the edge distance (IEEE
-   division), the collision decision (certified crossing, else the correctly
-   rounded log and division), the collision's new x and mu, or the crossing's
-   x; it returns -sig_a * di and the new cell index.  The caller then forms
-   dw = (1 - mc_exp_k_row(arg, row, K)) * wmc, wmc -= dw, index = index_new,
-   as mc_event does.  The operations and their order are mc_event's. */
+   reference does.  Results are identical either way. */
 __device__ __forceinline__ double mc_event_decide(mc_state &p, const mc_cell cell, const double dx,
                                                   const mc_coef &K, bool &collided,
                                                   int &index_new) {

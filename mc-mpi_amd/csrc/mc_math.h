@@ -143,7 +143,7 @@ MC_FN mc_coef mc_coef_default(void) {
    correctly rounded quotient by Markstein's theorem (y within half an ulp of
    1/b, q1 within 1 ulp of a/b).  For |b| >= 2^-60 the fmas stay in the
    normal range while 2^-900 <= |q0| <= 2^900; otherwise (a = 0 among them)
-   the IEEE division is used.  (mc_event uses the quotient only for
+   the IEEE division is used.  (The events use the quotient only for
    |mu| > EPS_PRECISION, far above 2^-60.) */
 MC_FN double mc_div_by_rcp(double a, double b, double y) {
   const double q0 = a * y;

@@ -2,21 +2,21 @@
  * mc_walk.h -- one transport event of Layer::particle_step
  * (src/layer.cpp:123-190) as the persistent kernels run it: a short common
  * step for the event that provably crosses its cell, and the general event
- * (mc_event's operations) for everything else.
+ * (mc_event_decide's operations) for everything else.
  *
  * What bounds these kernels is the number of vector instructions per event:
  * gfx950 issues one 64-bit (or three-operand) wave64 instruction per SIMD
  * every 4.25 cycles, and a wave on its own one every 8.5 whatever the
  * instruction, so the count sets both the rate of a full chip and the time of
  * a lone long history.  The common step has about half the instructions of
- * mc_event:
+ * the event written out in full (mc_device.h):
  *  - the state is kept in the form the step uses: the doubled RNG state (the
  *    generator is a map mod 2^64 with no mask, and its top 32 bits are h's),
  *    1/mu as a pair, the next edge's number as a double, the cell as an
  *    offset in the layer;
  *  - the collision test needs only 20 bits of h: 1 + h (truncated) + sig_i *
  *    di_edge < 2 - 2^-18 implies 1 - h > sig_i * di_edge * (1 + 2^-40), the
- *    certificate of mc_event;
+ *    certificate of mc_event_decide;
  *  - the absorbed fraction is a rounding on a fixed grid (mc_absorb_thin,
  *    mc_absorb_row), with no exp to full relative accuracy;
  *  - the deposit is split into two limbs by floating-point adds and summed by
@@ -53,7 +53,7 @@ __device__ __forceinline__ void mc_walk_turn(mc_walk &p, int32_t index) {
   const bool back = p.mu < 0;
   p.st8 = back ? -8 : 8;
   p.fs = back ? -1.0 : 1.0;
-  p.fe = (double)(back ? index : index + 1);
+  p.fe = (double)index + (back ? 0.0 : 1.0);
   p.rh = 1.0 / p.mu;
   p.rl = mc_fma(-p.mu, p.rh, 1.0) * p.rh;
   const double mu = __builtin_fabs(p.mu), x = __builtin_fabs(p.x);
@@ -66,7 +66,9 @@ __device__ __forceinline__ void mc_walk_from(mc_walk &w, const mc_state &p, cons
   w.x = p.x;
   w.mu = p.mu;
   w.wmc = p.wmc;
-  w.c8 = (p.index - L.index_start) * 8;
+  /* a history outside the layer ends at once; the edge's number keeps its index */
+  const int64_t c = (int64_t)p.index - L.index_start;
+  w.c8 = c < 0 ? -8 : 8 * (c < L.m ? (int32_t)c : L.m);
   mc_walk_turn(w, p.index);
 }
 
@@ -75,7 +77,7 @@ __device__ __forceinline__ void mc_walk_to(mc_state &p, const mc_walk &w, const 
   p.x = w.x;
   p.mu = w.mu;
   p.wmc = w.wmc;
-  p.index = (w.c8 >> 3) + L.index_start;
+  p.index = (int32_t)(w.fe - (w.st8 > 0 ? 1.0 : 0.0));
 }
 
 __device__ __forceinline__ bool mc_walk_alive(const mc_walk &w, const mc_layer_k &L) {
@@ -188,8 +190,9 @@ __device__ __forceinline__ mc_mask mc_walk_cross(mc_walk &p, mc_mask run, const 
   return ok & mc_lanes(__builtin_fabs(rem) < K.rem_max);
 }
 
-/* The general event, after mc_walk_cross has drawn: mc_event's operations.
-   Returns the deposit; coll, di as mc_event's. */
+/* The general event, after mc_walk_cross has drawn: mc_event_decide's
+   operations and the absorption.  Returns the deposit; coll: whether it
+   collided, di: the flight. */
 __device__ __forceinline__ double mc_walk_general(mc_walk &p, const mc_cell cell, const double dx,
                                                   bool &coll, double &di) {
   const mc_coef K = mc_coef_default();

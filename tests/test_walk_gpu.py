@@ -374,3 +374,29 @@ def test_tally_copies(ctx, oracle, m):
         assert np.array_equal(result, o["result"])
         assert st["events"] == int(o["events"].sum())
         assert np.array_equal(w, o["tally_exact"])
+
+
+@pytest.mark.parametrize("kernel", ["history", "event"])
+@pytest.mark.parametrize("lo", [0, 700, -5000])
+def test_particles_outside_the_layer(ctx, oracle, lo, kernel):
+    """Indices next to the layer and as far as 32 bits go: such a history ends
+    at once, with its index as it was."""
+    import mcgpu
+    m, n = 40, 400
+    _say(f"outside the layer lo={lo} {kernel}")
+    sigs, ar, dx, bank = _case(m, n, 17, 1.0)
+    far = np.array([-1, m, 1 << 28, 1 << 29, (1 << 29) + 5, 3 << 29, -(1 << 29), -(1 << 29) + 7,
+                    (1 << 31) - 1, -(1 << 31)])
+    bank["index"] += lo
+    bank["x"] = (bank["index"] + 0.25) * dx
+    bank["index"][::3] = np.clip(far[np.arange(134) % 10] + lo, -(1 << 31), (1 << 31) - 1)
+    o = oracle.simulate_bank(64, lo, lo + m, dx, 1e-2, sigs, ar, bank, nthread=8)
+    b, w = bank.copy(), np.zeros(m)
+    result, st, rc = ctx.simulate(b, sigs, ar, w, lo, lo + m, dx, 1e-2,
+                                  options=mcgpu.make_options(kernel))
+    assert rc == 0
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f]), f
+    assert np.array_equal(result, o["result"])
+    assert st["events"] == int(o["events"].sum())
+    assert np.array_equal(w, o["tally_exact"])
