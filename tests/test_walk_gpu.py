@@ -390,7 +390,7 @@ def test_particles_outside_the_layer(ctx, oracle, lo, kernel):
     bank["index"] += lo
     bank["x"] = (bank["index"] + 0.25) * dx
     bank["index"][::3] = np.clip(far[np.arange(134) % 10] + lo, -(1 << 31), (1 << 31) - 1)
-    o = oracle.simulate_bank(64, lo, lo + m, dx, 1e-2, sigs, ar, bank, nthread=8)
+    o = oracle.simulate_bank(64, lo, m, dx, 1e-2, sigs, ar, bank, nthread=8)
     b, w = bank.copy(), np.zeros(m)
     result, st, rc = ctx.simulate(b, sigs, ar, w, lo, lo + m, dx, 1e-2,
                                   options=mcgpu.make_options(kernel))
