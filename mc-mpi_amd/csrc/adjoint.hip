@@ -137,7 +137,9 @@ __global__ void k_setup_cells(int m, const double *sig_a, const double *sig_i, m
 }
 
 __global__ void k_finalize2(int m, const unsigned long long *fx, const uint32_t *flags,
-                            double *ga, double *gi) {
+                            double *ga, double *gi, const mc_counters *ctr,
+                            mc_counters *host_ctr) {
+  mc_counters_to_host(ctr, host_ctr);
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < m) {
     ga[c] = ga[c] + mc_fx_finalize(fx[c], fx[m + c], flags[c]);
@@ -145,15 +147,15 @@ __global__ void k_finalize2(int m, const unsigned long long *fx, const uint32_t 
   }
 }
 
-__global__ void k_finalize1(int m, const unsigned long long *fx, const uint32_t *flags,
-                            double *w) {
+__global__ void k_finalize1(int m, const unsigned long long *fx, const uint32_t *flags, double *w,
+                            const mc_counters *ctr, mc_counters *host_ctr) {
+  mc_counters_to_host(ctr, host_ctr);
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < m) w[c] = w[c] + mc_fx_finalize(fx[c], fx[m + c], flags[c]);
 }
 
+/* the counters that the finalizing kernel has handed over */
 int read_counters(mcgpu_context *ctx, hipStream_t s, mcgpu_stats *stats) {
-  MC_HIP(ctx, hipMemcpyAsync(ctx->host_counters, ctx->counters, sizeof(mc_counters),
-                             hipMemcpyDeviceToHost, s));
   MC_HIP(ctx, hipStreamSynchronize(s));
   const mc_counters *hc = (const mc_counters *)ctx->host_counters;
   if (stats) {
@@ -274,7 +276,7 @@ int mcgpu_forward_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *bank,
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
   hipLaunchKernelGGL(k_finalize1, dim3((m + 255) / 256), dim3(256), 0, s, m,
                      (const unsigned long long *)ctx->fx, (const uint32_t *)ctx->flags,
-                     weights_absorbed);
+                     weights_absorbed, a.ctr, (mc_counters *)ctx->host_counters);
   MC_HIP(ctx, hipGetLastError());
   return read_counters(ctx, s, stats);
 }
@@ -323,7 +325,7 @@ int mcgpu_adjoint_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *initial
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
   hipLaunchKernelGGL(k_finalize2, dim3((m + 255) / 256), dim3(256), 0, s, m,
                      (const unsigned long long *)ctx->fx, (const uint32_t *)ctx->flags,
-                     grad_sig_a, grad_sig_i);
+                     grad_sig_a, grad_sig_i, a.ctr, (mc_counters *)ctx->host_counters);
   MC_HIP(ctx, hipGetLastError());
   return read_counters(ctx, s, stats);
 }

@@ -321,7 +321,9 @@ __global__ void k_batch_cells_setup(int64_t total, const double *sig_a, const do
 
 /* out_k[c] += the k-th accumulator (k < n_out) */
 __global__ void k_batch_cells_finalize(int64_t total, const unsigned long long *fx,
-                                       const uint32_t *flags, double *out0, double *out1) {
+                                       const uint32_t *flags, double *out0, double *out1,
+                                       const mc_counters *ctr, mc_counters *host_ctr) {
+  mc_counters_to_host(ctr, host_ctr);
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= total) return;
   out0[c] = out0[c] + mc_fx_finalize(fx[c], fx[total + c], flags[c]);
@@ -387,9 +389,8 @@ int build_tables(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
   return MCGPU_OK;
 }
 
+/* the counters that the finalizing kernel has handed over */
 int read_batch_counters(mcgpu_context *ctx, hipStream_t s, mcgpu_stats *stats) {
-  MC_HIP(ctx, hipMemcpyAsync(ctx->host_counters, ctx->counters, sizeof(mc_counters),
-                             hipMemcpyDeviceToHost, s));
   MC_HIP(ctx, hipStreamSynchronize(s));
   const mc_counters *hc = (const mc_counters *)ctx->host_counters;
   if (stats) {
@@ -513,7 +514,8 @@ int mcgpu_forward_cells_batch(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_s
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
   hipLaunchKernelGGL(k_batch_cells_finalize, dim3((unsigned)((total_cells + 255) / 256)), dim3(256),
                      0, s, total_cells, (const unsigned long long *)ctx->fx,
-                     (const uint32_t *)ctx->flags, weights_absorbed, (double *)nullptr);
+                     (const uint32_t *)ctx->flags, weights_absorbed, (double *)nullptr, a.ctr,
+                     (mc_counters *)ctx->host_counters);
   MC_HIP(ctx, hipGetLastError());
   return read_batch_counters(ctx, s, stats);
 }
@@ -548,7 +550,8 @@ int mcgpu_adjoint_cells_batch(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_s
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
   hipLaunchKernelGGL(k_batch_cells_finalize, dim3((unsigned)((total_cells + 255) / 256)), dim3(256),
                      0, s, total_cells, (const unsigned long long *)ctx->fx,
-                     (const uint32_t *)ctx->flags, grad_sig_a, grad_sig_i);
+                     (const uint32_t *)ctx->flags, grad_sig_a, grad_sig_i, a.ctr,
+                     (mc_counters *)ctx->host_counters);
   MC_HIP(ctx, hipGetLastError());
   return read_batch_counters(ctx, s, stats);
 }

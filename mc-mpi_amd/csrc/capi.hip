@@ -74,7 +74,8 @@ __global__ void k_setup(int m, const double *sigs, const double *ar, mc_cell *ce
 }
 
 __global__ void k_finalize(int m, const unsigned long long *fx, const uint32_t *flags,
-                           double *weights) {
+                           double *weights, const mc_counters *ctr, mc_counters *host_ctr) {
+  mc_counters_to_host(ctr, host_ctr);
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < m) weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[m + c], flags[c]);
 }
@@ -159,9 +160,9 @@ int transport(mcgpu_context *ctx, mc_transport_args &a, const mcgpu_options *opt
   }
   if (rc) return rc;
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
-  if ((rc = mc_launch_finalize(ctx, a.L.m, a.fx, a.flags, d_weights, s))) return rc;
-  MC_HIP(ctx, hipMemcpyAsync(ctx->host_counters, ctx->counters, sizeof(mc_counters),
-                             hipMemcpyDeviceToHost, s));
+  if ((rc = mc_launch_finalize(ctx, a.L.m, a.fx, a.flags, d_weights, a.ctr,
+                               (mc_counters *)ctx->host_counters, s)))
+    return rc;
   MC_HIP(ctx, hipStreamSynchronize(s));
   float ms = 0.f;
   if (stats) (void)hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
@@ -186,8 +187,10 @@ int mc_launch_setup(mcgpu_context *ctx, int m, const double *sigs, const double 
 }
 
 int mc_launch_finalize(mcgpu_context *ctx, int m, const unsigned long long *fx,
-                       const uint32_t *flags, double *weights, hipStream_t s) {
-  hipLaunchKernelGGL(k_finalize, dim3(grid_for(m, 256)), dim3(256), 0, s, m, fx, flags, weights);
+                       const uint32_t *flags, double *weights, const mc_counters *ctr,
+                       mc_counters *host_ctr, hipStream_t s) {
+  hipLaunchKernelGGL(k_finalize, dim3(grid_for(m, 256)), dim3(256), 0, s, m, fx, flags, weights,
+                     ctr, host_ctr);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
 }

@@ -108,9 +108,13 @@ __global__ void k_cyc_cells(int64_t total, const double *sigs, const double *ar,
   if (c < total) cells[c] = mc_make_cell(sigs[c], ar[c]);
 }
 
+/* before a cycle's transport; `words` of the cycle's tables come from pinned
+   memory (a copy of its own waits some 20 us between two kernels) */
 __global__ void k_cyc_clear(int64_t total, unsigned long long *fx, uint32_t *flags,
-                            mc_counters *ctr) {
+                            mc_counters *ctr, const unsigned long long *from,
+                            unsigned long long *to, int64_t words) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (int64_t i = c; i < words; i += (int64_t)gridDim.x * blockDim.x) to[i] = from[i];
   if (c < total) {
     fx[c] = 0;
     fx[total + c] = 0;
@@ -219,7 +223,9 @@ __global__ __launch_bounds__(CHUNK) void k_cyc_scan(const rank_in *rin, const ch
 /* The exchange plan, one thread per rank: where each rank's escapes go and
    what each bank receives, in the reference's phase order. */
 __global__ void k_cyc_plan(int R, int64_t S, const rank_in *rin, const rank_tot *tot,
-                           rank_sum *sum) {
+                           rank_sum *sum, rank_sum *host_sum, const mc_counters *ctr,
+                           mc_counters *host_ctr) {
+  mc_counters_to_host(ctr, host_ctr);
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= R) return;
   const rank_in ri = rin[q];
@@ -254,6 +260,7 @@ __global__ void k_cyc_plan(int R, int64_t S, const rank_in *rin, const rank_tot 
   }
   s.new_size = s.keep + from_left + from_right;
   sum[q] = s;
+  host_sum[q] = s; /* pinned */
 }
 
 /* escapes of a chunk into the rank's buffers, in ascending iteration order */
@@ -620,7 +627,8 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
     MC_HIP(ctx, hipMemcpyAsync(d_tiles, h_tiles.data(), sizeof(mc_tile_k) * h_tiles.size(),
                                hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_cyc_clear, dim3(blocks_for(G * m, 256)), dim3(256), 0, s, G * m, d_fx,
-                       d_flags, d_ctr);
+                       d_flags, d_ctr, (const unsigned long long *)nullptr,
+                       (unsigned long long *)nullptr, (int64_t)0);
     MC_HIP(ctx, hipGetLastError());
     const mcgpu_bank bank{work.p.seed, work.p.x, work.p.mu, work.p.wmc, work.p.index};
     MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
@@ -1023,9 +1031,12 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
       }
       ri.chunk_count = (int32_t)(n_chunks - ri.chunk_first);
     }
-    MC_HIP(ctx, hipMemcpyAsync(d_tiles, h_table, table_bytes, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_cyc_clear, dim3(blocks_for(tc, 256)), dim3(256), 0, s, tc, d_fx, d_flags,
-                       d_ctr);
+    static_assert(sizeof(mc_tile_k) % 8 == 0 && sizeof(chunk_k) % 8 == 0 &&
+                      sizeof(rank_in) % 8 == 0, "tables in 8-byte words");
+    hipLaunchKernelGGL(k_cyc_clear, dim3(blocks_for(std::max(tc, (int64_t)(table_bytes / 8)), 256)),
+                       dim3(256), 0, s, tc, d_fx, d_flags, d_ctr,
+                       (const unsigned long long *)h_table, (unsigned long long *)d_tiles,
+                       (int64_t)(table_bytes / 8));
     MC_HIP(ctx, hipGetLastError());
     const mcgpu_bank bank{pool.p.seed, pool.p.x, pool.p.mu, pool.p.wmc, pool.p.index};
     MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
@@ -1047,7 +1058,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
                        (const chunk_cnt *)d_cnt, d_off, d_tot);
     MC_HIP(ctx, hipGetLastError());
     hipLaunchKernelGGL(k_cyc_plan, dim3(blocks_for(R, 256)), dim3(256), 0, s, R, S,
-                       (const rank_in *)d_rin, (const rank_tot *)d_tot, d_sum);
+                       (const rank_in *)d_rin, (const rank_tot *)d_tot, d_sum, h_sum, d_ctr, h_ctr);
     MC_HIP(ctx, hipGetLastError());
     if (n_chunks > 0) {
       hipLaunchKernelGGL(k_cyc_scatter, dim3((unsigned)n_chunks), dim3(CHUNK), 0, s,
@@ -1059,8 +1070,6 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
                        (const rank_in *)d_rin, (const rank_sum *)d_sum, pool.p, esc.p);
     MC_HIP(ctx, hipGetLastError());
     MC_HIP(ctx, hipEventRecord(ev_send, s));
-    MC_HIP(ctx, hipMemcpyAsync(h_sum, d_sum, sizeof(rank_sum) * R, hipMemcpyDeviceToHost, s));
-    MC_HIP(ctx, hipMemcpyAsync(h_ctr, d_ctr, sizeof(mc_counters), hipMemcpyDeviceToHost, s));
     MC_HIP(ctx, hipStreamSynchronize(s));
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);

@@ -26,6 +26,15 @@ struct mc_counters {
   unsigned long long aux[8];     /* kernel-specific (event kernel pass data) */
 };
 
+/* The last kernel of a call hands the counters to the host (pinned memory),
+   without a copy of their own.  host: null, or the pinned words. */
+__device__ __forceinline__ void mc_counters_to_host(const mc_counters *ctr, mc_counters *host) {
+  static_assert(sizeof(mc_counters) % 8 == 0 && sizeof(mc_counters) / 8 <= 64, "one wave");
+  if (host && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < sizeof(mc_counters) / 8)
+    reinterpret_cast<unsigned long long *>(host)[threadIdx.x] =
+        reinterpret_cast<const unsigned long long *>(ctr)[threadIdx.x];
+}
+
 struct mcgpu_context {
   int device = 0;
   int num_cus = 0;
@@ -150,14 +159,16 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
    mc_launch_setup:    cells[c] = (sigs*ar, sigs*(1-ar)), tally words and
                        flags of m cells and the counter block zeroed (a
                        kernel, no memset);
-   mc_launch_finalize: weights[c] += the tally of cell c, rounded once;
+   mc_launch_finalize: weights[c] += the tally of cell c, rounded once; the
+                       counters to host_ctr (pinned) if given;
    mc_status_from_counters: stats from the counter block read back (with
                        the kernel time given) and the call's status. */
 int mc_launch_setup(mcgpu_context *ctx, int m, const double *sigs, const double *ar,
                     mc_cell *cells, unsigned long long *fx, uint32_t *flags, mc_counters *ctr,
                     hipStream_t s);
 int mc_launch_finalize(mcgpu_context *ctx, int m, const unsigned long long *fx,
-                       const uint32_t *flags, double *weights, hipStream_t s);
+                       const uint32_t *flags, double *weights, const mc_counters *ctr,
+                       mc_counters *host_ctr, hipStream_t s);
 int mc_status_from_counters(mcgpu_context *ctx, const mc_counters &hc, float kernel_ms,
                             mcgpu_stats *stats);
 

@@ -150,7 +150,7 @@ extern "C" int mcgpu_simulate_device_noalloc(int64_t n, const mcgpu_bank *bank,
   a.ctr = ctr;
   a.max_events = o.max_events_per_history ? o.max_events_per_history : (1ULL << 27);
   if (n > 0 && (rc = mc_launch_history(&tmp, a, o, s))) return rc;
-  if ((rc = mc_launch_finalize(&tmp, (int)m, fx, flags, weights_absorbed, s))) return rc;
+  if ((rc = mc_launch_finalize(&tmp, (int)m, fx, flags, weights_absorbed, ctr, nullptr, s))) return rc;
   mc_counters hc;
   if (hipMemcpyAsync(&hc, ctr, sizeof hc, hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess) {
