@@ -366,7 +366,7 @@ int build_tables(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
       t.begin = h.particle_offset + p0;
       t.end = h.particle_offset + std::min(h.n, p0 + tile_size);
       tiles.push_back(t);
-      work.push_back((double)(t.end - t.begin) * (double)m);
+      work.push_back(mc_tile_work(t.end - t.begin, m));
     }
   }
   std::vector<size_t> order(tiles.size());

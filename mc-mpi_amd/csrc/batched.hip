@@ -317,7 +317,7 @@ int batch_tiles(mcgpu_batch *b) {
       t.begin = h.particle_offset + p0;
       t.end = h.particle_offset + std::min(h.n, p0 + Ts);
       tiles.push_back(t);
-      work.push_back((double)(t.end - t.begin) * (double)m);
+      work.push_back(mc_tile_work(t.end - t.begin, m));
     }
   }
   std::vector<size_t> order(tiles.size());

@@ -461,7 +461,7 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
   /* work buffer and per-cycle tallies of one group */
   const int64_t pcap = std::max(S, std::min<int64_t>(all, (int64_t)1 << 26));
   const int64_t gcap = std::max<int64_t>(1, ((int64_t)1 << 23) / m);
-  const int64_t max_tiles = pcap / (o.particles_per_lane > 0 ? T : block) + gcap + 1;
+  const int64_t max_tiles = pcap / T + sh.grid + 2 * gcap + 2; /* mc_tile_size */
 
   cycle_mem mem;
   auto dalloc = [&](void **p, size_t bytes) -> int {
@@ -779,7 +779,10 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
     return MCGPU_OK;
   };
   const int64_t tc = total_cells;
-  const int64_t max_tiles = (int64_t)R * ((S + T - 1) / T);
+  const int64_t most = 16 * (int64_t)block; /* of a tile (mc_tile_size) */
+  const int64_t max_tiles = o.particles_per_lane > 0
+                                ? (int64_t)R * ((S + T - 1) / T)
+                                : (int64_t)R * (S / most + 2) + sh.grid + 2;
   const int64_t max_chunks = (int64_t)R * ((S + CHUNK - 1) / CHUNK);
   mc_cell *d_cells;
   unsigned long long *d_fx;
@@ -1004,7 +1007,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
       const int64_t n = std::min(size[r], S);
       const int64_t end = base[r] + size[r];
       const int64_t Tr =
-          o.particles_per_lane > 0 ? T : mc_tile_size(16 * block, share, n, m_of(r), block);
+          o.particles_per_lane > 0 ? T : mc_tile_size(most, share, n, m_of(r), block);
       for (int64_t p0 = end - n; p0 < end; p0 += Tr) {
         mc_tile_k t;
         t.slab = r;

@@ -213,7 +213,10 @@ struct mc_batched_shape {
 /* Histories of a tile of a slab of n histories and m cells: n in equal tiles
    of at most `most`, or, when `share` (a block's part of all slabs' histories
    x cells) is given, of at most that (few or uneven slabs), though of at least
-   one history per thread of the block.  A block waits for its tile's longest
+   one history per four threads (a quarter of a CU's waves run twice as fast as
+   all of them: 120 slabs of 20 to 2,000 histories 15.2 -> 11.5 ms against one
+   per thread).  So there are at most as many tiles as blocks, n / most and one
+   for each slab.  A block waits for its tile's longest
    history, several times the mean one, so small tiles cost more than they
    balance.  In tiles of 4/3, 1, 1/1.3, 1/2 and 1/3 of a part: 512 slabs of 32
    to 8,192 cells 39.8, 39.3, 41.8, 45.5 and 46.5 ms; forward and adjoint of 64
@@ -224,11 +227,19 @@ struct mc_batched_shape {
 inline int64_t mc_tile_size(int64_t most, double share, int64_t n, int m, int block) {
   double fit = (double)most;
   if (share > 0.0 && share / m < fit) fit = share / m;
-  if (fit < (double)block) fit = (double)block;
+  if (fit < (double)block / 4) fit = (double)block / 4;
   const int64_t tiles = (int64_t)((double)n / fit) + ((double)n / fit > (int64_t)((double)n / fit));
   if (tiles <= 1) return n > 0 ? n : 1;
   return ((n + tiles - 1) / tiles + 63) / 64 * 64;
 }
+
+/* What tiles are sorted by, the largest first: about the time of a tile of n
+   histories of m cells, whose longest history counts as much as some 10,000
+   mean ones do on a full block.  Sorted by n m, small tiles of many cells came
+   last and the whole launch waited for them: 512 slabs 38.7 -> 32.6 ms, 80
+   slabs 14.3 -> 10.5 ms (1,000, 3,000 and 30,000 in place of 10,000: the
+   same). */
+inline double mc_tile_work(int64_t n, int m) { return ((double)n + 1e4) * (double)m; }
 
 /* Launch shape for slabs of up to max_m cells; block 0 takes the size with
    the most resident waves, grid <= 0 resident blocks per CU x CUs. */
