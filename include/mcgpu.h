@@ -202,7 +202,8 @@ typedef struct mcgpu_batch mcgpu_batch;
 /* Build a plan: copies the slab table to the device, orders the tiles
    (largest work first) and captures setup + transport + finalize into a
    hipGraph.  opt: block_size, grid_blocks, events_per_refill and
-   particles_per_lane (tile = particles_per_lane * block_size particles).
+   particles_per_lane (tile = particles_per_lane * block_size particles;
+   0: tiles of a block's part of the work).
    Slabs of any cell count: a tile keeps its slab's tally (and cross
    sections) in LDS when they fit and adds to the global tally otherwise. */
 int mcgpu_batch_create(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
@@ -393,7 +394,8 @@ typedef struct mcgpu_cycle_stats {
    sigs, absorption_rates, weights_absorbed: host arrays of total_cells (the
    ranks' cells at their cell_offset); weights_absorbed is added to.
    nb_particles_per_cycle must be in [1, 1000000] (MAX_PARTICLES_VECTOR).
-   opt: block_size (default 256), particles_per_lane (default 1),
+   opt: block_size (default 256), particles_per_lane (default: tiles of a
+   block's part of the cycle's particles),
    events_per_refill, grid_blocks and max_events_per_history of the
    transport launch.  Returns MCGPU_ERR_ARG (and leaves the ranks' outputs
    as of the last cycle) if max_cycles > 0 cycles pass without termination.

@@ -345,7 +345,7 @@ int build_tables(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
   *max_m = 0;
   *max_particle = 0;
   const int64_t most = (int64_t)(ppl > 0 ? ppl : 16) * block;
-  double share = 0.0; /* automatic: at most 16 histories per lane (mc_tile_size) */
+  double share = 0.0; /* automatic: mc_tile_size */
   if (ppl <= 0)
     for (int s = 0; s < n_slabs; ++s)
       share += (double)slabs[s].n * ((double)slabs[s].max_index - slabs[s].min_index) / grid;

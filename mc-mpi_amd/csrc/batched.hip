@@ -302,7 +302,7 @@ int batch_tiles(mcgpu_batch *b) {
   mcgpu_context *ctx = b->ctx;
   const int ppl = b->opt.particles_per_lane > 0 ? b->opt.particles_per_lane : 16;
   const int64_t T = (int64_t)ppl * b->block;
-  double share = 0.0; /* automatic: at most 16 histories per lane (mc_tile_size) */
+  double share = 0.0; /* automatic: mc_tile_size */
   if (b->opt.particles_per_lane <= 0)
     for (const mcgpu_slab &h : b->host_slabs)
       share += (double)h.n * (h.max_index - h.min_index) / b->grid;
@@ -528,8 +528,10 @@ int mcgpu_batch_autotune(mcgpu_batch *b, int32_t n_candidates, double *times_ms,
   struct cand {
     int block, ppl, refill;
   };
-  static const cand cands[] = {{1024, 16, 8}, {1024, 4, 8}, {1024, 64, 8}, {512, 16, 8},
-                               {1024, 16, 32}, {512, 64, 8}, {256, 64, 8}, {1024, 1, 8}};
+  /* the first: the automatic shape (tiles of a block's part, the interval
+     adapted per wave) */
+  static const cand cands[] = {{0, 0, 0},      {1024, 16, 8}, {1024, 4, 8},  {1024, 64, 8},
+                               {1024, 16, 32}, {512, 16, 8},  {256, 64, 8},  {1024, 1, 8}};
   const int n_all = (int)(sizeof(cands) / sizeof(cands[0]));
   const int nc = n_candidates > 0 && n_candidates < n_all ? n_candidates : n_all;
   /* device copies of everything a run overwrites */
@@ -584,6 +586,7 @@ int mcgpu_batch_autotune(mcgpu_batch *b, int32_t n_candidates, double *times_ms,
   b->opt.events_per_refill = cands[best_i].refill;
   b->opt.grid_blocks = 0;
   if (!rc) rc = batch_capture(b);
+  if (cands[best_i].ppl == 0) b->opt.events_per_refill = b->opt.particles_per_lane = 0;
   (void)hipFree(save);
   if (!rc && chosen) *chosen = b->opt;
   return rc;

@@ -212,21 +212,28 @@ struct mc_batched_shape {
 
 /* Histories of a tile of a slab of n histories and m cells: n in equal tiles
    of at most `most`, or, when `share` (a block's part of all slabs' histories
-   x cells) is given, of at most that (few or uneven slabs), though of at least
-   one history per four threads (a quarter of a CU's waves run twice as fast as
-   all of them: 120 slabs of 20 to 2,000 histories 15.2 -> 11.5 ms against one
-   per thread).  So there are at most as many tiles as blocks, n / most and one
-   for each slab.  A block waits for its tile's longest
-   history, several times the mean one, so small tiles cost more than they
-   balance.  In tiles of 4/3, 1, 1/1.3, 1/2 and 1/3 of a part: 512 slabs of 32
-   to 8,192 cells 39.8, 39.3, 41.8, 45.5 and 46.5 ms; forward and adjoint of 64
-   slabs of 50,000 histories on 1,000 cells 27.1, 24.3, 26.0, 28.0 and 29.5 ms;
-   the cycle loop of 20 cycles of 100,000 histories with one rank 8.7 ms in
-   whole parts, 9.2 in halves, 13.3 in tiles of 4,096 (half the blocks without
-   one). */
+   x cells) is given, of at most that part (few or uneven slabs), up to four
+   times `most` where that is a quarter of the part (many), though of at least
+   one history per four threads.  So there are at most as many tiles as blocks,
+   and n / most and one for each slab.
+   A block waits for its tile's longest history, several times the mean one,
+   so small tiles cost more than they balance.  In tiles of 4/3, 1, 1/1.3, 1/2
+   and 1/3 of a part: 512 slabs of 32 to 8,192 cells 39.8, 39.3, 41.8, 45.5 and
+   46.5 ms; forward and adjoint of 64 slabs of 50,000 histories on 1,000 cells
+   27.1, 24.3, 26.0, 28.0 and 29.5 ms; the cycle loop of 20 cycles of 100,000
+   histories with one rank 8.7 ms in whole parts, 9.2 in halves, 13.3 in tiles
+   of 4,096 (half the blocks without one).  4,096 slabs of 5.8e8 histories 2.56
+   s with `most` (16 a thread) and 2.36 with up to four times that, where 512
+   slabs lose without the quarter (32.3 and 37.4 ms).  A quarter of a CU's
+   waves run twice as fast as all of them: 120 slabs of 20 to 2,000 histories
+   15.2 ms with at least one history per thread, 11.5 with one per four. */
 inline int64_t mc_tile_size(int64_t most, double share, int64_t n, int m, int block) {
   double fit = (double)most;
-  if (share > 0.0 && share / m < fit) fit = share / m;
+  if (share > 0.0) {
+    const double part = share / m;
+    if (part / 4.0 > fit) fit = part / 4.0 < 4.0 * fit ? part / 4.0 : 4.0 * fit;
+    if (part < fit) fit = part;
+  }
   if (fit < (double)block / 4) fit = (double)block / 4;
   const int64_t tiles = (int64_t)((double)n / fit) + ((double)n / fit > (int64_t)((double)n / fit));
   if (tiles <= 1) return n > 0 ? n : 1;
@@ -235,11 +242,12 @@ inline int64_t mc_tile_size(int64_t most, double share, int64_t n, int m, int bl
 
 /* What tiles are sorted by, the largest first: about the time of a tile of n
    histories of m cells, whose longest history counts as much as some 10,000
-   mean ones do on a full block.  Sorted by n m, small tiles of many cells came
+   mean ones do on a full block, and whose collisions, load and store as much
+   as some 240 crossings each.  Sorted by n m, small tiles of many cells came
    last and the whole launch waited for them: 512 slabs 38.7 -> 32.6 ms, 80
    slabs 14.3 -> 10.5 ms (1,000, 3,000 and 30,000 in place of 10,000: the
    same). */
-inline double mc_tile_work(int64_t n, int m) { return ((double)n + 1e4) * (double)m; }
+inline double mc_tile_work(int64_t n, int m) { return ((double)n + 1e4) * ((double)m + 240.0); }
 
 /* Launch shape for slabs of up to max_m cells; block 0 takes the size with
    the most resident waves, grid <= 0 resident blocks per CU x CUs. */
