@@ -52,10 +52,10 @@ BYTES_PER_EVENT = 72  # algorithmic: the 36-byte particle state read + written p
 #    an upper bound on HBM bytes, since the Infinity Cache (MALL) in front of
 #    HBM can serve them;
 #  - VALU wave-instructions (SQ_INSTS_VALU).
-MEASURED_TRAFFIC_PER_EVENT = {"history": 0.0616, "event": 19.89}
-# (the event kernel's VALU figure is of a 1e8-particle run, the size bench.py
-# times: at 1e7 the end of the bank, with its partly empty chunks, weighs more)
-MEASURED_VALU_PER_EVENT = {"history": 1.620, "event": 2.918}
+MEASURED_TRAFFIC_PER_EVENT = {"history": 0.312, "event": 19.71}
+# (the VALU figures are of 1e8-particle runs, the size bench.py times: at 1e7
+# the end of the bank, with its partly idle waves, weighs more: 1.050 and 2.813)
+MEASURED_VALU_PER_EVENT = {"history": 0.943, "event": 2.869}
 # gfx950 issues one wave64 VALU instruction per SIMD every 4 cycles:
 # 256 CUs x 4 SIMDs x 2.4 GHz / 4 = 6.144e11 wave-instructions/s.
 VALU_PEAK_WAVE_INSTR = 256 * 4 * 2.4e9 / 4
@@ -76,8 +76,9 @@ def roofline(kernel, events, seconds):
     Both kernels are reported against VALU issue: `frac` is the issue rate
     (measured wave-instructions per event x events/s) over gfx950's 6.144e11
     wave-instructions/s, and the bytes are a side field (`hbm`).
-    history kernel: the state stays in registers (about 0.06 B/event of
-      traffic); bound by VALU issue.
+    history kernel: the state stays in registers (about 0.3 B/event of
+      traffic: histories parked between the layer's two windows); bound by
+      VALU issue and the LDS pipe together.
     event kernel: every event reloads and stores its particle, but the
       fields a pass touches (about 3.7 MB per XCD for the four-slot pools)
       stay in L2: about 3.4 B/event read and 16.5 B/event written reach the
@@ -98,8 +99,9 @@ def roofline(kernel, events, seconds):
            "peak": HBM_PEAK_GBS, "unit": "GB/s"}
     valu = valu_rate(kernel, events, seconds)
     if kernel == "history":
-        note = ("history kernel: one history per lane, state in registers; bound by FP64 VALU "
-                "issue (frac = measured wave-instructions/event x events/s / 6.144e11); ")
+        note = ("history kernel: one history per lane, state in registers; bound by VALU issue "
+                "and the LDS pipe together (frac = measured wave-instructions/event x events/s / "
+                "6.144e11); ")
     else:
         note = ("event kernel: one event per live particle per pass, state reloaded each event "
                 "from per-wave pools whose touched fields stay in L2; frac = measured "

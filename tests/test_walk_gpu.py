@@ -400,3 +400,27 @@ def test_particles_outside_the_layer(ctx, oracle, lo, kernel):
     assert np.array_equal(result, o["result"])
     assert st["events"] == int(o["events"].sum())
     assert np.array_equal(w, o["tally_exact"])
+
+
+def test_long_run_with_scores(ctx, oracle):
+    """The same for a device bank with counts and per-history scores, whose
+    targets take LDS too: 9,000 cells in three windows."""
+    import mcgpu
+    import torch
+    m, n = 9000, 9000
+    rng = np.random.default_rng(81)
+    sa, ss, g = rng.lognormal(0.5, 0.5, m), rng.lognormal(0, 0.5, m), rng.uniform(-1, 1, m)
+    _, _, dx, bank = _case(m, n, 82, 1.0)
+    _say("cells that do not fit, scores")
+    o = oracle.forward_cells(0, m, dx, 1e-1, sa, ss, bank, g=g)
+    db = mcgpu.bank_to_device(bank)
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+    w, sc, dr = dev(np.zeros(m)), dev(np.full(n, 7.0)), dev(np.zeros(n, np.int8))
+    ctx.forward_cells(db, dev(sa), dev(ss), w, 0, m, dx, 1e-1, g=dev(g), history_score=sc,
+                      result=dr, options=mcgpu.make_options("history", grid_blocks=2))
+    b = mcgpu.bank_from_device(db)
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f]), f
+    assert np.array_equal(dr.cpu().numpy().astype(np.int32), o["result"])
+    assert np.array_equal(w.cpu().numpy(), o["tally_exact"])
+    assert np.array_equal(sc.cpu().numpy().view(np.uint64), o["score"].view(np.uint64))
