@@ -218,7 +218,8 @@ int mcgpu_batch_options(const mcgpu_batch *batch, mcgpu_options *opt);
 /*
  * Autotuner: times the plan's transport for each candidate launch shape
  * (block size x particles per lane x events per refill, up to n_candidates
- * of the built-in list) on the plan's own inputs, restoring the bank and
+ * of the built-in list, the automatic shape first: particles_per_lane and
+ * events_per_refill 0) on the plan's own inputs, restoring the bank and
  * weights from a device copy between trials, then re-captures the graph with
  * the fastest.  On return the bank and weights hold their original values.
  * times_ms (may be NULL) receives each candidate's time.
