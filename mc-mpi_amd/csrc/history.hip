@@ -595,24 +595,25 @@ __global__ __launch_bounds__(1024) void k_history_windows(mc_transport_args a, m
         win.list + sh.first, win, &blk, w, 0, false};
     window_io<SCORE> io{a, win, w, &blk, 0.0, -1};
     const uint64_t i = queue.open.q.next + __lane_id();
-    int64_t j = -1;
-    const uint64_t at =
-        mc_scale_place(0, queue.open.q.n, (uint64_t)threadIdx.x * sh.blocks + sh.block,
-                       (uint64_t)blockDim.x * sh.blocks);
-    if (i < queue.open.q.end) {
-      j = queue.list[i];
-    } else if (at < queue.open.q.n) { /* its own share is short: one of all */
-      j = queue.list[at];
+    int k = -1023;
+    auto look = [&](int64_t j) {
+      const int of = mc_ceil_log2(ld_shared(a.aos ? &a.aos[j].wmc : &a.soa.wmc[j]));
+      k = of > k ? of : k;
+    };
+    if (listed) { /* the first histories, and one anywhere in the list */
+      const uint64_t at =
+          mc_scale_place(0, queue.open.q.n, (uint64_t)threadIdx.x * sh.blocks + sh.block,
+                         (uint64_t)blockDim.x * sh.blocks);
+      if (i < queue.open.q.end) look(queue.list[i]);
+      if (at < queue.open.q.n) look(queue.list[at]);
     } else { /* threads look at the run's first histories; none is taken yet */
       const uint32_t next = (uint32_t)blk.run, end = (uint32_t)(blk.run >> 32);
       if (threadIdx.x < end - next) {
         const uint32_t v =
             ld_shared(&win.parked[(size_t)w * win.cap + (next + threadIdx.x) % win.cap]);
-        if (v != MC_NOT_PUT) j = v;
+        if (v != MC_NOT_PUT) look(v);
       }
     }
-    int k = -1023;
-    if (j >= 0) k = mc_ceil_log2(ld_shared(a.aos ? &a.aos[j].wmc : &a.soa.wmc[j]));
     history_block<true, LDS_CELLS, SCORE>(a, L, off, io, queue, k, 0, refill_k);
   }
 }

@@ -510,10 +510,12 @@ __device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, m
    count);
    on_event as in mc_walk_many; moves(k) is called before every (at most) k
    events per lane, k <= k_max.
-   refill_k: events between refills; 0: adapted per wave from the lanes found
-   idle at each refill (many idle: the histories are short against the
-   interval, halve it; almost none: double it, since each refill costs a pass
-   through this loop). */
+   refill_k: events between refills; 0: adapted per wave, from a quarter of the
+   layer's cells (8 to 128; a history crosses about as many as there are; 4 M
+   on 50 cells 1.50 -> 1.42 ms, 200 slabs of 32 cells 0.73 -> 0.61), by the
+   lanes found idle at each refill (many idle: the histories are short against
+   the interval, halve it; almost none: double it, since each refill costs a
+   pass through this loop). */
 template <bool PAD, typename IO, typename Queue, typename Event, typename Moves>
 __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_layer_k &L,
                                              const mc_walk_k &K, const mc_cell *cells,
@@ -532,7 +534,7 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
   uint64_t ev = 0, before = 0; /* events of the lane's history; those before this call */
   uint32_t col = 0;
   const bool adapt = refill_k <= 0;
-  int kk = adapt ? 128 : refill_k;
+  int kk = adapt ? (L.m < 512 ? (L.m > 32 ? L.m >> 2 : 8) : 128) : refill_k;
   int wait = 1;
   /* wave-uniform bound on every lane's event count (a waiting event counted);
      recomputed exactly (the largest in the wave) when an interval could reach
