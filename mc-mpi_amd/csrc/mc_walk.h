@@ -511,11 +511,11 @@ __device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, m
    on_event as in mc_walk_many; moves(k) is called before every (at most) k
    events per lane, k <= k_max.
    refill_k: events between refills; 0: adapted per wave, from a quarter of the
-   layer's cells (8 to 128; a history crosses about as many as there are; 4 M
-   on 50 cells 1.50 -> 1.42 ms, 200 slabs of 32 cells 0.73 -> 0.61), by the
-   lanes found idle at each refill (many idle: the histories are short against
-   the interval, halve it; almost none: double it, since each refill costs a
-   pass through this loop). */
+   layer's cells (8 to 128; with the waiting lanes below 4 M histories on 50
+   cells 1.50 -> 1.38 ms, 200 slabs of 32 cells 0.73 -> 0.53), by the lanes
+   found idle at each refill (many idle: the histories are short against the
+   interval, halve it; almost none: double it, since each refill costs a pass
+   through this loop). */
 template <bool PAD, typename IO, typename Queue, typename Event, typename Moves>
 __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_layer_k &L,
                                              const mc_walk_k &K, const mc_cell *cells,
@@ -534,8 +534,9 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
   uint64_t ev = 0, before = 0; /* events of the lane's history; those before this call */
   uint32_t col = 0;
   const bool adapt = refill_k <= 0;
-  int kk = adapt ? (L.m < 512 ? (L.m > 32 ? L.m >> 2 : 8) : 128) : refill_k;
+  int kk = adapt ? 128 : refill_k;
   int wait = 1;
+  bool first = true; /* no histories taken yet */
   /* wave-uniform bound on every lane's event count (a waiting event counted);
      recomputed exactly (the largest in the wave) when an interval could reach
      the cap, which then shortens the interval: no history passes the cap */
@@ -550,6 +551,16 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
       }
       if (need) {
         const int64_t i = queue.take(need);
+        if (!queue.more()) {
+          if (adapt) kk = 256; /* no refill to come */
+        } else if (first) {
+          /* from the layer's cells: a history crosses about as many as there
+             are; in short ones it collides in many of its events, and those
+             may wait for each other at once */
+          if (adapt && L.m < 512) kk = L.m > 32 ? L.m >> 2 : 8;
+          if (L.m < 128) wait = L.m < 64 ? 12 : 4;
+        }
+        first = false;
         bool on = false;
         if (!has && i >= 0) {
           mc_state in;
