@@ -28,6 +28,8 @@
  *    tally is an exact sum (fixed point, 2^-88 resolution), rounded once to
  *    double and then added, so it is independent of thread scheduling.
  *  - All arithmetic is IEEE binary64; log and exp are correctly rounded.
+ *  - A layer (or slab) has 1 to 2^31 - 1 cells; other ranges of indices return
+ *    MCGPU_ERR_ARG.
  *  - Functions taking a `void *stream` accept a hipStream_t; NULL is HIP's
  *    default (null) stream.  mcgpu_simulate (host buffers) uses the
  *    context's own stream.  No torch or HIP types appear in signatures.

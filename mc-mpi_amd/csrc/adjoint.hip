@@ -48,7 +48,8 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ mc_scale s_scale;
   __shared__ unsigned long long s_tot[MC_TOTALS];
-  const mc_walk_k K = mc_walk_live(a.L);
+  constexpr int U = LDS_T ? MC_IN_LDS : MC_IN_MEMORY;
+  const mc_walk_k K = mc_walk_live<U>(a.L);
   mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
   const int m = a.L.m;
   double2 *tab = reinterpret_cast<double2 *>(smem);
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
                  mc_grad_mover{G, G.every});
   } else {
     constexpr int MODE = LDS_T ? MC_GRAD_CARRY : MC_GRAD_GLOBAL;
-    mc_walk_bank<LDS_C>(io, queue, a.L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
+    mc_walk_bank<LDS_C, U>(io, queue, a.L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
                  [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
                      double wmc) {
                    mc_grad_event<MODE>(io, G, g, lanes, c8, cell, coll, di, dw, wmc);
@@ -121,8 +122,8 @@ __global__ __launch_bounds__(1024) void k_adjoint(adj_args a, int refill_k, int 
 __global__ void k_setup_cells(int m, const double *sig_a, const double *sig_i, mc_cell *cells,
                               unsigned long long *fx, int fx_words_per_cell, uint32_t *flags,
                               int flag_words_per_cell, mc_counters *ctr) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < m) {
+  const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < (size_t)m) {
     mc_cell k;
     k.sig_a = sig_a[c];
     k.sig_i = sig_i[c];
@@ -145,18 +146,18 @@ __global__ void k_finalize2(int m, const unsigned long long *fx, const uint32_t 
                             double *ga, double *gi, const mc_counters *ctr,
                             mc_counters *host_ctr) {
   mc_counters_to_host(ctr, host_ctr);
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < m) {
-    ga[c] = ga[c] + mc_fx_finalize(fx[c], fx[m + c], flags[c]);
-    gi[c] = gi[c] + mc_fx_finalize(fx[2 * m + c], fx[3 * m + c], flags[m + c]);
+  const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
+  if (c < n) {
+    ga[c] = ga[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
+    gi[c] = gi[c] + mc_fx_finalize(fx[2 * n + c], fx[3 * n + c], flags[n + c]);
   }
 }
 
 __global__ void k_finalize1(int m, const unsigned long long *fx, const uint32_t *flags, double *w,
                             const mc_counters *ctr, mc_counters *host_ctr) {
   mc_counters_to_host(ctr, host_ctr);
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < m) w[c] = w[c] + mc_fx_finalize(fx[c], fx[m + c], flags[c]);
+  const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
+  if (c < n) w[c] = w[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
 }
 
 /* the counters that the finalizing kernel has handed over */
@@ -185,7 +186,7 @@ int cells_setup(mcgpu_context *ctx, int m, const double *sig_a, const double *si
   if ((rc = mc_ensure(ctx, &ctx->cells, &ctx->cells_bytes, sizeof(mc_cell) * (size_t)m))) return rc;
   if ((rc = mc_ensure(ctx, &ctx->fx, &ctx->fx_bytes, 8 * (size_t)fx_words * m))) return rc;
   if ((rc = mc_ensure(ctx, &ctx->flags, &ctx->flags_bytes, 4 * (size_t)flag_words * m))) return rc;
-  hipLaunchKernelGGL(k_setup_cells, dim3((m + 255) / 256), dim3(256), 0, s, m, sig_a, sig_i,
+  hipLaunchKernelGGL(k_setup_cells, dim3(((unsigned)m + 255) / 256), dim3(256), 0, s, m, sig_a, sig_i,
                      (mc_cell *)ctx->cells, (unsigned long long *)ctx->fx, fx_words,
                      (uint32_t *)ctx->flags, flag_words, (mc_counters *)ctx->counters);
   MC_HIP(ctx, hipGetLastError());
@@ -244,12 +245,13 @@ int mcgpu_forward_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *bank,
                         void *stream) {
   if (!ctx) return MCGPU_ERR_ARG;
   ctx->err.clear();
-  if (n < 0 || !bank || !sig_a || !sig_i || !weights_absorbed || max_index <= min_index ||
+  if (n < 0 || !bank || !sig_a || !sig_i || !weights_absorbed ||
+      mc_layer_cells(min_index, max_index) == 0 ||
       (history_score && !g))
     return mc_fail(ctx, MCGPU_ERR_ARG, "forward_cells: bad arguments");
   MC_HIP(ctx, hipSetDevice(ctx->device));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int m = max_index - min_index;
+  const int m = mc_layer_cells(min_index, max_index);
   int rc = cells_setup(ctx, m, sig_a, sig_i, 2, 1, s);
   if (rc) return rc;
   mcgpu_options o;
@@ -279,7 +281,7 @@ int mcgpu_forward_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *bank,
     if (rc) return rc;
   }
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
-  hipLaunchKernelGGL(k_finalize1, dim3((m + 255) / 256), dim3(256), 0, s, m,
+  hipLaunchKernelGGL(k_finalize1, dim3(((unsigned)m + 255) / 256), dim3(256), 0, s, m,
                      (const unsigned long long *)ctx->fx, (const uint32_t *)ctx->flags,
                      weights_absorbed, a.ctr, (mc_counters *)ctx->host_counters);
   MC_HIP(ctx, hipGetLastError());
@@ -295,13 +297,13 @@ int mcgpu_adjoint_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *initial
   if (!ctx) return MCGPU_ERR_ARG;
   ctx->err.clear();
   if (n < 0 || !initial || !sig_a || !sig_i || !g || !grad_sig_a || !grad_sig_i ||
-      max_index <= min_index)
+      mc_layer_cells(min_index, max_index) == 0)
     return mc_fail(ctx, MCGPU_ERR_ARG, "adjoint_cells: bad arguments");
   if (n > 0 && (!initial->seed || !initial->x || !initial->mu || !initial->wmc || !initial->index))
     return mc_fail(ctx, MCGPU_ERR_ARG, "adjoint_cells: bank has a null array");
   MC_HIP(ctx, hipSetDevice(ctx->device));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int m = max_index - min_index;
+  const int m = mc_layer_cells(min_index, max_index);
   int rc = cells_setup(ctx, m, sig_a, sig_i, 4, 2, s);
   if (rc) return rc;
   mcgpu_options o;
@@ -328,7 +330,7 @@ int mcgpu_adjoint_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *initial
     if (rc) return rc;
   }
   MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
-  hipLaunchKernelGGL(k_finalize2, dim3((m + 255) / 256), dim3(256), 0, s, m,
+  hipLaunchKernelGGL(k_finalize2, dim3(((unsigned)m + 255) / 256), dim3(256), 0, s, m,
                      (const unsigned long long *)ctx->fx, (const uint32_t *)ctx->flags,
                      grad_sig_a, grad_sig_i, a.ctr, (mc_counters *)ctx->host_counters);
   MC_HIP(ctx, hipGetLastError());

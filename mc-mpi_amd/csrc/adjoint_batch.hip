@@ -187,12 +187,13 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
                    },
                    [](int) {});
     } else {
-      mc_walk_bank<false>(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
-                   s_tot,
-                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+      mc_walk_bank<false, MC_IN_MEMORY>(
+                   io, queue, b.L, mc_walk_live<MC_IN_MEMORY>(b.L), a.cells + b.cell_off, tab,
+                   refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
                      if (mc_in(lanes)) {
-                       mc_tally(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
-                       if (SCORE) io.score = io.score + *mc_word(gg, c8) * dw;
+                       mc_tally(fx_lo, fx_hi, flags, status, c, dw);
+                       if (SCORE) io.score = io.score + gg[c] * dw;
                      }
                    },
                    [](int) {});
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
     const btile b = read_tile(a, t);
     const int m = b.L.m;
     const bool in_lds = m <= a.lds_max_m; /* block-uniform */
-    mc_cell *lc = reinterpret_cast<mc_cell *>(G.t + 4 * m);
+    mc_cell *lc = reinterpret_cast<mc_cell *>(G.t + 4 * (size_t)m);
     double *lg = reinterpret_cast<double *>(lc + m + 2);
     const double *gg = a.g + b.cell_off;
     G.fx = a.fx + b.cell_off;
@@ -281,11 +282,12 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
                    },
                    [](int) {});
     else
-      mc_walk_bank<false>(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30, a.max_events,
-                   s_tot,
-                   [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
+      mc_walk_bank<false, MC_IN_MEMORY>(
+                   io, queue, b.L, mc_walk_live<MC_IN_MEMORY>(b.L), a.cells + b.cell_off, tab,
+                   refill_k, 1 << 30, a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &cell, bool coll, double di, double dw,
                        double wmc) {
-                     mc_grad_event<MC_GRAD_GLOBAL>(io, G, gg, lanes, c8, cell, coll, di, dw, wmc);
+                     mc_grad_event<MC_GRAD_GLOBAL>(io, G, gg, lanes, c, cell, coll, di, dw, wmc);
                    },
                    [](int) {});
     __syncthreads();
@@ -351,7 +353,7 @@ int build_tables(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
       share += (double)slabs[s].n * ((double)slabs[s].max_index - slabs[s].min_index) / grid;
   for (int s = 0; s < n_slabs; ++s) {
     const mcgpu_slab &h = slabs[s];
-    const int m = h.max_index - h.min_index;
+    const int m = mc_layer_cells(h.min_index, h.max_index);
     if (m <= 0 || h.n < 0 || h.cell_offset < 0 || h.cell_offset + m > total_cells ||
         h.particle_offset < 0)
       return mc_fail(ctx, MCGPU_ERR_ARG, "batch: invalid slab descriptor");
@@ -438,7 +440,7 @@ int batch_prepare(mcgpu_context *ctx, K kern, int32_t n_slabs, const mcgpu_slab 
   memset(a, 0, sizeof *a);
   int max_m = 0;
   for (int s_ = 0; s_ < n_slabs; ++s_)
-    max_m = std::max(max_m, slabs[s_].max_index - slabs[s_].min_index);
+    max_m = std::max(max_m, (int)mc_layer_cells(slabs[s_].min_index, slabs[s_].max_index));
   /* LDS for the largest slab that fits; larger slabs use the global accumulators */
   const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES - MC_PAD_BYTES; /* static LDS */
   a->lds_max_m = (int)std::min<size_t>((size_t)max_m, budget / lds_bytes_per_cell);

@@ -155,9 +155,11 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
                    },
                    [](int) {});
     } else {
-      mc_walk_bank<false>(io, queue, L, K, gc, tab, refill_k, 1 << 30, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
-                     if (mc_in(lanes)) mc_tally(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
+      mc_walk_bank<false, MC_IN_MEMORY>(
+                   io, queue, L, mc_walk_live<MC_IN_MEMORY>(L), gc, tab, refill_k, 1 << 30,
+                   a.max_events, s_tot,
+                   [&](mc_mask lanes, int c, const mc_cell &, bool, double, double dw, double) {
+                     if (mc_in(lanes)) mc_tally(fx_lo, fx_hi, flags, status, c, dw);
                    },
                    [](int) {});
     }
@@ -305,12 +307,12 @@ int batch_tiles(mcgpu_batch *b) {
   double share = 0.0; /* automatic: mc_tile_size */
   if (b->opt.particles_per_lane <= 0)
     for (const mcgpu_slab &h : b->host_slabs)
-      share += (double)h.n * (h.max_index - h.min_index) / b->grid;
+      share += (double)h.n * mc_layer_cells(h.min_index, h.max_index) / b->grid;
   std::vector<mc_tile_k> tiles;
   std::vector<double> work;
   for (size_t s = 0; s < b->host_slabs.size(); ++s) {
     const mcgpu_slab &h = b->host_slabs[s];
-    const int m = h.max_index - h.min_index;
+    const int m = mc_layer_cells(h.min_index, h.max_index);
     const int64_t Ts = b->opt.particles_per_lane > 0 ? T : mc_tile_size(T, share, h.n, m, b->block);
     for (int64_t p0 = 0; p0 < h.n; p0 += Ts) {
       mc_tile_k t;
@@ -466,7 +468,7 @@ int mcgpu_batch_create(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *sl
   int rc = MCGPU_OK;
   for (int s = 0; s < n_slabs && !rc; ++s) {
     const mcgpu_slab &h = slabs[s];
-    const int m = h.max_index - h.min_index;
+    const int m = mc_layer_cells(h.min_index, h.max_index);
     if (m <= 0 || h.n < 0 || h.cell_offset < 0 || h.cell_offset + m > total_cells ||
         h.particle_offset < 0)
       rc = mc_fail(ctx, MCGPU_ERR_ARG, "batch: invalid slab descriptor");

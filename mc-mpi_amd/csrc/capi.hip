@@ -54,11 +54,11 @@ namespace {
 
 __global__ void k_setup(int m, const double *sigs, const double *ar, mc_cell *cells,
                         unsigned long long *fx, uint32_t *flags, mc_counters *ctr) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < m) {
+  const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
+  if (c < n) {
     cells[c] = mc_make_cell(sigs[c], ar[c]);
     fx[c] = 0;
-    fx[m + c] = 0;
+    fx[n + c] = 0;
     flags[c] = 0;
   }
   if (c == 0) {
@@ -76,8 +76,8 @@ __global__ void k_setup(int m, const double *sigs, const double *ar, mc_cell *ce
 __global__ void k_finalize(int m, const unsigned long long *fx, const uint32_t *flags,
                            double *weights, const mc_counters *ctr, mc_counters *host_ctr) {
   mc_counters_to_host(ctr, host_ctr);
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < m) weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[m + c], flags[c]);
+  const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
+  if (c < n) weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
 }
 
 __global__ void k_rng_real_step(int64_t n, uint64_t *seeds, double *reals) {
@@ -171,6 +171,8 @@ int transport(mcgpu_context *ctx, mc_transport_args &a, const mcgpu_options *opt
 
 int check_layer(mcgpu_context *ctx, int32_t min_index, int32_t max_index, double dx) {
   if (max_index <= min_index) return mc_fail(ctx, MCGPU_ERR_ARG, "max_index must exceed min_index");
+  if (mc_layer_cells(min_index, max_index) == 0)
+    return mc_fail(ctx, MCGPU_ERR_ARG, "a layer has at most 2^31 - 1 cells");
   (void)dx;
   return MCGPU_OK;
 }
@@ -312,7 +314,7 @@ int mcgpu_simulate(mcgpu_context *ctx, int32_t n, mcgpu_particle *particles, con
   int rc = check_layer(ctx, min_index, max_index, dx);
   if (rc) return rc;
   MC_HIP(ctx, hipSetDevice(ctx->device));
-  const int m = max_index - min_index;
+  const int m = mc_layer_cells(min_index, max_index);
   hipStream_t s = ctx->stream;
   if ((rc = mc_ensure(ctx, &ctx->sig_in, &ctx->sig_in_bytes, 16 * (size_t)m))) return rc;
   if ((rc = mc_ensure(ctx, &ctx->w_in, &ctx->w_in_bytes, 8 * (size_t)m))) return rc;
@@ -365,7 +367,7 @@ int mcgpu_simulate_device(mcgpu_context *ctx, int64_t n, const mcgpu_bank *bank,
   if (rc) return rc;
   MC_HIP(ctx, hipSetDevice(ctx->device));
   hipStream_t s = pick(ctx, stream);
-  const int m = max_index - min_index;
+  const int m = mc_layer_cells(min_index, max_index);
   if ((rc = prepare(ctx, m, sigs, absorption_rates, s))) return rc;
   mc_transport_args a;
   memset(&a, 0, sizeof a);

@@ -721,7 +721,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
   int max_m = 0;
   for (int r = 0; r < R; ++r) {
     const mcgpu_cycle_rank &k = ranks[r];
-    const int64_t m = (int64_t)k.max_index - k.min_index;
+    const int64_t m = mc_layer_cells(k.min_index, k.max_index);
     if (m <= 0 || k.cell_offset < 0 || k.cell_offset + m > total_cells || k.n_particles < 0 ||
         (k.n_particles > 0 && !k.particles) || k.nb_particles_create < 0 || !(k.dx > 0))
       return mc_fail(ctx, MCGPU_ERR_ARG, "sync_cycle: invalid rank descriptor");

@@ -708,7 +708,8 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
     const rsrc_t src = half_rsrc(mine + cur * half_bytes, P);
     pool_queue queue{src, F_CW, n_pool, 0};
     pool_io<COLL> io{v, src, L, P, pass, 0u, 0u};
-    const mc_walk_k W = mc_walk_live(L);
+    constexpr int U = LDS_TALLY ? MC_IN_LDS : MC_IN_MEMORY;
+    const mc_walk_k W = mc_walk_live<U>(L);
     const mc_cell *cells = LDS_CELLS ? cells_l : a.cells;
     const double2 *tab = reinterpret_cast<const double2 *>(mc_abs_tab);
     unsigned long long *fx_lo = a.fx, *fx_hi = a.fx + m;
@@ -721,9 +722,10 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
                    },
                    moves);
     else
-      mc_walk_bank<false>(io, queue, L, W, cells, tab, 0, 1 << 30, max_ev, s_tot,
+      mc_walk_bank<false, U>(io, queue, L, W, cells, tab, 0, 1 << 30, max_ev, s_tot,
                    [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
-                     if (mc_in(lanes)) mc_tally(t_lo, t_hi, flags, status, c8 >> 3, dw);
+                     if (mc_in(lanes))
+                       mc_tally(t_lo, t_hi, flags, status, mc_cell_of<U>(c8), dw);
                    },
                    [](int) {});
   }

@@ -475,7 +475,8 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ mc_scale s_scale;
   __shared__ unsigned long long s_tot[MC_TOTALS];
-  const mc_walk_k K = mc_walk_live(L);
+  constexpr int U = LDS_TALLY ? MC_IN_LDS : MC_IN_MEMORY;
+  const mc_walk_k K = mc_walk_live<U>(L);
   const int m = L.m;
   double2 *tab = reinterpret_cast<double2 *>(smem);
   mc_tab_fill(tab);
@@ -508,7 +509,9 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
   uint32_t *flags = a.flags + off;
   unsigned int *status = &a.ctr->status;
   const mc_block_tally B = mc_block_tally_for(m, s_scale, blockDim.x >> 6);
-  if (LDS_TALLY && B.limbs) { /* block-uniform */
+  bool limbs = false;
+  if constexpr (LDS_TALLY) limbs = B.limbs;
+  if (limbs) { /* block-uniform */
     mc_walk_bank<LDS_CELLS>(io, queue, L, K, cells, tab, refill_k, B.every, a.max_events, s_tot,
                  [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
                    mc_tally_limbs(mine, B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
@@ -519,11 +522,11 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
     mc_limbs_move(T, B.S.L, m, threadIdx.x, blockDim.x, fx_lo, fx_hi);
   } else {
     unsigned long long *lo = LDS_TALLY ? t0 : fx_lo, *hi = LDS_TALLY ? t1 : fx_hi;
-    mc_walk_bank<LDS_CELLS>(io, queue, L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
+    mc_walk_bank<LDS_CELLS, U>(io, queue, L, K, cells, tab, refill_k, 1 << 30, a.max_events, s_tot,
                  [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
                    if (mc_in(lanes)) {
-                     mc_tally(lo, hi, flags, status, c8 >> 3, dw);
-                     if (SCORE) io.score = io.score + *mc_word(g, c8) * dw;
+                     mc_tally(lo, hi, flags, status, mc_cell_of<U>(c8), dw);
+                     if (SCORE) io.score = io.score + *mc_word<U>(g, c8) * dw;
                    }
                  },
                  [](int) {});

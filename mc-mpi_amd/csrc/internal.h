@@ -58,6 +58,13 @@ struct mcgpu_context {
   void *tables = nullptr;     size_t tables_bytes = 0;    /* batched calls: slab + tile tables */
 };
 
+/* the cells of a layer [min_index, max_index): 0 if there are none, or more than
+   the 2^31 - 1 that its 32-bit cell numbers take */
+static inline int32_t mc_layer_cells(int32_t min_index, int32_t max_index) {
+  const int64_t m = (int64_t)max_index - min_index;
+  return m > 0 && m <= INT32_MAX ? (int32_t)m : 0;
+}
+
 /* grow-only device buffer */
 int mc_ensure(mcgpu_context *ctx, void **buf, size_t *cap, size_t need);
 int mc_fail(mcgpu_context *ctx, int status, const char *what, hipError_t e = hipSuccess);

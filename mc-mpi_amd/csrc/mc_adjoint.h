@@ -59,8 +59,8 @@ __device__ __forceinline__ void mc_grad_add(const mc_grad_tally &G, int which, m
   lanes &= mc_lanes(v != 0.0); /* (NaN differs from 0) */
   unsigned long long *fx = G.fx + 2 * which * G.stride;
   uint32_t *flags = which ? G.flags_i : G.flags_a;
-  if (MODE == MC_GRAD_GLOBAL) {
-    if (mc_in(lanes)) mc_tally<true>(fx, fx + G.stride, flags, G.status, c8 >> 3, v);
+  if (MODE == MC_GRAD_GLOBAL) { /* c8 in units of MC_IN_MEMORY */
+    if (mc_in(lanes)) mc_tally<true>(fx, fx + G.stride, flags, G.status, c8, v);
     return;
   }
   if (MODE == MC_GRAD_CARRY) {
@@ -152,7 +152,7 @@ __device__ __forceinline__ void mc_grad_event(mc_grad_io<HAVE_SCORE> &io, const 
                                               const mc_cell &cell, bool coll, double di, double dw,
                                               double wmc) {
   double gc = 0.0;
-  if (mc_in(lanes)) gc = *mc_word(g, c8);
+  if (mc_in(lanes)) gc = *mc_word<MODE == MC_GRAD_GLOBAL ? MC_IN_MEMORY : MC_IN_LDS>(g, c8);
   if (!HAVE_SCORE) {
     const mc_mask first = lanes & mc_lanes(io.phase == 0);
     if (mc_in(first)) io.T = io.T + gc * dw;

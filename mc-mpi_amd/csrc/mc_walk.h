@@ -36,9 +36,14 @@ struct mc_walk {
   double x, mu, wmc;
   double rh, rl;  /* 1/mu = rh + rl, rh = RN(1/mu); rh = NaN: no common step */
   double fe, fs;  /* number of the next edge, +-1 */
-  int32_t c8, st8; /* 8 times the cell's offset in the layer (a byte offset of
-                      8-byte words; twice that of cells), +-8 */
+  int32_t c8, st8; /* U times the cell's offset in the layer, +-U (see below) */
 };
+
+/* U, the unit of c8 and st8.  8 where the tally is in LDS (c8 is then the byte
+   offset of its words, half that of cells); 1 where it is in memory, in layers
+   of any number of cells: 8 times a cell's offset needs a 32nd bit from 2^28
+   cells on.  The global tally's two atomics hide the wider address. */
+constexpr int MC_IN_LDS = 8, MC_IN_MEMORY = 1;
 
 /* Edge distances are formed without range checks: with dx, x and mu in these
    bounds a = xn - x is 0 or at least 2^-752 (a difference of doubles that are
@@ -49,9 +54,10 @@ struct mc_walk {
 #define MC_WALK_DX_MAX 0x1p600
 #define MC_WALK_MU_MAX 0x1p64
 
+template <int U>
 __device__ __forceinline__ void mc_walk_turn(mc_walk &p, int32_t index) {
   const bool back = p.mu < 0;
-  p.st8 = back ? -8 : 8;
+  p.st8 = back ? -U : U;
   p.fs = back ? -1.0 : 1.0;
   p.fe = (double)index + (back ? 0.0 : 1.0);
   p.rh = 1.0 / p.mu;
@@ -61,6 +67,7 @@ __device__ __forceinline__ void mc_walk_turn(mc_walk &p, int32_t index) {
     p.rh = __builtin_nan("");
 }
 
+template <int U>
 __device__ __forceinline__ void mc_walk_from(mc_walk &w, const mc_state &p, const mc_layer_k &L) {
   w.s2 = p.seed << 1;
   w.x = p.x;
@@ -68,8 +75,8 @@ __device__ __forceinline__ void mc_walk_from(mc_walk &w, const mc_state &p, cons
   w.wmc = p.wmc;
   /* a history outside the layer ends at once; the edge's number keeps its index */
   const int64_t c = (int64_t)p.index - L.index_start;
-  w.c8 = c < 0 ? -8 : 8 * (c < L.m ? (int32_t)c : L.m);
-  mc_walk_turn(w, p.index);
+  w.c8 = c < 0 ? -U : U * (c < L.m ? (int32_t)c : L.m);
+  mc_walk_turn<U>(w, p.index);
 }
 
 __device__ __forceinline__ void mc_walk_to(mc_state &p, const mc_walk &w, const mc_layer_k &L) {
@@ -80,8 +87,9 @@ __device__ __forceinline__ void mc_walk_to(mc_state &p, const mc_walk &w, const 
   p.index = (int32_t)(w.fe - (w.st8 > 0 ? 1.0 : 0.0));
 }
 
+template <int U>
 __device__ __forceinline__ bool mc_walk_alive(const mc_walk &w, const mc_layer_k &L) {
-  return (w.wmc >= L.min_weight) && (uint32_t)w.c8 < 8u * (uint32_t)L.m;
+  return (w.wmc >= L.min_weight) && (uint32_t)w.c8 < (uint32_t)U * (uint32_t)L.m;
 }
 
 __device__ __forceinline__ void mc_walk_draw(uint64_t &s2) {
@@ -106,10 +114,11 @@ struct mc_walk_k {
   double sure_max;  /* 2 - 2^-18 */
   double three4;    /* 3/4 */
   double dx, min_weight;
-  uint32_t m8, top8; /* 8 m, 8 (m - 1) */
+  uint32_t m8, top8; /* U m, U (m - 1) */
   uint32_t one;      /* exponent field of 1.0 */
 };
 
+template <int U = MC_IN_LDS>
 __device__ __forceinline__ mc_walk_k mc_walk_live(const mc_layer_k &L) {
   mc_walk_k K;
   K.A = mc_abs_coef_default();
@@ -118,8 +127,8 @@ __device__ __forceinline__ mc_walk_k mc_walk_live(const mc_layer_k &L) {
   K.three4 = 0.75;
   K.dx = L.dx;
   K.min_weight = L.min_weight;
-  K.m8 = 8u * (uint32_t)L.m;
-  K.top8 = K.m8 - 8u;
+  K.m8 = (uint32_t)U * (uint32_t)L.m;
+  K.top8 = K.m8 - (uint32_t)U;
   K.one = 0x3FFu;
   asm volatile("" : "+v"(K.A.c7), "+s"(K.A.c6), "+s"(K.A.c5), "+s"(K.A.c4), "+s"(K.A.c3));
   asm volatile("" : "+s"(K.rem_max), "+s"(K.sure_max), "+s"(K.three4));
@@ -140,17 +149,25 @@ typedef unsigned long long mc_mask;
 __device__ __forceinline__ mc_mask mc_lanes(bool b) { return __builtin_amdgcn_ballot_w64(b); }
 __device__ __forceinline__ bool mc_in(mc_mask m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-/* the cell of c8 (in [0, 8 m)): an unsigned 32-bit byte offset, so that a
-   global load takes the uniform base in scalar registers */
+/* the cell of c8 (in [0, U m)).  U = 8: an unsigned 32-bit byte offset, so that
+   a global load takes the uniform base in scalar registers */
+template <int U>
 __device__ __forceinline__ mc_cell mc_cell_at(const mc_cell *cells, uint32_t c8) {
+  if (U == MC_IN_MEMORY) return cells[c8];
   return *reinterpret_cast<const mc_cell *>(reinterpret_cast<const char *>(cells) + (c8 << 1));
 }
 
-/* word c8 / 8 of an array of 8-byte words */
-template <typename T> __device__ __forceinline__ T *mc_word(T *base, int c8) {
+/* the cell's offset in the layer, and its word in an array of 8-byte words */
+template <int U> __device__ __forceinline__ int mc_cell_of(int c8) {
+  return U == MC_IN_LDS ? c8 >> 3 : c8;
+}
+template <int U = MC_IN_LDS, typename T> __device__ __forceinline__ T *mc_word(T *base, int c8) {
+  if (U == MC_IN_MEMORY) return base + c8;
   return reinterpret_cast<T *>(reinterpret_cast<char *>(base) + c8);
 }
-template <typename T> __device__ __forceinline__ const T *mc_word(const T *base, int c8) {
+template <int U = MC_IN_LDS, typename T>
+__device__ __forceinline__ const T *mc_word(const T *base, int c8) {
+  if (U == MC_IN_MEMORY) return base + c8;
   return reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + c8);
 }
 
@@ -193,6 +210,7 @@ __device__ __forceinline__ mc_mask mc_walk_cross(mc_walk &p, mc_mask run, const 
 /* The general event, after mc_walk_cross has drawn: mc_event_decide's
    operations and the absorption.  Returns the deposit; coll: whether it
    collided, di: the flight. */
+template <int U>
 __device__ __forceinline__ double mc_walk_general(mc_walk &p, const mc_cell cell, const double dx,
                                                   bool &coll, double &di) {
   const mc_coef K = mc_coef_default();
@@ -217,7 +235,7 @@ __device__ __forceinline__ double mc_walk_general(mc_walk &p, const mc_cell cell
     mc_walk_draw(p.s2);
     p.mu = 2 * mc_walk_h(p.s2) - 1;
     /* the index from the edge ahead: fe is index + 1 moving up, index moving down */
-    mc_walk_turn(p, (int32_t)p.fe - (p.st8 > 0 ? 1 : 0));
+    mc_walk_turn<U>(p, (int32_t)p.fe - (p.st8 > 0 ? 1 : 0));
   } else {
     p.x = xn;
     p.fe += p.fs;
@@ -264,7 +282,7 @@ __device__ __forceinline__ mc_mask mc_sets_out(mc_mask &fresh) {
    lanes whose drawn event waits for the general form; `fresh`: lanes that set
    out one after the other, one per event; all wave-uniform masks, disjoint).
    on_event(lanes, c8, cell, coll, di, dw, wmc) is called by the whole wave for
-   an event of `lanes` in cell c8 / 8 (wmc: the weight after it).  ei counts a
+   an event of `lanes` in cell c8 / U (wmc: the weight after it).  ei counts a
    lane's events, col its collisions.  Returns how often the general event ran.
    Every lane computes the common step (lanes not in `run` on whatever they
    hold); only the lanes of a certified crossing commit it.  A history's end
@@ -281,17 +299,18 @@ __device__ __forceinline__ mc_mask mc_sets_out(mc_mask &fresh) {
    58.9 -> 48.2 ms, 8 M on 4,000 cells (bound by LDS: the counter of its active
    cycles stood at 90 % of the time) 81.0 -> 64.6 ms; 1,000 on 1,000 cells,
    where the longest history's events follow one another, 1.09 -> 0.92 ms. */
-template <bool PAD, typename F>
+template <bool PAD, int U, typename F>
 __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &pend,
                                             mc_mask &fresh, int ki, int wait,
                                             const mc_cell *cells, const double2 *tab,
                                             const mc_walk_k &K, uint32_t &ei, uint32_t &col,
                                             F on_event) {
+  static_assert(!PAD || U == MC_IN_LDS, "cells in LDS, tally in LDS");
   int general = 0;
   auto cell_of = [&](int c8) {
     if (PAD) /* c8 >= -8 */
       return *reinterpret_cast<const mc_cell *>(reinterpret_cast<const char *>(cells) + 2 * c8);
-    return mc_cell_at(cells, (uint32_t)c8 < K.top8 ? (uint32_t)c8 : K.top8);
+    return mc_cell_at<U>(cells, (uint32_t)c8 < K.top8 ? (uint32_t)c8 : K.top8);
   };
   for (;;) {
     const int live = __popcll(run | pend | fresh);
@@ -357,8 +376,8 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
       bool coll = false;
       double di = 0.0, dw = 0.0;
       if (mc_in(pend)) {
-        cell = mc_cell_at(cells, (uint32_t)c8);
-        dw = mc_walk_general(p, cell, K.dx, coll, di);
+        cell = mc_cell_at<U>(cells, (uint32_t)c8);
+        dw = mc_walk_general<U>(p, cell, K.dx, coll, di);
         ++ei;
         col += coll ? 1u : 0u;
       }
@@ -516,7 +535,7 @@ __device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, m
    found idle at each refill (many idle: the histories are short against the
    interval, halve it; almost none: double it, since each refill costs a pass
    through this loop). */
-template <bool PAD, typename IO, typename Queue, typename Event, typename Moves>
+template <bool PAD, int U = MC_IN_LDS, typename IO, typename Queue, typename Event, typename Moves>
 __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_layer_k &L,
                                              const mc_walk_k &K, const mc_cell *cells,
                                              const double2 *tab, int refill_k, int k_max,
@@ -565,10 +584,10 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
         if (!has && i >= 0) {
           mc_state in;
           ev = io.load(i, in);
-          mc_walk_from(p, in, L);
+          mc_walk_from<U>(p, in, L);
           idx = i;
           has = true;
-          on = mc_walk_alive(p, L) && ev < max_events;
+          on = mc_walk_alive<U>(p, L) && ev < max_events;
           if (IO::RESUMES) before = ev;
           col = 0;
         }
@@ -605,7 +624,7 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
     moves(ki + 1);
     uint32_t ei = 0; /* events of this interval */
     const int general =
-        mc_walk_many<PAD>(p, run, pend, fresh, ki, wait, cells, tab, K, ei, col, on_event);
+        mc_walk_many<PAD, U>(p, run, pend, fresh, ki, wait, cells, tab, K, ei, col, on_event);
     wait = mc_walk_wait(wait, general, ki);
     ev += ei;
     const bool on = mc_in(run | fresh), waits = mc_in(pend);
@@ -622,8 +641,8 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
       atomicAdd(&s_tot[1], (unsigned long long)col);
       has = io.store(idx, out, code, ev, col);
       if (has) {
-        mc_walk_from(p, out, L);
-        again = mc_walk_alive(p, L);
+        mc_walk_from<U>(p, out, L);
+        again = mc_walk_alive<U>(p, L);
         ev = before = 0;
         col = 0;
       }
