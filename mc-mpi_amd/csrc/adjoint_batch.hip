@@ -106,14 +106,15 @@ template <bool SCORE> struct fwd_io {
     score = 0.0;
     return 0;
   }
-  __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t, uint32_t) {
+  __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t ev, uint32_t) {
+    if (a.result8) a.result8[i] = (int8_t)code;
+    if (SCORE) a.score_out[i] = score;
+    if (ev == 0) return false; /* its state stays as it came (store_state) */
     a.bank.seed[i] = p.seed;
     a.bank.x[i] = p.x;
     a.bank.mu[i] = p.mu;
     a.bank.wmc[i] = p.wmc;
     a.bank.index[i] = p.index;
-    if (a.result8) a.result8[i] = (int8_t)code;
-    if (SCORE) a.score_out[i] = score;
     return false;
   }
 };

@@ -65,13 +65,14 @@ struct tile_io {
     p.index = a.soa.index[i];
     return 0;
   }
-  __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t, uint32_t) {
+  __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t ev, uint32_t) {
+    if (a.result8) a.result8[i] = (int8_t)code;
+    if (ev == 0) return false; /* its state stays as it came (store_state) */
     a.soa.seed[i] = p.seed;
     a.soa.x[i] = p.x;
     a.soa.mu[i] = p.mu;
     a.soa.wmc[i] = p.wmc;
     a.soa.index[i] = p.index;
-    if (a.result8) a.result8[i] = (int8_t)code;
     return false;
   }
 };

@@ -51,7 +51,7 @@ template <bool SCORE> struct bank_io {
   }
   __device__ __forceinline__ bool store(int64_t i, mc_state &p, int code, uint64_t ev,
                                         uint32_t col) {
-    store_state(a, i, p, code);
+    store_state(a, i, p, code, ev != 0);
     if (a.events) a.events[i] = ev;
     if (a.collisions) a.collisions[i] = col;
     if (SCORE) a.score[i] = score;
@@ -190,7 +190,7 @@ template <bool SCORE> struct window_io {
     if (a.collisions) st_shared(&a.collisions[j], ld_shared(&a.collisions[j]) + col);
     if (SCORE) st_shared(&a.score[j], score);
     if (to < 0) {
-      store_state(a, j, p, code);
+      store_state(a, j, p, code, ev != 0);
       if (a.events) a.events[j] = ev;
       win.at[j] = -1;
       atomicAdd(&blk->done, 1u);

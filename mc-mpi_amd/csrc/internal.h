@@ -111,23 +111,27 @@ static __device__ __forceinline__ void load_state(const mc_transport_args &a, in
   }
 }
 
+/* moved: the history had an event; else its state in the bank stays as it came
+   (the walk keeps 63 bits of the seed) */
 static __device__ __forceinline__ void store_state(const mc_transport_args &a, int64_t i,
-                                            const mc_state &p, int code) {
+                                            const mc_state &p, int code, bool moved) {
   if (a.aos) {
+    if (a.result32) a.result32[i] = code;
+    if (!moved) return;
     mcgpu_particle *q = a.aos + i;
     q->seed = p.seed;
     q->x = p.x;
     q->mu = p.mu;
     q->wmc = p.wmc;
     q->index = p.index;
-    if (a.result32) a.result32[i] = code;
   } else {
+    if (a.result8) a.result8[i] = (int8_t)code;
+    if (!moved) return;
     a.soa.seed[i] = p.seed;
     a.soa.x[i] = p.x;
     a.soa.mu[i] = p.mu;
     a.soa.wmc[i] = p.wmc;
     a.soa.index[i] = p.index;
-    if (a.result8) a.result8[i] = (int8_t)code;
   }
 }
 
