@@ -33,6 +33,7 @@
 #include "internal.h"
 #include <algorithm>
 
+#include "mc_ring.h"
 #include "mc_walk.h"
 
 namespace {
@@ -83,6 +84,11 @@ template <bool SCORE> struct bank_io {
    208 ms in two windows (now 161; 234 in one, whose cells do not fit). */
 constexpr int MC_MAX_WINDOWS = 64;
 
+/* between rings, which would otherwise lie a power of two apart: 8 M histories
+   on 10,000 cells 169.8 ms without, 163.4 with (163.3 with rings of as many
+   slots as histories) */
+constexpr uint32_t MC_RING_PAD = 1056;
+
 struct mc_windows {
   int32_t nw, W;            /* window w: cells [w W, (w + 1) W) of the layer */
   uint32_t *count;          /* [nw] histories at the sweep's start */
@@ -91,16 +97,20 @@ struct mc_windows {
   int32_t *at;              /* [n] the cell of a parked history, -1 when finished */
   uint64_t *ev;             /* [n] its events so far */
   /* histories parked in the course of a sweep: window w's are a ring of cap
-     slots at parked + w cap, put[w] - got[w] of them waiting */
-  uint32_t *parked, *put, *got; /* [nw cap], [nw], [nw] */
+     slots (mc_ring.h) at ring(w), put[w] - got[w] of them waiting */
+  uint32_t *parked, *put, *got; /* [nw (cap + MC_RING_PAD)], [nw], [nw] */
   uint32_t *blocks;             /* [nw] blocks that transport window w */
   uint32_t *left;               /* histories not known to be finished */
   uint32_t cap;
   int patience; /* looks of an idle block before it ends */
+  __device__ __forceinline__ uint32_t *ring(int w) const {
+    return parked + (size_t)w * (cap + MC_RING_PAD);
+  }
 };
 constexpr uint32_t MC_NOT_PUT = 0xFFFFFFFFu;
 
-/* the rings' words of a call at most (2 GiB) */
+/* histories x windows of a call with rings at most (2 GiB, 4 GiB where the
+   histories are just above a power of two) */
 constexpr size_t MC_RING_WORDS = (size_t)1 << 29;
 
 /* words of different windows lie on different lines */
@@ -108,7 +118,7 @@ constexpr int MC_WINDOW_STEP = 32;
 
 /* LDS words of a block */
 struct mc_window_block {
-  unsigned long long run; /* the block's run of parked histories: next, end << 32 */
+  unsigned long long run; /* the block's run of parked histories (mc_ring.h) */
   unsigned int looked;    /* clock of the last look at the windows' counts */
   int looking;
   int busy;               /* lanes with a history */
@@ -231,7 +241,7 @@ template <bool SCORE> struct window_io {
     uint32_t base = 0;
     if (rank == 0) base = atomicAdd(&win.put[v * MC_WINDOW_STEP], (uint32_t)__popcll(lanes));
     base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-    st_shared(&win.parked[(size_t)v * win.cap + (base + rank) % win.cap], (uint32_t)j);
+    st_shared(win.ring(v) + mc_ring_slot(base + rank, win.cap), (uint32_t)j);
   }
 };
 
@@ -255,7 +265,7 @@ __device__ __forceinline__ unsigned long long mc_window_claim(const mc_windows &
     uint32_t size = share > want ? share : want;
     size = size < have ? size : have;
     const uint32_t was = atomicCAS(got, at, at + size);
-    if (was == at) return (unsigned long long)at | ((unsigned long long)(at + size) << 32);
+    if (was == at) return mc_ring_run(at, size);
     at = was;
   }
   return 0;
@@ -286,12 +296,10 @@ struct mc_window_queue {
     const uint32_t cnt = (uint32_t)__popcll(need);
     uint32_t next = 0, have = 0;
     if (__lane_id() == 0 && win.cap) {
-      unsigned long long run = ld_block(&blk->run);
-      if ((int32_t)((uint32_t)(run >> 32) - (uint32_t)run) > 0) {
-        run = atomicAdd(&blk->run, (unsigned long long)cnt); /* next stays below 2^32: see look */
-        next = (uint32_t)run;
-        const int32_t d = (int32_t)((uint32_t)(run >> 32) - next);
-        have = d > 0 ? (uint32_t)d : 0u;
+      if (mc_ring_left(ld_block(&blk->run)) != 0) {
+        const unsigned long long run = atomicAdd(&blk->run, (unsigned long long)cnt);
+        next = mc_ring_next(run);
+        have = mc_ring_left(run);
       }
     }
     next = (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
@@ -299,7 +307,7 @@ struct mc_window_queue {
     const uint32_t rank = (uint32_t)mc_mbcnt64(need);
     starved = have < cnt;
     if (mc_in(need) && rank < have) {
-      uint32_t *slot = win.parked + (size_t)w * win.cap + (next + rank) % win.cap;
+      uint32_t *slot = win.ring(w) + mc_ring_slot(next + rank, win.cap);
       uint32_t v = MC_NOT_PUT;
       /* put[] counts it, so its number is on the way; if it does not come in
          time, it stays for the next sweep */
@@ -322,8 +330,7 @@ struct mc_window_queue {
     return __builtin_amdgcn_readfirstlane(ld_block(&blk->leave)) != 0 && !open.more();
   }
   __device__ __forceinline__ bool has_run() const {
-    const unsigned long long run = ld_block(&blk->run);
-    return (int32_t)((uint32_t)(run >> 32) - (uint32_t)run) > 0;
+    return mc_ring_left(ld_block(&blk->run)) != 0;
   }
   __device__ __forceinline__ void look() {
     const unsigned int now = (unsigned int)__builtin_readcyclecounter();
@@ -403,7 +410,7 @@ __global__ void k_windows_clear(mc_windows win, uint32_t *cursor) {
   win.count[t] = 0;
   cursor[t] = 0;
   win.next[t] = 0;
-  win.put[t * MC_WINDOW_STEP] = win.got[t * MC_WINDOW_STEP] = 0;
+  win.put[t * MC_WINDOW_STEP] = win.got[t * MC_WINDOW_STEP] = MC_RING_START;
   win.blocks[t * MC_WINDOW_STEP] = 0;
   if (t == 0) *win.left = 0;
 }
@@ -442,7 +449,8 @@ template <bool OPEN> __global__ void k_windows_count(mc_transport_args a, mc_win
 __global__ void k_windows_list(int64_t n, mc_windows win, uint32_t *list, uint32_t *cursor) {
   __shared__ uint32_t s_n[MC_MAX_WINDOWS], s_at[MC_MAX_WINDOWS];
   const int t = threadIdx.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + t; i < (size_t)win.nw * win.cap;
+  const size_t words = win.cap ? (size_t)win.nw * (win.cap + MC_RING_PAD) : 0;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + t; i < words;
        i += (size_t)gridDim.x * blockDim.x)
     win.parked[i] = MC_NOT_PUT;
   for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < n;
@@ -610,10 +618,9 @@ __global__ __launch_bounds__(1024) void k_history_windows(mc_transport_args a, m
       if (i < queue.open.q.end) look(queue.list[i]);
       if (at < queue.open.q.n) look(queue.list[at]);
     } else { /* threads look at the run's first histories; none is taken yet */
-      const uint32_t next = (uint32_t)blk.run, end = (uint32_t)(blk.run >> 32);
-      if (threadIdx.x < end - next) {
-        const uint32_t v =
-            ld_shared(&win.parked[(size_t)w * win.cap + (next + threadIdx.x) % win.cap]);
+      if (threadIdx.x < mc_ring_left(blk.run)) {
+        const uint32_t v = ld_shared(
+            win.ring(w) + mc_ring_slot(mc_ring_next(blk.run) + threadIdx.x, win.cap));
         if (v != MC_NOT_PUT) look(v);
       }
     }
@@ -683,11 +690,12 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   const int resident = per_cu * ctx->num_cus, grid = o.grid_blocks > 0 ? o.grid_blocks : resident;
   const int k = o.events_per_refill > 0 ? o.events_per_refill : 0;
 
-  /* ev[n], at[n], list[n], parked[nw cap], queue counters, counts, cursors,
+  /* ev[n], at[n], list[n], parked (the rings), queue counters, counts, cursors,
      left, and put, got, blocks a line apart */
   const size_t n = (size_t)a.n;
-  const size_t cap = n * (size_t)nw <= MC_RING_WORDS ? n : 0; /* 0: no ring */
-  const size_t words = (16 * n + 4 * cap * (size_t)nw + 255) / 256 * 256;
+  const size_t cap = n * (size_t)nw <= MC_RING_WORDS ? mc_ring_cap((uint32_t)n) : 0; /* 0: no ring */
+  const size_t rings = cap ? (cap + MC_RING_PAD) * (size_t)nw : 0;
+  const size_t words = (16 * n + 4 * rings + 255) / 256 * 256;
   int rc = mc_ensure(ctx, &ctx->work, &ctx->work_bytes,
                      words + (20 + 12 * MC_WINDOW_STEP) * MC_MAX_WINDOWS);
   if (rc) return rc;
