@@ -215,7 +215,9 @@ int mcgpu_batch_create(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *sl
 /* Launch the captured graph on `stream` and wait; stats may be NULL. */
 int mcgpu_batch_run(mcgpu_batch *batch, void *stream, mcgpu_stats *stats);
 int mcgpu_batch_destroy(mcgpu_batch *batch);
-/* The options a plan was built with (after autotuning, the chosen ones). */
+/* The options a plan was built with (after autotuning, the chosen ones): its
+   block size and grid; events_per_refill and particles_per_lane are 0 where
+   they are automatic.  A plan built from them has the same launch shape. */
 int mcgpu_batch_options(const mcgpu_batch *batch, mcgpu_options *opt);
 /*
  * Autotuner: times the plan's transport for each candidate launch shape

@@ -292,7 +292,7 @@ struct mcgpu_batch {
   size_t lds = 0;
   int lds_cells_max_m = 0;
   int lds_tally_max_m = 0;
-  int block = 1024, grid = 0, refill = 8;
+  int block = 1024, grid = 0;
   hipStream_t stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -345,7 +345,6 @@ int batch_tiles(mcgpu_batch *b) {
 
 int batch_capture(mcgpu_batch *b) {
   mcgpu_context *ctx = b->ctx;
-  b->refill = b->opt.events_per_refill > 0 ? b->opt.events_per_refill : 8;
   int rc;
   mc_batched_shape sh;
   if ((rc = mc_batched_plan_shape(ctx, b->max_m, b->opt.block_size > 0 ? b->opt.block_size : 0,
@@ -394,8 +393,9 @@ int batch_capture(mcgpu_batch *b) {
   MC_HIP(ctx, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
   b->opt.block_size = b->block;
   b->opt.grid_blocks = b->grid;
-  b->opt.events_per_refill = b->refill;
-  if (b->opt.particles_per_lane <= 0) b->opt.particles_per_lane = 16;
+  /* 0 where the plan adapts (mcgpu_batch_options) */
+  b->opt.events_per_refill = std::max(b->opt.events_per_refill, 0);
+  b->opt.particles_per_lane = std::max(b->opt.particles_per_lane, 0);
   return MCGPU_OK;
 }
 
@@ -589,7 +589,6 @@ int mcgpu_batch_autotune(mcgpu_batch *b, int32_t n_candidates, double *times_ms,
   b->opt.events_per_refill = cands[best_i].refill;
   b->opt.grid_blocks = 0;
   if (!rc) rc = batch_capture(b);
-  if (cands[best_i].ppl == 0) b->opt.events_per_refill = b->opt.particles_per_lane = 0;
   (void)hipFree(save);
   if (!rc && chosen) *chosen = b->opt;
   return rc;

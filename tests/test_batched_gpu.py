@@ -183,3 +183,37 @@ def test_autotune_restores_inputs_and_keeps_results(ctx):
     assert _same_bank(mcgpu.bank_from_device(d_bank), ref_bank)
     assert np.array_equal(d_w.cpu().numpy().view(np.uint64), ref_w.view(np.uint64))
     batch.close()
+
+
+def test_options_are_the_plans_own(ctx):
+    """A plan reports the shape that runs: 0 where the interval and the tiles
+    are automatic, the same from create and from the autotuner, the caller's
+    numbers where there were any; a plan built from them reports them again."""
+    import mcgpu
+    slabs, sigs, ar, bank = _batch_inputs(24, 0.02, EXTRA[:2])
+    ref_bank, ref_res, ref_w = _unbatched(ctx, slabs, sigs, ar, bank)
+    given = dict(block_size=256, grid_blocks=40, events_per_refill=16, particles_per_lane=3)
+
+    def plan(options):
+        d_sigs, d_ar, d_w, d_bank, d_res = _device(slabs, sigs, ar, bank)
+        batch = mcgpu.Batch(ctx, slabs, d_sigs, d_ar, d_w, d_bank, d_res, options=options)
+        opt = batch.options()
+        batch.run()
+        assert _same_bank(mcgpu.bank_from_device(d_bank), ref_bank)
+        assert np.array_equal(d_w.cpu().numpy().view(np.uint64), ref_w.view(np.uint64))
+        batch.close()
+        return opt
+
+    auto = plan(None)
+    assert auto["events_per_refill"] == 0 and auto["particles_per_lane"] == 0
+    assert auto["block_size"] > 0 and auto["grid_blocks"] > 0
+    shape = {k: auto[k] for k in given}
+    assert plan(mcgpu.make_options(**shape)) == auto
+    own = plan(mcgpu.make_options(**given))
+    assert {k: own[k] for k in given} == given
+    # the autotuner's first candidate is the automatic shape
+    d_sigs, d_ar, d_w, d_bank, d_res = _device(slabs, sigs, ar, bank)
+    batch = mcgpu.Batch(ctx, slabs, d_sigs, d_ar, d_w, d_bank, d_res)
+    _, chosen = batch.autotune(1)
+    assert chosen == batch.options() == auto
+    batch.close()
