@@ -171,7 +171,8 @@ typedef struct {
 #define MC_FX_HI36 ((uint32_t)((1023 - 36) << 20)) /* high word of 2^-36 */
 #define MC_FX_HI88 ((uint32_t)((1023 - 88) << 20)) /* high word of 2^-88 */
 
-/* terms below 2^V, -35 <= V <= 15 */
+/* terms below 2^V, -35 <= V <= 14: v + c1 stays in c1's binade while
+   2^V <= c1 / 3, which fails at V = 15 */
 MC_FN_HD mc_fx_split mc_fx_split_for(int V) {
   mc_fx_split S;
   S.L = 44 + (V >> 1);

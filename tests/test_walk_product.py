@@ -177,6 +177,15 @@ def test_limbs_equal_the_fixed_point_term(pw, oracle, V):
     assert lg + L - 1 <= 63 and lg + V + 88 - L <= 64
 
 
+@pytest.mark.parametrize("V", [-35, 5, 13, 14])
+def test_limbs_to_the_ends_of_the_stated_range(pw, oracle, V):
+    """mc_fx_split_for's range; one further, terms next to 2^V come out wrong."""
+    test_limbs_equal_the_fixed_point_term(pw, oracle, V)
+    if V == 14:
+        with pytest.raises(AssertionError):
+            test_limbs_equal_the_fixed_point_term(pw, oracle, V + 1)
+
+
 @pytest.mark.parametrize("V", [-30, -3, 0, 2, 5])
 def test_signed_limbs_equal_the_fixed_point_term(pw, oracle, V):
     """The same for terms of either sign (the gradients')."""
