@@ -930,7 +930,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
         hm[i] = q.mu;
         hw[i] = q.wmc;
         hi[i] = q.index;
-        }
+      }
       const int64_t b = base[r];
       MC_HIP(ctx, hipMemcpyAsync(pool.p.seed + b, hs.data(), 8 * n, hipMemcpyHostToDevice, s));
       MC_HIP(ctx, hipMemcpyAsync(pool.p.x + b, hx.data(), 8 * n, hipMemcpyHostToDevice, s));

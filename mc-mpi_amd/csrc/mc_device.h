@@ -95,16 +95,12 @@ __device__ __forceinline__ void mc_fx_atomic_add(unsigned long long *lo_word,
 /* The same without the test of the whole term: both words are added even
    when zero (adding zero changes nothing; the transport's deposits are
    almost never zero, and the tests and their branches cost more than the
-   rare extra atomic).  HI_COND: the high word only when it changes -- for
-   particle weights below 2^-24, whose deposits add nothing there but their
-   carries; then the skipped atomic costs more than the test. */
-template <bool HI_COND>
+   rare extra atomic). */
 __device__ __forceinline__ void mc_fx_atomic_add_always(unsigned long long *lo_word,
                                                         unsigned long long *hi_word, mc_fx v) {
   const unsigned long long old = atomicAdd(lo_word, (unsigned long long)v.lo);
   const unsigned long long carry = (old + v.lo < old) ? 1ULL : 0ULL;
-  const unsigned long long h = (unsigned long long)v.hi + carry;
-  if (!HI_COND || h) atomicAdd(hi_word, h);
+  atomicAdd(hi_word, (unsigned long long)v.hi + carry);
 }
 
 /* --------------------------------------------------------- particle state */
@@ -238,7 +234,7 @@ __device__ __forceinline__ unsigned long long mc_wave_sum(unsigned long long v) 
    transport's non-negative deposits). */
 /* on_flags(g) records the flag word g of a term the general conversion
    flagged (never called for the common terms) */
-template <bool SIGNED = false, bool HI_COND = false, typename OnFlags>
+template <bool SIGNED = false, typename OnFlags>
 __device__ __forceinline__ void mc_tally_with(unsigned long long *lo, unsigned long long *hi, int c,
                                               double dw, OnFlags on_flags) {
   mc_fx v;
@@ -252,13 +248,13 @@ __device__ __forceinline__ void mc_tally_with(unsigned long long *lo, unsigned l
   if (SIGNED)
     mc_fx_atomic_add(&lo[c], &hi[c], v);
   else
-    mc_fx_atomic_add_always<HI_COND>(&lo[c], &hi[c], v);
+    mc_fx_atomic_add_always(&lo[c], &hi[c], v);
 }
 
-template <bool SIGNED = false, bool HI_COND = false>
+template <bool SIGNED = false>
 __device__ __forceinline__ void mc_tally(unsigned long long *lo, unsigned long long *hi,
                                          uint32_t *flags, unsigned int *status, int c, double dw) {
-  mc_tally_with<SIGNED, HI_COND>(lo, hi, c, dw, [&](uint32_t g) {
+  mc_tally_with<SIGNED>(lo, hi, c, dw, [&](uint32_t g) {
     atomicOr(&flags[c], g);
     if (g & 8u) atomicOr(status, 2u);
   });
