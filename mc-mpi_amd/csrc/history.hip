@@ -551,23 +551,65 @@ __device__ __forceinline__ void history_block(const mc_transport_args &a, const 
   if (threadIdx.x == 0) mc_totals_out(s_tot, a.ctr);
 }
 
+/* mc_ceil_log2 of the largest weight among the wave's first histories and one
+   anywhere */
+__device__ __forceinline__ int look_at_weights(const mc_transport_args &a, const mc_queue &q) {
+  int k = -1023;
+  auto look = [&](uint64_t i, uint64_t end) {
+    const int of = i < end ? mc_ceil_log2(a.aos ? a.aos[i].wmc : a.soa.wmc[i]) : -1023;
+    k = of > k ? of : k;
+  };
+  look(q.next + __lane_id(), q.end);
+  look(mc_scale_place(0, (uint64_t)a.n, (uint64_t)threadIdx.x * gridDim.x + blockIdx.x,
+                      (uint64_t)blockDim.x * gridDim.x), (uint64_t)a.n);
+  return k;
+}
+
 template <bool LDS_TALLY, bool LDS_CELLS, bool SCORE>
 __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refill_k, int per_cu,
                                                   int sh) {
   mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
   bank_io<SCORE> io{a, 0.0};
-  int k = -1023;
-  if (LDS_TALLY) { /* the first histories, and one anywhere */
-    auto look = [&](uint64_t i, uint64_t end) {
-      const int of = i < end ? mc_ceil_log2(a.aos ? a.aos[i].wmc : a.soa.wmc[i]) : -1023;
-      k = of > k ? of : k;
-    };
-    look(queue.q.next + __lane_id(), queue.q.end);
-    look(mc_scale_place(0, (uint64_t)a.n, (uint64_t)threadIdx.x * gridDim.x + blockIdx.x,
-                        (uint64_t)blockDim.x * gridDim.x), (uint64_t)a.n);
-  }
+  const int k = LDS_TALLY ? look_at_weights(a, queue.q) : -1023;
   history_block<LDS_TALLY, LDS_CELLS, SCORE>(a, a.L, 0, io, queue, k, LDS_CELLS ? sh : 0,
                                              refill_k);
+}
+
+/* the tally of the first `most` cells in all of the block's LDS (mc_full_tally) */
+__global__ __launch_bounds__(1024) void k_history_full(mc_transport_args a, int refill_k,
+                                                       int per_cu, int most) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ mc_scale s_scale;
+  __shared__ unsigned long long s_tot[MC_TOTALS];
+  mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
+  bank_io<false> io{a, 0.0};
+  const int k = look_at_weights(a, queue.q);
+  const mc_walk_k K = mc_walk_live(a.L);
+  mc_full_tally F;
+  F.t = reinterpret_cast<unsigned long long *>(smem);
+  F.m = a.L.m < most ? a.L.m : most;
+  for (int c = threadIdx.x; c < 2 * F.m; c += blockDim.x) F.t[c] = 0;
+  if (threadIdx.x < MC_TOTALS) s_tot[threadIdx.x] = 0;
+  if (threadIdx.x == 0) mc_scale_clear(&s_scale);
+  __syncthreads();
+  atomicMax(&s_scale.w, k);
+  mc_scale_cells(&s_scale, a.cells, a.L.m, a.L.dx);
+  __syncthreads();
+  F.B = mc_block_tally_for(a.L.m, s_scale, blockDim.x >> 6);
+  F.fx_lo = a.fx;
+  F.fx_hi = a.fx + a.L.m;
+  F.flags = a.flags;
+  F.status = &a.ctr->status;
+  F.left = F.B.every;
+  mc_walk_bank<false>(io, queue, a.L, K, a.cells, reinterpret_cast<const double2 *>(mc_abs_tab),
+               refill_k, F.every(), a.max_events, s_tot,
+               [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                 F.add(lanes, c8, dw);
+               },
+               [&](int n) { F.moves(n); });
+  __syncthreads();
+  F.out();
+  if (threadIdx.x == 0) mc_totals_out(s_tot, a.ctr);
 }
 
 /* one sweep over the windows of a wide layer */
@@ -634,16 +676,10 @@ constexpr size_t window_lds(size_t W, bool cells, bool score) {
          (cells ? sizeof(mc_cell) * W + MC_PAD_BYTES + (score ? 8 * W : 0) : 0);
 }
 
-template <bool T, bool C, bool S>
-int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-               hipStream_t s, size_t lds) {
-  auto kern = k_history<T, C, S>;
-  int sh = 0;
-  if (C) {
-    const size_t other = lds - 16 * (size_t)a.L.m;
-    lds = mc_lds_with_copies(lds, a.L.m);
-    sh = mc_limbs_copies(a.L.m, lds - other);
-  }
+/* last: the kernel's last argument */
+template <typename K>
+int launch_kernel(mcgpu_context *ctx, K kern, const mc_transport_args &a, const mcgpu_options &o,
+                  hipStream_t s, size_t lds, int last) {
   if (lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -663,9 +699,21 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
     if (a.n < grid) grid = (int)(a.n > 0 ? a.n : 1); /* a block per history at most */
   }
   int k = o.events_per_refill > 0 ? o.events_per_refill : 0; /* 0: adaptive */
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k, per_cu, sh);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k, per_cu, last);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
+}
+
+template <bool T, bool C, bool S>
+int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
+               hipStream_t s, size_t lds) {
+  int sh = 0;
+  if (C) {
+    const size_t other = lds - 16 * (size_t)a.L.m;
+    lds = mc_lds_with_copies(lds, a.L.m);
+    sh = mc_limbs_copies(a.L.m, lds - other);
+  }
+  return launch_kernel(ctx, k_history<T, C, S>, a, o, s, lds, sh);
 }
 
 /* Sweeps over a wide layer's windows, cells in LDS or not, until no history is
@@ -801,5 +849,8 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
   }
   if (lds_cells) return launch_one<true, true, false>(ctx, a, o, s, tally + cells);
   if (lds_tally) return launch_one<true, false, false>(ctx, a, o, s, tally);
+  const size_t most = budget / 16; /* cells of a tally in all of LDS */
+  if (m <= most + MC_FULL_BEYOND)
+    return launch_kernel(ctx, k_history_full, a, o, s, 16 * std::min(m, most), (int)most);
   return launch_one<false, false, false>(ctx, a, o, s, MC_TAB_BYTES);
 }

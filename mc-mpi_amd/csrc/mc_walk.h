@@ -854,6 +854,55 @@ struct mc_mover {
   }
 };
 
+/* A tally that takes all of a block's LDS: the layer's first m cells, as limbs
+   or as words with carry, the rows of mc_abs_tab read from memory; terms of the
+   few cells beyond go to the global tally.  For layers whose tally fits LDS but
+   not beside the rows (10,136 to 10,240 cells) where they cannot go in windows:
+   with every term in the global tally 200,000 histories on 10,180 cells take
+   176 ms, 2 M on thick ones 150; so 17.6 and 1.1 (10,240 cells, 16 of them
+   beyond: 22.3; 10,100, beside the rows: 16.1). */
+constexpr int MC_FULL_BEYOND = 16;
+
+struct mc_full_tally {
+  unsigned long long *t; /* LDS */
+  int m;
+  mc_block_tally B;
+  unsigned long long *fx_lo, *fx_hi;
+  uint32_t *flags;
+  unsigned int *status;
+  int left;
+  __device__ __forceinline__ mc_limbs limbs() const { return mc_limbs_at(t, m, 0); }
+  /* events between two calls of moves */
+  __device__ __forceinline__ int every() const { return B.limbs ? B.every : 1 << 30; }
+  __device__ __forceinline__ void moves(int k) {
+    if (!B.limbs) return;
+    if (left < k) { /* wave-uniform */
+      mc_limbs_move(limbs(), B.S.L, m, __lane_id(), 64, fx_lo, fx_hi);
+      left = B.every;
+    }
+    left -= k;
+  }
+  __device__ __forceinline__ void add(mc_mask lanes, int c8, double dw) const {
+    const mc_mask beyond = lanes & mc_lanes(c8 >= 8 * m);
+    if (beyond != 0) { /* wave-uniform */
+      if (mc_in(beyond)) mc_tally(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
+      lanes &= ~beyond;
+    }
+    if (B.limbs)
+      mc_tally_limbs(limbs(), B.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+    else if (mc_in(lanes))
+      mc_tally(t, t + m, flags, status, c8 >> 3, dw);
+  }
+  /* to the global tally, by all threads after a barrier */
+  __device__ __forceinline__ void out() const {
+    if (B.limbs)
+      mc_limbs_move(limbs(), B.S.L, m, threadIdx.x, blockDim.x, fx_lo, fx_hi);
+    else
+      for (int c = threadIdx.x; c < m; c += blockDim.x)
+        mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx{t[c], t[m + c]});
+  }
+};
+
 /* the m cells at `from` into LDS at `to`, with the pads of mc_walk_many's PAD
    (MC_PAD_BYTES more than the cells); returns the first cell's address */
 constexpr size_t MC_PAD_BYTES = 2 * sizeof(mc_cell);

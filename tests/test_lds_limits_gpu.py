@@ -1,0 +1,96 @@
+"""GPU: layers and slabs whose tally just fits a block's LDS, beside the rows of
+the absorbed fraction, without them, and with a few cells beyond: bit-identical
+to the oracle, and no step in time."""
+import ctypes as C
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+
+
+def _case(m, n, wmc, thick=1.0):
+    from mcgpu import PARTICLE, configs
+    rng = np.random.default_rng(m + n)
+    sigs, ar = thick * rng.lognormal(0.3, 0.6, m), rng.uniform(0.05, 0.95, m)
+    bank = np.zeros(n, dtype=PARTICLE)
+    bank["seed"] = configs.seed_chain(n)
+    bank["index"] = rng.integers(0, m, n)
+    bank["index"][::3] = m - 1 - rng.integers(0, 40, len(bank[::3]))  # the last cells
+    bank["x"] = (bank["index"] + rng.random(n)) / m
+    bank["mu"] = rng.uniform(-1, 1, n)
+    bank["wmc"] = wmc
+    return sigs, ar, 1.0 / m, bank
+
+
+def _noalloc(bank, sigs, ar, w, m, dx, min_w, result=None):
+    import torch
+    import mcgpu
+    from mcgpu import _bank_struct, _ptr, lib
+    b, opt = _bank_struct(bank), mcgpu.make_options()
+    rc = lib().mcgpu_simulate_device_noalloc(
+        bank["x"].numel(), C.byref(b), _ptr(sigs), _ptr(ar), _ptr(w), 0, m, dx, min_w,
+        _ptr(result), None, None, C.byref(opt), None, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+
+
+def _dev(x):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+@pytest.mark.parametrize("wmc", [1.0, 50.0])
+@pytest.mark.parametrize("m", [10_135, 10_136, 10_224, 10_225, 10_240, 10_241])
+@pytest.mark.parametrize("how", ["noalloc", "one_block"])
+def test_layers_whose_tally_fills_lds(ctx, oracle, how, m, wmc):
+    """Without allocation, and on one block (too few for windows)."""
+    import mcgpu
+    _say(f"tally fills LDS {how} m={m} weights {wmc}")
+    n, min_w = 600, 0.05 * wmc
+    sigs, ar, dx, bank = _case(m, n, wmc, 30.0)
+    o = oracle.simulate_bank(64, 0, m, dx, min_w, sigs, ar, bank, nthread=8)
+    db, dw, dr = mcgpu.bank_to_device(bank), _dev(np.zeros(m)), _dev(np.zeros(n, np.int8))
+    if how == "noalloc":
+        _noalloc(db, _dev(sigs), _dev(ar), dw, m, dx, min_w, dr)
+    else:
+        ctx.simulate_device(db, _dev(sigs), _dev(ar), dw, 0, m, dx, min_w, result=dr,
+                            options=mcgpu.make_options("history", grid_blocks=1))
+    b = mcgpu.bank_from_device(db)
+    for f in ("seed", "x", "mu", "wmc", "index"):
+        assert np.array_equal(b[f], o["bank"][f]), f
+    assert np.array_equal(dr.cpu().numpy().astype(np.int32), o["result"])
+    assert np.array_equal(dw.cpu().numpy(), o["tally_exact"])
+
+
+def _fastest(run, prepare, times=4):
+    import torch
+    best = 1e9
+    for _ in range(times):
+        prepare()
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        run()
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+def test_no_step_in_time_where_the_tally_fills_lds():
+    """Thick cells, 300,000 histories from one face: with every term in the
+    global tally 10,200 cells take some 77 times as long as 10,100."""
+    import mcgpu
+    t = {}
+    for m in (10_100, 10_200):
+        sigs, ar, dx, bank = _case(m, 300_000, 1.0, 1000.0)
+        bank["index"], bank["x"], bank["mu"] = 0, 0.0, np.abs(bank["mu"])
+        init, ds, da, w = mcgpu.bank_to_device(bank), _dev(sigs), _dev(ar), _dev(np.zeros(m))
+        work = {k: v.clone() for k, v in init.items()}
+        t[m] = _fastest(lambda: _noalloc(work, ds, da, w, m, dx, 1e-3),
+                        lambda: [work[k].copy_(v) for k, v in init.items()])
+        _say(f"no allocation, {m} thick cells: {1e3 * t[m]:.3f} ms")
+    assert t[10_200] < 3 * t[10_100]
