@@ -80,7 +80,10 @@ struct tile_io {
 /* The tile loop is the history kernel's (mc_walk_bank) with the tile's LDS
    counter as its queue; the tally and cell pointers are LDS or global in
    branches of their own, so every access compiles to the matching
-   instruction. */
+   instruction.  WIDE: some slabs' tallies do not fit LDS beside the rows of
+   the absorbed fraction; those that fit without them take all of LDS
+   (mc_full_tally), the others the global tally. */
+template <bool WIDE>
 __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_tile;
@@ -95,6 +98,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
   if (tid < MC_TOTALS) s_tot[tid] = 0;
   if (tid == 0) mc_scale_clear(&s_scale);
   tile_io io{a};
+  bool rows = true; /* in LDS */
 
   for (;;) {
     if (tid == 0) s_tile = (int)atomicAdd(&a.ctr->next, 1ull);
@@ -119,9 +123,21 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     unsigned long long *t1 = t0 + m; /* words with carry: one copy */
     mc_cell *lc = reinterpret_cast<mc_cell *>(t0 + (2 * (size_t)m << sh));
     const mc_cell *gc = a.cells + cell_off;
+    const int most = (int)(a.lds / 16);
+    const bool full = WIDE && !lds_tally && m <= most + MC_FULL_BEYOND; /* block-uniform */
     if (lds_tally) {
       for (int c = tid; c < 2 * m << sh; c += B) t0[c] = 0;
       if (lds_cells) lc = mc_cells_fill(lc, gc, m);
+    }
+    mc_full_tally F;
+    F.t = reinterpret_cast<unsigned long long *>(smem);
+    F.m = m < most ? m : most;
+    if (WIDE) {
+      if (full)
+        for (int c = tid; c < 2 * F.m; c += B) F.t[c] = 0;
+      else if (!rows)
+        mc_tab_fill(tab);
+      rows = !full;
     }
     if (tid == 0) s_next = (unsigned long long)tile.begin;
     /* the tile's weights, from one history per thread (as the history kernel) */
@@ -129,7 +145,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
       const uint64_t i = mc_scale_place(tile.begin, tile.end, tid, B);
       if (i < (uint64_t)tile.end) atomicMax(&s_scale.w, mc_ceil_log2(a.soa.wmc[i]));
     }
-    if (lds_tally && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, gc, m, L.dx);
+    if ((lds_tally || full) && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, gc, m, L.dx);
     __syncthreads();
 
     const mc_walk_k K = mc_walk_live(L);
@@ -155,7 +171,20 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
                      if (mc_in(lanes)) mc_tally(t0, t1, flags, status, c8 >> 3, dw);
                    },
                    [](int) {});
-    } else {
+    } else if (full) {
+      F.B = bt;
+      F.fx_lo = fx_lo;
+      F.fx_hi = fx_hi;
+      F.flags = flags;
+      F.status = status;
+      F.left = bt.every;
+      mc_walk_bank<false>(io, queue, L, K, gc, reinterpret_cast<const double2 *>(mc_abs_tab),
+                   refill_k, F.every(), a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                     F.add(lanes, c8, dw);
+                   },
+                   [&](int n) { F.moves(n); });
+    } else if (WIDE) {
       mc_walk_bank<false, MC_IN_MEMORY>(
                    io, queue, L, mc_walk_live<MC_IN_MEMORY>(L), gc, tab, refill_k, 1 << 30,
                    a.max_events, s_tot,
@@ -175,6 +204,8 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
         v.hi = t1[c];
         mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], v);
       }
+    } else if (full) {
+      F.out();
     }
     if (tid == 0) mc_scale_clear(&s_scale);
     __syncthreads();
@@ -209,6 +240,10 @@ __global__ void k_batch_finalize(int64_t total, const unsigned long long *fx,
   if (c < total) weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[total + c], flags[c]);
 }
 
+void (*batched_kernel(const mc_batched_shape &sh))(batch_args, int) {
+  return sh.wide ? k_batched<true> : k_batched<false>;
+}
+
 } // namespace
 
 int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, int refill,
@@ -225,15 +260,17 @@ int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, in
   sh.lds = mc_lds_with_copies(lds + MC_TAB_BYTES, max_m);
   sh.lds_cells_max_m = (int)((lds - MC_PAD_BYTES) / 32);
   sh.lds_tally_max_m = (int)(lds / 16);
+  sh.wide = max_m > sh.lds_tally_max_m;
+  const auto kern = batched_kernel(sh);
   if (sh.lds > 65536)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k_batched),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds);
   int per_cu = 0;
-  if (block == 0) block = mc_auto_block(k_batched, sh.lds, &per_cu);
+  if (block == 0) block = mc_auto_block(kern, sh.lds, &per_cu);
   sh.block = block;
   sh.grid = grid;
   if (sh.grid <= 0) {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batched, block, sh.lds) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, sh.lds) !=
             hipSuccess ||
         per_cu < 1)
       per_cu = 1;
@@ -263,7 +300,7 @@ int mc_launch_batched(mcgpu_context *ctx, const mc_batched_shape &sh, const mc_s
   a.result8 = result8;
   a.ctr = ctr;
   a.max_events = max_events;
-  hipLaunchKernelGGL(k_batched, dim3(sh.grid), dim3(sh.block), sh.lds, s, a, sh.refill);
+  hipLaunchKernelGGL(batched_kernel(sh), dim3(sh.grid), dim3(sh.block), sh.lds, s, a, sh.refill);
   MC_HIP(ctx, hipGetLastError());
   return MCGPU_OK;
 }
@@ -383,7 +420,7 @@ int batch_capture(mcgpu_batch *b) {
   MC_HIP(ctx, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   hipLaunchKernelGGL(k_batch_setup, dim3((unsigned)((tc + 255) / 256)), dim3(256), 0, b->stream,
                      tc, b->sigs, b->ar, b->d_cells, b->d_fx, b->d_flags, b->d_ctr);
-  hipLaunchKernelGGL(k_batched, dim3(sh.grid), dim3(sh.block), sh.lds, b->stream, a,
+  hipLaunchKernelGGL(batched_kernel(sh), dim3(sh.grid), dim3(sh.block), sh.lds, b->stream, a,
                      sh.refill);
   hipLaunchKernelGGL(k_batch_finalize, dim3((unsigned)((tc + 255) / 256)), dim3(256), 0,
                      b->stream, tc, (const unsigned long long *)b->d_fx,

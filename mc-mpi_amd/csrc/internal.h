@@ -219,6 +219,7 @@ struct mc_batched_shape {
   size_t lds;          /* dynamic LDS bytes per block */
   int lds_cells_max_m; /* slabs with m <= this stage their cells in LDS */
   int lds_tally_max_m; /* slabs with m <= this keep their tally in LDS */
+  bool wide;           /* some slab's tally does not fit beside the rows */
 };
 
 /* Histories of a tile of a slab of n histories and m cells: n in equal tiles

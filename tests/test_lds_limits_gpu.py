@@ -94,3 +94,51 @@ def test_no_step_in_time_where_the_tally_fills_lds():
                         lambda: [work[k].copy_(v) for k, v in init.items()])
         _say(f"no allocation, {m} thick cells: {1e3 * t[m]:.3f} ms")
     assert t[10_200] < 3 * t[10_100]
+
+
+@pytest.mark.parametrize("wmc", [1.0, 50.0])
+@pytest.mark.parametrize("grid", [0, 2])
+def test_slabs_whose_tally_fills_lds(ctx, oracle, grid, wmc):
+    """Slabs around the limits in one plan, small ones between them: on two
+    blocks each takes slabs of every kind, the rows put back after each."""
+    import mcgpu
+    _say(f"slabs that fill LDS grid={grid} weights {wmc}")
+    ms, n, min_w = [10_135, 300, 10_136, 10_224, 40, 10_225, 10_240, 2000, 10_241, 33], 250, 0.05 * wmc
+    cases = [_case(m, n, wmc, 30.0 * m / 10_000) for m in ms]
+    off = np.concatenate([[0], np.cumsum(ms)])
+    slabs = [(0, m, 1.0 / m, min_w, int(off[s]), s * n, n) for s, m in enumerate(ms)]
+    sigs, ar = (np.concatenate([c[k] for c in cases]) for k in (0, 1))
+    db = mcgpu.bank_to_device(np.concatenate([c[3] for c in cases]))
+    dw, dr = _dev(np.zeros(off[-1])), _dev(np.zeros(n * len(ms), np.int8))
+    plan = mcgpu.Batch(ctx, slabs, _dev(sigs), _dev(ar), dw, db, dr,
+                       options=mcgpu.make_options(grid_blocks=grid))
+    plan.run()
+    plan.close()
+    b, w, r = mcgpu.bank_from_device(db), dw.cpu().numpy(), dr.cpu().numpy()
+    for s, (m, (sg, a, dx, bank)) in enumerate(zip(ms, cases)):
+        o = oracle.simulate_bank(64, 0, m, dx, min_w, sg, a, bank, nthread=8)
+        part = slice(s * n, (s + 1) * n)
+        for f in ("seed", "x", "mu", "wmc", "index"):
+            assert np.array_equal(b[f][part], o["bank"][f]), (m, f)
+        assert np.array_equal(r[part].astype(np.int32), o["result"]), m
+        assert np.array_equal(w[off[s]:off[s + 1]], o["tally_exact"]), m
+
+
+def test_no_step_in_time_where_a_slabs_tally_fills_lds(ctx):
+    """As for layers: four slabs of thick cells."""
+    import mcgpu
+    t = {}
+    for m in (10_100, 10_200):
+        n = 100_000
+        cases = [_case(m, n, 1.0, 1000.0) for _ in range(4)]
+        for _, _, _, bank in cases:
+            bank["index"], bank["x"], bank["mu"] = 0, 0.0, np.abs(bank["mu"])
+        sigs, ar = (np.concatenate([c[k] for c in cases]) for k in (0, 1))
+        init = mcgpu.bank_to_device(np.concatenate([c[3] for c in cases]))
+        work = {k: v.clone() for k, v in init.items()}
+        plan = mcgpu.Batch(ctx, [(0, m, 1.0 / m, 1e-3, s * m, s * n, n) for s in range(4)],
+                           _dev(sigs), _dev(ar), _dev(np.zeros(4 * m)), work)
+        t[m] = _fastest(plan.run, lambda: [work[k].copy_(v) for k, v in init.items()])
+        plan.close()
+        _say(f"batch, {m} thick cells: {1e3 * t[m]:.3f} ms")
+    assert t[10_200] < 3 * t[10_100]
