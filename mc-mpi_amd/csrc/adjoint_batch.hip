@@ -10,7 +10,8 @@
  *    them by their time (mc_tile_work), the longest first;
  *  - a persistent block takes the next tile from a global counter, stages the
  *    slab's cells, target weights and (zeroed) fixed-point accumulators in
- *    LDS when they fit (otherwise it adds straight into the global ones),
+ *    LDS when they fit (if not, the accumulators alone, or it adds straight into
+ *    the global ones),
  *    runs the tile's histories with lanes refilled from an LDS counter, and
  *    adds its accumulators to the slab's global cells once per tile.
  * Per history the arithmetic is that of the single-slab kernels (the same
@@ -120,8 +121,11 @@ template <bool SCORE> struct fwd_io {
 };
 
 /* Forward: mcgpu_forward_cells per slab.  Per tile as the batched transport
-   (k_batched), with each history's score. */
-template <bool SCORE>
+   (k_batched), with each history's score.  WIDE: some slabs' cells do not fit
+   LDS beside the tally.  Those keep the tally there while it fits (10,135
+   cells) and read cells and targets through L2: eight slabs of 4,080 cells and
+   3,000 histories, with scores, 25.5 -> 7.3 ms; of 5,100, without, 23.0 -> 7.0. */
+template <bool SCORE, bool WIDE>
 __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_tile;
@@ -141,7 +145,7 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     if (t >= a.n_tiles) break;
     const btile b = read_tile(a, t);
     const int m = b.L.m;
-    const bool in_lds = m <= a.lds_max_m; /* block-uniform */
+    const bool in_lds = !WIDE || m <= a.lds_max_m; /* block-uniform */
     const int sh = in_lds ? mc_limbs_copies(m, a.lds - MC_TAB_BYTES - MC_PAD_BYTES -
                                                    (sizeof(mc_cell) + (SCORE ? 8 : 0)) * m)
                           : 0;
@@ -149,6 +153,12 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     unsigned long long *t1 = t0 + m; /* words with carry: one copy */
     mc_cell *lc = reinterpret_cast<mc_cell *>(t0 + (2 * (size_t)m << sh));
     double *lg = reinterpret_cast<double *>(lc + m + 2);
+    const bool lds_tally = WIDE && !in_lds && 16 * (int64_t)m <= (int64_t)a.lds - (int64_t)MC_TAB_BYTES;
+    mc_full_tally F;
+    F.t = t0;
+    F.m = m;
+    if (WIDE && lds_tally)
+      for (int c = tid; c < 2 * m; c += B) t0[c] = 0;
     if (in_lds) {
       for (int c = tid; c < 2 * m << sh; c += B) t0[c] = 0;
       for (int c = tid; c < m; c += B) {
@@ -161,7 +171,7 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
       const uint64_t i = mc_scale_place(b.begin, b.end, tid, B);
       if (i < (uint64_t)b.end) atomicMax(&s_scale.w, mc_ceil_log2(a.bank.wmc[i]));
     }
-    if (in_lds && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, a.cells + b.cell_off, m, b.L.dx);
+    if ((in_lds || lds_tally) && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, a.cells + b.cell_off, m, b.L.dx);
     __syncthreads();
 
     const mc_walk_k K = mc_walk_live(b.L);
@@ -171,14 +181,28 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     uint32_t *flags = a.flags + b.cell_off;
     unsigned int *status = &a.ctr->status;
     const double *gg = SCORE ? a.g + b.cell_off : nullptr;
-    if (in_lds && bt.limbs) {
+    if (WIDE && lds_tally) {
+      F.B = bt;
+      F.fx_lo = fx_lo;
+      F.fx_hi = fx_hi;
+      F.flags = flags;
+      F.status = status;
+      F.left = bt.every;
+      mc_walk_bank<false>(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, F.every(),
+                   a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+                     F.add(lanes, c8, dw);
+                     if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(gg, c8) * dw;
+                   },
+                   [&](int n) { F.moves(n); });
+    } else if (!(WIDE && !in_lds) && bt.limbs) {
       mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot,
                    [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
                      mc_tally_limbs(mine, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
                      if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(lg, c8) * dw;
                    },
                    mc_mover{T, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every});
-    } else if (in_lds) { /* weights too heavy for the limbs */
+    } else if (!WIDE || in_lds) { /* weights too heavy for the limbs */
       mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
                    [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
                      if (mc_in(lanes)) {
@@ -200,7 +224,9 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
                    [](int) {});
     }
     __syncthreads();
-    if (in_lds) {
+    if (WIDE && lds_tally) {
+      F.out();
+    } else if (!WIDE || in_lds) {
       if (bt.limbs)
         mc_limbs_move(T, bt.S.L, m, tid, B, fx_lo, fx_hi);
       else
@@ -213,8 +239,9 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
   if (tid == 0) mc_totals_out(s_tot, a.ctr);
 }
 
-/* Adjoint: mcgpu_adjoint_cells per slab (replay from the initial bank). */
-template <bool HAVE_SCORE>
+/* Adjoint: mcgpu_adjoint_cells per slab (replay from the initial bank).  WIDE
+   as above (5,067 cells): eight slabs of 2,910 cells 22.1 -> 6.9 ms. */
+template <bool HAVE_SCORE, bool WIDE>
 __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_tile;
@@ -237,7 +264,8 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
     if (t >= a.n_tiles) break;
     const btile b = read_tile(a, t);
     const int m = b.L.m;
-    const bool in_lds = m <= a.lds_max_m; /* block-uniform */
+    const bool in_lds = !WIDE || m <= a.lds_max_m; /* block-uniform */
+    const bool lds_tally = WIDE && !in_lds && 32 * (int64_t)m <= (int64_t)a.lds - (int64_t)MC_TAB_BYTES;
     mc_cell *lc = reinterpret_cast<mc_cell *>(G.t + 4 * (size_t)m);
     double *lg = reinterpret_cast<double *>(lc + m + 2);
     const double *gg = a.g + b.cell_off;
@@ -245,18 +273,18 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
     G.flags_a = a.flags + b.cell_off;
     G.flags_i = a.flags + a.total + b.cell_off;
     G.m = m;
-    if (in_lds) {
+    if (in_lds || lds_tally) {
       int kg = -1023;
       for (int c = tid; c < m; c += B) {
         for (int w = 0; w < 4; ++w) G.t[w * m + c] = 0;
         const double v = gg[c];
-        lg[c] = v;
+        if (in_lds) lg[c] = v;
         const int k = mc_ceil_log2(v);
         kg = k > kg ? k : kg;
       }
       atomicMax(&s_scale.g, kg);
       mc_scale_scatter(&s_scale, a.cells + b.cell_off, m);
-      lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
+      if (in_lds) lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
     }
     if (tid == 0) s_next = b.begin;
     {
@@ -282,7 +310,23 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
                      mc_grad_event<MC_GRAD_CARRY>(io, G, lg, lanes, c8, cell, coll, di, dw, wmc);
                    },
                    [](int) {});
-    else
+    else if (WIDE && lds_tally && limbs)
+      mc_walk_bank<false>(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, G.every,
+                   a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
+                       double wmc) {
+                     mc_grad_event<MC_GRAD_LIMBS>(io, G, gg, lanes, c8, cell, coll, di, dw, wmc);
+                   },
+                   mc_grad_mover{G, G.every});
+    else if (WIDE && lds_tally)
+      mc_walk_bank<false>(io, queue, b.L, K, a.cells + b.cell_off, tab, refill_k, 1 << 30,
+                   a.max_events, s_tot,
+                   [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
+                       double wmc) {
+                     mc_grad_event<MC_GRAD_CARRY>(io, G, gg, lanes, c8, cell, coll, di, dw, wmc);
+                   },
+                   [](int) {});
+    else if (WIDE)
       mc_walk_bank<false, MC_IN_MEMORY>(
                    io, queue, b.L, mc_walk_live<MC_IN_MEMORY>(b.L), a.cells + b.cell_off, tab,
                    refill_k, 1 << 30, a.max_events, s_tot,
@@ -292,7 +336,7 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
                    },
                    [](int) {});
     __syncthreads();
-    if (in_lds) mc_grad_move(G, tid, B, limbs);
+    if (in_lds || lds_tally) mc_grad_move(G, tid, B, limbs);
     if (tid == 0) mc_scale_clear(&s_scale);
     __syncthreads();
   }
@@ -425,6 +469,24 @@ int launch_persistent(mcgpu_context *ctx, K kern, const bcell_args &a, const mcg
   return MCGPU_OK;
 }
 
+/* the LDS for a slab's cells, beside the rows and the kernels' static LDS */
+size_t batch_budget(const mcgpu_context *ctx) {
+  return ctx->lds_per_block - 256 - MC_TAB_BYTES - MC_PAD_BYTES;
+}
+
+int largest_slab(int32_t n_slabs, const mcgpu_slab *slabs) {
+  int m = 0;
+  for (int s = 0; s < n_slabs; ++s)
+    m = std::max(m, (int)mc_layer_cells(slabs[s].min_index, slabs[s].max_index));
+  return m;
+}
+
+/* whether some slab's cells do not fit LDS */
+bool batch_wide(const mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
+                size_t lds_bytes_per_cell) {
+  return (size_t)largest_slab(n_slabs, slabs) > batch_budget(ctx) / lds_bytes_per_cell;
+}
+
 /* Common set-up of both batched calls: options and launch shape of `kern`,
    tables, cells, accumulators, LDS size.  fx_words / flag_words: accumulator
    words per cell. */
@@ -439,13 +501,12 @@ int batch_prepare(mcgpu_context *ctx, K kern, int32_t n_slabs, const mcgpu_slab 
   if (o->block_size > 1024 || o->block_size % 64)
     return mc_fail(ctx, MCGPU_ERR_ARG, "block_size must be a multiple of 64 and <= 1024");
   memset(a, 0, sizeof *a);
-  int max_m = 0;
-  for (int s_ = 0; s_ < n_slabs; ++s_)
-    max_m = std::max(max_m, (int)mc_layer_cells(slabs[s_].min_index, slabs[s_].max_index));
-  /* LDS for the largest slab that fits; larger slabs use the global accumulators */
-  const size_t budget = ctx->lds_per_block - 256 - MC_TAB_BYTES - MC_PAD_BYTES; /* static LDS */
+  int max_m = largest_slab(n_slabs, slabs);
+  /* LDS for the largest slab that fits; all of it if there are larger ones */
+  const size_t budget = batch_budget(ctx);
   a->lds_max_m = (int)std::min<size_t>((size_t)max_m, budget / lds_bytes_per_cell);
-  *lds = MC_TAB_BYTES + MC_PAD_BYTES + lds_bytes_per_cell * (size_t)a->lds_max_m;
+  *lds = MC_TAB_BYTES + MC_PAD_BYTES +
+         (max_m > a->lds_max_m ? budget : lds_bytes_per_cell * (size_t)a->lds_max_m);
   if (flag_words == 1) *lds = mc_lds_with_copies(*lds, a->lds_max_m); /* the forward */
   a->lds = (uint32_t)*lds;
   if (*lds > 65536)
@@ -506,9 +567,12 @@ int mcgpu_forward_cells_batch(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_s
   bcell_args a;
   size_t lds = 0;
   const bool score = history_score != nullptr;
-  const auto kern = score ? k_forward_cells_batch<true> : k_forward_cells_batch<false>;
+  const int per_cell = score ? 40 : 32;
+  const bool wide = batch_wide(ctx, n_slabs, slabs, per_cell);
+  const auto kern = score ? (wide ? k_forward_cells_batch<true, true> : k_forward_cells_batch<true, false>)
+                          : (wide ? k_forward_cells_batch<false, true> : k_forward_cells_batch<false, false>);
   int rc = batch_prepare(ctx, kern, n_slabs, slabs, total_cells, bank, sig_a, sig_i, 2, 1,
-                         score ? 40 : 32, opt, s, &o, &a, &lds);
+                         per_cell, opt, s, &o, &a, &lds);
   if (rc) return rc;
   a.g = g;
   a.score_out = history_score;
@@ -543,7 +607,10 @@ int mcgpu_adjoint_cells_batch(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_s
   mcgpu_options o;
   bcell_args a;
   size_t lds = 0;
-  const auto kern = history_score ? k_adjoint_cells_batch<true> : k_adjoint_cells_batch<false>;
+  const bool wide = batch_wide(ctx, n_slabs, slabs, 56);
+  const auto kern = history_score
+                        ? (wide ? k_adjoint_cells_batch<true, true> : k_adjoint_cells_batch<true, false>)
+                        : (wide ? k_adjoint_cells_batch<false, true> : k_adjoint_cells_batch<false, false>);
   int rc = batch_prepare(ctx, kern, n_slabs, slabs, total_cells, initial, sig_a, sig_i, 4, 2, 56, opt,
                          s, &o, &a, &lds);
   if (rc) return rc;

@@ -142,3 +142,77 @@ def test_no_step_in_time_where_a_slabs_tally_fills_lds(ctx):
         plan.close()
         _say(f"batch, {m} thick cells: {1e3 * t[m]:.3f} ms")
     assert t[10_200] < 3 * t[10_100]
+
+
+@pytest.mark.parametrize("wmc", [1.0, 50.0])
+@pytest.mark.parametrize("score", [True, False])
+def test_gradient_slabs_around_the_lds_limits(ctx, oracle, score, wmc):
+    """Forward (with scores and without) and gradient of slabs on both sides of
+    every limit: cells and tallies in LDS, the tallies alone, neither; on two
+    blocks, each taking slabs of every kind."""
+    import mcgpu
+    import torch
+    _say(f"gradient slabs score={score} weights {wmc}")
+    ms, n, min_w = [2895, 2896, 300, 4053, 4054, 5066, 40, 5067, 5068, 10_135, 10_136], 60, 0.05 * wmc
+    rng = np.random.default_rng(12)
+    cases, g = [], []
+    for m in ms:
+        sigs, ar, dx, bank = _case(m, n, wmc, m / 300.0)
+        cases.append((sigs * ar, sigs * (1 - ar), dx, bank))
+        g.append(rng.uniform(-1, 1, m))
+    off = np.concatenate([[0], np.cumsum(ms)])
+    total = int(off[-1])
+    slabs = [(0, m, 1.0 / m, min_w, int(off[s]), s * n, n) for s, m in enumerate(ms)]
+    sa, si = (_dev(np.concatenate([c[k] for c in cases])) for k in (0, 1))
+    dg = _dev(np.concatenate(g))
+    init = mcgpu.bank_to_device(np.concatenate([c[3] for c in cases]))
+    work = {k: v.clone() for k, v in init.items()}
+    w, ga, gi = (torch.zeros(total, dtype=torch.float64, device="cuda") for _ in range(3))
+    sc = torch.empty(n * len(ms), dtype=torch.float64, device="cuda")
+    opt = mcgpu.make_options(grid_blocks=2)
+    ctx.forward_cells_batch(slabs, work, sa, si, w, g=dg if score else None,
+                            history_score=sc if score else None, options=opt)
+    ctx.adjoint_cells_batch(slabs, init, sa, si, dg, ga, gi, history_score=sc if score else None,
+                            options=opt)
+    same = lambda t, x: np.array_equal(t.cpu().numpy().view(np.uint64), x.view(np.uint64))  # noqa: E731
+    b = mcgpu.bank_from_device(work)
+    for s, m in enumerate(ms):
+        a_, i_, dx, bank = cases[s]
+        o = oracle.forward_cells(0, m, dx, min_w, a_, i_, bank, g=g[s])
+        oa, oi = oracle.adjoint_cells(0, m, dx, min_w, a_, i_, bank, g[s],
+                                      score=o["score"] if score else None)
+        cut, part = slice(off[s], off[s + 1]), slice(s * n, (s + 1) * n)
+        for f in ("seed", "x", "mu", "wmc", "index"):
+            assert np.array_equal(b[f][part], o["bank"][f]), (m, f)
+        assert same(w[cut], o["tally_exact"]), m
+        assert not score or same(sc[part], o["score"]), m
+        assert same(ga[cut], oa) and same(gi[cut], oi), m
+
+
+@pytest.mark.parametrize("what,below,above", [("forward", 5060, 5100), ("score", 4050, 4080),
+                                              ("adjoint", 2890, 2910)])
+def test_no_step_in_time_where_a_slabs_cells_fill_lds(ctx, what, below, above):
+    """Eight slabs of thick cells, all histories from one face, where the
+    global accumulators' adds to one word follow one another."""
+    import mcgpu
+    import torch
+    t = {}
+    for m in (below, above):
+        n, k = 50_000, 8
+        sigs, ar, dx, bank = _case(m, n, 1.0, 1000.0)
+        bank["index"], bank["x"], bank["mu"] = 0, 0.0, np.abs(bank["mu"])
+        sa, si = _dev(np.tile(sigs * ar, k)), _dev(np.tile(sigs * (1 - ar), k))
+        g = torch.ones(k * m, dtype=torch.float64, device="cuda")
+        init = mcgpu.bank_to_device(np.tile(bank, k))
+        work = {f: v.clone() for f, v in init.items()}
+        w, ga, gi = (torch.zeros(k * m, dtype=torch.float64, device="cuda") for _ in range(3))
+        sc = torch.zeros(k * n, dtype=torch.float64, device="cuda")
+        slabs = [(0, m, dx, 1e-3, s * m, s * n, n) for s in range(k)]
+        with_score = {"g": g, "history_score": sc} if what != "forward" else {}
+        run = lambda: ctx.forward_cells_batch(slabs, work, sa, si, w, **with_score)  # noqa: E731
+        if what == "adjoint":
+            run()
+            run = lambda: ctx.adjoint_cells_batch(slabs, init, sa, si, g, ga, gi, history_score=sc)  # noqa: E731
+        t[m] = _fastest(run, lambda: [work[f].copy_(v) for f, v in init.items()])
+        _say(f"{what} of slabs of {m} thick cells: {1e3 * t[m]:.3f} ms")
+    assert t[above] < 3 * t[below]
