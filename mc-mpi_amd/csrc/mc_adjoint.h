@@ -72,7 +72,7 @@ __device__ __forceinline__ void mc_grad_add(const mc_grad_tally &G, int which, m
   if (__builtin_expect(take != lanes, 0)) {
     bool small = false;
     if (mc_in(lanes & ~take)) {
-      small = mc_fx_split_signed_small(&v);
+      small = mc_fx_split_signed_small(&v) || mc_fx_split_signed_tiny(&v);
       if (!small) mc_tally_general(fx, fx + G.stride, flags, G.status, c8 >> 3, v);
     }
     take |= mc_lanes(small);

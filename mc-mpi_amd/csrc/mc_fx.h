@@ -208,7 +208,16 @@ MC_FN_HD int mc_fx_split_small(double *v) {
   return 1;
 }
 
-/* the limbs of a term that one of the two accepts */
+/* v in [0, 2^-88): rounded half up to 0 or 2^-88.  Other terms return 0. */
+MC_FN_HD int mc_fx_split_tiny(double *v) {
+  uint64_t b;
+  __builtin_memcpy(&b, v, 8);
+  if ((uint32_t)(b >> 32) >= MC_FX_HI88) return 0;
+  *v = *v < 0x1p-89 ? 0.0 : 0x1p-88;
+  return 1;
+}
+
+/* the limbs of a term that one of the three accepts */
 MC_FN_HD void mc_fx_split_limbs(double v, const mc_fx_split *S, uint64_t *n0, uint64_t *n1) {
   const double h = v + S->c1;
   const double rest = v - (h - S->c1);
@@ -245,6 +254,13 @@ MC_FN_HD int mc_fx_split_signed_direct(double v, const mc_fx_split *S) {
 MC_FN_HD int mc_fx_split_signed_small(double *v) {
   double a = __builtin_fabs(*v);
   if (!mc_fx_split_small(&a)) return 0;
+  *v = __builtin_copysign(a, *v);
+  return 1;
+}
+
+MC_FN_HD int mc_fx_split_signed_tiny(double *v) {
+  double a = __builtin_fabs(*v);
+  if (!mc_fx_split_tiny(&a)) return 0;
   *v = __builtin_copysign(a, *v);
   return 1;
 }

@@ -801,7 +801,7 @@ __device__ __forceinline__ void mc_tally_limbs(const mc_limbs &T, const mc_fx_sp
   if (__builtin_expect(take != lanes, 0)) { /* wave-uniform: small, large or special terms */
     bool small = false;
     if (mc_in(lanes & ~take)) {
-      small = mc_fx_split_small(&dw);
+      small = mc_fx_split_small(&dw) || mc_fx_split_tiny(&dw);
       if (!small) mc_tally_general(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
     }
     take |= mc_lanes(small);
