@@ -68,16 +68,12 @@ __device__ __forceinline__ void mc_grad_add(const mc_grad_tally &G, int which, m
     if (mc_in(lanes)) mc_tally<true>(t, t + G.m, flags, G.status, c8 >> 3, v);
     return;
   }
-  mc_mask take = lanes & mc_lanes(mc_fx_split_signed_direct(v, &G.S));
+  const mc_mask take = lanes & mc_lanes(mc_fx_split_signed_direct(v, &G.S));
   if (__builtin_expect(take != lanes, 0)) {
-    bool small = false;
-    if (mc_in(lanes & ~take)) {
-      small = mc_fx_split_signed_small(&v) || mc_fx_split_signed_tiny(&v);
-      if (!small) mc_tally_general(fx, fx + G.stride, flags, G.status, c8 >> 3, v);
-    }
-    take |= mc_lanes(small);
+    if (mc_in(lanes & ~take) && !mc_fx_split_signed_small(&v))
+      v = mc_tally_rest(fx, fx + G.stride, flags, G.status, c8 >> 3, v);
   }
-  if (mc_in(take)) {
+  if (mc_in(lanes)) {
     uint64_t n0, n1;
     mc_fx_split_limbs(v, &G.S, &n0, &n1);
     unsigned long long *t = mc_word(G.t + 2 * which * G.m, c8);

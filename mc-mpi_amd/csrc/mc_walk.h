@@ -736,16 +736,21 @@ __device__ __forceinline__ mc_block_tally mc_block_tally_for(int m, const mc_sca
   return B;
 }
 
-/* a term that neither limb conversion takes: to the global tally */
-__device__ __noinline__ static void mc_tally_general(unsigned long long *fx_lo,
-                                                     unsigned long long *fx_hi, uint32_t *flags,
-                                                     unsigned int *status, int c, double dw) {
+/* A term that neither limb conversion takes: rounded to the resolution if it
+   lies below, else to the global tally.  Returns what is left for the limbs.
+   (Out of line: with the rounding inline the cycle loop, whose light particles
+   often take mc_fx_split_small, went from 21.1 to 22.6 ms.) */
+__device__ __noinline__ static double mc_tally_rest(unsigned long long *fx_lo,
+                                                    unsigned long long *fx_hi, uint32_t *flags,
+                                                    unsigned int *status, int c, double dw) {
+  if (mc_fx_split_signed_tiny(&dw)) return dw;
   const mc_fx_flagged g = mc_fx_from_double_general(dw);
   if (g.flags) {
     atomicOr(&flags[c], g.flags);
     if (g.flags & 8u) atomicOr(status, 2u);
   }
   mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], g.v);
+  return 0.0;
 }
 
 /* A block's limb tally of m cells: 2^sh copies of every word, those of a cell
@@ -797,16 +802,12 @@ __device__ __forceinline__ void mc_tally_limbs(const mc_limbs &T, const mc_fx_sp
                                                unsigned long long *fx_hi, uint32_t *flags,
                                                unsigned int *status, mc_mask lanes, int c8,
                                                double dw) {
-  mc_mask take = lanes & mc_lanes(mc_fx_split_direct(dw, &S));
+  const mc_mask take = lanes & mc_lanes(mc_fx_split_direct(dw, &S));
   if (__builtin_expect(take != lanes, 0)) { /* wave-uniform: small, large or special terms */
-    bool small = false;
-    if (mc_in(lanes & ~take)) {
-      small = mc_fx_split_small(&dw) || mc_fx_split_tiny(&dw);
-      if (!small) mc_tally_general(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
-    }
-    take |= mc_lanes(small);
+    if (mc_in(lanes & ~take) && !mc_fx_split_small(&dw))
+      dw = mc_tally_rest(fx_lo, fx_hi, flags, status, c8 >> 3, dw);
   }
-  if (mc_in(take)) {
+  if (mc_in(lanes)) {
     uint64_t n0, n1;
     mc_fx_split_limbs(dw, &S, &n0, &n1);
     atomicAdd(mc_word(T.t0, c8 << T.sh), (unsigned long long)n0);
