@@ -130,11 +130,15 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_tile;
   __shared__ mc_scale s_scale;
+  __shared__ uint32_t s_thick;
   __shared__ unsigned long long s_next;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   const int B = blockDim.x, tid = threadIdx.x;
   if (tid < MC_TOTALS) s_tot[tid] = 0;
-  if (tid == 0) mc_scale_clear(&s_scale);
+  if (tid == 0) {
+    mc_scale_clear(&s_scale);
+    s_thick = 0;
+  }
   double2 *tab = reinterpret_cast<double2 *>(smem);
   mc_tab_fill(tab);
   unsigned long long *t0 = reinterpret_cast<unsigned long long *>(smem + MC_TAB_BYTES);
@@ -171,7 +175,9 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
       const uint64_t i = mc_scale_place(b.begin, b.end, tid, B);
       if (i < (uint64_t)b.end) atomicMax(&s_scale.w, mc_ceil_log2(a.bank.wmc[i]));
     }
-    if ((in_lds || lds_tally) && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, a.cells + b.cell_off, m, b.L.dx);
+    if ((in_lds || lds_tally) && m >= MC_THICK_CELLS)
+      mc_scale_cells(&s_scale, a.cells + b.cell_off, m, b.L.dx);
+    if (in_lds) mc_count_thick(&s_thick, a.cells + b.cell_off, m, b.L.dx);
     __syncthreads();
 
     const mc_walk_k K = mc_walk_live(b.L);
@@ -196,12 +202,17 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
                    },
                    [&](int n) { F.moves(n); });
     } else if (!(WIDE && !in_lds) && bt.limbs) {
-      mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
-                     mc_tally_limbs(mine, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
-                     if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(lg, c8) * dw;
-                   },
-                   mc_mover{T, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every});
+      auto limbs = [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
+        mc_tally_limbs(mine, bt.S, fx_lo, fx_hi, flags, status, lanes, c8, dw);
+        if (SCORE && mc_in(lanes)) io.score = io.score + *mc_word(lg, c8) * dw;
+      };
+      const mc_mover mover{T, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every};
+      if (2 * s_thick > (uint32_t)m) /* block-uniform */
+        mc_walk_bank<true, MC_IN_LDS, true>(io, queue, b.L, K, lc, tab, refill_k, bt.every,
+                     a.max_events, s_tot, limbs, mover);
+      else
+        mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
+                     mover);
     } else if (!WIDE || in_lds) { /* weights too heavy for the limbs */
       mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
                    [&](mc_mask lanes, int c8, const mc_cell &, bool, double, double dw, double) {
@@ -233,7 +244,10 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
         for (int c = tid; c < m; c += B)
           mc_fx_atomic_add(&fx_lo[c], &fx_hi[c], mc_fx{t0[c], t1[c]});
     }
-    if (tid == 0) mc_scale_clear(&s_scale);
+    if (tid == 0) {
+      mc_scale_clear(&s_scale);
+      s_thick = 0;
+    }
     __syncthreads();
   }
   if (tid == 0) mc_totals_out(s_tot, a.ctr);
@@ -246,11 +260,15 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_tile;
   __shared__ mc_scale s_scale;
+  __shared__ uint32_t s_thick;
   __shared__ unsigned long long s_next;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   const int B = blockDim.x, tid = threadIdx.x;
   if (tid < MC_TOTALS) s_tot[tid] = 0;
-  if (tid == 0) mc_scale_clear(&s_scale);
+  if (tid == 0) {
+    mc_scale_clear(&s_scale);
+    s_thick = 0;
+  }
   double2 *tab = reinterpret_cast<double2 *>(smem);
   mc_tab_fill(tab);
   mc_grad_tally G;
@@ -284,6 +302,7 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
       }
       atomicMax(&s_scale.g, kg);
       mc_scale_scatter(&s_scale, a.cells + b.cell_off, m);
+      if (in_lds) mc_count_thick(&s_thick, a.cells + b.cell_off, m, b.L.dx);
       if (in_lds) lc = mc_cells_fill(lc, a.cells + b.cell_off, m);
     }
     if (tid == 0) s_next = b.begin;
@@ -296,12 +315,15 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
     const mc_walk_k K = mc_walk_live(b.L);
     const bool limbs = mc_grad_split(G, s_scale, b.L.dx, B >> 6);
     mc_tile_queue queue{&s_next, b.end, false};
-    if (in_lds && limbs)
-      mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, G.every, a.max_events, s_tot,
-                   [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
-                       double wmc) {
-                     mc_grad_event<MC_GRAD_LIMBS>(io, G, lg, lanes, c8, cell, coll, di, dw, wmc);
-                   },
+    auto add = [&](mc_mask lanes, int c8, const mc_cell &cell, bool coll, double di, double dw,
+                   double wmc) {
+      mc_grad_event<MC_GRAD_LIMBS>(io, G, lg, lanes, c8, cell, coll, di, dw, wmc);
+    };
+    if (in_lds && limbs && 2 * s_thick > (uint32_t)m) /* block-uniform */
+      mc_walk_bank<true, MC_IN_LDS, true>(io, queue, b.L, K, lc, tab, refill_k, G.every,
+                   a.max_events, s_tot, add, mc_grad_mover{G, G.every});
+    else if (in_lds && limbs)
+      mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, G.every, a.max_events, s_tot, add,
                    mc_grad_mover{G, G.every});
     else if (in_lds)
       mc_walk_bank<true>(io, queue, b.L, K, lc, tab, refill_k, 1 << 30, a.max_events, s_tot,
@@ -337,7 +359,10 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
                    [](int) {});
     __syncthreads();
     if (in_lds || lds_tally) mc_grad_move(G, tid, B, limbs);
-    if (tid == 0) mc_scale_clear(&s_scale);
+    if (tid == 0) {
+      mc_scale_clear(&s_scale);
+      s_thick = 0;
+    }
     __syncthreads();
   }
   if (tid == 0) { /* this call counts events alone */

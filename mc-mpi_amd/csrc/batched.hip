@@ -88,6 +88,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_tile;
   __shared__ mc_scale s_scale;
+  __shared__ uint32_t s_thick;
   __shared__ unsigned long long s_next;
   __shared__ unsigned long long s_tot[MC_TOTALS];
   double2 *tab = reinterpret_cast<double2 *>(smem);
@@ -96,7 +97,10 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
   const int B = blockDim.x;
   const int tid = threadIdx.x;
   if (tid < MC_TOTALS) s_tot[tid] = 0;
-  if (tid == 0) mc_scale_clear(&s_scale);
+  if (tid == 0) {
+    mc_scale_clear(&s_scale);
+    s_thick = 0;
+  }
   tile_io io{a};
   bool rows = true; /* in LDS */
 
@@ -146,6 +150,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
       if (i < (uint64_t)tile.end) atomicMax(&s_scale.w, mc_ceil_log2(a.soa.wmc[i]));
     }
     if ((lds_tally || full) && m >= MC_THICK_CELLS) mc_scale_cells(&s_scale, gc, m, L.dx);
+    if (lds_cells) mc_count_thick(&s_thick, gc, m, L.dx);
     __syncthreads();
 
     const mc_walk_k K = mc_walk_live(L);
@@ -159,7 +164,10 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     };
     const mc_mover mover{T, fx_lo, fx_hi, m, bt.S.L, bt.every, bt.every};
     if (lds_tally && bt.limbs) {
-      if (lds_cells)
+      if (lds_cells && 2 * s_thick > (uint32_t)m) /* block-uniform */
+        mc_walk_bank<true, MC_IN_LDS, true>(io, queue, L, K, lc, tab, refill_k, bt.every,
+                     a.max_events, s_tot, limbs, mover);
+      else if (lds_cells)
         mc_walk_bank<true>(io, queue, L, K, lc, tab, refill_k, bt.every, a.max_events, s_tot, limbs,
                      mover);
       else
@@ -207,7 +215,10 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     } else if (full) {
       F.out();
     }
-    if (tid == 0) mc_scale_clear(&s_scale);
+    if (tid == 0) {
+      mc_scale_clear(&s_scale);
+      s_thick = 0;
+    }
     __syncthreads();
   }
   /* the break follows a barrier after the last tile's totals */
