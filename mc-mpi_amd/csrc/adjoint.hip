@@ -139,6 +139,7 @@ __global__ void k_setup_cells(int m, const double *sig_a, const double *sig_i, m
     ctr->n_right = 0;
     ctr->n_killed = 0;
     ctr->status = 0;
+    ctr->left = 0;
   }
 }
 
@@ -157,7 +158,7 @@ __global__ void k_finalize1(int m, const unsigned long long *fx, const uint32_t 
                             const mc_counters *ctr, mc_counters *host_ctr) {
   mc_counters_to_host(ctr, host_ctr);
   const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
-  if (c < n) w[c] = w[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
+  if (c < n && ctr->left == 0) w[c] = w[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
 }
 
 /* the counters that the finalizing kernel has handed over */
@@ -276,16 +277,21 @@ int mcgpu_forward_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *bank,
   a.g = g;
   a.score = history_score;
   MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
-  if (n > 0) {
-    rc = o.kernel == MCGPU_KERNEL_EVENT ? mc_launch_event(ctx, a, o, s) : mc_launch_history(ctx, a, o, s);
-    if (rc) return rc;
-  }
-  MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
-  hipLaunchKernelGGL(k_finalize1, dim3(((unsigned)m + 255) / 256), dim3(256), 0, s, m,
-                     (const unsigned long long *)ctx->fx, (const uint32_t *)ctx->flags,
-                     weights_absorbed, a.ctr, (mc_counters *)ctx->host_counters);
-  MC_HIP(ctx, hipGetLastError());
-  return read_counters(ctx, s, stats);
+  int sweep = 0;
+  do {
+    if (n > 0) {
+      rc = o.kernel == MCGPU_KERNEL_EVENT ? mc_launch_event(ctx, a, o, s)
+                                          : mc_launch_history(ctx, a, o, s, sweep++);
+      if (rc) return rc;
+    }
+    MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
+    hipLaunchKernelGGL(k_finalize1, dim3(((unsigned)m + 255) / 256), dim3(256), 0, s, m,
+                       (const unsigned long long *)ctx->fx, (const uint32_t *)ctx->flags,
+                       weights_absorbed, a.ctr, (mc_counters *)ctx->host_counters);
+    MC_HIP(ctx, hipGetLastError());
+    rc = read_counters(ctx, s, stats);
+  } while (rc != MCGPU_ERR_HIP && ((const mc_counters *)ctx->host_counters)->left != 0);
+  return rc;
 }
 
 int mcgpu_adjoint_cells(mcgpu_context *ctx, int64_t n, const mcgpu_bank *initial,

@@ -69,7 +69,7 @@ __global__ void k_setup(int m, const double *sigs, const double *ar, mc_cell *ce
     ctr->n_right = 0;
     ctr->n_killed = 0;
     ctr->status = 0;
-    for (int i = 0; i < 8; ++i) ctr->aux[i] = 0;
+    ctr->left = 0;
   }
 }
 
@@ -77,7 +77,8 @@ __global__ void k_finalize(int m, const unsigned long long *fx, const uint32_t *
                            double *weights, const mc_counters *ctr, mc_counters *host_ctr) {
   mc_counters_to_host(ctr, host_ctr);
   const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
-  if (c < n) weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
+  if (c < n && ctr->left == 0)
+    weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
 }
 
 __global__ void k_rng_real_step(int64_t n, uint64_t *seeds, double *reals) {
@@ -149,21 +150,23 @@ int transport(mcgpu_context *ctx, mc_transport_args &a, const mcgpu_options *opt
   a.ctr = (mc_counters *)ctx->counters;
   a.max_events = o.max_events_per_history ? o.max_events_per_history : (1ULL << 27);
   MC_HIP(ctx, hipEventRecord(ctx->ev0, s));
-  int rc = MCGPU_OK;
-  if (a.n > 0) {
-    if (o.kernel == MCGPU_KERNEL_HISTORY)
-      rc = mc_launch_history(ctx, a, o, s);
-    else if (o.kernel == MCGPU_KERNEL_EVENT)
-      rc = mc_launch_event(ctx, a, o, s);
-    else
-      rc = mc_fail(ctx, MCGPU_ERR_ARG, "unknown options.kernel");
-  }
-  if (rc) return rc;
-  MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
-  if ((rc = mc_launch_finalize(ctx, a.L.m, a.fx, a.flags, d_weights, a.ctr,
-                               (mc_counters *)ctx->host_counters, s)))
-    return rc;
-  MC_HIP(ctx, hipStreamSynchronize(s));
+  int rc = MCGPU_OK, sweep = 0;
+  do {
+    if (a.n > 0) {
+      if (o.kernel == MCGPU_KERNEL_HISTORY)
+        rc = mc_launch_history(ctx, a, o, s, sweep++);
+      else if (o.kernel == MCGPU_KERNEL_EVENT)
+        rc = mc_launch_event(ctx, a, o, s);
+      else
+        rc = mc_fail(ctx, MCGPU_ERR_ARG, "unknown options.kernel");
+    }
+    if (rc) return rc;
+    MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
+    if ((rc = mc_launch_finalize(ctx, a.L.m, a.fx, a.flags, d_weights, a.ctr,
+                                 (mc_counters *)ctx->host_counters, s)))
+      return rc;
+    MC_HIP(ctx, hipStreamSynchronize(s));
+  } while (((const mc_counters *)ctx->host_counters)->left != 0);
   float ms = 0.f;
   if (stats) (void)hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
   return mc_status_from_counters(ctx, *(const mc_counters *)ctx->host_counters, ms, stats);

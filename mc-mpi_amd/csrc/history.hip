@@ -716,12 +716,13 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
   return launch_kernel(ctx, k_history<T, C, S>, a, o, s, lds, sh);
 }
 
-/* Sweeps over a wide layer's windows, cells in LDS or not, until no history is
-   parked.  Scratch from the context (16 bytes per history and 4 per history
-   and window); MCGPU_ERR_NOMEM: there is none. */
+/* A sweep over a wide layer's windows, cells in LDS or not; ctr->left counts the
+   histories that it has not finished (usually none).  Scratch from the context
+   (16 bytes per history and 4 per history and window); MCGPU_ERR_NOMEM: there is
+   none. */
 template <bool LDS_CELLS, bool S>
 int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-                   hipStream_t s, int nw) {
+                   hipStream_t s, int nw, int sweep) {
   auto kern = k_history_windows<LDS_CELLS, S>;
   const int W = (a.L.m + nw - 1) / nw;
   const size_t lds = window_lds((size_t)W, LDS_CELLS, S);
@@ -739,13 +740,13 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   const int k = o.events_per_refill > 0 ? o.events_per_refill : 0;
 
   /* ev[n], at[n], list[n], parked (the rings), queue counters, counts, cursors,
-     left, and put, got, blocks a line apart */
+     and put, got, blocks a line apart */
   const size_t n = (size_t)a.n;
   const size_t cap = n * (size_t)nw <= MC_RING_WORDS ? mc_ring_cap((uint32_t)n) : 0; /* 0: no ring */
   const size_t rings = cap ? (cap + MC_RING_PAD) * (size_t)nw : 0;
   const size_t words = (16 * n + 4 * rings + 255) / 256 * 256;
   int rc = mc_ensure(ctx, &ctx->work, &ctx->work_bytes,
-                     words + (20 + 12 * MC_WINDOW_STEP) * MC_MAX_WINDOWS);
+                     words + (16 + 12 * MC_WINDOW_STEP) * MC_MAX_WINDOWS);
   if (rc) return rc;
   unsigned char *base = (unsigned char *)ctx->work;
   mc_windows win;
@@ -763,31 +764,24 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   win.next = (unsigned long long *)(base + words);
   win.count = (uint32_t *)(win.next + MC_MAX_WINDOWS);
   uint32_t *cursor = win.count + MC_MAX_WINDOWS;
-  win.left = cursor + MC_MAX_WINDOWS;
-  win.put = win.left + MC_MAX_WINDOWS;
+  win.left = &a.ctr->left;
+  win.put = cursor + MC_MAX_WINDOWS;
   win.got = win.put + MC_MAX_WINDOWS * MC_WINDOW_STEP;
   win.blocks = win.got + MC_MAX_WINDOWS * MC_WINDOW_STEP;
   const unsigned blocks = (unsigned)std::min<size_t>((n + 1023) / 1024, 4 * (size_t)ctx->num_cus);
 
-  for (bool first = true;; first = false) {
-    hipLaunchKernelGGL(k_windows_clear, dim3(1), dim3(64), 0, s, win, cursor);
-    MC_HIP(ctx, hipGetLastError());
-    if (first)
-      hipLaunchKernelGGL(k_windows_count<true>, dim3(blocks), dim3(1024), 0, s, a, win);
-    else
-      hipLaunchKernelGGL(k_windows_count<false>, dim3(blocks), dim3(1024), 0, s, a, win);
-    MC_HIP(ctx, hipGetLastError());
-    if (!first) { /* the first sweep's histories are all of them */
-      uint32_t left = 0;
-      MC_HIP(ctx, hipMemcpyAsync(&left, win.left, 4, hipMemcpyDeviceToHost, s));
-      MC_HIP(ctx, hipStreamSynchronize(s));
-      if (left == 0) return MCGPU_OK;
-    }
-    hipLaunchKernelGGL(k_windows_list, dim3(blocks), dim3(1024), 0, s, a.n, win, list, cursor);
-    MC_HIP(ctx, hipGetLastError());
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, win, k, per_cu);
-    MC_HIP(ctx, hipGetLastError());
-  }
+  hipLaunchKernelGGL(k_windows_clear, dim3(1), dim3(64), 0, s, win, cursor);
+  MC_HIP(ctx, hipGetLastError());
+  if (sweep == 0)
+    hipLaunchKernelGGL(k_windows_count<true>, dim3(blocks), dim3(1024), 0, s, a, win);
+  else
+    hipLaunchKernelGGL(k_windows_count<false>, dim3(blocks), dim3(1024), 0, s, a, win);
+  MC_HIP(ctx, hipGetLastError());
+  hipLaunchKernelGGL(k_windows_list, dim3(blocks), dim3(1024), 0, s, a.n, win, list, cursor);
+  MC_HIP(ctx, hipGetLastError());
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, win, k, per_cu);
+  MC_HIP(ctx, hipGetLastError());
+  return MCGPU_OK;
 }
 
 /* the windows of a layer of m cells */
@@ -799,19 +793,19 @@ int windows_of(size_t m, size_t budget, bool cells, bool score) {
 
 template <bool S>
 int launch_wide(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-                hipStream_t s, size_t budget) {
+                hipStream_t s, size_t budget, int sweep) {
   const int all = windows_of((size_t)a.L.m, budget, true, S);
   const int tally = windows_of((size_t)a.L.m, budget, false, S);
   const int limit = o.grid_blocks > 0 ? std::min(o.grid_blocks, MC_MAX_WINDOWS) : MC_MAX_WINDOWS;
-  if (all <= limit) return launch_windows<true, S>(ctx, a, o, s, all);
-  if (tally > 1 && tally <= limit) return launch_windows<false, S>(ctx, a, o, s, tally);
+  if (all <= limit) return launch_windows<true, S>(ctx, a, o, s, all, sweep);
+  if (tally > 1 && tally <= limit) return launch_windows<false, S>(ctx, a, o, s, tally, sweep);
   return MCGPU_ERR_NOMEM;
 }
 
 } // namespace
 
 int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-                      hipStream_t s) {
+                      hipStream_t s, int sweep) {
   const size_t m = (size_t)a.L.m;
   const size_t tally = 16 * m + MC_TAB_BYTES, cells = sizeof(mc_cell) * m + MC_PAD_BYTES;
   const size_t budget = ctx->lds_per_block - 256; /* the kernel's static LDS */
@@ -836,8 +830,8 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
   const bool block_ok = o.block_size <= 1024 && o.block_size % 64 == 0;
   if ((!lds_tally || long_run) && !ctx->quiet && a.n < (int64_t)0xFFFFFFFFu && block_ok &&
       !(a.score && !a.g)) {
-    const int rc = a.score ? launch_wide<true>(ctx, a, o, s, budget)
-                           : launch_wide<false>(ctx, a, o, s, budget);
+    const int rc = a.score ? launch_wide<true>(ctx, a, o, s, budget, sweep)
+                           : launch_wide<false>(ctx, a, o, s, budget, sweep);
     if (rc != MCGPU_ERR_NOMEM) return rc;
     ctx->err.clear();
   }

@@ -22,8 +22,7 @@ struct mc_counters {
   unsigned long long n_right;
   unsigned long long n_killed;
   unsigned int status;           /* bit 0: event cap hit, bit 1: tally range */
-  unsigned int pad_;
-  unsigned long long aux[8];     /* kernel-specific (event kernel pass data) */
+  unsigned int left;             /* windows: histories not known to be finished */
 };
 
 /* The last kernel of a call hands the counters to the host (pinned memory),
@@ -162,16 +161,18 @@ static inline int mc_auto_block(K kern, size_t lds, int *per_cu) {
   return best;
 }
 
+/* sweep: 0, or, where ctr->left is not 0 after it, the number of the sweep over a
+   wide layer's windows that goes on with the histories left */
 int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-                      hipStream_t s);
+                      hipStream_t s, int sweep = 0);
 
 /* The steps of one transport call around the kernel (capi.hip), on buffers
    the caller provides:
    mc_launch_setup:    cells[c] = (sigs*ar, sigs*(1-ar)), tally words and
                        flags of m cells and the counter block zeroed (a
                        kernel, no memset);
-   mc_launch_finalize: weights[c] += the tally of cell c, rounded once; the
-                       counters to host_ctr (pinned) if given;
+   mc_launch_finalize: weights[c] += the tally of cell c, rounded once, unless
+                       ctr->left; the counters to host_ctr (pinned) if given;
    mc_status_from_counters: stats from the counter block read back (with
                        the kernel time given) and the call's status. */
 int mc_launch_setup(mcgpu_context *ctx, int m, const double *sigs, const double *ar,
