@@ -255,6 +255,23 @@ __device__ __forceinline__ int mc_walk_wait(int wait, int general, int iteration
   return wait > 1 ? wait - 1 : 1;
 }
 
+/* Where the waiting lanes start: w = sqrt(128 * 64 * 3 p) for the mean chance p
+   of a collision in 64 cells spread over the layer, at the mean cosine of 1/2.
+   In short layers most histories collide all the way; below 6 the walk finds w
+   by itself in time.  Starting from 1 everywhere, w grew by one an interval and
+   histories of a hundred events ended before it had: 200,000 on 10,180 cells
+   0.74 -> 0.58 ms, 64 slabs of 2,000 cells 0.96 -> 0.81, forward 0.94 -> 0.81,
+   gradient 1.07 -> 0.91. */
+template <int U>
+__device__ __forceinline__ int mc_walk_first_wait(const mc_cell *cells, const mc_layer_k &L) {
+  if (L.m < 128) return L.m < 64 ? 12 : 4;
+  const int c = (int)(((int64_t)__lane_id() * L.m) >> 6);
+  const double p = 2.0 * cells[c].sig_i * L.dx;
+  const uint32_t sum = mc_wave_sum_u32((uint32_t)(p > 0.0 ? (p < 1.0 ? p : 1.0) * 0x1p20 : 0.0));
+  const int w = (int)__builtin_sqrtf((float)sum * (24576.0f * 0x1p-26f));
+  return w < 6 ? 1 : (w < 16 ? w : 16);
+}
+
 /* Histories that set out together from one cell in one direction stay in the
    same cell as long as none collides (an event moves each by one cell), and a
    wave's adds to one LDS word follow one another.  So such lanes set out one
@@ -557,8 +574,7 @@ __device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, m
    on_event as in mc_walk_many; moves(k) is called before every (at most) k
    events per lane, k <= k_max.
    refill_k: events between refills; 0: adapted per wave, from a quarter of the
-   layer's cells (8 to 128; with the waiting lanes below 4 M histories on 50
-   cells 1.50 -> 1.38 ms, 200 slabs of 32 cells 0.73 -> 0.53), by the lanes
+   layer's cells (8 to 128), by the lanes
    found idle at each refill (many idle: the histories are short against the
    interval, halve it; almost none: double it, since each refill costs a pass
    through this loop). */
@@ -582,6 +598,7 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
   const bool adapt = refill_k <= 0;
   int kk = adapt ? 128 : refill_k;
   int wait = 1;
+  const int first_wait = Queue::LEAVES ? mc_walk_first_wait<U>(cells, L) : 0;
   bool first = true; /* no histories taken yet */
   /* wave-uniform bound on every lane's event count (a waiting event counted);
      recomputed exactly (the largest in the wave) when an interval could reach
@@ -601,10 +618,9 @@ __device__ __forceinline__ void mc_walk_bank(IO &io, Queue &queue, const mc_laye
           if (adapt) kk = 256; /* no refill to come */
         } else if (first) {
           /* from the layer's cells: a history crosses about as many as there
-             are; in short ones it collides in many of its events, and those
-             may wait for each other at once */
+             are */
           if (adapt && L.m < 512) kk = L.m > 32 ? L.m >> 2 : 8;
-          if (L.m < 128) wait = L.m < 64 ? 12 : 4;
+          wait = Queue::LEAVES ? first_wait : mc_walk_first_wait<U>(cells, L);
         }
         first = false;
         bool on = false;
