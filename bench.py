@@ -52,10 +52,10 @@ BYTES_PER_EVENT = 72  # algorithmic: the 36-byte particle state read + written p
 #    an upper bound on HBM bytes, since the Infinity Cache (MALL) in front of
 #    HBM can serve them;
 #  - VALU wave-instructions (SQ_INSTS_VALU).
-MEASURED_TRAFFIC_PER_EVENT = {"history": 0.312, "event": 19.71}
+MEASURED_TRAFFIC_PER_EVENT = {"history": 0.313, "event": 19.71}
 # (the VALU figures are of 1e8-particle runs, the size bench.py times: at 1e7
 # the end of the bank, with its partly idle waves, weighs more: 1.050 and 2.813)
-MEASURED_VALU_PER_EVENT = {"history": 0.943, "event": 2.869}
+MEASURED_VALU_PER_EVENT = {"history": 0.945, "event": 2.870}
 # gfx950 issues one wave64 VALU instruction per SIMD every 4 cycles:
 # 256 CUs x 4 SIMDs x 2.4 GHz / 4 = 6.144e11 wave-instructions/s.
 VALU_PEAK_WAVE_INSTR = 256 * 4 * 2.4e9 / 4

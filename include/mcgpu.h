@@ -36,6 +36,16 @@
  *  - Every call returns after its work has finished.  A context (and a
  *    batch plan) holds scratch buffers reused by its calls: use it from one
  *    thread at a time; separate contexts are independent.
+ *  - Device memory of a context: its buffers grow to what the largest call so
+ *    far needed and a quarter more, and are given back by
+ *    mcgpu_context_destroy.  Per cell 36 bytes (gradients 56); mcgpu_simulate 24
+ *    more and 44 per particle.  With the history kernel, layers of more than 10,135
+ *    cells, and long runs (many histories per lane) of layers of 5,067 cells on
+ *    (4,054 with scores), take 16 bytes per history and, while histories x
+ *    windows are at most 2^29, 4 to 8 per history and window (a window holds
+ *    5,066 cells, or 4,053; at most 4 GiB in all).  Where the device has not got
+ *    them, the call does without: slower, with the same results.  The event
+ *    kernel keeps about 100 MB.
  */
 #ifndef MCGPU_H
 #define MCGPU_H
@@ -331,6 +341,9 @@ int mcgpu_create_particles(mcgpu_context *ctx, uint64_t seed, int64_t first, int
  * All ranks' transports of one cycle share one launch (the batched
  * kernel's work queue), and banks, escape buffers and the exchange stay in
  * device memory: per cycle the host reads back one small summary.
+ * The call allocates its device memory and gives it back: banks with room for
+ * every particle in every rank up to 1 GiB in all at once (less if the device
+ * has not got it, and more as the banks grow), 37 bytes a particle.
  * Per history and per cycle the arithmetic is that of mcgpu_simulate, so
  * the tallies (one rounding into weights_absorbed per rank and cycle, as
  * Layer::simulate adds its call's tally) and the counts are bit-identical to

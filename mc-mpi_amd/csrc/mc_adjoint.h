@@ -35,8 +35,8 @@ __device__ __forceinline__ void mc_scale_scatter(mc_scale *s, const mc_cell *cel
    weight times a flight, or, where the history collides, 1 / sig_i: 1, 64
    cells (terms above need |mu| < 1/64, one crossing in 4,096) or 1 over the
    largest sig_i, whichever is most.  Larger terms go to fx.  Returns whether
-   limbs serve (an interval of at least 128 events per lane between moves); if
-   not, t holds words with carry. */
+   limbs serve (an interval of at least 64 events per lane between moves, with 16
+   waves and k = 5); if not, t holds words with carry. */
 __device__ __forceinline__ bool mc_grad_split(mc_grad_tally &G, const mc_scale &s, double dx,
                                               int waves) {
   const int flight = mc_ceil_log2(dx) + 6, b = __builtin_amdgcn_readfirstlane(s.b);

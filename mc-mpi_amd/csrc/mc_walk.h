@@ -176,8 +176,9 @@ __device__ __forceinline__ const T *mc_word(const T *base, int c8) {
    the lanes whose event certainly is that crossing, u certified; for the
    others mc_walk_general finishes the event.  run: the lanes that matter.
    tab: the rows of mc_abs_tab (LDS).
-   A quotient from rh = NaN fails every test.  A negative quotient (a particle beyond its edge) fails
-   the range of y, unless sig_a is 0, where nothing is absorbed either way. */
+   A quotient from rh = NaN fails every test.  A negative quotient (a particle
+   beyond its edge) fails the range of y: a negative y, and -0 where sig_a is 0,
+   have the sign bit set. */
 __device__ __forceinline__ mc_mask mc_walk_cross(mc_walk &p, mc_mask run, const mc_cell cell,
                                                  const double2 *tab, const mc_walk_k &K,
                                                  double &xn, double &q, double &u) {
