@@ -204,7 +204,7 @@ int launch_adj(mcgpu_context *ctx, const adj_args &a, const mcgpu_options &o, hi
   int per_cu = 0;
   int block = o.block_size;
   if (block <= 0) {
-    block = mc_auto_block(kern, lds, &per_cu);
+    block = mc_auto_block(ctx, kern, lds, &per_cu);
   } else if (block > 1024 || block % 64) {
     return mc_fail(ctx, MCGPU_ERR_ARG, "block_size must be a multiple of 64 and <= 1024");
   } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, lds) !=

@@ -448,20 +448,19 @@ int build_tables(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *slabs,
   std::vector<size_t> order(tiles.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return work[x] > work[y]; });
-  std::vector<btile_k> sorted(tiles.size());
-  for (size_t i = 0; i < order.size(); ++i) sorted[i] = tiles[order[i]];
+  /* both tables in one copy */
   const size_t slab_bytes = (sizeof(bslab_k) * ks.size() + 255) / 256 * 256;
-  const size_t bytes = slab_bytes + sizeof(btile_k) * (sorted.size() + 1);
-  int rc = mc_ensure(ctx, &ctx->tables, &ctx->tables_bytes, bytes);
+  std::vector<unsigned char> both(slab_bytes + sizeof(btile_k) * tiles.size());
+  memcpy(both.data(), ks.data(), sizeof(bslab_k) * ks.size());
+  for (size_t i = 0; i < order.size(); ++i)
+    memcpy(both.data() + slab_bytes + sizeof(btile_k) * i, &tiles[order[i]], sizeof(btile_k));
+  int rc = mc_ensure(ctx, &ctx->tables, &ctx->tables_bytes, both.size() + sizeof(btile_k));
   if (rc) return rc;
   unsigned char *base = (unsigned char *)ctx->tables;
-  MC_HIP(ctx, hipMemcpy(base, ks.data(), sizeof(bslab_k) * ks.size(), hipMemcpyHostToDevice));
-  if (!sorted.empty())
-    MC_HIP(ctx, hipMemcpy(base + slab_bytes, sorted.data(), sizeof(btile_k) * sorted.size(),
-                          hipMemcpyHostToDevice));
+  MC_HIP(ctx, hipMemcpy(base, both.data(), both.size(), hipMemcpyHostToDevice));
   *d_slabs = (const bslab_k *)base;
   *d_tiles = (const btile_k *)(base + slab_bytes);
-  *n_tiles = (int32_t)sorted.size();
+  *n_tiles = (int32_t)tiles.size();
   return MCGPU_OK;
 }
 
@@ -539,7 +538,7 @@ int batch_prepare(mcgpu_context *ctx, K kern, int32_t n_slabs, const mcgpu_slab 
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds);
   int per_cu = 0;
   if (o->block_size <= 0)
-    o->block_size = mc_auto_block(kern, *lds, &per_cu);
+    o->block_size = mc_auto_block(ctx, kern, *lds, &per_cu);
   else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, o->block_size, *lds) !=
                hipSuccess || per_cu < 1)
     per_cu = 1;

@@ -277,7 +277,7 @@ int mc_batched_plan_shape(mcgpu_context *ctx, int max_m, int block, int grid, in
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.lds);
   int per_cu = 0;
-  if (block == 0) block = mc_auto_block(kern, sh.lds, &per_cu);
+  if (block == 0) block = mc_auto_block(ctx, kern, sh.lds, &per_cu);
   sh.block = block;
   sh.grid = grid;
   if (sh.grid <= 0) {

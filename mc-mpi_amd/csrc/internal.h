@@ -34,6 +34,13 @@ __device__ __forceinline__ void mc_counters_to_host(const mc_counters *ctr, mc_c
         reinterpret_cast<const unsigned long long *>(ctr)[threadIdx.x];
 }
 
+/* the launch shape of a persistent kernel with so much LDS (mc_auto_block) */
+struct mc_block_shape {
+  const void *kern = nullptr;
+  size_t lds = 0;
+  int block = 0, per_cu = 0;
+};
+
 struct mcgpu_context {
   int device = 0;
   int num_cus = 0;
@@ -42,6 +49,10 @@ struct mcgpu_context {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::string err;
+
+  /* shapes found by the last calls, the oldest replaced */
+  mc_block_shape shapes[8];
+  unsigned next_shape = 0;
 
   /* grow-only scratch (device) */
   void *cells = nullptr;      size_t cells_bytes = 0;     /* mc_cell[m] */
@@ -140,9 +151,17 @@ static __device__ __forceinline__ void store_state(const mc_transport_args &a, i
    registers and LDS); ties go to the smaller block.  With LDS-resident
    tables a small block can leave most of the CU idle: 56 KB per block fits
    two blocks in 160 KB, 8 waves at 256 threads but 16 at 512.
-   *per_cu receives the resident blocks per CU of the choice (at least 1). */
+   *per_cu receives the resident blocks per CU of the choice (at least 1).
+   The context keeps the last shapes: the calculator's three answers take some
+   10 us of a small call's 300. */
 template <typename K>
-static inline int mc_auto_block(K kern, size_t lds, int *per_cu) {
+static inline int mc_auto_block(mcgpu_context *ctx, K kern, size_t lds, int *per_cu) {
+  const void *key = reinterpret_cast<const void *>(kern);
+  for (const mc_block_shape &s : ctx->shapes)
+    if (s.kern == key && s.lds == lds) {
+      *per_cu = s.per_cu;
+      return s.block;
+    }
   int best = 256, best_waves = -1, best_per_cu = 1;
   for (int b = 256; b <= 1024; b *= 2) {
     int pc = 0;
@@ -158,6 +177,7 @@ static inline int mc_auto_block(K kern, size_t lds, int *per_cu) {
     }
   }
   *per_cu = best_per_cu;
+  if (best_waves > 0) ctx->shapes[ctx->next_shape++ % 8] = {key, lds, best, best_per_cu};
   return best;
 }
 
