@@ -210,11 +210,11 @@ __device__ __forceinline__ mc_mask mc_walk_cross(mc_walk &p, mc_mask run, const 
 
 /* The general event, after mc_walk_cross has drawn: mc_event_decide's
    operations and the absorption.  Returns the deposit; coll: whether it
-   collided, di: the flight. */
-template <int U>
+   collided, di: the flight.  THICK: for mc_walk_thick, which divides by rh alone
+   (after a collision |mu| is below 1, and mc_div_by_rcp tests the rest). */
+template <int U, bool THICK = false>
 __device__ __forceinline__ double mc_walk_general(mc_walk &p, const mc_cell cell, const double dx,
-                                                  bool &coll, double &di) {
-  const mc_coef K = mc_coef_default();
+                                                  const mc_coef &K, bool &coll, double &di) {
   const double h = mc_walk_h(p.s2);
   const double xn = p.fe * dx;
   const bool flat = !(p.mu < -MC_EPS || MC_EPS < p.mu);
@@ -235,8 +235,16 @@ __device__ __forceinline__ double mc_walk_general(mc_walk &p, const mc_cell cell
     p.x += di * p.mu;
     mc_walk_draw(p.s2);
     p.mu = 2 * mc_walk_h(p.s2) - 1;
-    /* the index from the edge ahead: fe is index + 1 moving up, index moving down */
-    mc_walk_turn<U>(p, (int32_t)p.fe - (p.st8 > 0 ? 1 : 0));
+    if (THICK) {
+      const bool back = p.mu < 0;
+      const double fs = back ? -1.0 : 1.0;
+      p.st8 = back ? -U : U;
+      p.fe = mc_fma(0.5, fs - p.fs, p.fe); /* the same cell's other edge, or this one */
+      p.fs = fs;
+      p.rh = 1.0 / p.mu;
+    } else { /* the index from the edge ahead: fe is index + 1 moving up, index moving down */
+      mc_walk_turn<U>(p, (int32_t)p.fe - (p.st8 > 0 ? 1 : 0));
+    }
   } else {
     p.x = xn;
     p.fe += p.fs;
@@ -395,7 +403,7 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
       double di = 0.0, dw = 0.0;
       if (mc_in(pend)) {
         cell = mc_cell_at<U>(cells, (uint32_t)c8);
-        dw = mc_walk_general<U>(p, cell, K.dx, coll, di);
+        dw = mc_walk_general<U>(p, cell, K.dx, mc_coef_default(), coll, di);
         ++ei;
         col += coll ? 1u : 0u;
       }
@@ -410,12 +418,22 @@ __device__ __forceinline__ int mc_walk_many(mc_walk &p, mc_mask &run, mc_mask &p
 }
 
 /* mc_walk_many for thick cells, where most events are general ones: no common
-   step before them, every lane's event a general one.  (Within mc_walk_many, as
-   a mode of its own, this made the common loop 5 to 10 % slower.) */
+   step before them, every lane's event a general one.  Bound by the general
+   event's instructions, some 300 of them.  (Within mc_walk_many, as a mode of
+   its own, this made the common loop 5 to 10 % slower.)  Its coefficients and
+   dx stay in registers; with dx among the scalar ones the kernels' arguments
+   came back from their spills at each event.  Histories of 2,300 events, all
+   collisions, on 100 cells, by the history kernel with mc_walk_many and so: one
+   2.86 and 1.70 ms, 20,000 of them 3.91 and 2.34, 2 M of 340 events 42.3 and
+   25.7. */
 template <int U, typename F>
 __device__ __forceinline__ void mc_walk_thick(mc_walk &p, mc_mask &run, mc_mask &fresh, int ki,
                                               const mc_cell *cells, const mc_walk_k &K,
                                               uint32_t &ei, uint32_t &col, F on_event) {
+  mc_coef C = mc_coef_default();
+  double dx = K.dx;
+  asm volatile("" : "+v"(C.l8), "+v"(C.l7), "+v"(C.l6), "+v"(C.l5), "+v"(C.l4), "+v"(C.l3));
+  asm volatile("" : "+s"(C.e5), "+s"(C.e4), "+s"(C.e3), "+s"(C.ziv), "+v"(dx));
   run |= fresh;
   fresh = 0;
   for (; ki > 0 && run != 0; --ki) { /* wave-uniform */
@@ -427,7 +445,7 @@ __device__ __forceinline__ void mc_walk_thick(mc_walk &p, mc_mask &run, mc_mask 
     if (mc_in(run)) {
       cell = mc_cell_at<U>(cells, (uint32_t)c8);
       mc_walk_draw(p.s2);
-      dw = mc_walk_general<U>(p, cell, K.dx, coll, di);
+      dw = mc_walk_general<U, true>(p, cell, dx, C, coll, di);
       ++ei;
       col += coll ? 1u : 0u;
     }
