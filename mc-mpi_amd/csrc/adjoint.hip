@@ -46,7 +46,7 @@ struct adj_args {
 __device__ __forceinline__ void events_out(unsigned long long *s_tot, mc_counters *ctr) {
   if (threadIdx.x != 0) return;
   s_tot[1] = s_tot[2] = s_tot[3] = s_tot[4] = 0;
-  mc_totals_out(s_tot, ctr);
+  mc_totals_out(s_tot, ctr, mc_counter_copy());
 }
 
 /* LDS_T: the two limb tallies in LDS; LDS_C: the cells and target weights too */
@@ -153,22 +153,13 @@ __global__ void k_setup_cells(int m, const double *sig_a, const double *sig_i, m
     for (int w = 0; w < fx_words_per_cell; ++w) fx[(size_t)w * m + c] = 0;
     for (int w = 0; w < flag_words_per_cell; ++w) flags[(size_t)w * m + c] = 0;
   }
-  if (c == 0) {
-    ctr->next = 0;
-    ctr->events = 0;
-    ctr->collisions = 0;
-    ctr->n_left = 0;
-    ctr->n_right = 0;
-    ctr->n_killed = 0;
-    ctr->status = 0;
-    ctr->left = 0;
-  }
+  mc_counters_clear(ctr, (uint64_t)c);
 }
 
 __global__ void k_finalize2(int m, const unsigned long long *fx, const uint32_t *flags,
-                            double *ga, double *gi, const mc_counters *ctr,
+                            double *ga, double *gi, mc_counters *ctr,
                             mc_counters *host_ctr) {
-  mc_counters_to_host(ctr, host_ctr);
+  mc_counters_fold(ctr, host_ctr);
   const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
   if (c < n) {
     ga[c] = ga[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
@@ -177,8 +168,8 @@ __global__ void k_finalize2(int m, const unsigned long long *fx, const uint32_t 
 }
 
 __global__ void k_finalize1(int m, const unsigned long long *fx, const uint32_t *flags, double *w,
-                            const mc_counters *ctr, mc_counters *host_ctr) {
-  mc_counters_to_host(ctr, host_ctr);
+                            mc_counters *ctr, mc_counters *host_ctr) {
+  mc_counters_fold(ctr, host_ctr);
   const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
   if (c < n && ctr->left == 0) w[c] = w[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
 }

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(1024) void k_forward_cells_batch(bcell_args a, int 
     }
     __syncthreads();
   }
-  if (tid == 0) mc_totals_out(s_tot, a.ctr);
+  if (tid == 0) mc_totals_out(s_tot, a.ctr, mc_counter_copy());
 }
 
 /* Adjoint: mcgpu_adjoint_cells per slab (replay from the initial bank).  WIDE
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(1024) void k_adjoint_cells_batch(bcell_args a, int 
   }
   if (tid == 0) { /* this call counts events alone */
     s_tot[1] = s_tot[2] = s_tot[3] = s_tot[4] = 0;
-    mc_totals_out(s_tot, a.ctr);
+    mc_totals_out(s_tot, a.ctr, mc_counter_copy());
   }
 }
 
@@ -384,22 +384,14 @@ __global__ void k_batch_cells_setup(int64_t total, const double *sig_a, const do
     for (int w = 0; w < fx_words; ++w) fx[(size_t)w * total + c] = 0;
     for (int w = 0; w < flag_words; ++w) flags[(size_t)w * total + c] = 0;
   }
-  if (c == 0) {
-    ctr->next = 0;
-    ctr->events = 0;
-    ctr->collisions = 0;
-    ctr->n_left = 0;
-    ctr->n_right = 0;
-    ctr->n_killed = 0;
-    ctr->status = 0;
-  }
+  mc_counters_clear(ctr, (uint64_t)c);
 }
 
 /* out_k[c] += the k-th accumulator (k < n_out) */
 __global__ void k_batch_cells_finalize(int64_t total, const unsigned long long *fx,
                                        const uint32_t *flags, double *out0, double *out1,
-                                       const mc_counters *ctr, mc_counters *host_ctr) {
-  mc_counters_to_host(ctr, host_ctr);
+                                       mc_counters *ctr, mc_counters *host_ctr) {
+  mc_counters_fold(ctr, host_ctr);
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= total) return;
   out0[c] = out0[c] + mc_fx_finalize(fx[c], fx[total + c], flags[c]);

@@ -222,7 +222,7 @@ __global__ __launch_bounds__(1024) void k_batched(batch_args a, int refill_k) {
     __syncthreads();
   }
   /* the break follows a barrier after the last tile's totals */
-  if (tid == 0) mc_totals_out(s_tot, a.ctr);
+  if (tid == 0) mc_totals_out(s_tot, a.ctr, mc_counter_copy());
 }
 
 __global__ void k_batch_setup(int64_t total, const double *sigs, const double *ar, mc_cell *cells,
@@ -234,19 +234,13 @@ __global__ void k_batch_setup(int64_t total, const double *sigs, const double *a
     fx[total + c] = 0;
     flags[c] = 0;
   }
-  if (c == 0) {
-    ctr->next = 0;
-    ctr->events = 0;
-    ctr->collisions = 0;
-    ctr->n_left = 0;
-    ctr->n_right = 0;
-    ctr->n_killed = 0;
-    ctr->status = 0;
-  }
+  mc_counters_clear(ctr, (uint64_t)c);
 }
 
 __global__ void k_batch_finalize(int64_t total, const unsigned long long *fx,
-                                 const uint32_t *flags, double *weights) {
+                                 const uint32_t *flags, double *weights, mc_counters *ctr,
+                                 mc_counters *host_ctr) {
+  mc_counters_fold(ctr, host_ctr);
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c < total) weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[total + c], flags[c]);
 }
@@ -435,7 +429,7 @@ int batch_capture(mcgpu_batch *b) {
                      sh.refill);
   hipLaunchKernelGGL(k_batch_finalize, dim3((unsigned)((tc + 255) / 256)), dim3(256), 0,
                      b->stream, tc, (const unsigned long long *)b->d_fx,
-                     (const uint32_t *)b->d_flags, b->weights);
+                     (const uint32_t *)b->d_flags, b->weights, b->d_ctr, b->h_ctr);
   hipError_t e = hipStreamEndCapture(b->stream, &b->graph);
   if (e != hipSuccess) return mc_fail(ctx, MCGPU_ERR_HIP, "hipStreamEndCapture", e);
   MC_HIP(ctx, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
@@ -452,7 +446,6 @@ int batch_launch(mcgpu_batch *b, hipStream_t s, mcgpu_stats *stats) {
   MC_HIP(ctx, hipEventRecord(b->e0, s));
   MC_HIP(ctx, hipGraphLaunch(b->exec, s));
   MC_HIP(ctx, hipEventRecord(b->e1, s));
-  MC_HIP(ctx, hipMemcpyAsync(b->h_ctr, b->d_ctr, sizeof(mc_counters), hipMemcpyDeviceToHost, s));
   MC_HIP(ctx, hipStreamSynchronize(s));
   if (stats) {
     float ms = 0.f;
@@ -542,7 +535,7 @@ int mcgpu_batch_create(mcgpu_context *ctx, int32_t n_slabs, const mcgpu_slab *sl
   B_HIP(hipMalloc(&b->d_cells, sizeof(mc_cell) * total_cells));
   B_HIP(hipMalloc(&b->d_fx, 16 * (size_t)total_cells));
   B_HIP(hipMalloc(&b->d_flags, 4 * (size_t)total_cells));
-  B_HIP(hipMalloc(&b->d_ctr, sizeof(mc_counters)));
+  B_HIP(hipMalloc(&b->d_ctr, MC_COUNTER_BYTES));
   B_HIP(hipHostMalloc(&b->h_ctr, sizeof(mc_counters), hipHostMallocDefault));
   B_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
   B_HIP(hipEventCreate(&b->e0));

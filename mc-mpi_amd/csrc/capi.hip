@@ -61,21 +61,12 @@ __global__ void k_setup(int m, const double *sigs, const double *ar, mc_cell *ce
     fx[n + c] = 0;
     flags[c] = 0;
   }
-  if (c == 0) {
-    ctr->next = 0;
-    ctr->events = 0;
-    ctr->collisions = 0;
-    ctr->n_left = 0;
-    ctr->n_right = 0;
-    ctr->n_killed = 0;
-    ctr->status = 0;
-    ctr->left = 0;
-  }
+  mc_counters_clear(ctr, (uint64_t)c);
 }
 
 __global__ void k_finalize(int m, const unsigned long long *fx, const uint32_t *flags,
-                           double *weights, const mc_counters *ctr, mc_counters *host_ctr) {
-  mc_counters_to_host(ctr, host_ctr);
+                           double *weights, mc_counters *ctr, mc_counters *host_ctr) {
+  mc_counters_fold(ctr, host_ctr);
   const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)m;
   if (c < n && ctr->left == 0)
     weights[c] = weights[c] + mc_fx_finalize(fx[c], fx[n + c], flags[c]);
@@ -192,7 +183,7 @@ int mc_launch_setup(mcgpu_context *ctx, int m, const double *sigs, const double 
 }
 
 int mc_launch_finalize(mcgpu_context *ctx, int m, const unsigned long long *fx,
-                       const uint32_t *flags, double *weights, const mc_counters *ctr,
+                       const uint32_t *flags, double *weights, mc_counters *ctr,
                        mc_counters *host_ctr, hipStream_t s) {
   hipLaunchKernelGGL(k_finalize, dim3(grid_for(m, 256)), dim3(256), 0, s, m, fx, flags, weights,
                      ctr, host_ctr);
@@ -276,7 +267,7 @@ int mcgpu_context_create(int device, mcgpu_context **out) {
   }
   if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
-      hipMalloc(&ctx->counters, sizeof(mc_counters)) != hipSuccess ||
+      hipMalloc(&ctx->counters, MC_COUNTER_BYTES) != hipSuccess ||
       hipHostMalloc(&ctx->host_counters, sizeof(mc_counters), hipHostMallocDefault) != hipSuccess) {
     rc = MCGPU_ERR_HIP;
   }

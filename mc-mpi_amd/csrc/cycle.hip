@@ -120,15 +120,7 @@ __global__ void k_cyc_clear(int64_t total, unsigned long long *fx, uint32_t *fla
     fx[total + c] = 0;
     flags[c] = 0;
   }
-  if (c == 0) {
-    ctr->next = 0;
-    ctr->events = 0;
-    ctr->collisions = 0;
-    ctr->n_left = 0;
-    ctr->n_right = 0;
-    ctr->n_killed = 0;
-    ctr->status = 0;
-  }
+  mc_counters_clear(ctr, (uint64_t)c);
 }
 
 __global__ void k_cyc_finalize(int64_t total, const unsigned long long *fx, const uint32_t *flags,
@@ -223,9 +215,9 @@ __global__ __launch_bounds__(CHUNK) void k_cyc_scan(const rank_in *rin, const ch
 /* The exchange plan, one thread per rank: where each rank's escapes go and
    what each bank receives, in the reference's phase order. */
 __global__ void k_cyc_plan(int R, int64_t S, const rank_in *rin, const rank_tot *tot,
-                           rank_sum *sum, rank_sum *host_sum, const mc_counters *ctr,
+                           rank_sum *sum, rank_sum *host_sum, mc_counters *ctr,
                            mc_counters *host_ctr) {
-  mc_counters_to_host(ctr, host_ctr);
+  mc_counters_fold(ctr, host_ctr);
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= R) return;
   const rank_in ri = rin[q];
@@ -391,7 +383,9 @@ __global__ void k_one_cells(int64_t G, int m, const double *sigs, const double *
 
 /* weights[c] += the tally of cycle g, rounded once, for g = 0 .. G-1 in order */
 __global__ void k_one_finalize(int m, int64_t G, const unsigned long long *fx,
-                               const uint32_t *flags, double *weights) {
+                               const uint32_t *flags, double *weights, mc_counters *ctr,
+                               mc_counters *host_ctr) {
+  mc_counters_fold(ctr, host_ctr);
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= m) return;
   const int64_t total = G * m;
@@ -481,7 +475,7 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
       (rc = dalloc((void **)&d_cells, sizeof(mc_cell) * (size_t)(gcap * m))) ||
       (rc = dalloc((void **)&d_fx, 16 * (size_t)(gcap * m))) ||
       (rc = dalloc((void **)&d_flags, 4 * (size_t)(gcap * m))) ||
-      (rc = dalloc((void **)&d_ctr, sizeof(mc_counters))) ||
+      (rc = dalloc((void **)&d_ctr, MC_COUNTER_BYTES)) ||
       (rc = dalloc((void **)&d_slabs, sizeof(mc_slab_k) * (size_t)gcap)) ||
       (rc = dalloc((void **)&d_tiles, sizeof(mc_tile_k) * (size_t)max_tiles)))
     return rc;
@@ -637,10 +631,10 @@ int sync_one_rank(mcgpu_context *ctx, mcgpu_cycle_rank &k, const double *sigs, c
       return rc;
     MC_HIP(ctx, hipEventRecord(ctx->ev1, s));
     hipLaunchKernelGGL(k_one_finalize, dim3(blocks_for(m, 256)), dim3(256), 0, s, m, G,
-                       (const unsigned long long *)d_fx, (const uint32_t *)d_flags, d_w);
+                       (const unsigned long long *)d_fx, (const uint32_t *)d_flags, d_w, d_ctr,
+                       (mc_counters *)h_ctr);
     MC_HIP(ctx, hipGetLastError());
     MC_HIP(ctx, hipEventRecord(ev_comp, s));
-    MC_HIP(ctx, hipMemcpyAsync(h_ctr, d_ctr, sizeof(mc_counters), hipMemcpyDeviceToHost, s));
     MC_HIP(ctx, hipStreamSynchronize(s)); /* also: h_slabs / h_tiles reusable */
     const mc_counters *hc = reinterpret_cast<const mc_counters *>(h_ctr);
     float ms = 0.f, comp_ms = 0.f;
@@ -803,7 +797,7 @@ extern "C" int mcgpu_sync_cycle(mcgpu_context *ctx, int32_t world_size, mcgpu_cy
   if ((rc = dalloc((void **)&d_cells, sizeof(mc_cell) * tc)) ||
       (rc = dalloc((void **)&d_fx, 16 * (size_t)tc)) ||
       (rc = dalloc((void **)&d_flags, 4 * (size_t)tc)) ||
-      (rc = dalloc((void **)&d_ctr, sizeof(mc_counters))) ||
+      (rc = dalloc((void **)&d_ctr, MC_COUNTER_BYTES)) ||
       (rc = dalloc((void **)&d_w, 8 * (size_t)tc)) ||
       (rc = dalloc((void **)&d_in, 16 * (size_t)tc)) ||
       (rc = dalloc((void **)&d_slabs, sizeof(mc_slab_k) * R)) ||

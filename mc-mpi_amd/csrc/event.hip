@@ -732,7 +732,7 @@ __global__ __launch_bounds__(EVENT_MAX_BLOCK) void k_event(mc_transport_args a,
 
   if (capped) atomicOr(&s_tot[5], 1ull);
   __syncthreads();
-  if (threadIdx.x == 0) mc_totals_out(s_tot, a.ctr);
+  if (threadIdx.x == 0) mc_totals_out(s_tot, a.ctr, mc_counter_copy());
   if (LDS_TALLY) {
     unsigned long long *fx = a.fx;
     if (limbs) {

@@ -573,13 +573,15 @@ struct mc_tile_queue {
    addresses of a full chip's 4,096 waves alone took 0.14 ms. */
 constexpr int MC_TOTALS = 6;
 
-/* by one thread of the block, after a barrier */
-__device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, mc_counters *ctr) {
-  if (s_tot[0]) atomicAdd(&ctr->events, s_tot[0]);
-  if (s_tot[1]) atomicAdd(&ctr->collisions, s_tot[1]);
-  if (s_tot[2]) atomicAdd(&ctr->n_left, s_tot[2]);
-  if (s_tot[3]) atomicAdd(&ctr->n_right, s_tot[3]);
-  if (s_tot[4]) atomicAdd(&ctr->n_killed, s_tot[4]);
+/* by one thread of the block, after a barrier; copy: of the totals */
+__device__ __forceinline__ void mc_totals_out(const unsigned long long *s_tot, mc_counters *ctr,
+                                              unsigned copy) {
+  unsigned long long *to = mc_counter_word(ctr, copy, 1);
+  if (s_tot[0]) atomicAdd(&to[0], s_tot[0]);
+  if (s_tot[1]) atomicAdd(&to[1], s_tot[1]);
+  if (s_tot[2]) atomicAdd(&to[2], s_tot[2]);
+  if (s_tot[3]) atomicAdd(&to[3], s_tot[3]);
+  if (s_tot[4]) atomicAdd(&to[4], s_tot[4]);
   if (s_tot[5]) atomicOr(&ctr->status, 1u);
 }
 

@@ -27,8 +27,7 @@
 
 namespace {
 
-constexpr size_t kCounterBytes = 256; /* the mc_counters block, padded */
-static_assert(sizeof(mc_counters) <= kCounterBytes, "counter block exceeds its slot");
+constexpr size_t kCounterBytes = MC_COUNTER_BYTES;
 constexpr size_t kMaxCells = MCGPU_NOALLOC_MAX_CELLS;
 /* counters | cells (16 B) | tally lo, hi (8 B each) | flags (4 B), per cell */
 constexpr size_t kCellsOff = kCounterBytes;
@@ -38,7 +37,7 @@ constexpr size_t kScratchBytes = kFlagsOff + 4 * kMaxCells;
 
 } // namespace
 
-/* The scratch array: 256 + 36 * MCGPU_NOALLOC_MAX_CELLS bytes (2.25 MiB) per
+/* The scratch array: 2048 + 36 * MCGPU_NOALLOC_MAX_CELLS bytes (2.25 MiB) per
    device.  Only kernels touch it, through the address below. */
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
