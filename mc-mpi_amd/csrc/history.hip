@@ -717,11 +717,7 @@ int launch_kernel(mcgpu_context *ctx, K kern, const mc_transport_args &a, const 
                  hipSuccess || per_cu < 1) {
     per_cu = 1;
   }
-  int grid = o.grid_blocks;
-  if (grid <= 0) {
-    grid = per_cu * ctx->num_cus;
-    if (a.n < grid) grid = (int)(a.n > 0 ? a.n : 1); /* a block per history at most */
-  }
+  const int grid = o.grid_blocks > 0 ? o.grid_blocks : mc_auto_grid(ctx, a.L.m, a.n, per_cu);
   int k = o.events_per_refill > 0 ? o.events_per_refill : 0; /* 0: adaptive */
   hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, k, per_cu, last);
   MC_HIP(ctx, hipGetLastError());

@@ -212,6 +212,19 @@ static inline int mc_auto_block(mcgpu_context *ctx, K kern, size_t lds, int *per
   return best;
 }
 
+/* Blocks of a persistent kernel for n histories in a layer of m cells: all that
+   the chip holds, a block per history at most, so that few histories spread over
+   it.  In a layer of a few cells all blocks move their tallies to the same words,
+   one after the other, and histories are short: one block per CU while that is a
+   wave per SIMD.  One cell, 20,000 histories, by a full grid and so, in us: 48 and
+   26 (1 event each), 82 and 70 (42); their gradients 86 and 47, 280 and 255.  Ten
+   cells 109 and 105, 64 cells 255 and 280. */
+static inline int mc_auto_grid(const mcgpu_context *ctx, int m, int64_t n, int per_cu) {
+  int grid = per_cu * ctx->num_cus;
+  if (m <= 8 && n <= 256 * (int64_t)ctx->num_cus) grid = ctx->num_cus;
+  return n < grid ? (int)(n > 0 ? n : 1) : grid;
+}
+
 /* sweep: 0, or, where ctr->left is not 0 after it, the number of the sweep over a
    wide layer's windows that goes on with the histories left */
 int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
