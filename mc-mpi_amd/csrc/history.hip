@@ -101,6 +101,7 @@ struct mc_windows {
   uint32_t *parked, *put, *got; /* [nw (cap + MC_RING_PAD)], [nw], [nw] */
   uint32_t *blocks;             /* [nw] blocks that transport window w */
   uint32_t *left;               /* histories not known to be finished */
+  uint32_t *thick;              /* thick cells, or null: not asked (k_history_if_thick) */
   uint32_t cap;
   int patience; /* looks of an idle block before it ends */
   __device__ __forceinline__ uint32_t *ring(int w) const {
@@ -413,6 +414,7 @@ __global__ void k_windows_clear(mc_windows win, uint32_t *cursor) {
   win.put[t * MC_WINDOW_STEP] = win.got[t * MC_WINDOW_STEP] = MC_RING_START;
   win.blocks[t * MC_WINDOW_STEP] = 0;
   if (t == 0) *win.left = 0;
+  if (t == 0 && win.thick) *win.thick = 0;
 }
 
 /* the histories of each window; OPEN: their first windows, from the bank */
@@ -437,6 +439,9 @@ template <bool OPEN> __global__ void k_windows_count(mc_transport_args a, mc_win
     }
     if (w >= 0) atomicAdd(&s_n[w / win.W], 1u);
   }
+  if (OPEN && win.thick)
+    mc_count_thick(win.thick, a.cells, a.L.m, a.L.dx, blockIdx.x * blockDim.x + threadIdx.x,
+                   gridDim.x * blockDim.x);
   __syncthreads();
   if (threadIdx.x < (unsigned)win.nw && s_n[threadIdx.x]) {
     atomicAdd(&win.count[threadIdx.x], s_n[threadIdx.x]);
@@ -599,6 +604,21 @@ __global__ __launch_bounds__(1024) void k_history(mc_transport_args a, int refil
                                              refill_k);
 }
 
+/* A long run on a layer whose tally fits LDS but not its cells, if they are thick:
+   k_history_windows leaves it, as their walk and windows do not go into one
+   kernel (history_block).  8,000 cells, 2 M histories of some 160 events, all
+   collisions, in two windows 21.6 ms, here 15.9. */
+template <bool SCORE>
+__global__ __launch_bounds__(1024) void k_history_if_thick(mc_transport_args a, int refill_k,
+                                                           int per_cu, const uint32_t *thick) {
+  if (2 * (int64_t)*thick <= a.L.m) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.ctr->left = 0;
+  mc_call_queue queue{mc_queue_open(a.n, per_cu, blockIdx.x, gridDim.x), &a.ctr->next};
+  bank_io<SCORE> io{a, 0.0};
+  const int k = look_at_weights(a, queue.q);
+  history_block<true, false, SCORE>(a, a.L, 0, io, queue, k, 0, refill_k);
+}
+
 /* the tally of the first `most` cells in all of the block's LDS (mc_full_tally) */
 __global__ __launch_bounds__(1024) void k_history_full(mc_transport_args a, int refill_k,
                                                        int per_cu, int most) {
@@ -640,6 +660,7 @@ __global__ __launch_bounds__(1024) void k_history_full(mc_transport_args a, int 
 template <bool LDS_CELLS, bool SCORE>
 __global__ __launch_bounds__(1024) void k_history_windows(mc_transport_args a, mc_windows win,
                                                           int refill_k, int per_cu) {
+  if (win.thick && 2 * (int64_t)*win.thick > a.L.m) return; /* k_history_if_thick's */
   __shared__ mc_window_block blk;
   const mc_window_share sh = mc_window_of(win);
   if (threadIdx.x == 0) {
@@ -701,9 +722,9 @@ constexpr size_t window_lds(size_t W, bool cells, bool score) {
 }
 
 /* last: the kernel's last argument */
-template <typename K>
+template <typename K, typename V>
 int launch_kernel(mcgpu_context *ctx, K kern, const mc_transport_args &a, const mcgpu_options &o,
-                  hipStream_t s, size_t lds, int last) {
+                  hipStream_t s, size_t lds, V last) {
   if (lds > 65536)
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -739,10 +760,10 @@ int launch_one(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_optio
 /* A sweep over a wide layer's windows, cells in LDS or not; ctr->left counts the
    histories that it has not finished (usually none).  Scratch from the context
    (16 bytes per history and 4 per history and window); MCGPU_ERR_NOMEM: there is
-   none. */
+   none.  ask: the tally fits LDS, and thick cells go to k_history_if_thick. */
 template <bool LDS_CELLS, bool S>
 int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-                   hipStream_t s, int nw, int sweep) {
+                   hipStream_t s, int nw, int sweep, bool ask) {
   auto kern = k_history_windows<LDS_CELLS, S>;
   const int W = (a.L.m + nw - 1) / nw;
   const size_t lds = window_lds((size_t)W, LDS_CELLS, S);
@@ -766,7 +787,7 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   const size_t rings = cap ? (cap + MC_RING_PAD) * (size_t)nw : 0;
   const size_t words = (16 * n + 4 * rings + 255) / 256 * 256;
   int rc = mc_ensure(ctx, &ctx->work, &ctx->work_bytes,
-                     words + (16 + 12 * MC_WINDOW_STEP) * MC_MAX_WINDOWS);
+                     words + (16 + 12 * MC_WINDOW_STEP) * MC_MAX_WINDOWS + 4);
   if (rc) return rc;
   unsigned char *base = (unsigned char *)ctx->work;
   mc_windows win;
@@ -788,6 +809,7 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   win.put = cursor + MC_MAX_WINDOWS;
   win.got = win.put + MC_MAX_WINDOWS * MC_WINDOW_STEP;
   win.blocks = win.got + MC_MAX_WINDOWS * MC_WINDOW_STEP;
+  win.thick = ask && sweep == 0 ? win.blocks + MC_MAX_WINDOWS * MC_WINDOW_STEP : nullptr;
   const unsigned blocks = (unsigned)std::min<size_t>((n + 1023) / 1024, 4 * (size_t)ctx->num_cus);
 
   hipLaunchKernelGGL(k_windows_clear, dim3(1), dim3(64), 0, s, win, cursor);
@@ -801,6 +823,9 @@ int launch_windows(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_o
   MC_HIP(ctx, hipGetLastError());
   hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, a, win, k, per_cu);
   MC_HIP(ctx, hipGetLastError());
+  if (win.thick)
+    return launch_kernel(ctx, k_history_if_thick<S>, a, o, s, MC_TAB_BYTES + 16 * (size_t)a.L.m,
+                         (const uint32_t *)win.thick);
   return MCGPU_OK;
 }
 
@@ -813,12 +838,12 @@ int windows_of(size_t m, size_t budget, bool cells, bool score) {
 
 template <bool S>
 int launch_wide(mcgpu_context *ctx, const mc_transport_args &a, const mcgpu_options &o,
-                hipStream_t s, size_t budget, int sweep) {
+                hipStream_t s, size_t budget, int sweep, bool ask) {
   const int all = windows_of((size_t)a.L.m, budget, true, S);
   const int tally = windows_of((size_t)a.L.m, budget, false, S);
   const int limit = o.grid_blocks > 0 ? std::min(o.grid_blocks, MC_MAX_WINDOWS) : MC_MAX_WINDOWS;
-  if (all <= limit) return launch_windows<true, S>(ctx, a, o, s, all, sweep);
-  if (tally > 1 && tally <= limit) return launch_windows<false, S>(ctx, a, o, s, tally, sweep);
+  if (all <= limit) return launch_windows<true, S>(ctx, a, o, s, all, sweep, ask);
+  if (tally > 1 && tally <= limit) return launch_windows<false, S>(ctx, a, o, s, tally, sweep, ask);
   return MCGPU_ERR_NOMEM;
 }
 
@@ -850,8 +875,8 @@ int mc_launch_history(mcgpu_context *ctx, const mc_transport_args &a, const mcgp
   const bool block_ok = o.block_size <= 1024 && o.block_size % 64 == 0;
   if ((!lds_tally || long_run) && !ctx->quiet && a.n < (int64_t)0xFFFFFFFFu && block_ok &&
       !(a.score && !a.g)) {
-    const int rc = a.score ? launch_wide<true>(ctx, a, o, s, budget, sweep)
-                           : launch_wide<false>(ctx, a, o, s, budget, sweep);
+    const int rc = a.score ? launch_wide<true>(ctx, a, o, s, budget, sweep, lds_tally)
+                           : launch_wide<false>(ctx, a, o, s, budget, sweep, lds_tally);
     if (rc != MCGPU_ERR_NOMEM) return rc;
     ctx->err.clear();
   }

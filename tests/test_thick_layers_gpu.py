@@ -72,6 +72,44 @@ def test_gradients_of_thick_layers(ctx, oracle, m, n, thick, kind, score):
     assert np.array_equal(gi.cpu().numpy(), oi)
 
 
+@pytest.mark.parametrize("thick", [10_000, 5001, 5000, 0])
+@pytest.mark.parametrize("cap,score", [(0, False), (0, True), (3, False)])
+def test_long_runs_of_thick_cells(ctx, oracle, thick, cap, score):
+    """10,000 cells fit LDS without the cross sections; long runs (here on two
+    blocks) go in two windows, those of thick cells in one."""
+    import mcgpu
+    m, n, min_w = 10_000, 9000, 0.05
+    _say(f"long run, {thick} of {m} cells thick, cap {cap} score {score}")
+    sa, si, dx, bank = _slab(m, n, thick, "both", seed=thick)
+    o = oracle.forward_cells(0, m, dx, min_w, sa, si, bank, g=np.linspace(-1, 1, m))
+    opt = mcgpu.make_options(grid_blocks=2, max_events_per_history=cap)
+    for _ in range(2):
+        db, dw, dr = mcgpu.bank_to_device(bank), _dev(np.zeros(m)), _dev(np.zeros(n, np.int8))
+        if score:
+            sc = _dev(np.zeros(n))
+            st = ctx.forward_cells(db, _dev(sa), _dev(si), dw, 0, m, dx, min_w,
+                                   g=_dev(np.linspace(-1, 1, m)), history_score=sc, result=dr,
+                                   options=opt)
+            assert np.array_equal(sc.cpu().numpy(), o["score"])
+            assert np.array_equal(dw.cpu().numpy(), o["tally_exact"])
+            continue
+        sigs, ar = sa + si, sa / (sa + si)
+        q = oracle.simulate_bank(64, 0, m, dx, min_w, sigs, ar, bank, nthread=8)
+        ev, col = _dev(np.zeros(n, np.int64)), _dev(np.zeros(n, np.int64))
+        st, _ = ctx.simulate_device(db, _dev(sigs), _dev(ar), dw, 0, m, dx, min_w, result=dr,
+                                    events=ev, collisions=col, options=opt,
+                                    allow=(mcgpu.ERR_EVENT_CAP,))
+        same = q["events"] <= cap if cap else np.ones(n, bool)
+        b, r = mcgpu.bank_from_device(db), dr.cpu().numpy().astype(np.int32)
+        assert np.all(r[~same] == 2) and np.array_equal(r[same], q["result"][same])
+        for f in ("seed", "x", "mu", "wmc", "index"):
+            assert np.array_equal(b[f][same], q["bank"][f][same], equal_nan=f == "x"), f
+        assert np.array_equal(ev.cpu().numpy()[same], q["events"][same].astype(np.int64))
+        assert st["events"] == int(ev.sum()) and st["collisions"] == int(col.sum())
+        if cap == 0:
+            assert np.array_equal(dw.cpu().numpy(), q["tally_exact"])
+
+
 def test_a_thick_layer_is_as_fast_as_a_thick_slab(ctx):
     """One history of some 2,300 collisions, by itself and as a batch of one slab:
     with the common step before every general event a layer takes half as long
