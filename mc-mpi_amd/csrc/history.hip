@@ -439,9 +439,14 @@ template <bool OPEN> __global__ void k_windows_count(mc_transport_args a, mc_win
     }
     if (w >= 0) atomicAdd(&s_n[w / win.W], 1u);
   }
-  if (OPEN && win.thick)
-    mc_count_thick(win.thick, a.cells, a.L.m, a.L.dx, blockIdx.x * blockDim.x + threadIdx.x,
-                   gridDim.x * blockDim.x);
+  if (OPEN && win.thick) {
+    uint32_t thick = 0;
+    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < a.L.m;
+         c += (int64_t)gridDim.x * blockDim.x)
+      thick += mc_thick(a.cells[c], a.L.dx) ? 1u : 0u;
+    thick = mc_wave_sum_u32(thick);
+    if (__lane_id() == 0 && thick != 0) atomicAdd(win.thick, thick);
+  }
   __syncthreads();
   if (threadIdx.x < (unsigned)win.nw && s_n[threadIdx.x]) {
     atomicAdd(&win.count[threadIdx.x], s_n[threadIdx.x]);

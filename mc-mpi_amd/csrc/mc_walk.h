@@ -766,25 +766,22 @@ struct mc_scale {
 /* by one thread, before a barrier */
 __device__ __forceinline__ void mc_scale_clear(mc_scale *s) { *s = {-1023, -1023, -1023, -1023}; }
 
-/* Adds to *count (cleared before) the cells with sig_i dx or sig_a dx above 1/2,
-   by whole waves: thread `first` of `step`, or all threads of a block.
+__device__ __forceinline__ bool mc_thick(const mc_cell k, double dx) {
+  return (k.sig_i > k.sig_a ? k.sig_i : k.sig_a) * dx > 0.5;
+}
+
+/* Adds to *count (LDS, cleared before a barrier) the cells with sig_i dx or sig_a
+   dx above 1/2, by all threads of a block.
    mc_walk_thick serves where they are more than half: at the mean cosine of 1/2
    two events in three collide there.  Batches of thick slabs without it and
    with, in ms: 300 slabs of 32 cells 1.24 and 0.90, 200 smaller ones 0.395 and
    0.298. */
 __device__ __forceinline__ void mc_count_thick(uint32_t *count, const mc_cell *cells, int m,
-                                               double dx, unsigned first, unsigned step) {
+                                               double dx) {
   uint32_t n = 0;
-  for (int64_t c = first; c < m; c += step) {
-    const mc_cell k = cells[c];
-    n += (k.sig_i > k.sig_a ? k.sig_i : k.sig_a) * dx > 0.5 ? 1u : 0u;
-  }
+  for (int c = threadIdx.x; c < m; c += blockDim.x) n += mc_thick(cells[c], dx) ? 1u : 0u;
   n = mc_wave_sum_u32(n);
   if (__lane_id() == 0 && n != 0) atomicAdd(count, n);
-}
-__device__ __forceinline__ void mc_count_thick(uint32_t *count, const mc_cell *cells, int m,
-                                               double dx) {
-  mc_count_thick(count, cells, m, dx, threadIdx.x, blockDim.x);
 }
 
 /* the weights of histories first .. end - 1, as one history per thread of
